@@ -349,7 +349,18 @@ static void long_rows_epi(const DeviceBsr<S> &a, const V *x, V *y, const V *b, i
 }
 
 template <int RB, int CB, typename S, typename V>
+static void wide_rows_epi(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
+    const dim3 grid(a.rows), block(WideRows<RB, CB, V>::THREADS);
+    if (epi == EPI_STORE) hipLaunchKernelGGL((wide_rows_kernel<RB, CB, S, V, EPI_STORE>), grid, block, 0, s, a.view(), x, y, b, st);
+    else if (epi == EPI_RESIDUAL) hipLaunchKernelGGL((wide_rows_kernel<RB, CB, S, V, EPI_RESIDUAL>), grid, block, 0, s, a.view(), x, y, b, st);
+    else hipLaunchKernelGGL((wide_rows_kernel<RB, CB, S, V, EPI_ADD>), grid, block, 0, s, a.view(), x, y, b, st);
+}
+
+template <int RB, int CB, typename S, typename V>
 static void long_rows_shape(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st, int rpw) {
+    if constexpr (RB == 6) {  // the restrictions and the coarse levels
+        if (rpw == WIDE_ROWS) return wide_rows_epi<RB, CB>(a, x, y, b, epi, s, st);
+    }
     if (rpw == 4) long_rows_epi<RB, CB, S, V, 4>(a, x, y, b, epi, s, st);
     else if (rpw == 2) long_rows_epi<RB, CB, S, V, 2>(a, x, y, b, epi, s, st);
     else long_rows_epi<RB, CB, S, V, 1>(a, x, y, b, epi, s, st);
@@ -483,20 +494,23 @@ template void tune_spmv<double, double>(DeviceSliced<double> &, int, hipStream_t
 
 namespace {
 
-// coarse_inverse_small_kernel for n <= COARSE_SMALL rows. Its LDS limit is raised once per
-// process, when a hierarchy forms its inverse (so never under a stream capture).
+// The coarsest solve's LDS limit is raised when a hierarchy with a factor is built (so never under
+// a stream capture).
 template <typename V>
-void raise_coarse_small() {
+void raise_coarse_solve() {
     static const bool raised = [] {
-        const int most = (int)coarse_small_lds(COARSE_SMALL);
-        SF_HIP(hipFuncSetAttribute((const void *)coarse_inverse_small_kernel<V>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
+        size_t most = 0;
+        for (uint32_t n = 1; n <= COARSE_MAX; ++n) most = std::max(most, coarse_solve_lds(n));
+        SF_HIP(hipFuncSetAttribute((const void *)coarse_solve_kernel<V>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
         return true;
     }();
     (void)raised;
 }
 template <typename V>
-void launch_coarse_small(uint32_t n, const double *inv, const V *b, V *x, hipStream_t s) {
-    hipLaunchKernelGGL(coarse_inverse_small_kernel<V>, dim3(1), dim3(COARSE_SMALL_THREADS), coarse_small_lds(n), s, n, inv, b, x);
+void launch_coarse_solve(size_t n, const double *packed, const V *b, V *x, uint32_t columns, hipStream_t s) {
+    if (n == 0) return;
+    hipLaunchKernelGGL(coarse_solve_kernel<V>, dim3(columns), dim3(COARSE_THREADS), coarse_solve_lds((uint32_t)n), s, (uint32_t)n, packed, b, x,
+                       columns);
 }
 
 // Chebyshev scalars computed in f64 as the reference's cycle does (cycle.rs:578-650,
@@ -524,10 +538,8 @@ struct LevelDev {
     DeviceBsr<S> a_rows;          // coarse levels: A in plain block rows, for the row kernels
     int cheb_rows = 0, residual_rows = 0;  // the same choice for the steps and residuals (by timing)
     DeviceBuffer<S> dinv;
-    DeviceBuffer<double> lt;      // coarsest: transposed Cholesky factor
-    DeviceBuffer<double> packed;  // coarsest: the factor packed by columns, for the LDS solve
+    DeviceBuffer<double> packed;  // coarsest: the Cholesky factor packed by columns (SF_COARSE_REFERENCE's solve)
     DeviceBuffer<double> inverse; // coarsest: the f64 inverse, by columns (SF_COARSE_INVERSE)
-    size_t lds_bytes = 0;         // nonzero when the LDS solve is used
     bool has_p = false, has_factor = false;
     double theta = 0;
     std::vector<std::pair<double, double>> steps;
@@ -640,47 +652,37 @@ class Hierarchy final : public DeviceMultigrid {
                 d.has_factor = true;
                 const size_t n = d.n;
                 if (n > COARSE_MAX) throw Error(SF_ERR_INTERNAL, "coarse factor larger than the device solve");
-                std::vector<double> lt(n * n, 0.0);
-                for (size_t i = 0; i < n; ++i)
-                    for (size_t k = 0; k <= i; ++k) lt[k * n + i] = h.factor[i * n + k];
-                d.lt.upload(lt, s);
                 if (coarse_mode == SF_COARSE_INVERSE) {
                     // inverse = L^-T L^-1 in f64 on the device (symmetric by construction): the
                     // columns of L^-1, then every entry, each in a fixed order
-                    DeviceBuffer<double> linv;
+                    std::vector<double> by_columns(n * n, 0.0);
+                    for (size_t i = 0; i < n; ++i)
+                        for (size_t k = 0; k <= i; ++k) by_columns[k * n + i] = h.factor[i * n + k];
+                    DeviceBuffer<double> lt, linv;
+                    lt.upload(by_columns, s);
                     std::vector<double> identity(n * n, 0.0);
                     for (size_t i = 0; i < n; ++i) identity[i * n + i] = 1.0;
                     linv.upload(identity, s);
                     d.inverse.resize(n * n);
                     for (size_t k = 0; k < n; ++k) {
                         hipLaunchKernelGGL(factor_inverse_finish_row_kernel, dim3(grid_for(k + 1, 256)), dim3(256), 0, s, (uint32_t)n,
-                                           (uint32_t)k, (const double *)d.lt.ptr, linv.ptr);
+                                           (uint32_t)k, (const double *)lt.ptr, linv.ptr);
                         if (k + 1 < n)
                             hipLaunchKernelGGL(factor_inverse_update_kernel, dim3(grid_for(k + 1, 256), (unsigned)(n - k - 1)), dim3(256), 0,
-                                               s, (uint32_t)n, (uint32_t)k, (const double *)d.lt.ptr, linv.ptr);
+                                               s, (uint32_t)n, (uint32_t)k, (const double *)lt.ptr, linv.ptr);
                     }
                     hipLaunchKernelGGL(factor_inverse_entries_kernel, dim3(grid_for(n * n, 256)), dim3(256), 0, s, (uint32_t)n,
                                        (const double *)linv.ptr, d.inverse.ptr);
-                    if (n <= COARSE_SMALL) raise_coarse_small<V>();
                     SF_HIP(hipGetLastError());
-                    SF_HIP(hipStreamSynchronize(s));  // linv is freed on return
+                    SF_HIP(hipStreamSynchronize(s));  // lt and linv are freed on return
                 }
-                const size_t need = (n * (n + 1) / 2 + 2 * n) * sizeof(double);
-                int dev = 0, limit = 0;
-                SF_HIP(hipGetDevice(&dev));
-                SF_HIP(hipDeviceGetAttribute(&limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-                if (need <= (size_t)limit) {
-                    std::vector<double> packed;
-                    packed.reserve(n * (n + 1) / 2);
-                    for (size_t k = 0; k < n; ++k)
-                        for (size_t i = k; i < n; ++i) packed.push_back(h.factor[i * n + k]);
-                    d.packed.upload(packed, s);
-                    d.lds_bytes = need;
-                    if (need > 65536) {
-                        SF_HIP(hipFuncSetAttribute((const void *)coarse_solve_lds_kernel<V>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
-                        SF_HIP(hipFuncSetAttribute((const void *)coarse_solve_lds_kernel<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
-                    }
-                }
+                std::vector<double> packed;
+                packed.reserve(n * (n + 1) / 2);
+                for (size_t k = 0; k < n; ++k)
+                    for (size_t i = k; i < n; ++i) packed.push_back(h.factor[i * n + k]);
+                d.packed.upload(packed, s);
+                raise_coarse_solve<V>();
+                raise_coarse_solve<double>();
             }
             for (auto *buf : {&d.b, &d.x, &d.d0, &d.d1, &d.r0, &d.r1, &d.res, &d.px}) buf->resize(d.n);
             SF_HIP(hipStreamSynchronize(s));
@@ -815,10 +817,7 @@ class Hierarchy final : public DeviceMultigrid {
     void coarse_solve(const double *b, double *x, hipStream_t s) override {
         LevelDev<S, V> &d = lv_.back();
         if (!d.has_factor) throw Error(SF_ERR_MG_COARSEST_NOT_FACTORED, "the coarsest level has no direct factorization", (int64_t)d.n);
-        if (d.lds_bytes)
-            hipLaunchKernelGGL(coarse_solve_lds_kernel<double>, dim3(1), dim3(WAVE), d.lds_bytes, s, (uint32_t)d.n, d.packed.ptr, b, x, 1u);
-        else
-            hipLaunchKernelGGL(coarse_solve_kernel<double>, dim3(1), dim3(WAVE), 0, s, (uint32_t)d.n, d.lt.ptr, b, x, 1u);
+        launch_coarse_solve<double>(d.n, d.packed.ptr, b, x, 1u, s);
         SF_HIP(hipGetLastError());
     }
 
@@ -977,10 +976,8 @@ class Hierarchy final : public DeviceMultigrid {
                 if (d.inverse.ptr)
                     hipLaunchKernelGGL(coarse_inverse_batch_kernel<V>, dim3(grid_for(d.n, coarse_rows(M))), dim3(256), 0, s, (uint32_t)d.n, M,
                                        coarse_rows(M), d.inverse.ptr, b, x);
-                else if (d.lds_bytes)
-                    hipLaunchKernelGGL(coarse_solve_lds_kernel<V>, dim3(M), dim3(WAVE), d.lds_bytes, s, (uint32_t)d.n, d.packed.ptr, b, x, M);
                 else
-                    hipLaunchKernelGGL(coarse_solve_kernel<V>, dim3(M), dim3(WAVE), 0, s, (uint32_t)d.n, d.lt.ptr, b, x, M);
+                    launch_coarse_solve<V>(d.n, d.packed.ptr, b, x, M, s);
             } else {
                 smooth_batch(d, b, x, nullptr, M, s);
             }
@@ -1046,11 +1043,12 @@ class Hierarchy final : public DeviceMultigrid {
                 SF_HIP(hipMemsetAsync(c.x.ptr, 0, c.n * sizeof(V), s));
                 d.r.batch_spmv = tune_batch(s, [&](int batch) { launch_spmv<S, V>(d.r, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s, batch); },
                                             {1, 2, 4, 8}, at + "restriction depth", "restriction " + shape_class(d.r) + vs_);
-                // the sliced product at its best depth (0) against 1, 2 or 4 rows per wavefront
-                d.restrict_rows = fastest(s, [&](int rpw) {
+                // the sliced product at its best depth (0) against 1, 2 or 4 rows per wavefront and
+                // four wavefronts per row
+                d.restrict_rows = forced_variant().load(std::memory_order_relaxed) == WIDE_ROWS ? WIDE_ROWS : fastest(s, [&](int rpw) {
                     if (!rpw) launch_spmv<S, V>(d.r, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s);
                     else launch_long_rows<S, V>(d.r_rows, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s, {nullptr, (V)0, nullptr, nullptr}, rpw);
-                }, {0, 1, 2, 4}, at + "restriction rows per wave", "restriction rows " + shape_class(d.r) + vs_);
+                }, {0, 1, 2, 4, WIDE_ROWS}, at + "restriction rows per wave", "restriction rows " + shape_class(d.r) + vs_);
                 d.p.batch_spmv = tune_batch(s, [&](int batch) { launch_spmv<S, V>(d.p, c.x.ptr, d.px.ptr, nullptr, EPI_ADD, s, batch); },
                                             {1, 2, 4, 8}, at + "prolongation depth", "prolongation " + shape_class(d.p) + vs_);
             }
@@ -1128,14 +1126,10 @@ class Hierarchy final : public DeviceMultigrid {
         LevelDev<S, V> &d = lv_[l];
         if (!d.has_p) {
             if (d.has_factor) {
-                if (d.inverse.ptr && d.n <= COARSE_SMALL)
-                    launch_coarse_small<V>((uint32_t)d.n, d.inverse.ptr, b, x, s);
-                else if (d.inverse.ptr)
-                    hipLaunchKernelGGL(coarse_inverse_kernel<V>, dim3(grid_for(d.n, 256)), dim3(256), 0, s, (uint32_t)d.n, d.inverse.ptr, b, x);
-                else if (d.lds_bytes)
-                    hipLaunchKernelGGL(coarse_solve_lds_kernel<V>, dim3(1), dim3(WAVE), d.lds_bytes, s, (uint32_t)d.n, d.packed.ptr, b, x, 1u);
+                if (d.inverse.ptr)
+                    hipLaunchKernelGGL(coarse_inverse_kernel<V>, dim3(grid_for(d.n, COARSE_ROWS)), dim3(256), 0, s, (uint32_t)d.n, d.inverse.ptr, b, x);
                 else
-                    hipLaunchKernelGGL(coarse_solve_kernel<V>, dim3(1), dim3(WAVE), 0, s, (uint32_t)d.n, d.lt.ptr, b, x, 1u);
+                    launch_coarse_solve<V>(d.n, d.packed.ptr, b, x, 1u, s);
             } else {
                 smooth(d, b, x, nullptr, s, false, started);
             }

@@ -83,7 +83,9 @@ void upload_bsr(DeviceBsr<T> &out, const HostBsr<double> &m, hipStream_t s);
 template <typename T>
 void build_bsr(DeviceBsr<T> &out, const HostBsr<double> &pattern, const double *values, hipStream_t s);
 // y = A x (epilogue per dev::Epilogue) with `rows_per_wave` block rows per wavefront
-// (long_rows_kernel: 1, 2 or 4).
+// (long_rows_kernel: 1, 2 or 4), or WIDE_ROWS: four wavefronts per block row (wide_rows_kernel).
+// sf_force_variant(WIDE_ROWS) forces the latter on every restriction.
+constexpr int WIDE_ROWS = 96;
 template <typename S, typename V>
 void launch_long_rows(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s,
                       dev::Start<S, V> start = {nullptr, (V)0, nullptr, nullptr}, int rows_per_wave = 1);

@@ -226,18 +226,44 @@ __device__ __forceinline__ uint32_t longest_of_wave(uint32_t len) {
     return len;
 }
 
-// Adds `n` terms in order onto `sum`, eight loads ahead.
-template <typename V>
+// `n` terms from `t` (LDS, 16-byte aligned) added in order onto `sum`. READS 16-byte reads are one
+// group; two groups alternate, the next one's reads issued before this one's additions (the barrier
+// keeps the compiler from moving them back), so the chain of additions never waits on LDS. The last
+// group is read whole -- `t` has room up to a multiple of a group -- and what lies past `n` is
+// replaced by -0.0, which added to any value leaves it as it is.
+template <int READS, typename V>
 __device__ __forceinline__ V add_terms(V sum, const V *t, uint32_t n) {
-    uint32_t i = 0;
-    for (; i + 8 <= n; i += 8) {
-        V v[8];
+    typedef V Quad __attribute__((ext_vector_type(16 / sizeof(V))));
+    constexpr uint32_t W = 16 / sizeof(V), GROUP = W * READS;
+    const uint32_t groups = (n + GROUP - 1) / GROUP;
+    if (groups == 0) return sum;
+    auto read = [&](Quad(&q)[READS], uint32_t g) {
+        const Quad *p = reinterpret_cast<const Quad *>(t) + (g < groups ? g : groups - 1) * READS;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = t[i + u];
+        for (int u = 0; u < READS; ++u) q[u] = p[u];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](const Quad(&q)[READS], uint32_t g) {
+        if ((g + 1) * GROUP <= n) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) sum = sum + v[u];
+            for (int u = 0; u < READS; ++u)
+#pragma unroll
+                for (uint32_t v = 0; v < W; ++v) sum = sum + q[u][v];
+        } else if (g < groups) {
+#pragma unroll
+            for (int u = 0; u < READS; ++u)
+#pragma unroll
+                for (uint32_t v = 0; v < W; ++v) sum = sum + (g * GROUP + u * W + v < n ? q[u][v] : (V)-0.0);
+        }
+    };
+    Quad a[READS], b[READS];
+    read(a, 0);
+    for (uint32_t g = 0; g < groups; g += 2) {
+        read(b, g + 1);
+        add(a, g);
+        read(a, g + 2);
+        add(b, g + 1);
     }
-    for (; i < n; ++i) sum = sum + t[i];
     return sum;
 }
 
@@ -252,7 +278,7 @@ template <int RB, int CB, typename S, typename V, int EPI, int RPW>
 __global__ __launch_bounds__(64) void long_rows_kernel(Bsr<S> a, const V *__restrict__ x, V *__restrict__ y,
                                                        const V *__restrict__ b, Start<S, V> then) {
     constexpr int LW = WAVE / RPW;
-    __shared__ V terms[RPW][RB][LW * CB];
+    __shared__ __align__(16) V terms[RPW][RB][LW * CB + 16 / sizeof(V)];  // rows on different banks
     __shared__ V values[RPW][RB];
     const int lane = threadIdx.x, g = lane / LW, sl = lane % LW;
     const uint32_t row = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW + (uint32_t)g;
@@ -274,7 +300,7 @@ __global__ __launch_bounds__(64) void long_rows_kernel(Bsr<S> a, const V *__rest
                 for (int q = 0; q < CB; ++q) terms[g][p][sl * CB + q] = widen<V>(blk[p * CB + q]) * xv[q];
         }
         __syncthreads();
-        if (sl < RB && k0 < len) sum = add_terms(sum, terms[g][sl], (len - k0 < (uint32_t)LW ? len - k0 : (uint32_t)LW) * CB);
+        if (sl < RB && k0 < len) sum = add_terms<4>(sum, (const V *)terms[g][sl], (len - k0 < (uint32_t)LW ? len - k0 : (uint32_t)LW) * CB);
         __syncthreads();
     }
     const bool owner = live && sl < RB;
@@ -301,6 +327,90 @@ __global__ __launch_bounds__(64) void long_rows_kernel(Bsr<S> a, const V *__rest
     }
 }
 
+// long_rows_kernel with one workgroup of four wavefronts per block row, for matrices whose rows
+// are so long (hundreds of blocks) and so few that one wavefront per row leaves the chip idle
+// through a chain of round trips. All four wavefronts load CHUNK blocks' values and x entries at
+// once and put their terms into one of two LDS buffers; then lane p of the first wavefront adds row
+// p's terms in stored order while the next chunk's loads are in flight (its block columns were
+// fetched a chunk before that). Bound by the ordered chain of additions: about 4 us for 350
+// blocks, where one wavefront's chunks of 64 took 21 us.
+template <int RB, int CB, typename V>
+struct WideRows {
+    static constexpr int THREADS = 256;
+    // a block is shared by PARTS threads, RB / PARTS rows each, so that both LDS buffers stay under 40 KB
+    static constexpr int PARTS = CB * sizeof(V) <= 12 ? 1 : CB * sizeof(V) <= 24 ? 2 : 3;
+    static constexpr int CHUNK = PARTS == 1 ? 256 : PARTS == 2 ? 128 : 64;
+    static constexpr int STRIDE = CHUNK * CB + 16 / sizeof(V);  // rows on different banks, 16-byte aligned
+    static_assert(RB % PARTS == 0 && CHUNK * PARTS <= THREADS, "whole rows per thread");
+};
+template <int RB, int CB, typename S, typename V, int EPI>
+__global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__restrict__ x, V *__restrict__ y, const V *__restrict__ b,
+                                                        Start<S, V> then) {
+    using W = WideRows<RB, CB, V>;
+    constexpr int RP = RB / W::PARTS;
+    __shared__ __align__(16) V terms[2][RB][W::STRIDE];
+    __shared__ V values[RB];
+    const uint32_t row = a.reverse ? xcd_reversed_block() : blockIdx.x;  // one workgroup per row: row < a.rows
+    const uint32_t start = a.starts[row], len = a.starts[row + 1] - start;
+    const uint32_t t = threadIdx.x, k = t / W::PARTS, p0 = (t % W::PARTS) * RP;
+    const bool loads = k < (uint32_t)W::CHUNK;
+    S v[RP * CB];
+    V xv[CB];
+    auto fetch = [&](uint32_t at, uint32_t col) {
+        if (loads && at < len) {
+            const S *blk = a.vals + ((size_t)(start + at) * RB + p0) * CB;
+#pragma unroll
+            for (int e = 0; e < RP * CB; ++e) v[e] = blk[e];
+#pragma unroll
+            for (int q = 0; q < CB; ++q) xv[q] = x[(size_t)col * CB + q];
+        }
+    };
+    uint32_t col = loads && k < len ? a.cols[start + k] : 0u;
+    fetch(k, col);
+    col = loads && k + W::CHUNK < len ? a.cols[start + k + W::CHUNK] : 0u;
+    V sum = (V)0;
+    int buf = 0;
+    for (uint32_t k0 = 0; k0 < len; k0 += W::CHUNK, buf ^= 1) {
+        if (loads && k0 + k < len) {
+#pragma unroll
+            for (int p = 0; p < RP; ++p)
+#pragma unroll
+                for (int q = 0; q < CB; ++q) terms[buf][p0 + p][k * CB + q] = widen<V>(v[p * CB + q]) * xv[q];
+        }
+        const uint32_t k1 = k0 + W::CHUNK, k2 = k1 + W::CHUNK;
+        if (k1 < len) {
+            fetch(k1 + k, col);
+            if (loads && k2 + k < len) col = a.cols[start + k2 + k];
+        }
+        // one barrier per chunk: this buffer is written again two chunks on, after the next barrier,
+        // which the adding wavefront reaches only once it has read it
+        __syncthreads();
+        if (t < (uint32_t)RB) sum = add_terms<8>(sum, (const V *)terms[buf][t], (len - k0 < (uint32_t)W::CHUNK ? len - k0 : (uint32_t)W::CHUNK) * CB);
+    }
+    const bool owner = t < (uint32_t)RB;
+    const size_t out = (size_t)row * RB + (owner ? t : 0);
+    if (owner) {
+        V value;
+        if (EPI == EPI_STORE) value = sum;
+        else if (EPI == EPI_RESIDUAL) value = b[out] - sum;
+        else value = y[out] + sum;
+        y[out] = value;
+        values[t] = value;
+    }
+    if (then.dinv) {  // uniform
+        __syncthreads();
+        if (owner) {
+            const S *drow = then.dinv + (size_t)row * RB * RB + (size_t)t * RB;
+            V z = (V)0;
+#pragma unroll
+            for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * values[q];
+            const V dv = z / then.theta;
+            then.d[out] = dv;
+            then.x[out] = dv;
+        }
+    }
+}
+
 // The fused Chebyshev step of cheb_step_kernel for levels with few rows, RPW block rows per
 // wavefront (one workgroup) as long_rows_kernel: the lanes form the terms of A d_in, lane p of a
 // row's group adds the row's terms in stored order, and the RB residuals of the block row meet in
@@ -312,7 +422,7 @@ __global__ __launch_bounds__(64) void cheb_rows_kernel(Bsr<S> a, const S *__rest
                                                        V *__restrict__ r_out, V *__restrict__ x, V *__restrict__ sum_into,
                                                        double *__restrict__ widen_into) {
     constexpr int LW = WAVE / RPW;
-    __shared__ V terms[RPW][RB][LW * RB];
+    __shared__ __align__(16) V terms[RPW][RB][LW * RB + 16 / sizeof(V)];  // rows on different banks
     __shared__ V r_new[RPW][RB];
     const int lane = threadIdx.x, g = lane / LW, sl = lane % LW;
     const uint32_t row = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW + (uint32_t)g;
@@ -334,7 +444,7 @@ __global__ __launch_bounds__(64) void cheb_rows_kernel(Bsr<S> a, const S *__rest
                 for (int q = 0; q < RB; ++q) terms[g][p][sl * RB + q] = widen<V>(blk[p * RB + q]) * xv[q];
         }
         __syncthreads();
-        if (sl < RB && k0 < len) sum = add_terms(sum, terms[g][sl], (len - k0 < (uint32_t)LW ? len - k0 : (uint32_t)LW) * RB);
+        if (sl < RB && k0 < len) sum = add_terms<4>(sum, (const V *)terms[g][sl], (len - k0 < (uint32_t)LW ? len - k0 : (uint32_t)LW) * RB);
         __syncthreads();
     }
     const bool owner = live && sl < RB;
@@ -483,91 +593,99 @@ __global__ void convert_kernel(size_t n, const From *__restrict__ in, To *__rest
 }
 
 // The coarsest level's direct solve with the f64 Cholesky factor (block.rs:357-373), the
-// right-hand side widened from V and the solution rounded to V (cycle.rs:475-486). One
-// wavefront; `lt` is the factor transposed (column k of the factor contiguous) and the running
-// sums live in LDS. Forward substitution runs right-looking: once x_k is final every later row
-// subtracts its term, so each row still subtracts in ascending k, the reference's order. Back
-// substitution also subtracts each row's terms in ascending k, which can only start once every
-// later x is known: the lanes form the products, then one lane folds them in order.
+// right-hand side widened from V and the solution rounded to V (cycle.rs:475-486). `packed` is the
+// factor by columns (column k holds rows k..n-1 at offset k n - k (k - 1) / 2). Forward substitution
+// runs right-looking: once x_k is final every later row subtracts its term, so each row still
+// subtracts in ascending k, the reference's order. Back substitution also subtracts each row's terms
+// in ascending k, which can only start once every later x is known: the lanes form the negated
+// products, then every lane folds them in order (broadcast reads), so the row's value needs no
+// exchange before its division.
+//
+// The first wavefront solves, alone and with no barrier inside a panel; the other three bring the
+// next panel of `width` columns into the other LDS buffer meanwhile, so no step waits on global
+// memory. A factor that fits one buffer is one panel, read once for both substitutions. Bound by
+// the n^2 / 2 dependent subtractions of the back substitution and 2 n dependent divisions.
 constexpr uint32_t COARSE_MAX = 3072;
+constexpr uint32_t COARSE_THREADS = 256;
+constexpr uint32_t COARSE_PANEL = 6144;  // entries of one of the two panel buffers
+__host__ __device__ constexpr size_t packed_column(uint32_t n, uint32_t k) { return (size_t)k * n - ((size_t)k * (k - 1)) / 2; }
+// Columns per panel and LDS bytes: the whole factor where it fits two buffers' room, else two panels.
+__host__ __device__ constexpr uint32_t coarse_panel_width(uint32_t n) {
+    return packed_column(n, n) <= 2 * COARSE_PANEL ? n : COARSE_PANEL / n;
+}
+constexpr size_t coarse_solve_lds(uint32_t n) {
+    return ((coarse_panel_width(n) == n ? packed_column(n, n) + packed_column(n, n) % 2 : 2 * COARSE_PANEL) + (size_t)n + n % 2 + (n + 15) / 16 * 16) * sizeof(double);
+}
+// Orders this wavefront's LDS accesses before and after this point (LDS serves a wavefront's
+// accesses in order, so only the compiler has to be kept from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 // Several right-hand sides (row-interleaved, `stride` columns) take one workgroup each.
 template <typename V>
-__global__ __launch_bounds__(64) void coarse_solve_kernel(uint32_t n, const double *__restrict__ lt,
-                                                           const V *__restrict__ rhs, V *__restrict__ out, uint32_t stride) {
-    __shared__ double xs[COARSE_MAX];
-    __shared__ double prod[COARSE_MAX];
+__global__ __launch_bounds__(COARSE_THREADS) void coarse_solve_kernel(uint32_t n, const double *__restrict__ packed,
+                                                                      const V *__restrict__ rhs, V *__restrict__ out, uint32_t stride) {
+    extern __shared__ __align__(16) double smem[];
+    const uint32_t width = coarse_panel_width(n), panels = (n + width - 1) / width;
+    const size_t whole = packed_column(n, n);
+    double *xs = smem + (panels == 1 ? whole + whole % 2 : 2 * (size_t)COARSE_PANEL), *prod = xs + n + n % 2;
     const uint32_t t = threadIdx.x;
     rhs += blockIdx.x;
     out += blockIdx.x;
-    for (uint32_t i = t; i < n; i += WAVE) xs[i] = (double)rhs[(size_t)i * stride];
-    __syncthreads();
-    for (uint32_t k = 0; k < n; ++k) {
-        if (t == k % WAVE) xs[k] = xs[k] / lt[(size_t)k * n + k];
-        __syncthreads();
-        const double xv = xs[k];
-        const double *col = lt + (size_t)k * n;
-        for (uint32_t i = k + 1 + t; i < n; i += WAVE) xs[i] = xs[i] - col[i] * xv;
-        __syncthreads();
-    }
-    for (uint32_t ii = n; ii-- > 0;) {
-        const double *col = lt + (size_t)ii * n;
-        for (uint32_t k = ii + 1 + t; k < n; k += WAVE) prod[k] = col[k] * xs[k];
-        __syncthreads();
-        if (t == 0) {
-            double sum = xs[ii];
-            for (uint32_t k = ii + 1; k < n; ++k) sum = sum - prod[k];
-            xs[ii] = sum / col[ii];
+    // panel p into its buffer, by the threads from `first` on
+    auto bring = [&](uint32_t p, uint32_t first) {
+        const uint32_t k0 = p * width, k1 = k0 + width < n ? k0 + width : n;
+        const size_t at = packed_column(n, k0), entries = packed_column(n, k1) - at;
+        double *to = smem + (size_t)(p & 1u) * COARSE_PANEL;
+        const uint32_t step = COARSE_THREADS - first;
+        for (size_t e = t - first; e < entries; e += 8 * (size_t)step) {
+            double v[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) v[u] = e + u * step < entries ? packed[at + e + u * step] : 0.0;
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u)
+                if (e + u * step < entries) to[e + u * step] = v[u];
         }
-        __syncthreads();
-    }
-    for (uint32_t i = t; i < n; i += WAVE) out[(size_t)i * stride] = (V)xs[i];
-}
-
-// The same solve with the factor held in LDS, packed by columns (column k holds rows k..n-1 at
-// offset k n - k (k - 1) / 2), so no step of either substitution waits on global memory. Used
-// when the packed factor and two vectors fit in one workgroup's LDS.
-__device__ __forceinline__ size_t packed_column(uint32_t n, uint32_t k) { return (size_t)k * n - ((size_t)k * (k - 1)) / 2; }
-
-template <typename V>
-__global__ __launch_bounds__(64) void coarse_solve_lds_kernel(uint32_t n, const double *__restrict__ packed,
-                                                               const V *__restrict__ rhs, V *__restrict__ out, uint32_t stride) {
-    extern __shared__ double smem[];
-    const size_t np = (size_t)n * (n + 1) / 2;
-    double *l = smem, *xs = smem + np, *prod = xs + n;
-    const uint32_t t = threadIdx.x;
-    rhs += blockIdx.x;
-    out += blockIdx.x;
-    for (size_t i = t; i < np; i += WAVE) l[i] = packed[i];
-    for (uint32_t i = t; i < n; i += WAVE) xs[i] = (double)rhs[(size_t)i * stride];
+    };
+    bring(0, 0);
+    for (uint32_t i = t; i < n; i += COARSE_THREADS) xs[i] = (double)rhs[(size_t)i * stride];
     __syncthreads();
-    for (uint32_t k = 0; k < n; ++k) {
-        const double *col = l + packed_column(n, k) - k;  // col[i] = L[i][k]
-        if (t == k % WAVE) xs[k] = xs[k] / col[k];
-        __syncthreads();
-        const double xv = xs[k];
-        for (uint32_t i = k + 1 + t; i < n; i += WAVE) xs[i] = xs[i] - col[i] * xv;
-        __syncthreads();
-    }
-    for (uint32_t ii = n; ii-- > 0;) {
-        const double *col = l + packed_column(n, ii) - ii;
-        for (uint32_t k = ii + 1 + t; k < n; k += WAVE) prod[k] = col[k] * xs[k];
-        __syncthreads();
-        if (t == 0) {
-            double sum = xs[ii];
-            uint32_t k = ii + 1;
-            for (; k + 8 <= n; k += 8) {
-                double p[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) p[u] = prod[k + u];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) sum = sum - p[u];
+    for (uint32_t p = 0; p < panels; ++p) {
+        const uint32_t k0 = p * width, k1 = k0 + width < n ? k0 + width : n;
+        if (t >= WAVE) {
+            if (p + 1 < panels) bring(p + 1, WAVE);
+        } else {
+            const double *col = smem + (size_t)(p & 1u) * COARSE_PANEL;  // col[i - k] = L[i][k]
+            for (uint32_t k = k0; k < k1; col += n - k, ++k) {
+                const double xv = xs[k] / col[0];  // every lane the same quotient
+                wave_lds_fence();
+                if (t == 0) xs[k] = xv;
+                for (uint32_t i = k + 1 + t; i < n; i += WAVE) xs[i] = xs[i] - col[i - k] * xv;
+                wave_lds_fence();
             }
-            for (; k < n; ++k) sum = sum - prod[k];
-            xs[ii] = sum / col[ii];
         }
         __syncthreads();
     }
-    for (uint32_t i = t; i < n; i += WAVE) out[(size_t)i * stride] = (V)xs[i];
+    for (uint32_t p = panels; p-- > 0;) {
+        const uint32_t k0 = p * width, k1 = k0 + width < n ? k0 + width : n;
+        if (t >= WAVE) {
+            if (p > 0) bring(p - 1, WAVE);
+        } else {
+            const double *col = smem + (size_t)(p & 1u) * COARSE_PANEL + (packed_column(n, k1) - packed_column(n, k0));
+            for (uint32_t ii = k1; ii-- > k0;) {
+                col -= n - ii;
+                for (uint32_t k = ii + 1 + t; k < n; k += WAVE) prod[k - ii - 1] = -(col[k - ii] * xs[k]);
+                wave_lds_fence();
+                const double xv = add_terms<8>(xs[ii], (const double *)prod, n - 1 - ii) / col[0];
+                wave_lds_fence();
+                if (t == 0) xs[ii] = xv;
+                wave_lds_fence();
+            }
+        }
+        __syncthreads();
+    }
+    for (uint32_t i = t; i < n; i += COARSE_THREADS) out[(size_t)i * stride] = (V)xs[i];
 }
 
 // The coarsest level's solve as a product with the f64 inverse (stored by columns: inv[k n + i]
@@ -613,70 +731,37 @@ static __global__ __launch_bounds__(256) void factor_inverse_entries_kernel(uint
     inv[(size_t)j * n + i] = v;
 }
 
+// out = inv b, R rows per workgroup. inv is symmetric bit for bit (entry (i, j) and entry (j, i) add
+// the same products in the same order), so a row's entries are read as its column's, contiguous. All
+// threads form a chunk of the rows' terms into LDS with every load in flight at once; then lane r of
+// the first wavefront adds row r's terms in ascending k from zero. Bound by that chain of n additions.
+constexpr uint32_t COARSE_ROWS = 4, COARSE_CHUNK = 1024;
 template <typename V>
-__global__ __launch_bounds__(256) void coarse_inverse_kernel(uint32_t n, const double *__restrict__ inv,
-                                                             const V *__restrict__ rhs, V *__restrict__ out) {
-    __shared__ double bs[256];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void coarse_inverse_kernel(uint32_t n, const double *__restrict__ inv, const V *__restrict__ rhs,
+                                                             V *__restrict__ out) {
+    __shared__ __align__(16) double terms[COARSE_ROWS][COARSE_CHUNK + 2];
+    const uint32_t t = threadIdx.x, i0 = blockIdx.x * COARSE_ROWS;
+    const uint32_t rows = n - i0 < COARSE_ROWS ? n - i0 : COARSE_ROWS;
     double sum = 0.0;
-    for (uint32_t k0 = 0; k0 < n; k0 += 256) {
-        if (k0 + threadIdx.x < n) bs[threadIdx.x] = (double)rhs[k0 + threadIdx.x];
-        __syncthreads();
-        const uint32_t kmax = n - k0 < 256u ? n - k0 : 256u;
-        if (i < n) {
-            // 32 loads in flight (the column is latency-bound), then their terms in ascending k
-            uint32_t kk = 0;
-            for (; kk + 32 <= kmax; kk += 32) {
-                double a[32];
+    for (uint32_t k0 = 0; k0 < n; k0 += COARSE_CHUNK) {
+        constexpr uint32_t PER = COARSE_CHUNK / 256;
+        double a[COARSE_ROWS][PER], bk[PER];
 #pragma unroll
-                for (int u = 0; u < 32; ++u) a[u] = inv[(size_t)(k0 + kk + u) * n + i];
+        for (uint32_t j = 0; j < PER; ++j) {
+            const uint32_t k = k0 + t + 256 * j;
+            bk[j] = k < n ? (double)rhs[k] : 0.0;
 #pragma unroll
-                for (int u = 0; u < 32; ++u) sum = sum + a[u] * bs[kk + u];
-            }
-            for (; kk + 8 <= kmax; kk += 8) {
-                double a[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) a[u] = inv[(size_t)(k0 + kk + u) * n + i];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) sum = sum + a[u] * bs[kk + u];
-            }
-            for (; kk < kmax; ++kk) sum = sum + inv[(size_t)(k0 + kk) * n + i] * bs[kk];
+            for (uint32_t r = 0; r < COARSE_ROWS; ++r) a[r][j] = k < n && r < rows ? inv[(size_t)(i0 + r) * n + k] : 0.0;
         }
+        if (k0) __syncthreads();  // the chunk before has been added
+#pragma unroll
+        for (uint32_t j = 0; j < PER; ++j)
+#pragma unroll
+            for (uint32_t r = 0; r < COARSE_ROWS; ++r) terms[r][t + 256 * j] = a[r][j] * bk[j];
         __syncthreads();
+        if (t < rows) sum = add_terms<8>(sum, (const double *)terms[t], n - k0 < COARSE_CHUNK ? n - k0 : COARSE_CHUNK);
     }
-    if (i < n) out[i] = (V)sum;
-}
-
-// The same product for a coarse level of at most COARSE_SMALL rows (the plate's has 102): one
-// workgroup brings the whole inverse (at most 128 KB) and the right-hand side into LDS with every
-// load in flight at once, then thread i adds its row's terms in ascending k from zero.
-constexpr uint32_t COARSE_SMALL = 128;
-constexpr uint32_t COARSE_SMALL_THREADS = 1024;
-constexpr size_t coarse_small_lds(uint32_t n) { return ((size_t)n * n + n) * sizeof(double); }
-template <typename V>
-__global__ __launch_bounds__(COARSE_SMALL_THREADS) void coarse_inverse_small_kernel(uint32_t n, const double *__restrict__ inv,
-                                                                                     const V *__restrict__ rhs, V *__restrict__ out) {
-    extern __shared__ double ls[];  // the n x n inverse, then the n right-hand-side entries
-    constexpr int PER = COARSE_SMALL * COARSE_SMALL / COARSE_SMALL_THREADS;
-    const uint32_t t = threadIdx.x, nn = n * n;
-    double a[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const uint32_t e = t + COARSE_SMALL_THREADS * j;
-        a[j] = e < nn ? inv[e] : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const uint32_t e = t + COARSE_SMALL_THREADS * j;
-        if (e < nn) ls[e] = a[j];
-    }
-    if (t < n) ls[nn + t] = (double)rhs[t];
-    __syncthreads();
-    if (t < n) {
-        double sum = 0.0;
-        for (uint32_t k = 0; k < n; ++k) sum = sum + ls[(size_t)k * n + t] * ls[nn + k];
-        out[t] = (V)sum;
-    }
+    if (t < rows) out[i0 + t] = (V)sum;
 }
 
 // ---- conjugate gradient vectors -------------------------------------------------------------
