@@ -339,13 +339,13 @@ template void build_bsr<float>(DeviceBsr<float> &, const HostBsr<double> &, cons
 template void upload_bsr<double>(DeviceBsr<double> &, const HostBsr<double> &, hipStream_t);
 template void upload_bsr<float>(DeviceBsr<float> &, const HostBsr<double> &, hipStream_t);
 
-template <int RB, int CB, typename S, typename V, int RPW>
+template <int RB, int CB, int RPW, int U, typename S, typename V>
 static void long_rows_epi(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
     const dim3 grid((a.rows + RPW - 1) / RPW), block(WAVE);
-    if (epi == EPI_STORE) hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_STORE, RPW>), grid, block, 0, s, a.view(), x, y, b, st);
+    if (epi == EPI_STORE) hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_STORE, RPW, U>), grid, block, 0, s, a.view(), x, y, b, st);
     else if (epi == EPI_RESIDUAL)
-        hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_RESIDUAL, RPW>), grid, block, 0, s, a.view(), x, y, b, st);
-    else hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_ADD, RPW>), grid, block, 0, s, a.view(), x, y, b, st);
+        hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_RESIDUAL, RPW, U>), grid, block, 0, s, a.view(), x, y, b, st);
+    else hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_ADD, RPW, U>), grid, block, 0, s, a.view(), x, y, b, st);
 }
 
 template <int RB, int CB, typename S, typename V>
@@ -361,9 +361,9 @@ static void long_rows_shape(const DeviceBsr<S> &a, const V *x, V *y, const V *b,
     if constexpr (RB == 6) {  // the restrictions and the coarse levels
         if (rpw == WIDE_ROWS) return wide_rows_epi<RB, CB>(a, x, y, b, epi, s, st);
     }
-    if (rpw == 4) long_rows_epi<RB, CB, S, V, 4>(a, x, y, b, epi, s, st);
-    else if (rpw == 2) long_rows_epi<RB, CB, S, V, 2>(a, x, y, b, epi, s, st);
-    else long_rows_epi<RB, CB, S, V, 1>(a, x, y, b, epi, s, st);
+    with_rows_form<RB * CB * (int)sizeof(V)>(rpw, [&](auto rows, auto blocks) {
+        long_rows_epi<RB, CB, decltype(rows)::value, decltype(blocks)::value>(a, x, y, b, epi, s, st);
+    });
 }
 
 template <typename S, typename V>
@@ -535,7 +535,7 @@ struct LevelDev {
     DeviceSliced<S> a, p, r;
     DeviceBsr<S> r_rows;          // the same transpose in plain block rows, for long_rows_kernel
     int restrict_rows = 0;  // 0: the sliced restriction; else long_rows_kernel with this many rows per wave (by timing)
-    DeviceBsr<S> a_rows;          // coarse levels: A in plain block rows, for the row kernels
+    DeviceBsr<S> a_rows;          // coarse levels and small systems: A in plain block rows, for the row kernels
     int cheb_rows = 0, residual_rows = 0;  // the same choice for the steps and residuals (by timing)
     DeviceBuffer<S> dinv;
     DeviceBuffer<double> packed;  // coarsest: the Cholesky factor packed by columns (SF_COARSE_REFERENCE's solve)
@@ -587,7 +587,7 @@ class Hierarchy final : public DeviceMultigrid {
                 h.fetch_values();
                 upload_sliced(d.a, h.a, s);
             }
-            if (l > 0) {
+            if (l > 0 || h.a.blocks() <= ROWS_BLOCKS) {
                 if (adev) build_bsr(d.a_rows, h.a, adev, s);
                 else upload_bsr(d.a_rows, h.a, s);
             }
@@ -993,22 +993,19 @@ class Hierarchy final : public DeviceMultigrid {
         smooth_batch(d, d.mres.ptr, d.mpx.ptr, x, M, s);
     }
 
-    template <int RPW>
-    static void launch_cheb_rows_rpw(LevelDev<S, V> &d, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out, V *x,
-                                     V *into, hipStream_t s, double *widen) {
-        const dim3 grid((d.a_rows.rows + RPW - 1) / RPW), block(WAVE);
-        if (d.rb == 3)
-            hipLaunchKernelGGL((cheb_rows_kernel<3, S, V, RPW>), grid, block, 0, s, d.a_rows.view(), d.dinv.ptr, d_in, r_in, keep, stp,
-                               d_out, r_out, x, into, widen);
-        else
-            hipLaunchKernelGGL((cheb_rows_kernel<6, S, V, RPW>), grid, block, 0, s, d.a_rows.view(), d.dinv.ptr, d_in, r_in, keep, stp,
-                               d_out, r_out, x, into, widen);
+    template <int RB>
+    static void launch_cheb_rows_rb(LevelDev<S, V> &d, int form, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out, V *x,
+                                    V *into, hipStream_t s, double *widen) {
+        with_rows_form<RB * RB * (int)sizeof(V)>(form, [&](auto rows, auto blocks) {
+            constexpr int RPW = decltype(rows)::value, U = decltype(blocks)::value;
+            hipLaunchKernelGGL((cheb_rows_kernel<RB, S, V, RPW, U>), dim3((d.a_rows.rows + RPW - 1) / RPW), dim3(WAVE), 0, s, d.a_rows.view(),
+                               d.dinv.ptr, d_in, r_in, keep, stp, d_out, r_out, x, into, widen);
+        });
     }
-    static void launch_cheb_rows(LevelDev<S, V> &d, int rpw, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out, V *x,
+    static void launch_cheb_rows(LevelDev<S, V> &d, int form, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out, V *x,
                                  V *into, hipStream_t s, double *widen = nullptr) {
-        if (rpw == 4) launch_cheb_rows_rpw<4>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
-        else if (rpw == 2) launch_cheb_rows_rpw<2>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
-        else launch_cheb_rows_rpw<1>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+        if (d.rb == 3) launch_cheb_rows_rb<3>(d, form, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+        else launch_cheb_rows_rb<6>(d, form, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
     }
 
     // Picks each level's batch depths, kernel forms and start fusions by timing its own kernels
@@ -1026,16 +1023,15 @@ class Hierarchy final : public DeviceMultigrid {
             d.a.batch_spmv = tune_batch(s, [&](int batch) { launch_spmv<S, V>(d.a, d.x.ptr, d.res.ptr, d.b.ptr, EPI_RESIDUAL, s, batch); },
                                         {1, 2, 4, 8}, at + "residual depth", "residual " + a_class);
             if (d.a_rows.rows) {
-                // each kernel against its row-per-wavefront forms with 1, 2 or 4 rows per wavefront
-                // (all the same bits); 0 is the sliced kernel
+                // each kernel against its rows_sum forms (all the same bits); 0 is the sliced kernel
                 d.cheb_rows = fastest(s, [&](int rpw) {
                     if (!rpw) launch_cheb_step(d, d.a.batch_cheb, d.d0.ptr, d.b.ptr, (V)0, (V)0, d.d1.ptr, d.r0.ptr, d.x.ptr, nullptr, s);
                     else launch_cheb_rows(d, rpw, d.d0.ptr, d.b.ptr, (V)0, (V)0, d.d1.ptr, d.r0.ptr, d.x.ptr, nullptr, s);
-                }, {0, 1, 2, 4}, at + "step rows per wave", "step rows " + a_class);
+                }, rows_forms(d.rb * d.rb * sizeof(V)), at + "step rows per wave", "step rows " + a_class);
                 d.residual_rows = fastest(s, [&](int rpw) {
                     if (!rpw) launch_spmv<S, V>(d.a, d.x.ptr, d.res.ptr, d.b.ptr, EPI_RESIDUAL, s);
                     else launch_long_rows<S, V>(d.a_rows, d.x.ptr, d.res.ptr, d.b.ptr, EPI_RESIDUAL, s, {nullptr, (V)0, nullptr, nullptr}, rpw);
-                }, {0, 1, 2, 4}, at + "residual rows per wave", "residual rows " + a_class);
+                }, rows_forms(d.rb * d.rb * sizeof(V)), at + "residual rows per wave", "residual rows " + a_class);
             }
             if (d.has_p) {
                 LevelDev<S, V> &c = lv_[l + 1];
@@ -1043,12 +1039,14 @@ class Hierarchy final : public DeviceMultigrid {
                 SF_HIP(hipMemsetAsync(c.x.ptr, 0, c.n * sizeof(V), s));
                 d.r.batch_spmv = tune_batch(s, [&](int batch) { launch_spmv<S, V>(d.r, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s, batch); },
                                             {1, 2, 4, 8}, at + "restriction depth", "restriction " + shape_class(d.r) + vs_);
-                // the sliced product at its best depth (0) against 1, 2 or 4 rows per wavefront and
-                // four wavefronts per row
+                // the sliced product at its best depth (0) against the rows_sum forms and four
+                // wavefronts per row
+                std::vector<int> restrict_forms = rows_forms(d.r.rb * d.r.cb * sizeof(V));
+                restrict_forms.push_back(WIDE_ROWS);
                 d.restrict_rows = forced_variant().load(std::memory_order_relaxed) == WIDE_ROWS ? WIDE_ROWS : fastest(s, [&](int rpw) {
                     if (!rpw) launch_spmv<S, V>(d.r, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s);
                     else launch_long_rows<S, V>(d.r_rows, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s, {nullptr, (V)0, nullptr, nullptr}, rpw);
-                }, {0, 1, 2, 4, WIDE_ROWS}, at + "restriction rows per wave", "restriction rows " + shape_class(d.r) + vs_);
+                }, restrict_forms, at + "restriction rows per wave", "restriction rows " + shape_class(d.r) + vs_);
                 d.p.batch_spmv = tune_batch(s, [&](int batch) { launch_spmv<S, V>(d.p, c.x.ptr, d.px.ptr, nullptr, EPI_ADD, s, batch); },
                                             {1, 2, 4, 8}, at + "prolongation depth", "prolongation " + shape_class(d.p) + vs_);
             }
@@ -1233,7 +1231,28 @@ void DeviceSystem::build_from_device_values(hipStream_t s) {
     SF_HIP(hipStreamSynchronize(s));
     clock.lap("system layout build");
     tune_spmv<double, double>(sliced, EPI_STORE, s);
+    if (rb == 3 && host.blocks() <= ROWS_BLOCKS && sliced.slices) {
+        // a small system's product by rows, on the values as they were assembled
+        std::vector<uint32_t> starts(host.starts.begin(), host.starts.end());
+        rows.rb = rows.cb = 3;
+        rows.rows = (uint32_t)host.rows;
+        rows.starts.upload(starts, s);
+        rows.cols.upload(host.columns.empty() ? std::vector<uint32_t>{0} : host.columns, s);
+        rows.borrowed = values.ptr;
+        DeviceBuffer<double> x(std::max<size_t>(host.cols * 3, 1)), y(std::max<size_t>(host.rows * 3, 1));
+        SF_HIP(hipMemsetAsync(x.ptr, 0, x.bytes(), s));
+        rows_form = fastest(s, [&](int form) {
+            if (!form) launch_spmv<double, double>(sliced, x.ptr, y.ptr, nullptr, EPI_STORE, s);
+            else launch_long_rows<double, double>(rows, x.ptr, y.ptr, nullptr, EPI_STORE, s, {nullptr, 0.0, nullptr, nullptr}, form);
+        }, rows_forms(9 * sizeof(double)), "system rows per wave", "system rows " + shape_class(sliced));
+        SF_HIP(hipStreamSynchronize(s));
+    }
     clock.lap("system product tuning");
+}
+
+void DeviceSystem::multiply(const double *x, double *y, hipStream_t s) const {
+    if (rows_form) launch_long_rows<double, double>(rows, x, y, nullptr, EPI_STORE, s, {nullptr, 0.0, nullptr, nullptr}, rows_form);
+    else launch_spmv<double, double>(sliced, x, y, nullptr, EPI_STORE, s);
 }
 
 // ---- the conjugate gradient -------------------------------------------------------------------
@@ -1430,7 +1449,7 @@ void DevicePcg::iterate() {
     hipStream_t s = ctx_->stream;
     PcgScalars *sc = scalars_.ptr;
     const int token = Profiler::get().begin(1, s, (double)a_.sliced.algorithmic_matrix_bytes() + 2.0 * n_ * 8);
-    launch_spmv<double, double>(a_.sliced, p_.ptr, ap_.ptr, nullptr, EPI_STORE, s);
+    a_.multiply(p_.ptr, ap_.ptr, s);
     Profiler::get().end(1, token, s);
     const uint32_t tag = ++readbacks_;
     if (dot_order_ == SF_DOT_TREE) {

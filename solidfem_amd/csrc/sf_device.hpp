@@ -69,11 +69,12 @@ struct DeviceBsr {
     uint32_t rows = 0;
     DeviceBuffer<uint32_t> starts, cols;
     DeviceBuffer<T> vals;
+    const T *borrowed = nullptr;  // values held elsewhere, for as long as this matrix (else null)
     mutable uint32_t passes = 0;  // launches so far, for the alternating traversal
     // Every other pass takes each XCD's rows in reverse order (SOLIDFEM_ROWS_PING_PONG=0: never).
     dev::Bsr<T> view() const {
         const uint32_t reverse = rows_ping_pong() ? (passes++ & 1u) : 0u;
-        return {starts.ptr, cols.ptr, vals.ptr, rows, reverse};
+        return {starts.ptr, cols.ptr, borrowed ? borrowed : vals.ptr, rows, reverse};
     }
     static bool rows_ping_pong();
 };
@@ -82,13 +83,42 @@ void upload_bsr(DeviceBsr<T> &out, const HostBsr<double> &m, hipStream_t s);
 // The same from `pattern` with its values already on the device (f64, row-major blocks).
 template <typename T>
 void build_bsr(DeviceBsr<T> &out, const HostBsr<double> &pattern, const double *values, hipStream_t s);
-// y = A x (epilogue per dev::Epilogue) with `rows_per_wave` block rows per wavefront
-// (long_rows_kernel: 1, 2 or 4), or WIDE_ROWS: four wavefronts per block row (wide_rows_kernel).
+// The forms of the row kernels: block rows per wavefront + 256 * (blocks a lane loads at once - 1),
+// or WIDE_ROWS: four wavefronts per block row (wide_rows_kernel, restrictions only).
 // sf_force_variant(WIDE_ROWS) forces the latter on every restriction.
 constexpr int WIDE_ROWS = 96;
+constexpr int rows_form_code(int rows, int blocks) { return rows + 256 * (blocks - 1); }
+// The forms worth timing against the sliced kernel (0) for blocks of `bytes` in the vector's
+// precision: a lane keeps U blocks in registers and a wavefront 64 U of them in LDS.
+inline std::vector<int> rows_forms(size_t bytes) {
+    std::vector<int> f{0, 1, 2, 4};
+    if (bytes <= 144) f.insert(f.end(), {rows_form_code(2, 2), rows_form_code(4, 2)});
+    if (bytes <= 72) f.insert(f.end(), {rows_form_code(4, 4), rows_form_code(8, 4)});
+    return f;
+}
+// Calls f(rows per wavefront, blocks per lane) as compile-time constants for one of rows_forms(BYTES).
+template <int BYTES, typename F>
+void with_rows_form(int form, F &&f) {
+    using std::integral_constant;
+    if constexpr (BYTES <= 72) {
+        if (form == rows_form_code(4, 4)) return f(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+        if (form == rows_form_code(8, 4)) return f(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+    }
+    if constexpr (BYTES <= 144) {
+        if (form == rows_form_code(2, 2)) return f(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+        if (form == rows_form_code(4, 2)) return f(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+    }
+    if (form == 4) return f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+    if (form == 2) return f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    return f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+}
+// Systems of at most this many blocks also keep their finest level in plain block rows for the row
+// kernels, whose latency is shorter. Four rows per wavefront against the sliced kernel, f32 step: 9.0
+// against 10.3 us at 0.5M blocks, 16.4 against 16.3 us at 0.97M (f64 vectors), 61 against 59 us at 6.9M.
+constexpr size_t ROWS_BLOCKS = 1u << 20;
 template <typename S, typename V>
 void launch_long_rows(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s,
-                      dev::Start<S, V> start = {nullptr, (V)0, nullptr, nullptr}, int rows_per_wave = 1);
+                      dev::Start<S, V> start = {nullptr, (V)0, nullptr, nullptr}, int form = 1);
 
 // Builds a sliced matrix from row-major f64 blocks already on the device (`src_values`).
 template <typename T>
@@ -242,6 +272,10 @@ struct DeviceSystem {
     HostBsr<double> host;  // block (or scalar) rows with f64 values, as assembled
     DeviceBuffer<double> values;  // row-major blocks on the device (assembly output)
     DeviceSliced<double> sliced;
+    DeviceBsr<double> rows;  // a small system's pattern over `values`, for the row kernels
+    int rows_form = 0;       // the product's form: 0 sliced, else of the row kernels (by timing)
+    // y = A x
+    void multiply(const double *x, double *y, hipStream_t s) const;
     void upload_from_host(hipStream_t s);
     void build_from_device_values(hipStream_t s);
 };

@@ -267,56 +267,89 @@ __device__ __forceinline__ V add_terms(V sum, const V *t, uint32_t n) {
     return sum;
 }
 
-// y = A x with an epilogue (as spmv_kernel) for matrices with few, long rows -- the stored
-// transposes of the prolongators, whose rows gather every fine row of an aggregate's
-// neighbourhood, and the coarse levels. One wavefront (one workgroup) takes RPW block rows,
-// 64 / RPW lanes each: the lanes load that many blocks at once and form their terms A[p][q] x[q]
-// into LDS; then lane p of the row's group adds the row's terms in stored block order and column
-// order, from zero -- the summation of spmv_kernel and of the reference, so the same bits, with
-// one memory round trip per 64 / RPW blocks instead of one per few blocks.
-template <int RB, int CB, typename S, typename V, int EPI, int RPW>
+// The sums of RPW block rows of one wavefront (one workgroup), 64 / RPW lanes each: every lane loads
+// U blocks and the x entries they meet, all in flight at once, and forms their terms A[p][q] x[q] into
+// LDS; then lane p of a row's group adds row p's terms in stored block order and column order, from
+// zero -- the summation of spmv_kernel and of the reference, so the same bits, with one memory round
+// trip per U * 64 / RPW blocks instead of one per few blocks. The sum is lane p's of each group.
+template <int RB, int CB, typename V, int RPW, int U>
+struct RowTerms {
+    static constexpr int LW = WAVE / RPW, CHUNK = LW * U;
+    V t[RPW][RB][CHUNK * CB + 16 / sizeof(V)];  // rows on different banks
+};
+template <int RB, int CB, int RPW, int U, typename S, typename V>
+__device__ __forceinline__ V rows_sum(const Bsr<S> &a, RowTerms<RB, CB, V, RPW, U> &terms, int g, int sl, uint32_t start, uint32_t len,
+                                      const V *__restrict__ x) {
+    using T = RowTerms<RB, CB, V, RPW, U>;
+    const uint32_t longest = longest_of_wave<RPW>(len);
+    V sum = (V)0;
+    for (uint32_t k0 = 0; k0 < longest; k0 += T::CHUNK) {
+        uint32_t col[U];
+        S v[U][RB * CB];
+        V xv[U][CB];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t k = k0 + sl + u * T::LW;
+            if (k < len) {
+                col[u] = a.cols[start + k];
+                const S *blk = a.vals + (size_t)(start + k) * RB * CB;
+#pragma unroll
+                for (int e = 0; e < RB * CB; ++e) v[u][e] = blk[e];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k0 + sl + u * T::LW < len) {
+#pragma unroll
+                for (int q = 0; q < CB; ++q) xv[u][q] = x[(size_t)col[u] * CB + q];
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k0 + sl + u * T::LW < len) {
+#pragma unroll
+                for (int p = 0; p < RB; ++p)
+#pragma unroll
+                    for (int q = 0; q < CB; ++q) terms.t[g][p][(sl + u * T::LW) * CB + q] = widen<V>(v[u][p * CB + q]) * xv[u][q];
+            }
+        __syncthreads();
+        if (sl < RB && k0 < len)
+            sum = add_terms<4>(sum, (const V *)terms.t[g][sl], (len - k0 < (uint32_t)T::CHUNK ? len - k0 : (uint32_t)T::CHUNK) * CB);
+        __syncthreads();
+    }
+    return sum;
+}
+
+// y = A x with an epilogue (as spmv_kernel) by rows_sum, for matrices with few or long rows: the
+// stored transposes of the prolongators, whose rows gather every fine row of an aggregate's
+// neighbourhood, the coarse levels, and systems too small to fill the chip with a lane per row.
+template <int RB, int CB, typename S, typename V, int EPI, int RPW, int U>
 __global__ __launch_bounds__(64) void long_rows_kernel(Bsr<S> a, const V *__restrict__ x, V *__restrict__ y,
                                                        const V *__restrict__ b, Start<S, V> then) {
     constexpr int LW = WAVE / RPW;
-    __shared__ __align__(16) V terms[RPW][RB][LW * CB + 16 / sizeof(V)];  // rows on different banks
+    __shared__ __align__(16) RowTerms<RB, CB, V, RPW, U> terms;
     __shared__ V values[RPW][RB];
     const int lane = threadIdx.x, g = lane / LW, sl = lane % LW;
     const uint32_t row = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW + (uint32_t)g;
     const bool live = row < a.rows;
     const uint32_t start = live ? a.starts[row] : 0u, len = live ? a.starts[row + 1] - start : 0u;
-    const uint32_t longest = longest_of_wave<RPW>(len);
-    V sum = (V)0;
-    for (uint32_t k0 = 0; k0 < longest; k0 += LW) {
-        const uint32_t k = k0 + sl;
-        if (k < len) {
-            const uint32_t col = a.cols[start + k];
-            const S *blk = a.vals + (size_t)(start + k) * RB * CB;
-            V xv[CB];
-#pragma unroll
-            for (int q = 0; q < CB; ++q) xv[q] = x[(size_t)col * CB + q];
-#pragma unroll
-            for (int p = 0; p < RB; ++p)
-#pragma unroll
-                for (int q = 0; q < CB; ++q) terms[g][p][sl * CB + q] = widen<V>(blk[p * CB + q]) * xv[q];
-        }
-        __syncthreads();
-        if (sl < RB && k0 < len) sum = add_terms<4>(sum, (const V *)terms[g][sl], (len - k0 < (uint32_t)LW ? len - k0 : (uint32_t)LW) * CB);
-        __syncthreads();
-    }
     const bool owner = live && sl < RB;
     const size_t out = (size_t)row * RB + (owner ? sl : 0);
+    // what the epilogue reads is fetched before the sums
+    const V before = !owner || EPI == EPI_STORE ? (V)0 : EPI == EPI_RESIDUAL ? b[out] : y[out];
+    S drow[RB];
+    if (then.dinv && owner) {
+#pragma unroll
+        for (int q = 0; q < RB; ++q) drow[q] = then.dinv[(size_t)row * RB * RB + (size_t)sl * RB + q];
+    }
+    const V sum = rows_sum<RB, CB, RPW, U, S, V>(a, terms, g, sl, start, len, x);
     if (owner) {
-        V value;
-        if (EPI == EPI_STORE) value = sum;
-        else if (EPI == EPI_RESIDUAL) value = b[out] - sum;
-        else value = y[out] + sum;
+        const V value = EPI == EPI_STORE ? sum : EPI == EPI_RESIDUAL ? before - sum : before + sum;
         y[out] = value;
         values[g][sl] = value;
     }
     if (then.dinv) {  // uniform
         __syncthreads();
         if (owner) {
-            const S *drow = then.dinv + (size_t)row * RB * RB + (size_t)sl * RB;
             V z = (V)0;
 #pragma unroll
             for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * values[g][q];
@@ -411,58 +444,48 @@ __global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__res
     }
 }
 
-// The fused Chebyshev step of cheb_step_kernel for levels with few rows, RPW block rows per
-// wavefront (one workgroup) as long_rows_kernel: the lanes form the terms of A d_in, lane p of a
-// row's group adds the row's terms in stored order, and the RB residuals of the block row meet in
-// LDS for the block-Jacobi product (summed over q in order from zero). The same bits as
-// cheb_step_kernel.
-template <int RB, typename S, typename V, int RPW>
+// The fused Chebyshev step of cheb_step_kernel by rows_sum: lane p of a row's group holds A d_in, and
+// the RB residuals of the block row meet in LDS for the block-Jacobi product (summed over q in order
+// from zero). The same bits as cheb_step_kernel.
+template <int RB, typename S, typename V, int RPW, int U>
 __global__ __launch_bounds__(64) void cheb_rows_kernel(Bsr<S> a, const S *__restrict__ dinv, const V *__restrict__ d_in,
                                                        const V *__restrict__ r_in, V keep, V step, V *__restrict__ d_out,
                                                        V *__restrict__ r_out, V *__restrict__ x, V *__restrict__ sum_into,
                                                        double *__restrict__ widen_into) {
     constexpr int LW = WAVE / RPW;
-    __shared__ __align__(16) V terms[RPW][RB][LW * RB + 16 / sizeof(V)];  // rows on different banks
+    __shared__ __align__(16) RowTerms<RB, RB, V, RPW, U> terms;
     __shared__ V r_new[RPW][RB];
     const int lane = threadIdx.x, g = lane / LW, sl = lane % LW;
     const uint32_t row = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW + (uint32_t)g;
     const bool live = row < a.rows;
     const uint32_t start = live ? a.starts[row] : 0u, len = live ? a.starts[row + 1] - start : 0u;
-    const uint32_t longest = longest_of_wave<RPW>(len);
-    V sum = (V)0;
-    for (uint32_t k0 = 0; k0 < longest; k0 += LW) {
-        const uint32_t k = k0 + sl;
-        if (k < len) {
-            const uint32_t col = a.cols[start + k];
-            const S *blk = a.vals + (size_t)(start + k) * RB * RB;
-            V xv[RB];
-#pragma unroll
-            for (int q = 0; q < RB; ++q) xv[q] = d_in[(size_t)col * RB + q];
-#pragma unroll
-            for (int p = 0; p < RB; ++p)
-#pragma unroll
-                for (int q = 0; q < RB; ++q) terms[g][p][sl * RB + q] = widen<V>(blk[p * RB + q]) * xv[q];
-        }
-        __syncthreads();
-        if (sl < RB && k0 < len) sum = add_terms<4>(sum, (const V *)terms[g][sl], (len - k0 < (uint32_t)LW ? len - k0 : (uint32_t)LW) * RB);
-        __syncthreads();
-    }
     const bool owner = live && sl < RB;
     const size_t i = (size_t)row * RB + (owner ? sl : 0);
-    if (owner) r_new[g][sl] = r_in[i] - sum;
+    // what the step reads besides the matrix is fetched before the sums
+    V r_old = (V)0, d_old = (V)0, x_old = (V)0, into = (V)0;
+    S drow[RB];
+    if (owner) {
+        r_old = r_in[i];
+        d_old = d_in[i];
+        x_old = x[i];
+        if (sum_into) into = sum_into[i];
+#pragma unroll
+        for (int q = 0; q < RB; ++q) drow[q] = dinv[(size_t)row * RB * RB + (size_t)sl * RB + q];
+    }
+    const V sum = rows_sum<RB, RB, RPW, U, S, V>(a, terms, g, sl, start, len, d_in);
+    if (owner) r_new[g][sl] = r_old - sum;
     __syncthreads();
     if (owner) {
-        const S *drow = dinv + (size_t)row * RB * RB + (size_t)sl * RB;
         V z = (V)0;
 #pragma unroll
         for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * r_new[g][q];
-        const V dn = keep * d_in[i] + step * z;
-        const V xn = x[i] + dn;
+        const V dn = keep * d_old + step * z;
+        const V xn = x_old + dn;
         d_out[i] = dn;
         r_out[i] = r_new[g][sl];
         x[i] = xn;
         if (sum_into) {
-            const V total = sum_into[i] + xn;
+            const V total = into + xn;
             sum_into[i] = total;
             if (widen_into) widen_into[i] = (double)total;
         }
