@@ -267,6 +267,70 @@ __device__ __forceinline__ V add_terms(V sum, const V *t, uint32_t n) {
     return sum;
 }
 
+// Adds onto acc, in order, the 16 bytes of terms that lanes FIRST .. FIRST + 3 of the lane's row of 16
+// hold, one instruction a term: the term comes from its lane with the addition. For double that is
+// fma(t, 1, acc), the same value, the product being exact. One block of instructions: between two
+// blocks the compiler would put a wait state each.
+template <int FIRST>
+__device__ __forceinline__ void add_from_lanes(float &acc, float x, float y, float z, float w) {
+#define SF_ADD(N)                                                                          \
+    "v_add_f32_dpp %0, %1, %0 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"           \
+    "v_add_f32_dpp %0, %2, %0 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"           \
+    "v_add_f32_dpp %0, %3, %0 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"           \
+    "v_add_f32_dpp %0, %4, %0 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"
+    asm("s_nop 1\n" SF_ADD(5) SF_ADD(6) SF_ADD(7) SF_ADD(8)
+        : "+v"(acc)
+        : "v"(x), "v"(y), "v"(z), "v"(w), "n"(FIRST), "n"(FIRST + 1), "n"(FIRST + 2), "n"(FIRST + 3));
+#undef SF_ADD
+}
+template <int FIRST>
+__device__ __forceinline__ void add_from_lanes(double &acc, double x, double y) {
+#define SF_ADD(N)                                                                             \
+    "v_fmac_f64_dpp %0, %1, %3 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"             \
+    "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"
+    asm("s_nop 1\n" SF_ADD(4) SF_ADD(5) SF_ADD(6) SF_ADD(7)
+        : "+v"(acc)
+        : "v"(x), "v"(y), "v"(1.0), "n"(FIRST), "n"(FIRST + 1), "n"(FIRST + 2), "n"(FIRST + 3));
+#undef SF_ADD
+}
+template <int FIRST, typename Quad>
+__device__ __forceinline__ void add_from_lanes(float &acc, const Quad &q) {
+    add_from_lanes<FIRST>(acc, q[0], q[1], q[2], q[3]);
+}
+template <int FIRST, typename Quad>
+__device__ __forceinline__ void add_from_lanes(double &acc, const Quad &q) {
+    add_from_lanes<FIRST>(acc, q[0], q[1]);
+}
+// add_terms with a row of 16 lanes per sum (four sums a wavefront, every lane of it active, `n` the
+// same for all four): one 16-byte read per lane brings 16 lanes' terms, and each addition takes its
+// term from the lane that holds it. Where few lanes add, a 16-byte LDS read is what a lane waits on:
+// 33-40 cycles for two doubles or four floats, against 5 to 6 for an addition. A lane of its own per
+// sum took 16.6 cycles a double, 10 a float. `t` has room up to a multiple of 16 reads; what lies past
+// `n` is replaced by -0.0. The sum is in every lane of the row.
+template <typename V>
+__device__ __forceinline__ V add_row_terms(V sum, const V *t, uint32_t n) {
+    constexpr uint32_t W = 16 / sizeof(V), GROUP = 16 * W;
+    typedef V Quad __attribute__((ext_vector_type(16 / sizeof(V))));
+    const uint32_t c = threadIdx.x % 16u, groups = (n + GROUP - 1) / GROUP;
+    if (groups == 0) return sum;
+    const Quad *p = reinterpret_cast<const Quad *>(t) + c;
+    Quad next = p[0];
+    for (uint32_t g = 0; g < groups; ++g) {
+        Quad q = next;
+        next = p[(g + 1 < groups ? g + 1 : g) * 16];
+        const uint32_t left = n - g * GROUP;
+        if (left < GROUP) {
+#pragma unroll
+            for (uint32_t v = 0; v < W; ++v) q[v] = c * W + v < left ? q[v] : (V)-0.0;
+        }
+        add_from_lanes<0>(sum, q);
+        if (left > 4 * W) add_from_lanes<4>(sum, q);
+        if (left > 8 * W) add_from_lanes<8>(sum, q);
+        if (left > 12 * W) add_from_lanes<12>(sum, q);
+    }
+    return sum;
+}
+
 // The sums of RPW block rows of one wavefront (one workgroup), 64 / RPW lanes each: every lane loads
 // U blocks and the x entries they meet, all in flight at once, and forms their terms A[p][q] x[q] into
 // LDS; then lane p of a row's group adds row p's terms in stored block order and column order, from
@@ -363,10 +427,11 @@ __global__ __launch_bounds__(64) void long_rows_kernel(Bsr<S> a, const V *__rest
 // long_rows_kernel with one workgroup of four wavefronts per block row, for matrices whose rows
 // are so long (hundreds of blocks) and so few that one wavefront per row leaves the chip idle
 // through a chain of round trips. All four wavefronts load CHUNK blocks' values and x entries at
-// once and put their terms into one of two LDS buffers; then lane p of the first wavefront adds row
-// p's terms in stored order while the next chunk's loads are in flight (its block columns were
-// fetched a chunk before that). Bound by the ordered chain of additions: about 4 us for 350
-// blocks, where one wavefront's chunks of 64 took 21 us.
+// once and put their terms into one of two LDS buffers; then each row of 16 lanes of the first
+// wavefronts adds one of the block row's RB rows' terms in stored order (add_row_terms) while the
+// next chunk's loads are in flight (its block columns were fetched a chunk before that). Bound by the
+// ordered chain of additions: 73 rows of 350 blocks, f32, took 21 us a wavefront per row and 11 us
+// with a lane per sum here.
 template <int RB, int CB, typename V>
 struct WideRows {
     static constexpr int THREADS = 256;
@@ -387,6 +452,18 @@ __global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__res
     const uint32_t start = a.starts[row], len = a.starts[row + 1] - start;
     const uint32_t t = threadIdx.x, k = t / W::PARTS, p0 = (t % W::PARTS) * RP;
     const bool loads = k < (uint32_t)W::CHUNK;
+    // the row of 16 lanes t / 16 adds row p of the block row (whole wavefronts: rows past RB repeat the last)
+    const bool adds = t / WAVE < (uint32_t)(RB + 3) / 4;
+    const uint32_t p = t / 16 < (uint32_t)RB ? t / 16 : RB - 1;
+    const bool owner = t / 16 < (uint32_t)RB && t % 16 == 0;
+    const size_t out = (size_t)row * RB + p;
+    // what the epilogue reads is fetched before the sums
+    const V before = !owner || EPI == EPI_STORE ? (V)0 : EPI == EPI_RESIDUAL ? b[out] : y[out];
+    S drow[RB];
+    if (then.dinv && owner) {
+#pragma unroll
+        for (int q = 0; q < RB; ++q) drow[q] = then.dinv[(size_t)row * RB * RB + (size_t)p * RB + q];
+    }
     S v[RP * CB];
     V xv[CB];
     auto fetch = [&](uint32_t at, uint32_t col) {
@@ -406,9 +483,9 @@ __global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__res
     for (uint32_t k0 = 0; k0 < len; k0 += W::CHUNK, buf ^= 1) {
         if (loads && k0 + k < len) {
 #pragma unroll
-            for (int p = 0; p < RP; ++p)
+            for (int r = 0; r < RP; ++r)
 #pragma unroll
-                for (int q = 0; q < CB; ++q) terms[buf][p0 + p][k * CB + q] = widen<V>(v[p * CB + q]) * xv[q];
+                for (int q = 0; q < CB; ++q) terms[buf][p0 + r][k * CB + q] = widen<V>(v[r * CB + q]) * xv[q];
         }
         const uint32_t k1 = k0 + W::CHUNK, k2 = k1 + W::CHUNK;
         if (k1 < len) {
@@ -416,24 +493,18 @@ __global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__res
             if (loads && k2 + k < len) col = a.cols[start + k2 + k];
         }
         // one barrier per chunk: this buffer is written again two chunks on, after the next barrier,
-        // which the adding wavefront reaches only once it has read it
+        // which the adding wavefronts reach only once they have read it
         __syncthreads();
-        if (t < (uint32_t)RB) sum = add_terms<8>(sum, (const V *)terms[buf][t], (len - k0 < (uint32_t)W::CHUNK ? len - k0 : (uint32_t)W::CHUNK) * CB);
+        if (adds) sum = add_row_terms(sum, (const V *)terms[buf][p], (len - k0 < (uint32_t)W::CHUNK ? len - k0 : (uint32_t)W::CHUNK) * CB);
     }
-    const bool owner = t < (uint32_t)RB;
-    const size_t out = (size_t)row * RB + (owner ? t : 0);
     if (owner) {
-        V value;
-        if (EPI == EPI_STORE) value = sum;
-        else if (EPI == EPI_RESIDUAL) value = b[out] - sum;
-        else value = y[out] + sum;
+        const V value = EPI == EPI_STORE ? sum : EPI == EPI_RESIDUAL ? before - sum : before + sum;
         y[out] = value;
-        values[t] = value;
+        values[p] = value;
     }
     if (then.dinv) {  // uniform
         __syncthreads();
         if (owner) {
-            const S *drow = then.dinv + (size_t)row * RB * RB + (size_t)t * RB;
             V z = (V)0;
 #pragma unroll
             for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * values[q];
@@ -621,29 +692,40 @@ __global__ void convert_kernel(size_t n, const From *__restrict__ in, To *__rest
 // runs right-looking: once x_k is final every later row subtracts its term, so each row still
 // subtracts in ascending k, the reference's order. Back substitution also subtracts each row's terms
 // in ascending k, which can only start once every later x is known: the lanes form the negated
-// products, then every lane folds them in order (broadcast reads), so the row's value needs no
-// exchange before its division.
+// products of all but the latest x while that one is still being computed, and every row of 16 lanes
+// folds them in order (add_row_terms), so the row's value needs no exchange before its division.
 //
 // The first wavefront solves, alone and with no barrier inside a panel; the other three bring the
 // next panel of `width` columns into the other LDS buffer meanwhile, so no step waits on global
-// memory. A factor that fits one buffer is one panel, read once for both substitutions. Bound by
-// the n^2 / 2 dependent subtractions of the back substitution and 2 n dependent divisions.
+// memory. A factor that fits one buffer is one panel, read once for both substitutions. Forward, a
+// block of 64 rows stays in registers, one per lane, for its own columns, then the later rows take
+// those columns' terms. Bound by the n^2 / 2 dependent subtractions of the back substitution and 2 n
+// dependent divisions (100 cycles each): n = 90 took 104 us with every step through LDS and a lane
+// folding the products.
 constexpr uint32_t COARSE_MAX = 3072;
 constexpr uint32_t COARSE_THREADS = 256;
-constexpr uint32_t COARSE_PANEL = 6144;  // entries of one of the two panel buffers
+constexpr uint32_t COARSE_PANEL = 5600;  // entries of one of the two panel buffers
 __host__ __device__ constexpr size_t packed_column(uint32_t n, uint32_t k) { return (size_t)k * n - ((size_t)k * (k - 1)) / 2; }
 // Columns per panel and LDS bytes: the whole factor where it fits two buffers' room, else two panels.
 __host__ __device__ constexpr uint32_t coarse_panel_width(uint32_t n) {
     return packed_column(n, n) <= 2 * COARSE_PANEL ? n : COARSE_PANEL / n;
 }
+// Entries of one of the two product buffers: whole groups of add_row_terms.
+__host__ __device__ constexpr uint32_t coarse_products(uint32_t n) { return (n + 31) / 32 * 32; }
 constexpr size_t coarse_solve_lds(uint32_t n) {
-    return ((coarse_panel_width(n) == n ? packed_column(n, n) + packed_column(n, n) % 2 : 2 * COARSE_PANEL) + (size_t)n + n % 2 + (n + 15) / 16 * 16) * sizeof(double);
+    return ((coarse_panel_width(n) == n ? packed_column(n, n) + packed_column(n, n) % 2 : 2 * COARSE_PANEL) + (size_t)n + n % 2 + 2 * coarse_products(n)) * sizeof(double);
 }
 // Orders this wavefront's LDS accesses before and after this point (LDS serves a wavefront's
 // accesses in order, so only the compiler has to be kept from moving them).
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+// v of `lane`, the same lane for the whole wavefront.
+__device__ __forceinline__ double lane_value(double v, uint32_t lane) {
+    const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+    const uint32_t low = __builtin_amdgcn_readlane((uint32_t)bits, lane), high = __builtin_amdgcn_readlane((uint32_t)(bits >> 32), lane);
+    return __builtin_bit_cast(double, (uint64_t)high << 32 | low);
 }
 // Several right-hand sides (row-interleaved, `stride` columns) take one workgroup each.
 template <typename V>
@@ -653,7 +735,7 @@ __global__ __launch_bounds__(COARSE_THREADS) void coarse_solve_kernel(uint32_t n
     const uint32_t width = coarse_panel_width(n), panels = (n + width - 1) / width;
     const size_t whole = packed_column(n, n);
     double *xs = smem + (panels == 1 ? whole + whole % 2 : 2 * (size_t)COARSE_PANEL), *prod = xs + n + n % 2;
-    const uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x, room = coarse_products(n);
     rhs += blockIdx.x;
     out += blockIdx.x;
     // panel p into its buffer, by the threads from `first` on
@@ -673,36 +755,86 @@ __global__ __launch_bounds__(COARSE_THREADS) void coarse_solve_kernel(uint32_t n
     };
     bring(0, 0);
     for (uint32_t i = t; i < n; i += COARSE_THREADS) xs[i] = (double)rhs[(size_t)i * stride];
+    // adding -0.0 changes nothing, and a buffer's products grow by two a step: what lies past them is
+    // never anything else
+    for (uint32_t i = t; i < 2 * room; i += COARSE_THREADS) prod[i] = -0.0;
     __syncthreads();
     for (uint32_t p = 0; p < panels; ++p) {
         const uint32_t k0 = p * width, k1 = k0 + width < n ? k0 + width : n;
         if (t >= WAVE) {
             if (p + 1 < panels) bring(p + 1, WAVE);
         } else {
-            const double *col = smem + (size_t)(p & 1u) * COARSE_PANEL;  // col[i - k] = L[i][k]
-            for (uint32_t k = k0; k < k1; col += n - k, ++k) {
-                const double xv = xs[k] / col[0];  // every lane the same quotient
+            const double *panel = smem + (size_t)(p & 1u) * COARSE_PANEL;
+            const double *col = panel;  // col[i - k] = L[i][k]
+            for (uint32_t kb = k0; kb < k1; kb += WAVE) {
+                const uint32_t ke = k1 - kb < (uint32_t)WAVE ? k1 : kb + WAVE, i = kb + t;
+                const double *const block = col;
+                double y = i < n ? xs[i] : 0.0;
+                double diagonal = col[0], below = i < n ? col[t] : 0.0;
+                for (uint32_t k = kb; k < ke; ++k) {
+                    // the next column's entries are read before this one's division
+                    const double d = diagonal, l = below;
+                    col += n - k;
+                    if (k + 1 < ke) {
+                        diagonal = col[0];
+                        below = i > k && i < n ? col[i - k - 1] : 0.0;
+                    }
+                    const double xv = lane_value(y, k - kb) / d;
+                    if (i == k) y = xv;
+                    else if (i > k) y = y - l * xv;
+                }
+                if (i < n) xs[i] = y;
                 wave_lds_fence();
-                if (t == 0) xs[k] = xv;
-                for (uint32_t i = k + 1 + t; i < n; i += WAVE) xs[i] = xs[i] - col[i - k] * xv;
+                for (uint32_t later = kb + WAVE + t; later < n; later += WAVE) {
+                    double v = xs[later];
+                    const double *c = block;
+#pragma unroll 8
+                    for (uint32_t k = kb; k < ke; ++k) {
+                        v = v - c[later - k] * xs[k];
+                        c += n - k;
+                    }
+                    xs[later] = v;
+                }
                 wave_lds_fence();
             }
         }
         __syncthreads();
     }
+    double latest = 0.0;  // x of the row below the current one
     for (uint32_t p = panels; p-- > 0;) {
         const uint32_t k0 = p * width, k1 = k0 + width < n ? k0 + width : n;
         if (t >= WAVE) {
             if (p > 0) bring(p - 1, WAVE);
         } else {
             const double *col = smem + (size_t)(p & 1u) * COARSE_PANEL + (packed_column(n, k1) - packed_column(n, k0));
+            // row ii's products with every x but the latest: k from ii + 2; c is its column
+            auto products = [&](uint32_t ii, const double *c) {
+                double *to = prod + (ii & 1u) * room;
+                for (uint32_t k = ii + 2 + t; k < n; k += 2 * WAVE) {
+                    const bool more = k + WAVE < n;
+                    const double l0 = c[k - ii], x0 = xs[k], l1 = more ? c[k + WAVE - ii] : 0.0, x1 = more ? xs[k + WAVE] : 0.0;
+                    to[k - ii - 2] = -(l0 * x0);
+                    if (more) to[k + WAVE - ii - 2] = -(l1 * x1);
+                }
+            };
+            products(k1 - 1, col - (n - (k1 - 1)));
+            double d_next = col[-(int)(n - (k1 - 1))], first_next = k1 < n ? col[1 - (int)(n - (k1 - 1))] : 0.0, y_next = xs[k1 - 1];
             for (uint32_t ii = k1; ii-- > k0;) {
                 col -= n - ii;
-                for (uint32_t k = ii + 1 + t; k < n; k += WAVE) prod[k - ii - 1] = -(col[k - ii] * xs[k]);
+                const double d = d_next, first = first_next, y = y_next;
+                if (ii > k0) {
+                    const double *c = col - (n - (ii - 1));
+                    products(ii - 1, c);  // with the x of row ii + 1 by now
+                    d_next = c[0];
+                    first_next = c[1];
+                    y_next = xs[ii - 1];
+                }
                 wave_lds_fence();
-                const double xv = add_terms<8>(xs[ii], (const double *)prod, n - 1 - ii) / col[0];
+                double v = ii + 1 < n ? y + -(first * latest) : y;
+                v = add_row_terms(v, (const double *)(prod + (ii & 1u) * room), ii + 2 < n ? n - ii - 2 : 0u);
+                latest = v / d;
                 wave_lds_fence();
-                if (t == 0) xs[ii] = xv;
+                if (t == 0) xs[ii] = latest;
                 wave_lds_fence();
             }
         }
@@ -756,8 +888,9 @@ static __global__ __launch_bounds__(256) void factor_inverse_entries_kernel(uint
 
 // out = inv b, R rows per workgroup. inv is symmetric bit for bit (entry (i, j) and entry (j, i) add
 // the same products in the same order), so a row's entries are read as its column's, contiguous. All
-// threads form a chunk of the rows' terms into LDS with every load in flight at once; then lane r of
-// the first wavefront adds row r's terms in ascending k from zero. Bound by that chain of n additions.
+// threads form a chunk of the rows' terms into LDS with every load in flight at once; then row r of 16
+// lanes of the first wavefront adds row r's terms in ascending k from zero. Bound by that chain of n
+// additions; n = 438 took 17.5 us with one lane per row walking its column.
 constexpr uint32_t COARSE_ROWS = 4, COARSE_CHUNK = 1024;
 template <typename V>
 __global__ __launch_bounds__(256) void coarse_inverse_kernel(uint32_t n, const double *__restrict__ inv, const V *__restrict__ rhs,
@@ -782,9 +915,9 @@ __global__ __launch_bounds__(256) void coarse_inverse_kernel(uint32_t n, const d
 #pragma unroll
             for (uint32_t r = 0; r < COARSE_ROWS; ++r) terms[r][t + 256 * j] = a[r][j] * bk[j];
         __syncthreads();
-        if (t < rows) sum = add_terms<8>(sum, (const double *)terms[t], n - k0 < COARSE_CHUNK ? n - k0 : COARSE_CHUNK);
+        if (t < WAVE) sum = add_row_terms(sum, (const double *)terms[t / 16], n - k0 < COARSE_CHUNK ? n - k0 : COARSE_CHUNK);
     }
-    if (t < rows) out[i0 + t] = (V)sum;
+    if (t < WAVE && t % 16 == 0 && t / 16 < rows) out[i0 + t / 16] = (V)sum;
 }
 
 // ---- conjugate gradient vectors -------------------------------------------------------------

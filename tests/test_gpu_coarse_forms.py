@@ -31,7 +31,8 @@ def serial(first, terms):
     return np.add.accumulate(np.concatenate([[first], terms]))[-1]
 
 
-# 54 and 108 unknowns: one panel; 162, the first past it: two; 600: panels of 10 columns; 1260: of 4, and two chunks of 1024
+# 54 and 108 unknowns: one panel; 162, the first past it: two; 600: panels of 9 columns; 1260: of 4, and two chunks of 1024;
+# 64 columns of the inverse's product are past the form of eight sums a workgroup from 600 on, 3 columns within it
 @pytest.mark.parametrize("divisions", [(1, 1, 1), (2, 1, 1), (3, 1, 1), (4, 2, 2), (6, 3, 2)])
 def test_coarse_solves_follow_their_serial_orders(ctx, divisions):
     ref = refcpu.Problem(loaded([float(d) for d in divisions], list(divisions)))
@@ -58,6 +59,7 @@ def test_coarse_solves_follow_their_serial_orders(ctx, divisions):
         inverse = np.vstack([inverse, fast.apply_batch(np.eye(n)[first:first + 64])])
     assert np.array_equal(bits(inverse), bits(inverse.T))
     got = fast.apply(b[2])
+    assert np.array_equal(bits(fast.apply_batch(b)[2]), bits(got))
     assert np.array_equal(bits(got), bits([serial(0.0, inverse[:, i] * b[2]) for i in range(n)]))
 
 
