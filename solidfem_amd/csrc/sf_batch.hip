@@ -14,13 +14,13 @@ using namespace dev;
 static inline unsigned grid_for(size_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
 
 template <typename S>
-bool staged_candidate(const DeviceSliced<S> &a, uint32_t M, size_t vector_size) {
+bool staged_candidate(const DeviceSliced<S> &a, uint32_t M) {
     const bool long_rows = a.rows > 0 && a.blocks >= 40 * a.rows;
     const bool forced = forced_variant().load(std::memory_order_relaxed) == STAGED_FORM;
-    return (long_rows || forced) && (size_t)a.rb * M <= 256 && (size_t)STAGE_BLOCKS * a.cb * M * vector_size <= 48 * 1024;
+    return (long_rows || forced) && (size_t)a.rb * (M % 2 ? M : M / 2) <= 256;
 }
-template bool staged_candidate<double>(const DeviceSliced<double> &, uint32_t, size_t);
-template bool staged_candidate<float>(const DeviceSliced<float> &, uint32_t, size_t);
+template bool staged_candidate<double>(const DeviceSliced<double> &, uint32_t);
+template bool staged_candidate<float>(const DeviceSliced<float> &, uint32_t);
 
 std::vector<int> spmm_candidates(int rb, int cb, size_t value_size, uint32_t M, bool product, bool staged) {
     // Depths 1, 2, 4 of the lane-group kernels, NODE_FORM + depth for one wavefront per block
@@ -87,11 +87,21 @@ static void spmm_shape(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, c
     else spmm_depth<RB, CB, 1>(a, M, x, y, b, epi, s, depth, node_form(batch));
 }
 
+template <int RB, int CB, typename S, typename V, typename UNIT, int CPL>
+static void spmm_staged_unit(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s) {
+    const uint32_t units = (uint32_t)(CB * M * sizeof(V) / sizeof(UNIT));
+    const size_t lds = 2 * (size_t)stage_chunk(units, STAGE_UNITS<UNIT, V>) * units * sizeof(UNIT);
+    hipLaunchKernelGGL((spmm_staged_kernel<RB, CB, S, V, UNIT, CPL>), dim3((unsigned)((size_t)a.slices * Shape<RB>::NPW)), dim3(256), lds, s,
+                       a.batch_view(), M, epi, x, y, b);
+}
 template <int RB, int CB, typename S, typename V>
 static void spmm_staged(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s) {
-    const size_t lds = (size_t)STAGE_BLOCKS * CB * M * sizeof(V);
-    hipLaunchKernelGGL((spmm_staged_kernel<RB, CB, S, V>), dim3((unsigned)((size_t)a.slices * Shape<RB>::NPW)), dim3(256), lds, s,
-                       a.batch_view(), M, epi, x, y, b);
+    // 16-byte units where every block's x entries are whole aligned units; two columns per thread
+    // where M is even (its x entries then are pairs too)
+    const bool wide = (size_t)CB * M * sizeof(V) % 16 == 0 && (uintptr_t)x % 16 == 0;
+    if (wide && M % 2 == 0) spmm_staged_unit<RB, CB, S, V, uint4, 2>(a, M, x, y, b, epi, s);
+    else if (M % 2 == 0) spmm_staged_unit<RB, CB, S, V, V, 2>(a, M, x, y, b, epi, s);
+    else spmm_staged_unit<RB, CB, S, V, V, 1>(a, M, x, y, b, epi, s);
 }
 
 template <typename S, typename V>
@@ -106,7 +116,7 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
             SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));
             SF_HIP(hipMemsetAsync(ty.ptr, 0, ty.bytes(), s));
             tuned = tune_batch(s, [&](int depth) { launch_spmm<S, V>(a, M, tx.ptr, ty.ptr, ty.ptr, EPI_STORE, s, depth); },
-                               spmm_candidates(a.rb, a.cb, sizeof(S), M, true, staged_candidate(a, M, sizeof(V))), "",
+                               spmm_candidates(a.rb, a.cb, sizeof(S), M, true, staged_candidate(a, M)), "",
                                "batch product " + std::to_string(columns_log2(M)) + " " + shape_class(a) + "|" + std::to_string(sizeof(V)));
             SF_HIP(hipStreamSynchronize(s));
         }
@@ -114,7 +124,7 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
     }
     if (batch >= STAGED_FORM) {
         // the staged form where it fits, else one column and four blocks in flight per lane
-        if (staged_candidate(a, M, sizeof(V))) {
+        if (staged_candidate(a, M)) {
             if (a.rb == 3 && a.cb == 3) spmm_staged<3, 3>(a, M, x, y, b, epi, s);
             else if (a.rb == 6 && a.cb == 6) spmm_staged<6, 6>(a, M, x, y, b, epi, s);
             else if (a.rb == 3 && a.cb == 6) spmm_staged<3, 6>(a, M, x, y, b, epi, s);

@@ -248,16 +248,25 @@ __device__ __forceinline__ uint32_t node_of_wave(uint32_t order) {
 }
 
 // The same product with one workgroup per block row, for matrices of few, long rows (the stored
-// transposes of the coarse levels): the workgroup stages a chunk of STAGE_BLOCKS of the row's
-// blocks and the x entries they gather into LDS with loads that are all in flight at once, then
-// thread (p, m) adds the chunk's terms of row entry p and column m in the stored order -- a chunk
-// costs two round trips where a lane walking the row costs one per few blocks. Every sum is the
-// lane-group form's: from zero, blocks in order, block columns in order.
-constexpr int STAGE_BLOCKS = 32;
-template <int RB, int CB, typename S, typename V>
+// transposes of the coarse levels): the workgroup stages a chunk of the row's blocks and the x entries
+// they gather in LDS, all loads in flight at once, then thread (p, CPL columns from m) adds the chunk's
+// terms of row entry p in the stored order. The next chunk's values and x entries are on their way to
+// registers meanwhile, and the block columns of the one after it: a chunk costs its additions, not a
+// round trip, and one barrier (two LDS buffers). Every sum is the lane-group form's: from zero, blocks
+// in order, block columns in order. x moves in units of UNIT: 16 bytes where a block's CB * M entries
+// are whole units, else single entries.
+constexpr int STAGE_BLOCKS = 32;  // at most this many blocks a chunk
+template <typename UNIT, typename V>
+constexpr int STAGE_UNITS = sizeof(UNIT) == 16 && sizeof(V) < 16 ? 4 : 8;  // x units a thread holds
+// Blocks per chunk for `units` units of x per block.
+__host__ __device__ inline uint32_t stage_chunk(uint32_t units, uint32_t held) {
+    const uint32_t c = 256u * held / units;
+    return c < (uint32_t)STAGE_BLOCKS ? c : (uint32_t)STAGE_BLOCKS;
+}
+template <int RB, int CB, typename S, typename V, typename UNIT, int CPL>
 __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t M, int epi, const V *__restrict__ x,
                                                           V *__restrict__ y, const V *__restrict__ b) {
-    constexpr int NPW = Shape<RB>::NPW;
+    constexpr int NPW = Shape<RB>::NPW, LEN = RB * CB, UX = STAGE_UNITS<UNIT, V>, UV = (STAGE_BLOCKS * LEN + 255) / 256;
     const uint32_t pos = blockIdx.x;
     if (pos >= a.slices * (uint32_t)NPW) return;  // the whole workgroup leaves together
     const uint32_t row = a.perm[pos];
@@ -267,45 +276,82 @@ __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t 
     const uint32_t slot0 = a.slice_start[slice], len = a.row_len[pos];
     const uint32_t *__restrict__ cp = a.cols + (size_t)slot0 * NPW + j;
     const S *__restrict__ vp = a.vals + ((size_t)slot0 * WAVE + (size_t)j * RB) * CB;
-    __shared__ S values[STAGE_BLOCKS][RB * CB];
-    __shared__ uint32_t columns[STAGE_BLOCKS];
-    extern __shared__ unsigned char staged_x[];  // STAGE_BLOCKS x CB x M entries of x
-    V *xs = reinterpret_cast<V *>(staged_x);
-    const uint32_t t = threadIdx.x;
-    const bool computes = t < (uint32_t)RB * M;
-    const uint32_t p = computes ? t / M : 0, m = computes ? t % M : 0;
-    V sum = (V)0;
-    // a chunk's block columns are loaded during the chunk before it, so its values and its x
-    // entries are fetched together: one round trip per chunk
-    uint32_t column = t < (uint32_t)STAGE_BLOCKS && t < len ? cp[(size_t)t * NPW] : 0;
-    for (uint32_t k0 = 0; k0 < len; k0 += STAGE_BLOCKS) {
-        const uint32_t n = min((uint32_t)STAGE_BLOCKS, len - k0);
-        if (t < n) columns[t] = column;
-        __syncthreads();
-        const uint32_t k1 = k0 + STAGE_BLOCKS;
-        if (t < (uint32_t)STAGE_BLOCKS && k1 + t < len) column = cp[(size_t)(k1 + t) * NPW];
-        for (uint32_t e = t; e < n * RB * CB; e += blockDim.x) {
-            const uint32_t k = e / (RB * CB), r = e - k * (RB * CB);
-            values[k][r] = vp[(size_t)(k0 + k) * WAVE * CB + r];
+    __shared__ S values[2][STAGE_BLOCKS * LEN];
+    __shared__ uint32_t columns[2][STAGE_BLOCKS];
+    extern __shared__ __align__(16) unsigned char staged_x[];  // two buffers of chunk * CB * M entries of x
+    const uint32_t units = (uint32_t)(CB * M * sizeof(V) / sizeof(UNIT)), chunk = stage_chunk(units, UX);
+    UNIT *xs[2] = {reinterpret_cast<UNIT *>(staged_x), reinterpret_cast<UNIT *>(staged_x) + chunk * units};
+    const uint32_t t = threadIdx.x, across = M / CPL;
+    const bool computes = t < (uint32_t)RB * across;
+    const uint32_t p = computes ? t / across : 0, m = computes ? t % across * CPL : 0;
+    // this thread's units of a chunk: block k and unit r of its x
+    uint32_t uk[UX], ur[UX];
+#pragma unroll
+    for (int u = 0; u < UX; ++u) {
+        uk[u] = (t + 256u * u) / units;
+        ur[u] = (t + 256u * u) - uk[u] * units;
+        if (uk[u] >= chunk) uk[u] = NONE;
+    }
+    UNIT xv[UX];
+    S vv[UV];
+    auto fetch = [&](uint32_t k0, const uint32_t *cols) {
+        const uint32_t n = k0 < len ? min(chunk, len - k0) : 0u;
+#pragma unroll
+        for (int u = 0; u < UX; ++u)
+            if (uk[u] < n) xv[u] = reinterpret_cast<const UNIT *>(x + (size_t)cols[uk[u]] * CB * M)[ur[u]];
+#pragma unroll
+        for (int u = 0; u < UV; ++u) {
+            const uint32_t e = t + 256u * u, k = e / LEN;
+            if (k < n) vv[u] = vp[(size_t)(k0 + k) * WAVE * CB + (e - k * LEN)];
         }
-        for (uint32_t e = t; e < n * CB * M; e += blockDim.x) {
-            const uint32_t mm = e % M, kq = e / M;
-            const uint32_t k = kq / CB, q = kq - k * CB;
-            xs[e] = x[((size_t)columns[k] * CB + q) * M + mm];
-        }
+    };
+    V sum[CPL];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) sum[c] = (V)0;
+    if (t < chunk && t < len) columns[0][t] = cp[(size_t)t * NPW];
+    uint32_t column = t < chunk && chunk + t < len ? cp[(size_t)(chunk + t) * NPW] : 0;
+    __syncthreads();
+    fetch(0, columns[0]);
+    int buf = 0;
+    for (uint32_t k0 = 0; k0 < len; k0 += chunk, buf ^= 1) {
+        const uint32_t n = min(chunk, len - k0);
+#pragma unroll
+        for (int u = 0; u < UX; ++u)
+            if (uk[u] < n) xs[buf][t + 256u * u] = xv[u];
+#pragma unroll
+        for (int u = 0; u < UV; ++u)
+            if (t + 256u * u < n * LEN) values[buf][t + 256u * u] = vv[u];
+        if (t < chunk) columns[buf ^ 1][t] = column;
+        // one barrier per chunk: a buffer is written again two chunks on, which a wavefront reaches
+        // only after the barrier between, and so after the others have read it
         __syncthreads();
-        if (computes)
+        const uint32_t k2 = k0 + 2 * chunk;
+        if (t < chunk && k2 + t < len) column = cp[(size_t)(k2 + t) * NPW];
+        fetch(k0 + chunk, columns[buf ^ 1]);
+        if (computes) {
+            const V *xb = reinterpret_cast<const V *>(xs[buf]) + m;
+            const S *vb = values[buf] + p * CB;
+#pragma unroll 4
             for (uint32_t k = 0; k < n; ++k)
 #pragma unroll
-                for (int q = 0; q < CB; ++q) sum = sum + widen<V>(values[k][p * CB + q]) * xs[(k * CB + q) * M + m];
-        __syncthreads();
+                for (int q = 0; q < CB; ++q) {
+                    V xe[CPL];
+                    load_columns<CPL, V>(xb + (k * CB + q) * M, xe);
+                    const V v = widen<V>(vb[k * LEN + q]);
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) sum[c] = sum[c] + v * xe[c];
+                }
+        }
     }
     if (!computes) return;
     const size_t out = ((size_t)row * RB + p) * M + m;
-    V v = sum;
-    if (epi == EPI_RESIDUAL) v = b[out] - sum;
-    else if (epi == EPI_ADD) v = y[out] + sum;
-    y[out] = v;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        V v = sum[c];
+        if (epi == EPI_RESIDUAL) v = b[out + c] - sum[c];
+        else if (epi == EPI_ADD) v = y[out + c] + sum[c];
+        y[out + c] = v;
+    }
 }
 
 template <int RB, int CB, int BATCH, typename S, typename V>
@@ -523,6 +569,43 @@ __global__ __launch_bounds__(256) void coarse_inverse_batch_kernel(uint32_t n, u
         buf ^= 1;
     }
     if (m < M && i < n) out[(size_t)i * M + m] = (V)sum;
+}
+
+// The same product where it has few sums (row, column), too few to fill the chip with a thread each:
+// a workgroup takes eight of them, all threads form a chunk of their terms into LDS at once, and a row
+// of 16 lanes adds each sum's terms in ascending k (add_row_terms). n = 377 rows and 5 columns took
+// 20 us with the tiles above, 12 workgroups in a chain of round trips.
+constexpr uint32_t COARSE_SUMS = 8, COARSE_SUMS_CHUNK = 512;
+constexpr size_t COARSE_SUMS_MOST = 16384;  // sums up to which this form is taken: two waves of the chip's workgroups
+template <typename V>
+__global__ __launch_bounds__(256) void coarse_inverse_sums_kernel(uint32_t n, uint32_t M, const double *__restrict__ inv,
+                                                                  const V *__restrict__ rhs, V *__restrict__ out) {
+    __shared__ __align__(16) double terms[COARSE_SUMS][COARSE_SUMS_CHUNK + 2];
+    const uint32_t t = threadIdx.x, first = blockIdx.x * COARSE_SUMS, count = n * M;
+    double sum = 0.0;
+    for (uint32_t k0 = 0; k0 < n; k0 += COARSE_SUMS_CHUNK) {
+        constexpr uint32_t PER = COARSE_SUMS_CHUNK / 256;
+        double a[COARSE_SUMS][PER], bk[COARSE_SUMS][PER];
+#pragma unroll
+        for (uint32_t r = 0; r < COARSE_SUMS; ++r) {
+            const uint32_t e = first + r < count ? first + r : count - 1, i = e / M, m = e - i * M;
+#pragma unroll
+            for (uint32_t j = 0; j < PER; ++j) {
+                const uint32_t k = k0 + t + 256 * j;
+                a[r][j] = k < n ? inv[(size_t)i * n + k] : 0.0;
+                bk[r][j] = k < n ? (double)rhs[(size_t)k * M + m] : 0.0;
+            }
+        }
+        if (k0) __syncthreads();  // the chunk before has been added
+#pragma unroll
+        for (uint32_t r = 0; r < COARSE_SUMS; ++r)
+#pragma unroll
+            for (uint32_t j = 0; j < PER; ++j) terms[r][t + 256 * j] = a[r][j] * bk[r][j];
+        __syncthreads();
+        if (t < COARSE_SUMS * 16)
+            sum = add_row_terms(sum, (const double *)terms[t / 16], n - k0 < COARSE_SUMS_CHUNK ? n - k0 : COARSE_SUMS_CHUNK);
+    }
+    if (t < COARSE_SUMS * 16 && t % 16 == 0 && first + t / 16 < count) out[first + t / 16] = (V)sum;
 }
 
 // ---- conjugate gradient, M columns -----------------------------------------------------------

@@ -915,7 +915,7 @@ class Hierarchy final : public DeviceMultigrid {
             }, spmm_candidates(d.rb, d.rb, sizeof(S), M, false), "", "batch step " + group + shape_class(d.a) + vsize);
             d.mm_depth[lg][1] = tune_batch(s, [&](int batch) {
                 launch_spmm<S, V>(d.a, M, d.mx.ptr, d.mres.ptr, d.mb.ptr, EPI_RESIDUAL, s, batch);
-            }, spmm_candidates(d.rb, d.rb, sizeof(S), M, true, staged_candidate(d.a, M, sizeof(V))), "",
+            }, spmm_candidates(d.rb, d.rb, sizeof(S), M, true, staged_candidate(d.a, M)), "",
                "batch residual " + group + shape_class(d.a) + vsize);
             if (d.has_p) {
                 LevelDev<S, V> &c = lv_[l + 1];
@@ -924,11 +924,11 @@ class Hierarchy final : public DeviceMultigrid {
                 SF_HIP(hipMemsetAsync(c.mx.ptr, 0, cneed * sizeof(V), s));
                 d.mm_depth[lg][2] = tune_batch(s, [&](int batch) {
                     launch_spmm<S, V>(d.r, M, d.mres.ptr, c.mb.ptr, nullptr, EPI_STORE, s, batch);
-                }, spmm_candidates(d.r.rb, d.r.cb, sizeof(S), M, true, staged_candidate(d.r, M, sizeof(V))), "",
+                }, spmm_candidates(d.r.rb, d.r.cb, sizeof(S), M, true, staged_candidate(d.r, M)), "",
                    "batch restriction " + group + shape_class(d.r) + vsize);
                 d.mm_depth[lg][3] = tune_batch(s, [&](int batch) {
                     launch_spmm<S, V>(d.p, M, c.mx.ptr, d.mpx.ptr, nullptr, EPI_ADD, s, batch);
-                }, spmm_candidates(d.p.rb, d.p.cb, sizeof(S), M, true, staged_candidate(d.p, M, sizeof(V))), "",
+                }, spmm_candidates(d.p.rb, d.p.cb, sizeof(S), M, true, staged_candidate(d.p, M)), "",
                    "batch prolongation " + group + shape_class(d.p) + vsize);
             }
         }
@@ -973,7 +973,10 @@ class Hierarchy final : public DeviceMultigrid {
         const int lg = columns_log2(M);
         if (!d.has_p) {
             if (d.has_factor) {
-                if (d.inverse.ptr)
+                if (d.inverse.ptr && d.n * (size_t)M <= COARSE_SUMS_MOST)
+                    hipLaunchKernelGGL(coarse_inverse_sums_kernel<V>, dim3(grid_for(d.n * (size_t)M, COARSE_SUMS)), dim3(256), 0, s, (uint32_t)d.n, M,
+                                       d.inverse.ptr, b, x);
+                else if (d.inverse.ptr)
                     hipLaunchKernelGGL(coarse_inverse_batch_kernel<V>, dim3(grid_for(d.n, coarse_rows(M))), dim3(256), 0, s, (uint32_t)d.n, M,
                                        coarse_rows(M), d.inverse.ptr, b, x);
                 else

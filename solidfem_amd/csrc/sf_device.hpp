@@ -187,11 +187,11 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
 // The batch depths worth trying for a matrix's batched product.
 // The variant codes a batched product (`product`) or Chebyshev step is timed over for M columns.
 std::vector<int> spmm_candidates(int rb, int cb, size_t value_size, uint32_t M, bool product = true, bool staged = false);
-// Whether the staged form (STAGED_FORM) is a candidate for products by `a` with M columns of
-// `vector_size` bytes: rows of at least 40 blocks on average (or the form forced), at most 256
-// (row entry, column) pairs per row, and the staged entries of x within 48 KiB of LDS.
+// Whether the staged form (STAGED_FORM) is a candidate for products by `a` with M columns: rows of
+// at least 40 blocks on average (or the form forced) and at most 256 threads' sums per row (two
+// columns a thread where M is even).
 template <typename S>
-bool staged_candidate(const DeviceSliced<S> &a, uint32_t M, size_t vector_size);
+bool staged_candidate(const DeviceSliced<S> &a, uint32_t M);
 // Tunes a matrix's product on scratch vectors of its shape.
 template <typename S, typename V>
 void tune_spmv(DeviceSliced<S> &a, int epi, hipStream_t s);
