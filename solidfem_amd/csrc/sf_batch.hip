@@ -1,8 +1,10 @@
 // Several load cases over one matrix and one hierarchy: the batched block product and the
 // lockstep conjugate gradient whose every column repeats the single-column solve's bits.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstddef>
+#include <cstring>
 
 #include "sf_batch_kernels.hpp"
 #include "sf_device.hpp"
@@ -47,65 +49,65 @@ std::vector<int> spmm_candidates(int rb, int cb, size_t value_size, uint32_t M, 
 }
 
 template <int RB, int CB, int BATCH, int CPL, typename S, typename V>
-static void spmm_launch(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, bool node) {
+static void spmm_launch(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st, bool node) {
     if (node) {
         const size_t threads = (size_t)a.slices * Shape<RB>::NPW * WAVE;
         hipLaunchKernelGGL((spmm_node_kernel<RB, CB, BATCH, S, V>), dim3(grid_for(threads, 256)), dim3(256), 0, s, a.batch_view(), M, epi,
-                           x, y, b);
+                           x, y, b, st);
         return;
     }
     const int lg = columns_log2((M + CPL - 1) / CPL);
     const size_t threads = (size_t)a.slices * Shape<RB>::NPW << lg;
     hipLaunchKernelGGL((spmm_kernel<RB, CB, BATCH, S, V, CPL>), dim3(grid_for(threads, 256)), dim3(256), 0, s, a.batch_view(), lg, M, epi,
-                       x, y, b);
+                       x, y, b, st);
 }
 
 template <int RB, int CB, int CPL, typename S, typename V>
-static void spmm_depth(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int depth, bool node) {
+static void spmm_depth(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st, int depth, bool node) {
     switch (depth) {
-        case 1: spmm_launch<RB, CB, 1, CPL>(a, M, x, y, b, epi, s, node); break;
-        case 2: spmm_launch<RB, CB, 2, CPL>(a, M, x, y, b, epi, s, node); break;
+        case 1: spmm_launch<RB, CB, 1, CPL>(a, M, x, y, b, epi, s, st, node); break;
+        case 2: spmm_launch<RB, CB, 2, CPL>(a, M, x, y, b, epi, s, st, node); break;
         case 8:
             // eight blocks in flight: for one column per lane (long rows, few of them)
             if constexpr (CPL == 1) {
-                spmm_launch<RB, CB, 8, CPL>(a, M, x, y, b, epi, s, node);
+                spmm_launch<RB, CB, 8, CPL>(a, M, x, y, b, epi, s, st, node);
                 break;
             }
             [[fallthrough]];
-        default: spmm_launch<RB, CB, 4, CPL>(a, M, x, y, b, epi, s, node); break;
+        default: spmm_launch<RB, CB, 4, CPL>(a, M, x, y, b, epi, s, st, node); break;
     }
 }
 
 template <int RB, int CB, typename S, typename V>
-static void spmm_shape(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int batch) {
+static void spmm_shape(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st, int batch) {
     const int depth = form_depth(batch);
     int cpl = form_columns(batch);
     if (M % (uint32_t)cpl) cpl = 1;
-    if (cpl == 8) spmm_depth<RB, CB, 8>(a, M, x, y, b, epi, s, depth, false);
-    else if (cpl == 4) spmm_depth<RB, CB, 4>(a, M, x, y, b, epi, s, depth, false);
-    else if (cpl == 2) spmm_depth<RB, CB, 2>(a, M, x, y, b, epi, s, depth, false);
-    else spmm_depth<RB, CB, 1>(a, M, x, y, b, epi, s, depth, node_form(batch));
+    if (cpl == 8) spmm_depth<RB, CB, 8>(a, M, x, y, b, epi, s, st, depth, false);
+    else if (cpl == 4) spmm_depth<RB, CB, 4>(a, M, x, y, b, epi, s, st, depth, false);
+    else if (cpl == 2) spmm_depth<RB, CB, 2>(a, M, x, y, b, epi, s, st, depth, false);
+    else spmm_depth<RB, CB, 1>(a, M, x, y, b, epi, s, st, depth, node_form(batch));
 }
 
 template <int RB, int CB, typename S, typename V, typename UNIT, int CPL>
-static void spmm_staged_unit(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s) {
+static void spmm_staged_unit(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
     const uint32_t units = (uint32_t)(CB * M * sizeof(V) / sizeof(UNIT));
     const size_t lds = 2 * (size_t)stage_chunk(units, STAGE_UNITS<UNIT, V>) * units * sizeof(UNIT);
     hipLaunchKernelGGL((spmm_staged_kernel<RB, CB, S, V, UNIT, CPL>), dim3((unsigned)((size_t)a.slices * Shape<RB>::NPW)), dim3(256), lds, s,
-                       a.batch_view(), M, epi, x, y, b);
+                       a.batch_view(), M, epi, x, y, b, st);
 }
 template <int RB, int CB, typename S, typename V>
-static void spmm_staged(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s) {
+static void spmm_staged(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
     // 16-byte units where every block's x entries are whole aligned units; two columns per thread
     // where M is even (its x entries then are pairs too)
     const bool wide = (size_t)CB * M * sizeof(V) % 16 == 0 && (uintptr_t)x % 16 == 0;
-    if (wide && M % 2 == 0) spmm_staged_unit<RB, CB, S, V, uint4, 2>(a, M, x, y, b, epi, s);
-    else if (M % 2 == 0) spmm_staged_unit<RB, CB, S, V, V, 2>(a, M, x, y, b, epi, s);
-    else spmm_staged_unit<RB, CB, S, V, V, 1>(a, M, x, y, b, epi, s);
+    if (wide && M % 2 == 0) spmm_staged_unit<RB, CB, S, V, uint4, 2>(a, M, x, y, b, epi, s, st);
+    else if (M % 2 == 0) spmm_staged_unit<RB, CB, S, V, V, 2>(a, M, x, y, b, epi, s, st);
+    else spmm_staged_unit<RB, CB, S, V, V, 1>(a, M, x, y, b, epi, s, st);
 }
 
 template <typename S, typename V>
-void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int batch) {
+void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int batch, Start<S, V> st) {
     if (a.slices == 0 || M == 0) return;
     if (M > MAX_COLUMNS) throw Error(SF_ERR_INVALID_ARGUMENT, "more columns than a batch carries");
     if (batch == 0) {
@@ -125,10 +127,10 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
     if (batch >= STAGED_FORM) {
         // the staged form where it fits, else one column and four blocks in flight per lane
         if (staged_candidate(a, M)) {
-            if (a.rb == 3 && a.cb == 3) spmm_staged<3, 3>(a, M, x, y, b, epi, s);
-            else if (a.rb == 6 && a.cb == 6) spmm_staged<6, 6>(a, M, x, y, b, epi, s);
-            else if (a.rb == 3 && a.cb == 6) spmm_staged<3, 6>(a, M, x, y, b, epi, s);
-            else if (a.rb == 6 && a.cb == 3) spmm_staged<6, 3>(a, M, x, y, b, epi, s);
+            if (a.rb == 3 && a.cb == 3) spmm_staged<3, 3>(a, M, x, y, b, epi, s, st);
+            else if (a.rb == 6 && a.cb == 6) spmm_staged<6, 6>(a, M, x, y, b, epi, s, st);
+            else if (a.rb == 3 && a.cb == 6) spmm_staged<3, 6>(a, M, x, y, b, epi, s, st);
+            else if (a.rb == 6 && a.cb == 3) spmm_staged<6, 3>(a, M, x, y, b, epi, s, st);
             else batch = 4;
             if (batch >= STAGED_FORM) {
                 SF_HIP(hipGetLastError());
@@ -138,12 +140,12 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
             batch = 4;
         }
     }
-    if (a.rb == 3 && a.cb == 3) spmm_shape<3, 3>(a, M, x, y, b, epi, s, batch);
-    else if (a.rb == 6 && a.cb == 6) spmm_shape<6, 6>(a, M, x, y, b, epi, s, batch);
-    else if (a.rb == 3 && a.cb == 6) spmm_shape<3, 6>(a, M, x, y, b, epi, s, batch);
-    else if (a.rb == 6 && a.cb == 3) spmm_shape<6, 3>(a, M, x, y, b, epi, s, batch);
+    if (a.rb == 3 && a.cb == 3) spmm_shape<3, 3>(a, M, x, y, b, epi, s, st, batch);
+    else if (a.rb == 6 && a.cb == 6) spmm_shape<6, 6>(a, M, x, y, b, epi, s, st, batch);
+    else if (a.rb == 3 && a.cb == 6) spmm_shape<3, 6>(a, M, x, y, b, epi, s, st, batch);
+    else if (a.rb == 6 && a.cb == 3) spmm_shape<6, 3>(a, M, x, y, b, epi, s, st, batch);
     else if constexpr (std::is_same<S, double>::value && std::is_same<V, double>::value) {
-        if (a.rb == 1 && a.cb == 1) spmm_shape<1, 1>(a, M, x, y, b, epi, s, batch);
+        if (a.rb == 1 && a.cb == 1) spmm_shape<1, 1>(a, M, x, y, b, epi, s, st, batch);
         else throw Error(SF_ERR_INTERNAL, "unsupported block shape");
     } else {
         throw Error(SF_ERR_INTERNAL, "unsupported block shape");
@@ -152,11 +154,63 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
 }
 
 template void launch_spmm<double, double>(const DeviceSliced<double> &, uint32_t, const double *, double *, const double *, int,
-                                          hipStream_t, int);
+                                          hipStream_t, int, Start<double, double>);
 template void launch_spmm<float, double>(const DeviceSliced<float> &, uint32_t, const double *, double *, const double *, int,
-                                         hipStream_t, int);
+                                         hipStream_t, int, Start<float, double>);
 template void launch_spmm<float, float>(const DeviceSliced<float> &, uint32_t, const float *, float *, const float *, int,
-                                        hipStream_t, int);
+                                        hipStream_t, int, Start<float, float>);
+
+// Rows per wavefront of a rows form for M columns: its chains, 3 M a row, fit the 64 lanes.
+int rows_batch_rows(int form, uint32_t M) {
+    int rpw = form - ROWS_BATCH_FORM;
+    while (rpw > 1 && (uint32_t)rpw * 3 * M > (uint32_t)WAVE) rpw /= 2;
+    return rpw;
+}
+template <int MM, int RPW, typename S, typename V>
+static void rows_batch_launch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
+    hipLaunchKernelGGL((rows_batch_kernel<3, 3, MM, RPW, S, V>), dim3((a.rows + RPW - 1) / RPW), dim3(WAVE),
+                       ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, a.view(), M, epi, x, y, b, st);
+}
+template <int MM, typename S, typename V>
+static void rows_batch_rpw(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int rpw, Start<S, V> st) {
+    if (rpw == 4) rows_batch_launch<MM, 4>(a, M, x, y, b, epi, s, st);
+    else if (rpw == 2) rows_batch_launch<MM, 2>(a, M, x, y, b, epi, s, st);
+    else rows_batch_launch<MM, 1>(a, M, x, y, b, epi, s, st);
+}
+template <typename S, typename V>
+void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, Start<S, V> st) {
+    if (a.rows == 0 || M == 0) return;
+    if (a.rb != 3 || a.cb != 3 || M > ROWS_BATCH_COLUMNS) throw Error(SF_ERR_INTERNAL, "no rows form for this block shape or column count");
+    if (M <= 4) rows_batch_rpw<4>(a, M, x, y, b, epi, s, rows_batch_rows(form, M), st);
+    else rows_batch_rpw<8>(a, M, x, y, b, epi, s, rows_batch_rows(form, M), st);
+    SF_HIP(hipGetLastError());
+}
+template void launch_rows_batch<double, double>(const DeviceBsr<double> &, uint32_t, const double *, double *, const double *, int, hipStream_t, int,
+                                                Start<double, double>);
+template void launch_rows_batch<float, double>(const DeviceBsr<float> &, uint32_t, const double *, double *, const double *, int, hipStream_t, int,
+                                               Start<float, double>);
+template void launch_rows_batch<float, float>(const DeviceBsr<float> &, uint32_t, const float *, float *, const float *, int, hipStream_t, int,
+                                              Start<float, float>);
+
+void DeviceSystem::multiply_batch(uint32_t M, const double *x, double *y, hipStream_t s) const {
+    // the form by rows is chosen per group of column counts, as the sliced product's is
+    int &form = rows_mm[columns_log2(M)];
+    if (rows.rows == 0 || M > ROWS_BATCH_COLUMNS) form = 0;
+    else if (form < 0) {
+        DeviceBuffer<double> tx(host.cols * 3 * M), ty(host.rows * 3 * M);
+        SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));
+        launch_spmm<double, double>(sliced, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s);  // its own choice first
+        std::vector<int> forms = rows_batch_forms();
+        forms.insert(forms.begin(), 0);
+        form = tune_batch(s, [&](int f) {
+            if (!f) launch_spmm<double, double>(sliced, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s);
+            else launch_rows_batch<double, double>(rows, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s, f, {nullptr, 0.0, nullptr, nullptr});
+        }, forms, "", "batch system rows " + std::to_string(columns_log2(M)) + " " + shape_class(sliced));
+        SF_HIP(hipStreamSynchronize(s));
+    }
+    if (form) launch_rows_batch<double, double>(rows, M, x, y, nullptr, EPI_STORE, s, form, {nullptr, 0.0, nullptr, nullptr});
+    else launch_spmm<double, double>(sliced, M, x, y, nullptr, EPI_STORE, s);
+}
 
 // ---- the lockstep conjugate gradient ---------------------------------------------------------
 
@@ -171,12 +225,14 @@ DevicePcgBatch::DevicePcgBatch(std::shared_ptr<Context> ctx, const DeviceSystem 
     for (auto *buf : {&b_, &x_, &r_, &z_, &p_, &ap_, &tmp_, &tmp2_, &stage_}) buf->resize(total);
     scalars_.resize(m_);
     partials_.resize((size_t)DOT_BLOCKS * m_);
+    partials2_.resize((size_t)DOT_BLOCKS * m_);
     active_.resize(m_);
     mask_.resize(m_);
     col_.assign(m_, Column{});
-    SF_HIP(hipHostMalloc((void **)&pinned_, sizeof(PcgScalars) * m_, hipHostMallocDefault));
+    SF_HIP(hipHostMalloc((void **)&pinned_, sizeof(PcgScalars) * m_, hipHostMallocCoherent));
+    std::memset((void *)pinned_, 0, sizeof(PcgScalars) * m_);
+    SF_HIP(hipHostGetDevicePointer((void **)&mirror_, pinned_, 0));
     SF_HIP(hipHostMalloc((void **)&pinned_flags_, sizeof(uint32_t) * m_, hipHostMallocDefault));
-    SF_HIP(hipEventCreateWithFlags(&copied_, hipEventDisableTiming));
     static const bool lds_set = [] {
         const int bytes = (int)(DOT_THREADS * MAX_COLUMNS * sizeof(double));
         SF_HIP(hipFuncSetAttribute((const void *)dot_partials_batch_kernel<0>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
@@ -192,7 +248,6 @@ DevicePcgBatch::~DevicePcgBatch() {
     (void)hipStreamSynchronize(ctx_->stream);
     if (pinned_) (void)hipHostFree(pinned_);
     if (pinned_flags_) (void)hipHostFree(pinned_flags_);
-    if (copied_) (void)hipEventDestroy(copied_);
 }
 
 void DevicePcgBatch::upload_flags(uint32_t *device, const std::vector<uint32_t> &flags) {
@@ -215,7 +270,26 @@ const PcgScalars *DevicePcgBatch::read_scalars() {
     return pinned_;
 }
 
-void DevicePcgBatch::dot(const double *a, const double *b, size_t field, int kind, const uint32_t *mask, int mode) {
+// As DevicePcg::wait_for_tag, for every column's copy.
+void DevicePcgBatch::wait_for_tag(uint32_t tag) {
+    const auto start = std::chrono::steady_clock::now();
+    uint32_t m = 0;
+    for (uint64_t spins = 0; m < m_; ++spins) {
+        if (__atomic_load_n(&pinned_[m].tag, __ATOMIC_ACQUIRE) == tag) {
+            ++m;
+            continue;
+        }
+        if ((spins & 1023) == 1023 && std::chrono::steady_clock::now() - start > std::chrono::seconds(1)) break;
+    }
+    if (m == m_) return;
+    SF_HIP(hipStreamSynchronize(ctx_->stream));
+    for (m = 0; m < m_; ++m)
+        if (__atomic_load_n(&pinned_[m].tag, __ATOMIC_ACQUIRE) != tag)
+            throw Error(SF_ERR_INTERNAL, "the solver's scalars did not reach the host");
+}
+
+void DevicePcgBatch::dot(const double *a, const double *b, size_t field, int kind, const uint32_t *mask, int mode, PcgScalars *mirror,
+                         uint32_t tag) {
     hipStream_t s = ctx_->stream;
     if (dot_order_ == SF_DOT_REFERENCE) {
         if (mode == 0)
@@ -229,8 +303,10 @@ void DevicePcgBatch::dot(const double *a, const double *b, size_t field, int kin
         else
             hipLaunchKernelGGL((dot_partials_batch_kernel<1>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_, m_, a, b, partials_.ptr);
         hipLaunchKernelGGL(dot_final_batch_kernel, dim3(m_), dim3(DOT_THREADS), 0, s, DOT_BLOCKS, m_, (const double *)partials_.ptr,
-                           kind, (uint32_t)field, scalars_.ptr, mask);
+                           kind, (uint32_t)field, scalars_.ptr, mask, mirror, tag);
     }
+    if (dot_order_ == SF_DOT_REFERENCE && mirror)
+        hipLaunchKernelGGL(mirror_columns_kernel, dim3(1), dim3(WAVE), 0, s, m_, (const PcgScalars *)scalars_.ptr, mirror, tag);
     SF_HIP(hipGetLastError());
 }
 
@@ -251,7 +327,7 @@ void DevicePcgBatch::reset_direction(const uint32_t *mask) {
     const size_t total = n_ * m_;
     hipLaunchKernelGGL((copy_columns_kernel<double>), dim3(grid_for(total, 256)), dim3(256), 0, ctx_->stream, n_, m_, mask,
                        (const double *)z_.ptr, p_.ptr);
-    dot(r_.ptr, z_.ptr, offsetof(PcgScalars, rz), FINAL_STORE, mask);
+    dot(r_.ptr, z_.ptr, rz_slot_ ? offsetof(PcgScalars, rz_next) : offsetof(PcgScalars, rz), FINAL_STORE, mask);
 }
 
 void DevicePcgBatch::restart(const double *rhs) {
@@ -268,6 +344,7 @@ void DevicePcgBatch::restart(const double *rhs) {
     SF_HIP(hipMemsetAsync(z_.ptr, 0, total * 8, s));
     SF_HIP(hipMemsetAsync(p_.ptr, 0, total * 8, s));
     SF_HIP(hipMemsetAsync(scalars_.ptr, 0, sizeof(PcgScalars) * m_, s));
+    rz_slot_ = 0;
     dot(b_.ptr, b_.ptr, offsetof(PcgScalars, rr), FINAL_STORE, nullptr);
     const PcgScalars *h = read_scalars();
     std::vector<uint32_t> live(m_, 0);
@@ -294,20 +371,38 @@ void DevicePcgBatch::iterate() {
     const size_t total = n_ * m_;
     const unsigned g = grid_for(total, 256);
     const int token = Profiler::get().begin(4, s, (double)a_.sliced.algorithmic_matrix_bytes() + 2.0 * total * 8);
-    launch_spmm<double, double>(a_.sliced, m_, p_.ptr, ap_.ptr, nullptr, EPI_STORE, s);
+    a_.multiply_batch(m_, p_.ptr, ap_.ptr, s);
     Profiler::get().end(4, token, s);
-    dot(p_.ptr, ap_.ptr, offsetof(PcgScalars, curvature), FINAL_STORE, nullptr);
-    hipLaunchKernelGGL(pcg_update_batch_kernel, dim3(g), dim3(256), 0, s, n_, m_, scalars_.ptr, (const uint32_t *)active_.ptr,
-                       (const double *)p_.ptr, (const double *)ap_.ptr, x_.ptr, r_.ptr);
-    dot(r_.ptr, r_.ptr, offsetof(PcgScalars, rr), FINAL_STORE, nullptr);
-    SF_HIP(hipMemcpyAsync(pinned_, scalars_.ptr, sizeof(PcgScalars) * m_, hipMemcpyDeviceToHost, s));
-    SF_HIP(hipEventRecord(copied_, s));
-    precondition(r_.ptr, z_.ptr);
-    dot(r_.ptr, z_.ptr, 0, FINAL_RZ, active_.ptr);
-    hipLaunchKernelGGL(pcg_direction_batch_kernel, dim3(g), dim3(256), 0, s, n_, m_, (const PcgScalars *)scalars_.ptr,
-                       (const uint32_t *)active_.ptr, (const double *)z_.ptr, p_.ptr);
+    // the readback overlaps the V-cycle, as DevicePcg::iterate's
+    const uint32_t tag = ++readbacks_;
+    if (dot_order_ == SF_DOT_TREE && m_ <= FUSED_COLUMNS) {
+        // the same sums in the same order, formed by the kernels that use them
+        const size_t lds = (size_t)DOT_THREADS * m_ * sizeof(double);
+        hipLaunchKernelGGL((dot_partials_batch_kernel<0>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_, m_, (const double *)p_.ptr,
+                           (const double *)ap_.ptr, partials_.ptr);
+        hipLaunchKernelGGL(pcg_update_fused_batch_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_, m_, scalars_.ptr, rz_slot_,
+                           (const uint32_t *)active_.ptr, (const double *)partials_.ptr, (const double *)p_.ptr, (const double *)ap_.ptr,
+                           x_.ptr, r_.ptr, partials2_.ptr);
+        hipLaunchKernelGGL(dot_final_batch_kernel, dim3(m_), dim3(DOT_THREADS), 0, s, DOT_BLOCKS, m_, (const double *)partials2_.ptr,
+                           (int)FINAL_STORE, (uint32_t)offsetof(PcgScalars, rr), scalars_.ptr, (const uint32_t *)nullptr, mirror_, tag);
+        precondition(r_.ptr, z_.ptr);
+        hipLaunchKernelGGL((dot_partials_batch_kernel<0>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_, m_, (const double *)r_.ptr,
+                           (const double *)z_.ptr, partials_.ptr);
+        hipLaunchKernelGGL(pcg_direction_fused_batch_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, s, n_, m_, scalars_.ptr, rz_slot_,
+                           (const uint32_t *)active_.ptr, (const double *)partials_.ptr, (const double *)z_.ptr, p_.ptr);
+        rz_slot_ ^= 1u;
+    } else {
+        dot(p_.ptr, ap_.ptr, offsetof(PcgScalars, curvature), FINAL_STORE, nullptr);
+        hipLaunchKernelGGL(pcg_update_batch_kernel, dim3(g), dim3(256), 0, s, n_, m_, scalars_.ptr, (const uint32_t *)active_.ptr,
+                           (const double *)p_.ptr, (const double *)ap_.ptr, x_.ptr, r_.ptr);
+        dot(r_.ptr, r_.ptr, offsetof(PcgScalars, rr), FINAL_STORE, nullptr, 0, mirror_, tag);
+        precondition(r_.ptr, z_.ptr);
+        dot(r_.ptr, z_.ptr, 0, FINAL_RZ, active_.ptr);
+        hipLaunchKernelGGL(pcg_direction_batch_kernel, dim3(g), dim3(256), 0, s, n_, m_, (const PcgScalars *)scalars_.ptr,
+                           (const uint32_t *)active_.ptr, (const double *)z_.ptr, p_.ptr);
+    }
     SF_HIP(hipGetLastError());
-    SF_HIP(hipEventSynchronize(copied_));
+    wait_for_tag(tag);
     std::vector<PcgScalars> h(pinned_, pinned_ + m_);
     bool changed = false;
     std::vector<uint32_t> recheck(m_, 0);
@@ -468,7 +563,7 @@ void DevicePcgBatch::replace_columns(const std::vector<uint32_t> &columns, const
 
 size_t DevicePcgBatch::device_bytes() const {
     size_t bytes = 0;
-    for (const auto *buf : {&b_, &x_, &r_, &z_, &p_, &ap_, &tmp_, &tmp2_, &jacobi_, &stage_, &partials_}) bytes += buf->bytes();
+    for (const auto *buf : {&b_, &x_, &r_, &z_, &p_, &ap_, &tmp_, &tmp2_, &jacobi_, &stage_, &partials_, &partials2_}) bytes += buf->bytes();
     return bytes + scalars_.bytes() + active_.bytes() + mask_.bytes();
 }
 

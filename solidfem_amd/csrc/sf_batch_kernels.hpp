@@ -163,11 +163,33 @@ __device__ __forceinline__ void rows_product(const Sliced<S> &a, uint32_t slot0,
     for (int p = 0; p < RB; ++p) sum[p] = s[p][0];
 }
 
+// The Chebyshev start on CPL columns of block row `row`, whose values y a lane holds (Start,
+// cheb_start_batch_kernel): z = D^-1 y summed over the block row in order from zero, d = z / theta, x = d.
+template <int RB, int CPL, typename S, typename V>
+__device__ __forceinline__ void start_columns(const Start<S, V> &st, uint32_t row, uint32_t m0, uint32_t M, const V (&y)[RB][CPL]) {
+    const S *dr = st.dinv + (size_t)row * RB * RB;
+#pragma unroll
+    for (int p = 0; p < RB; ++p) {
+        V d[CPL];
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            V z = (V)0;
+#pragma unroll
+            for (int q = 0; q < RB; ++q) z = z + widen<V>(dr[p * RB + q]) * y[q][c];
+            d[c] = z / st.theta;
+        }
+        const size_t at = ((size_t)row * RB + p) * M + m0;
+        store_columns<CPL, V>(st.d + at, d);
+        store_columns<CPL, V>(st.x + at, d);
+    }
+}
+
 // Y = A X (STORE), Y = B - A X (RESIDUAL) or Y = Y + A X (ADD) for M columns: the batched form
-// of spmv_kernel (products, residuals, restriction over the stored transpose, prolongation).
+// of spmv_kernel (products, residuals, restriction over the stored transpose, prolongation),
+// optionally followed by the Chebyshev start on Y.
 template <int RB, int CB, int BATCH, typename S, typename V, int CPL>
 __global__ __launch_bounds__(256) void spmm_kernel(Sliced<S> a, int log2g, uint32_t M, int epi, const V *__restrict__ x,
-                                                   V *__restrict__ y, const V *__restrict__ b) {
+                                                   V *__restrict__ y, const V *__restrict__ b, Start<S, V> then) {
     // CPL > 1: lane m of the group takes the CPL columns from m * CPL (M a multiple of CPL)
     constexpr int NPW = Shape<RB>::NPW;
     const GroupLane g = group_lane(log2g, a.order);
@@ -192,7 +214,10 @@ __global__ __launch_bounds__(256) void spmm_kernel(Sliced<S> a, int log2g, uint3
             for (int c = 0; c < CPL; ++c) v[c] = epi == EPI_RESIDUAL ? v[c] - sum[p][c] : v[c] + sum[p][c];
         }
         store_columns<CPL, V>(y + out, v);
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) sum[p][c] = v[c];
     }
+    if (then.dinv) start_columns<RB, CPL, S, V>(then, row, m0, M, sum);
 }
 
 // The same product with one wavefront per block row: the row's position, block columns and block
@@ -265,7 +290,7 @@ __host__ __device__ inline uint32_t stage_chunk(uint32_t units, uint32_t held) {
 }
 template <int RB, int CB, typename S, typename V, typename UNIT, int CPL>
 __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t M, int epi, const V *__restrict__ x,
-                                                          V *__restrict__ y, const V *__restrict__ b) {
+                                                          V *__restrict__ y, const V *__restrict__ b, Start<S, V> then) {
     constexpr int NPW = Shape<RB>::NPW, LEN = RB * CB, UX = STAGE_UNITS<UNIT, V>, UV = (STAGE_BLOCKS * LEN + 255) / 256;
     const uint32_t pos = blockIdx.x;
     if (pos >= a.slices * (uint32_t)NPW) return;  // the whole workgroup leaves together
@@ -343,20 +368,42 @@ __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t 
                 }
         }
     }
-    if (!computes) return;
     const size_t out = ((size_t)row * RB + p) * M + m;
+    if (computes) {
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        V v = sum[c];
-        if (epi == EPI_RESIDUAL) v = b[out + c] - sum[c];
-        else if (epi == EPI_ADD) v = y[out + c] + sum[c];
-        y[out + c] = v;
+        for (int c = 0; c < CPL; ++c) {
+            if (epi == EPI_RESIDUAL) sum[c] = b[out + c] - sum[c];
+            else if (epi == EPI_ADD) sum[c] = y[out + c] + sum[c];
+            y[out + c] = sum[c];
+        }
+    }
+    if (!then.dinv) return;  // uniform
+    // the start: the block row's entries meet in LDS (RB * M entries: within the two x buffers of at
+    // least one block of CB >= 3 each), which every thread has done with after the barrier
+    V *row_values = reinterpret_cast<V *>(staged_x);
+    __syncthreads();
+    if (computes) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) row_values[p * M + m + c] = sum[c];
+    }
+    __syncthreads();
+    if (computes) {
+        const S *drow = then.dinv + (size_t)row * RB * RB + (size_t)p * RB;
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            V z = (V)0;
+#pragma unroll
+            for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * row_values[q * M + m + c];
+            const V dv = z / then.theta;
+            then.d[out + c] = dv;
+            then.x[out + c] = dv;
+        }
     }
 }
 
 template <int RB, int CB, int BATCH, typename S, typename V>
 __global__ __launch_bounds__(256) void spmm_node_kernel(Sliced<S> a, uint32_t M, int epi, const V *__restrict__ x,
-                                                        V *__restrict__ y, const V *__restrict__ b) {
+                                                        V *__restrict__ y, const V *__restrict__ b, Start<S, V> then) {
     constexpr int NPW = Shape<RB>::NPW;
     const uint32_t pos = node_of_wave(a.order);
     if (pos >= a.slices * (uint32_t)NPW) return;
@@ -365,20 +412,22 @@ __global__ __launch_bounds__(256) void spmm_node_kernel(Sliced<S> a, uint32_t M,
     V sum[RB];
     node_product<RB, CB, BATCH, S, V>(a, pos, m, M, x, row, sum);
     if (row == NONE || (uint32_t)m >= M) return;
+    V v[RB][1];
 #pragma unroll
     for (int p = 0; p < RB; ++p) {
         const size_t out = ((size_t)row * RB + p) * M + m;
-        if (epi == EPI_STORE) y[out] = sum[p];
-        else if (epi == EPI_RESIDUAL) y[out] = b[out] - sum[p];
-        else y[out] = y[out] + sum[p];
+        v[p][0] = epi == EPI_STORE ? sum[p] : epi == EPI_RESIDUAL ? b[out] - sum[p] : y[out] + sum[p];
+        y[out] = v[p][0];
     }
+    if (then.dinv) start_columns<RB, 1, S, V>(then, row, (uint32_t)m, M, v);
 }
 
 template <int RB, int BATCH, typename S, typename V>
 __global__ __launch_bounds__(256) void cheb_step_node_kernel(Sliced<S> a, uint32_t M, const S *__restrict__ dinv,
                                                              const V *__restrict__ d_in, const V *__restrict__ r_in, V keep,
                                                              V step, V *__restrict__ d_out, V *__restrict__ r_out,
-                                                             V *__restrict__ x, V *__restrict__ sum_into) {
+                                                             V *__restrict__ x, V *__restrict__ sum_into,
+                                                             double *__restrict__ widen_into) {
     constexpr int NPW = Shape<RB>::NPW;
     const uint32_t pos = node_of_wave(a.order);
     if (pos >= a.slices * (uint32_t)NPW) return;
@@ -402,7 +451,11 @@ __global__ __launch_bounds__(256) void cheb_step_node_kernel(Sliced<S> a, uint32
         d_out[i] = dn;
         r_out[i] = r_new[p];
         x[i] = xn;
-        if (sum_into) sum_into[i] = sum_into[i] + xn;
+        if (sum_into) {
+            const V total = sum_into[i] + xn;
+            sum_into[i] = total;
+            if (widen_into) widen_into[i] = (double)total;
+        }
     }
 }
 
@@ -461,6 +514,155 @@ __global__ __launch_bounds__(256) void cheb_start_batch_kernel(uint32_t rows, ui
     }
 }
 
+// The finest level's right-hand sides rounded in from f64 and the start on them (convert_start_kernel
+// per column). One thread per block row and column.
+template <int RB, typename S, typename V>
+__global__ __launch_bounds__(256) void convert_start_batch_kernel(uint32_t rows, uint32_t M, const double *__restrict__ r,
+                                                                  V *__restrict__ b, const S *__restrict__ dinv, V theta,
+                                                                  V *__restrict__ d, V *__restrict__ x) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (size_t)rows * M) return;
+    const uint32_t row = (uint32_t)(t / M), m = (uint32_t)(t - (size_t)row * M);
+    V bv[RB][1];
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        const size_t at = ((size_t)row * RB + q) * M + m;
+        bv[q][0] = (V)r[at];
+        b[at] = bv[q][0];
+    }
+    start_columns<RB, 1, S, V>(Start<S, V>{dinv, theta, d, x}, row, m, M, bv);
+}
+
+// ---- few columns of a small system ----
+
+// rows_sum for M <= MM columns: a wavefront (one workgroup) takes RPW block rows, 64 / RPW lanes each;
+// every lane loads a block and the M columns of the x entries it meets and forms their terms into LDS,
+// then lane c adds chain c's terms in stored order: row entry and column c % (RB M) of row c / (RB M),
+// RPW RB M <= 64. One round trip per 64 / RPW blocks, where a lane walking its row pays one per few.
+template <int RB, int CB, typename V, int RPW>
+constexpr int ROWS_BATCH_STRIDE = WAVE / RPW * CB + 16 / sizeof(V);  // entries of a chain's room
+template <int RB, int CB, int MM, int RPW, typename S, typename V>
+__device__ __forceinline__ V rows_sum_batch(const Bsr<S> &a, V *terms, uint32_t M, int g, int sl, uint32_t start, uint32_t len,
+                                            const V *__restrict__ x) {
+    constexpr int LW = WAVE / RPW, STRIDE = ROWS_BATCH_STRIDE<RB, CB, V, RPW>;
+    const uint32_t longest = longest_of_wave<RPW>(len), chain = threadIdx.x;
+    const bool adds = chain < (uint32_t)(RPW * RB) * M;
+    const uint32_t chain_len = (uint32_t)__shfl((int)len, adds ? (int)(chain / (RB * M)) * LW : 0, WAVE);
+    V sum = (V)0;
+    for (uint32_t k0 = 0; k0 < longest; k0 += LW) {
+        const uint32_t k = k0 + sl;
+        if (k < len) {
+            const uint32_t col = a.cols[start + k];
+            S v[RB * CB];
+            V xv[MM][CB];
+            const S *blk = a.vals + (size_t)(start + k) * RB * CB;
+#pragma unroll
+            for (int e = 0; e < RB * CB; ++e) v[e] = blk[e];
+#pragma unroll
+            for (int m = 0; m < MM; ++m)
+                if ((uint32_t)m < M) {
+#pragma unroll
+                    for (int q = 0; q < CB; ++q) xv[m][q] = x[((size_t)col * CB + q) * M + m];
+                }
+#pragma unroll
+            for (int m = 0; m < MM; ++m)
+                if ((uint32_t)m < M) {
+#pragma unroll
+                    for (int p = 0; p < RB; ++p)
+#pragma unroll
+                        for (int q = 0; q < CB; ++q)
+                            terms[(size_t)((g * RB + p) * M + m) * STRIDE + sl * CB + q] = widen<V>(v[p * CB + q]) * xv[m][q];
+                }
+        }
+        __syncthreads();
+        if (adds && k0 < chain_len)
+            sum = add_terms<4>(sum, (const V *)terms + (size_t)chain * STRIDE, (chain_len - k0 < (uint32_t)LW ? chain_len - k0 : (uint32_t)LW) * CB);
+        __syncthreads();
+    }
+    return sum;
+}
+
+template <int RB, int CB, int MM, int RPW, typename S, typename V>
+__global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, uint32_t M, int epi, const V *__restrict__ x, V *__restrict__ y,
+                                                        const V *__restrict__ b, Start<S, V> then) {
+    constexpr int LW = WAVE / RPW;
+    extern __shared__ __align__(16) unsigned char rows_terms[];
+    V *terms = reinterpret_cast<V *>(rows_terms);
+    __shared__ V values[WAVE];
+    const uint32_t lane = threadIdx.x, first = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW;
+    const uint32_t row = first + lane / LW;
+    const uint32_t start = row < a.rows ? a.starts[row] : 0u, len = row < a.rows ? a.starts[row + 1] - start : 0u;
+    // this lane's chain: row entry p of `own`, column m
+    const uint32_t per = RB * M, within = lane % per, p = within / M, m = within - p * M, own = first + lane / per;
+    const bool owner = lane < RPW * per && own < a.rows;
+    const size_t out = owner ? ((size_t)own * RB + p) * M + m : 0;
+    const V before = !owner || epi == EPI_STORE ? (V)0 : epi == EPI_RESIDUAL ? b[out] : y[out];
+    const V sum = rows_sum_batch<RB, CB, MM, RPW, S, V>(a, terms, M, (int)(lane / LW), (int)(lane % LW), start, len, x);
+    V value = (V)0;
+    if (owner) {
+        value = epi == EPI_STORE ? sum : epi == EPI_RESIDUAL ? before - sum : before + sum;
+        y[out] = value;
+    }
+    if (!then.dinv) return;  // uniform
+    values[lane] = value;
+    __syncthreads();
+    if (owner) {
+        const S *drow = then.dinv + (size_t)own * RB * RB + (size_t)p * RB;
+        const V *row_values = values + lane - within + m;
+        V z = (V)0;
+#pragma unroll
+        for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * row_values[q * M];
+        const V dv = z / then.theta;
+        then.d[out] = dv;
+        then.x[out] = dv;
+    }
+}
+
+template <int RB, int MM, int RPW, typename S, typename V>
+__global__ __launch_bounds__(64) void cheb_rows_batch_kernel(Bsr<S> a, uint32_t M, const S *__restrict__ dinv, const V *__restrict__ d_in,
+                                                             const V *__restrict__ r_in, V keep, V step, V *__restrict__ d_out,
+                                                             V *__restrict__ r_out, V *__restrict__ x, V *__restrict__ sum_into,
+                                                             double *__restrict__ widen_into) {
+    constexpr int LW = WAVE / RPW;
+    extern __shared__ __align__(16) unsigned char rows_terms[];
+    V *terms = reinterpret_cast<V *>(rows_terms);
+    __shared__ V r_new[WAVE];
+    const uint32_t lane = threadIdx.x, first = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW;
+    const uint32_t row = first + lane / LW;
+    const uint32_t start = row < a.rows ? a.starts[row] : 0u, len = row < a.rows ? a.starts[row + 1] - start : 0u;
+    const uint32_t per = RB * M, within = lane % per, p = within / M, m = within - p * M, own = first + lane / per;
+    const bool owner = lane < RPW * per && own < a.rows;
+    const size_t i = owner ? ((size_t)own * RB + p) * M + m : 0;
+    V r_old = (V)0, d_old = (V)0, x_old = (V)0, into = (V)0;
+    S drow[RB];
+    if (owner) {
+        r_old = r_in[i];
+        d_old = d_in[i];
+        x_old = x[i];
+        if (sum_into) into = sum_into[i];
+#pragma unroll
+        for (int q = 0; q < RB; ++q) drow[q] = dinv[(size_t)own * RB * RB + (size_t)p * RB + q];
+    }
+    const V sum = rows_sum_batch<RB, RB, MM, RPW, S, V>(a, terms, M, (int)(lane / LW), (int)(lane % LW), start, len, d_in);
+    r_new[lane] = r_old - sum;
+    __syncthreads();
+    if (!owner) return;
+    const V *row_r = r_new + lane - within + m;
+    V z = (V)0;
+#pragma unroll
+    for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * row_r[q * M];
+    const V dn = keep * d_old + step * z;
+    const V xn = x_old + dn;
+    d_out[i] = dn;
+    r_out[i] = r_new[lane];
+    x[i] = xn;
+    if (sum_into) {
+        const V total = into + xn;
+        sum_into[i] = total;
+        if (widen_into) widen_into[i] = (double)total;
+    }
+}
+
 // One later Chebyshev step for M columns, fused as cheb_step_kernel: ad = A d_in;
 // r_out = r_in - ad; z = D^-1 r_out (the lane holds its block row's residuals); d_out = keep d_in
 // + step z; x += d_out; with `sum_into`, sum_into += x (cycle.rs:611-650, :534-536, :655-674).
@@ -468,7 +670,8 @@ template <int RB, int BATCH, typename S, typename V, int CPL>
 __global__ __launch_bounds__(256) void cheb_step_batch_kernel(Sliced<S> a, int log2g, uint32_t M, const S *__restrict__ dinv,
                                                               const V *__restrict__ d_in, const V *__restrict__ r_in, V keep,
                                                               V step, V *__restrict__ d_out, V *__restrict__ r_out,
-                                                              V *__restrict__ x, V *__restrict__ sum_into) {
+                                                              V *__restrict__ x, V *__restrict__ sum_into,
+                                                              double *__restrict__ widen_into) {
     constexpr int NPW = Shape<RB>::NPW;
     const GroupLane g = group_lane(log2g, a.order);
     const uint32_t m0 = (uint32_t)g.m * CPL;
@@ -512,6 +715,12 @@ __global__ __launch_bounds__(256) void cheb_step_batch_kernel(Sliced<S> a, int l
 #pragma unroll
             for (int c = 0; c < CPL; ++c) acc[c] = acc[c] + xn[c];
             store_columns<CPL, V>(sum_into + i, acc);
+            if (widen_into) {
+                double w[CPL];
+#pragma unroll
+                for (int c = 0; c < CPL; ++c) w[c] = (double)acc[c];
+                store_columns<CPL, double>(widen_into + i, w);
+            }
         }
     }
 }
@@ -618,6 +827,27 @@ __global__ __launch_bounds__(256) void coarse_inverse_sums_kernel(uint32_t n, ui
 // coalesced: thread u takes column u % M of slots t = u / M, u / M + 256 / M, ..., eight slots at a
 // time, so that each grid-stride step has their sixteen loads in flight together.
 constexpr int DOT_CHUNK = 8;
+// The sums of a block's DOT_THREADS slots per column, from LDS, into the block's partials.
+__device__ __forceinline__ void reduce_slots(double *ls, uint32_t M, double *__restrict__ partials) {
+    const uint32_t u = threadIdx.x;
+    __syncthreads();
+    // the butterfly of wave_sum, as pairs: s[l] = s[l] + s[l + off] for l < off
+    for (uint32_t off = WAVE / 2; off > 0; off >>= 1) {
+        const uint32_t work = (DOT_THREADS / WAVE) * off * M;
+        for (uint32_t e = u; e < work; e += DOT_THREADS) {
+            const uint32_t m = e % M, rest = e / M, l = rest % off, w = rest / off;
+            const uint32_t t = w * WAVE + l;
+            ls[t * M + m] = ls[t * M + m] + ls[(t + off) * M + m];
+        }
+        __syncthreads();
+    }
+    for (uint32_t m = u; m < M; m += DOT_THREADS) {
+        double s = 0.0;
+        for (int w = 0; w < DOT_THREADS / WAVE; ++w) s = s + ls[(size_t)w * WAVE * M + m];
+        partials[(size_t)blockIdx.x * M + m] = s;
+    }
+}
+
 template <int MODE>
 __global__ __launch_bounds__(DOT_THREADS) void dot_partials_batch_kernel(size_t n, uint32_t M, const double *__restrict__ a,
                                                                           const double *__restrict__ b,
@@ -651,22 +881,7 @@ __global__ __launch_bounds__(DOT_THREADS) void dot_partials_batch_kernel(size_t 
                 if (t0 + j * groups < (uint32_t)DOT_THREADS) ls[(t0 + j * groups) * M + m] = v[j];
         }
     }
-    __syncthreads();
-    // the butterfly of wave_sum, as pairs: s[l] = s[l] + s[l + off] for l < off
-    for (uint32_t off = WAVE / 2; off > 0; off >>= 1) {
-        const uint32_t work = (DOT_THREADS / WAVE) * off * M;
-        for (uint32_t e = u; e < work; e += DOT_THREADS) {
-            const uint32_t m = e % M, rest = e / M, l = rest % off, w = rest / off;
-            const uint32_t t = w * WAVE + l;
-            ls[t * M + m] = ls[t * M + m] + ls[(t + off) * M + m];
-        }
-        __syncthreads();
-    }
-    for (uint32_t m = u; m < M; m += DOT_THREADS) {
-        double s = 0.0;
-        for (int w = 0; w < DOT_THREADS / WAVE; ++w) s = s + ls[(size_t)w * WAVE * M + m];
-        partials[(size_t)blockIdx.x * M + m] = s;
-    }
+    reduce_slots(ls, M, partials);
 }
 
 // What a batched final sum feeds, per column: STORE writes the column's `out` field (`field` is a
@@ -674,15 +889,138 @@ __global__ __launch_bounds__(DOT_THREADS) void dot_partials_batch_kernel(size_t 
 // `mask` entry is zero are left as they are.
 static __global__ __launch_bounds__(DOT_THREADS) void dot_final_batch_kernel(int parts, uint32_t M, const double *__restrict__ partials,
                                                                              int kind, uint32_t field, PcgScalars *s,
-                                                                             const uint32_t *__restrict__ mask) {
+                                                                             const uint32_t *__restrict__ mask, PcgScalars *mirror,
+                                                                             uint32_t tag) {
     const uint32_t m = blockIdx.x;
     double v = 0.0;
     for (int i = threadIdx.x; i < parts; i += blockDim.x) v = v + partials[(size_t)i * M + m];
     const double total = block_sum(v);
-    if (threadIdx.x == 0 && (!mask || mask[m])) {
+    if (threadIdx.x == 0) {
         PcgScalars *c = s + m;
-        if (kind == FINAL_STORE) *(double *)((char *)c + field) = total;
-        else dot_finish(FINAL_RZ, total, nullptr, c);
+        if (!mask || mask[m]) {
+            if (kind == FINAL_STORE) *(double *)((char *)c + field) = total;
+            else dot_finish(FINAL_RZ, total, nullptr, c);
+        }
+        // a column's scalars for the host, as dot_final_kernel's
+        if (mirror) mirror_scalars(c, mirror + m, tag);
+    }
+}
+
+// The scalars of all M columns for the host (the serial order's readback).
+static __global__ void mirror_columns_kernel(uint32_t M, const PcgScalars *s, PcgScalars *mirror, uint32_t tag) {
+    const uint32_t m = threadIdx.x;
+    if (m < M) mirror_scalars(s + m, mirror + m, tag);
+}
+
+// For few columns, the final sums formed by every block of the kernel that uses them, as tree_total
+// does for one: a launch less each. FUSED_COLUMNS: each block reads every column's 512 partials, which
+// costs more than the launch it saves from about nine columns on.
+constexpr uint32_t FUSED_COLUMNS = 8;
+__device__ __forceinline__ void tree_totals(uint32_t M, const double *__restrict__ partials, double (&totals)[FUSED_COLUMNS]) {
+    __shared__ double wsum[FUSED_COLUMNS][DOT_THREADS / WAVE];
+    for (uint32_t m = 0; m < M; ++m) {
+        double v = 0.0;
+        for (uint32_t i = threadIdx.x; i < (uint32_t)DOT_BLOCKS; i += DOT_THREADS) v = v + partials[(size_t)i * M + m];
+        v = wave_sum(v);
+        if (threadIdx.x % WAVE == 0) wsum[m][threadIdx.x / WAVE] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < M) {
+        double t = 0.0;
+        for (int w = 0; w < DOT_THREADS / WAVE; ++w) t = t + wsum[threadIdx.x][w];
+        totals[threadIdx.x] = t;
+    }
+    __syncthreads();
+}
+
+// pcg_update_fused_kernel for M <= FUSED_COLUMNS columns: p . A p from its partials, the update of
+// pcg_update_batch_kernel, and the partials of the new r . r over dot_partials_batch_kernel's slots.
+static __global__ __launch_bounds__(DOT_THREADS) void pcg_update_fused_batch_kernel(size_t n, uint32_t M, PcgScalars *__restrict__ s, uint32_t slot,
+                                                                                    const uint32_t *__restrict__ active,
+                                                                                    const double *__restrict__ pap_partials,
+                                                                                    const double *__restrict__ p,
+                                                                                    const double *__restrict__ ap, double *__restrict__ x,
+                                                                                    double *__restrict__ r, double *__restrict__ rr_partials) {
+    extern __shared__ double ls[];  // DOT_THREADS x M
+    __shared__ double totals[FUSED_COLUMNS];
+    tree_totals(M, pap_partials, totals);
+    const uint32_t u = threadIdx.x, groups = DOT_THREADS / M, m = u % M;
+    const double curvature = totals[m], rz = rz_in(s + m, slot);
+    const bool live_column = active[m] != 0;
+    const bool valid = !(isnan(curvature) || curvature <= 0.0 || !isfinite(rz));
+    const double alpha = rz / curvature;
+    if (blockIdx.x == 0 && u < M) {
+        s[m].curvature = curvature;
+        if (live_column) {
+            s[m].valid = valid ? 1 : 0;
+            s[m].alpha = alpha;
+        }
+    }
+    const bool moves = live_column && valid;
+    const size_t stride = (size_t)gridDim.x * DOT_THREADS;
+    if (u < groups * M) {
+        for (uint32_t t0 = u / M; t0 < (uint32_t)DOT_THREADS; t0 += DOT_CHUNK * groups) {
+            double v[DOT_CHUNK];
+#pragma unroll
+            for (int j = 0; j < DOT_CHUNK; ++j) v[j] = 0.0;
+            for (size_t base = (size_t)blockIdx.x * DOT_THREADS; base < n; base += stride) {
+                double rv[DOT_CHUNK], xv[DOT_CHUNK], pv[DOT_CHUNK], av[DOT_CHUNK];
+#pragma unroll
+                for (int j = 0; j < DOT_CHUNK; ++j) {
+                    const size_t i = base + t0 + (size_t)j * groups;
+                    if (t0 + j * groups < (uint32_t)DOT_THREADS && i < n) {
+                        rv[j] = r[i * M + m];
+                        if (moves) {
+                            xv[j] = x[i * M + m];
+                            pv[j] = p[i * M + m];
+                            av[j] = ap[i * M + m];
+                        }
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < DOT_CHUNK; ++j) {
+                    const size_t i = base + t0 + (size_t)j * groups;
+                    if (t0 + j * groups < (uint32_t)DOT_THREADS && i < n) {
+                        if (moves) {
+                            x[i * M + m] = xv[j] + alpha * pv[j];
+                            rv[j] = rv[j] + (-alpha) * av[j];
+                            r[i * M + m] = rv[j];
+                        }
+                        v[j] = v[j] + rv[j] * rv[j];
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < DOT_CHUNK; ++j)
+                if (t0 + j * groups < (uint32_t)DOT_THREADS) ls[(t0 + j * groups) * M + m] = v[j];
+        }
+    }
+    reduce_slots(ls, M, rr_partials);
+}
+
+// pcg_direction_fused_kernel for M <= FUSED_COLUMNS columns: r . z from its partials, beta, then
+// p = z + beta p in the active columns. Block 0 stores the next r . z in the other slot.
+static __global__ __launch_bounds__(DOT_THREADS) void pcg_direction_fused_batch_kernel(size_t n, uint32_t M, PcgScalars *__restrict__ s,
+                                                                                       uint32_t slot, const uint32_t *__restrict__ active,
+                                                                                       const double *__restrict__ rz_partials,
+                                                                                       const double *__restrict__ z, double *__restrict__ p) {
+    __shared__ double totals[FUSED_COLUMNS];
+    __shared__ double betas[FUSED_COLUMNS];
+    tree_totals(M, rz_partials, totals);
+    if (threadIdx.x < M) {
+        const uint32_t m = threadIdx.x;
+        const double beta = totals[m] / rz_in(s + m, slot);
+        betas[m] = beta;
+        if (blockIdx.x == 0 && active[m]) {
+            rz_in(s + m, slot ^ 1u) = totals[m];
+            s[m].beta = beta;
+        }
+    }
+    __syncthreads();
+    const size_t stride = (size_t)gridDim.x * DOT_THREADS;
+    for (size_t e = (size_t)blockIdx.x * DOT_THREADS + threadIdx.x; e < n * M; e += stride) {
+        const uint32_t m = (uint32_t)(e % M);
+        if (active[m]) p[e] = z[e] + betas[m] * p[e];
     }
 }
 

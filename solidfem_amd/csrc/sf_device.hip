@@ -789,10 +789,23 @@ class Hierarchy final : public DeviceMultigrid {
         if constexpr (std::is_same<V, double>::value) {
             cycle_batch(0, r, z, columns, s);
         } else {
-            const size_t n = lv_[0].n * (size_t)columns;
-            hipLaunchKernelGGL((convert_kernel<V, double>), dim3(grid_for(n, 256)), dim3(256), 0, s, n, r, min_.ptr);
-            cycle_batch(0, min_.ptr, mout_.ptr, columns, s);
-            hipLaunchKernelGGL((convert_kernel<double, V>), dim3(grid_for(n, 256)), dim3(256), 0, s, n, (const V *)mout_.ptr, z);
+            LevelDev<S, V> &d = lv_[0];
+            const size_t n = d.n * (size_t)columns;
+            if (d.has_p) {
+                // the rounding in with the first start, the widening out with the last step, as launch_apply
+                const unsigned g = grid_for(d.rows * (size_t)columns, 256);
+                if (d.rb == 3)
+                    hipLaunchKernelGGL((convert_start_batch_kernel<3, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, columns, r, min_.ptr,
+                                       d.dinv.ptr, (V)d.theta, d.md0.ptr, mout_.ptr);
+                else
+                    hipLaunchKernelGGL((convert_start_batch_kernel<6, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, columns, r, min_.ptr,
+                                       d.dinv.ptr, (V)d.theta, d.md0.ptr, mout_.ptr);
+                cycle_batch(0, min_.ptr, mout_.ptr, columns, s, true, z);
+            } else {
+                hipLaunchKernelGGL((convert_kernel<V, double>), dim3(grid_for(n, 256)), dim3(256), 0, s, n, r, min_.ptr);
+                cycle_batch(0, min_.ptr, mout_.ptr, columns, s);
+                hipLaunchKernelGGL((convert_kernel<double, V>), dim3(grid_for(n, 256)), dim3(256), 0, s, n, (const V *)mout_.ptr, z);
+            }
         }
         SF_HIP(hipGetLastError());
     }
@@ -848,43 +861,74 @@ class Hierarchy final : public DeviceMultigrid {
 
     template <int RB, int BATCH, int CPL>
     static void cheb_batch_launch(LevelDev<S, V> &d, uint32_t M, const V *d_in, const V *r_in, V keep, V stp, V *d_out,
-                                  V *r_out, V *x, V *into, hipStream_t s, bool node) {
+                                  V *r_out, V *x, V *into, hipStream_t s, bool node, double *widen) {
         if (node) {
             const size_t threads = (size_t)d.a.slices * Shape<RB>::NPW * WAVE;
             hipLaunchKernelGGL((cheb_step_node_kernel<RB, BATCH, S, V>), dim3(grid_for(threads, 256)), dim3(256), 0, s, d.a.batch_view(), M,
-                               d.dinv.ptr, d_in, r_in, keep, stp, d_out, r_out, x, into);
+                               d.dinv.ptr, d_in, r_in, keep, stp, d_out, r_out, x, into, widen);
             return;
         }
         const int lg = columns_log2((M + CPL - 1) / CPL);
         const size_t threads = (size_t)d.a.slices * Shape<RB>::NPW << lg;
         hipLaunchKernelGGL((cheb_step_batch_kernel<RB, BATCH, S, V, CPL>), dim3(grid_for(threads, 256)), dim3(256), 0, s, d.a.batch_view(),
-                           lg, M, d.dinv.ptr, d_in, r_in, keep, stp, d_out, r_out, x, into);
+                           lg, M, d.dinv.ptr, d_in, r_in, keep, stp, d_out, r_out, x, into, widen);
     }
     template <int RB, int CPL>
     static void cheb_batch_depth(LevelDev<S, V> &d, int depth, uint32_t M, const V *d_in, const V *r_in, V keep, V stp,
-                                 V *d_out, V *r_out, V *x, V *into, hipStream_t s, bool node) {
+                                 V *d_out, V *r_out, V *x, V *into, hipStream_t s, bool node, double *widen) {
         switch (depth) {
-            case 1: cheb_batch_launch<RB, 1, CPL>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node); break;
-            case 2: cheb_batch_launch<RB, 2, CPL>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node); break;
-            default: cheb_batch_launch<RB, 4, CPL>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node); break;
+            case 1: cheb_batch_launch<RB, 1, CPL>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node, widen); break;
+            case 2: cheb_batch_launch<RB, 2, CPL>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node, widen); break;
+            default: cheb_batch_launch<RB, 4, CPL>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node, widen); break;
         }
     }
     template <int RB>
     static void cheb_batch_rb(LevelDev<S, V> &d, int batch, uint32_t M, const V *d_in, const V *r_in, V keep, V stp,
-                              V *d_out, V *r_out, V *x, V *into, hipStream_t s) {
+                              V *d_out, V *r_out, V *x, V *into, hipStream_t s, double *widen) {
         const int depth = form_depth(batch);
         int cpl = form_columns(batch);
         if (M % (uint32_t)cpl) cpl = 1;
-        if (cpl == 8) cheb_batch_depth<RB, 8>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, false);
-        else if (cpl == 4) cheb_batch_depth<RB, 4>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, false);
-        else if (cpl == 2) cheb_batch_depth<RB, 2>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, false);
-        else cheb_batch_depth<RB, 1>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node_form(batch));
+        if (cpl == 8) cheb_batch_depth<RB, 8>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, false, widen);
+        else if (cpl == 4) cheb_batch_depth<RB, 4>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, false, widen);
+        else if (cpl == 2) cheb_batch_depth<RB, 2>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, false, widen);
+        else cheb_batch_depth<RB, 1>(d, depth, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, node_form(batch), widen);
     }
     static void launch_cheb_batch(LevelDev<S, V> &d, int batch, uint32_t M, const V *d_in, const V *r_in, V keep, V stp,
-                                  V *d_out, V *r_out, V *x, V *into, hipStream_t s) {
+                                  V *d_out, V *r_out, V *x, V *into, hipStream_t s, double *widen = nullptr) {
         if (d.a.slices == 0) return;
-        if (d.rb == 3) cheb_batch_rb<3>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s);
-        else cheb_batch_rb<6>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s);
+        if (batch > ROWS_BATCH_FORM) {
+            const int rpw = rows_batch_rows(batch, M);
+            if (M <= 4) cheb_rows_batch_rpw<4>(d, rpw, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+            else cheb_rows_batch_rpw<8>(d, rpw, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+        } else if (d.rb == 3) cheb_batch_rb<3>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+        else cheb_batch_rb<6>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+    }
+    template <int MM, int RPW>
+    static void cheb_rows_batch_launch(LevelDev<S, V> &d, uint32_t M, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out,
+                                       V *x, V *into, hipStream_t s, double *widen) {
+        hipLaunchKernelGGL((cheb_rows_batch_kernel<3, MM, RPW, S, V>), dim3((d.a_rows.rows + RPW - 1) / RPW), dim3(WAVE),
+                           ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, d.a_rows.view(), M, d.dinv.ptr, d_in,
+                           r_in, keep, stp, d_out, r_out, x, into, widen);
+    }
+    template <int MM>
+    static void cheb_rows_batch_rpw(LevelDev<S, V> &d, int rpw, uint32_t M, const V *d_in, const V *r_in, V keep, V stp, V *d_out,
+                                    V *r_out, V *x, V *into, hipStream_t s, double *widen) {
+        if (rpw == 4) cheb_rows_batch_launch<MM, 4>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+        else if (rpw == 2) cheb_rows_batch_launch<MM, 2>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+        else cheb_rows_batch_launch<MM, 1>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+    }
+    // Whether the forms by plain block rows are candidates for a level's steps and residuals.
+    static bool rows_batch_level(const LevelDev<S, V> &d, uint32_t M) { return d.rb == 3 && d.a_rows.rows && M <= ROWS_BATCH_COLUMNS; }
+    static std::vector<int> with_rows_batch(std::vector<int> forms, const LevelDev<S, V> &d, uint32_t M) {
+        if (rows_batch_level(d, M))
+            for (int f : rows_batch_forms()) forms.push_back(f);
+        return forms;
+    }
+    // res = b - A x for M columns, optionally with the start of the smoothing that follows.
+    static void residual_batch(LevelDev<S, V> &d, int form, uint32_t M, const V *x, const V *b, hipStream_t s,
+                               Start<S, V> st = {nullptr, (V)0, nullptr, nullptr}) {
+        if (form > ROWS_BATCH_FORM) launch_rows_batch<S, V>(d.a_rows, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
+        else launch_spmm<S, V>(d.a, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
     }
 
     // Sizes the column work vectors for M columns and tunes the batched kernels for M's group.
@@ -912,10 +956,10 @@ class Hierarchy final : public DeviceMultigrid {
             for (V *v : vs) SF_HIP(hipMemsetAsync(v, 0, need * sizeof(V), s));
             d.mm_depth[lg][0] = tune_batch(s, [&](int batch) {
                 launch_cheb_batch(d, batch, M, d.md0.ptr, d.mb.ptr, (V)0, (V)0, d.md1.ptr, d.mr0.ptr, d.mx.ptr, nullptr, s);
-            }, spmm_candidates(d.rb, d.rb, sizeof(S), M, false), "", "batch step " + group + shape_class(d.a) + vsize);
+            }, with_rows_batch(spmm_candidates(d.rb, d.rb, sizeof(S), M, false), d, M), "", "batch step " + group + shape_class(d.a) + vsize);
             d.mm_depth[lg][1] = tune_batch(s, [&](int batch) {
-                launch_spmm<S, V>(d.a, M, d.mx.ptr, d.mres.ptr, d.mb.ptr, EPI_RESIDUAL, s, batch);
-            }, spmm_candidates(d.rb, d.rb, sizeof(S), M, true, staged_candidate(d.a, M)), "",
+                residual_batch(d, batch, M, d.mx.ptr, d.mb.ptr, s);
+            }, with_rows_batch(spmm_candidates(d.rb, d.rb, sizeof(S), M, true, staged_candidate(d.a, M)), d, M), "",
                "batch residual " + group + shape_class(d.a) + vsize);
             if (d.has_p) {
                 LevelDev<S, V> &c = lv_[l + 1];
@@ -935,13 +979,16 @@ class Hierarchy final : public DeviceMultigrid {
         SF_HIP(hipStreamSynchronize(s));
     }
 
-    void smooth_batch(LevelDev<S, V> &d, const V *b, V *x, V *sum_into, uint32_t M, hipStream_t s) {
+    // smooth() for M columns.
+    void smooth_batch(LevelDev<S, V> &d, const V *b, V *x, V *sum_into, uint32_t M, hipStream_t s, bool started, double *widen = nullptr) {
         const int lg = columns_log2(M);
-        const unsigned g = grid_for(d.rows * (size_t)M, 256);
-        if (d.rb == 3)
-            hipLaunchKernelGGL((cheb_start_batch_kernel<3, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, M, d.dinv.ptr, b, (V)d.theta, d.md0.ptr, x);
-        else
-            hipLaunchKernelGGL((cheb_start_batch_kernel<6, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, M, d.dinv.ptr, b, (V)d.theta, d.md0.ptr, x);
+        if (!started) {
+            const unsigned g = grid_for(d.rows * (size_t)M, 256);
+            if (d.rb == 3)
+                hipLaunchKernelGGL((cheb_start_batch_kernel<3, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, M, d.dinv.ptr, b, (V)d.theta, d.md0.ptr, x);
+            else
+                hipLaunchKernelGGL((cheb_start_batch_kernel<6, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, M, d.dinv.ptr, b, (V)d.theta, d.md0.ptr, x);
+        }
         V *dd[2] = {d.md0.ptr, d.md1.ptr};
         V *rr[2] = {d.mr0.ptr, d.mr1.ptr};
         const size_t steps = d.steps.size();
@@ -958,17 +1005,20 @@ class Hierarchy final : public DeviceMultigrid {
             const V *d_in = dd[(k - 1) & 1];
             const V *r_in = k == 1 ? b : rr[(k - 1) & 1];
             const V keep = (V)d.steps[k - 1].first, stp = (V)d.steps[k - 1].second;
-            launch_cheb_batch(d, d.mm_depth[lg][0], M, d_in, r_in, keep, stp, dd[k & 1], rr[k & 1], x, k == steps ? sum_into : nullptr, s);
+            V *into = k == steps ? sum_into : nullptr;
+            launch_cheb_batch(d, d.mm_depth[lg][0], M, d_in, r_in, keep, stp, dd[k & 1], rr[k & 1], x, into, s, into ? widen : nullptr);
         }
         Profiler::get().end(3, token, s);
         if (steps == 0 && sum_into) {
             const size_t n = d.n * (size_t)M;
             hipLaunchKernelGGL((add_kernel<V>), dim3(grid_for(n, 256)), dim3(256), 0, s, n, sum_into, (const V *)x);
+            if (widen)
+                hipLaunchKernelGGL((convert_kernel<double, V>), dim3(grid_for(n, 256)), dim3(256), 0, s, n, (const V *)sum_into, widen);
         }
     }
 
     // cycle() for M columns.
-    void cycle_batch(size_t l, const V *b, V *x, uint32_t M, hipStream_t s) {
+    void cycle_batch(size_t l, const V *b, V *x, uint32_t M, hipStream_t s, bool started = false, double *widen = nullptr) {
         LevelDev<S, V> &d = lv_[l];
         const int lg = columns_log2(M);
         if (!d.has_p) {
@@ -982,18 +1032,21 @@ class Hierarchy final : public DeviceMultigrid {
                 else
                     launch_coarse_solve<V>(d.n, d.packed.ptr, b, x, M, s);
             } else {
-                smooth_batch(d, b, x, nullptr, M, s);
+                smooth_batch(d, b, x, nullptr, M, s, started);
             }
             return;
         }
         LevelDev<S, V> &c = lv_[l + 1];
-        smooth_batch(d, b, x, nullptr, M, s);
-        launch_spmm<S, V>(d.a, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, d.mm_depth[lg][1]);
-        launch_spmm<S, V>(d.r, M, d.mres.ptr, c.mb.ptr, nullptr, EPI_STORE, s, d.mm_depth[lg][2]);
-        cycle_batch(l + 1, c.mb.ptr, c.mx.ptr, M, s);
+        smooth_batch(d, b, x, nullptr, M, s, started);
+        residual_batch(d, d.mm_depth[lg][1], M, x, b, s);
+        // restriction and residual with the start of the smoothing that follows, as cycle()
+        const bool fuse = smooths_first(c);
+        const Start<S, V> first = {fuse ? c.dinv.ptr : nullptr, (V)c.theta, c.md0.ptr, c.mx.ptr};
+        launch_spmm<S, V>(d.r, M, d.mres.ptr, c.mb.ptr, nullptr, EPI_STORE, s, d.mm_depth[lg][2], first);
+        cycle_batch(l + 1, c.mb.ptr, c.mx.ptr, M, s, fuse);
         launch_spmm<S, V>(d.p, M, c.mx.ptr, x, nullptr, EPI_ADD, s, d.mm_depth[lg][3]);
-        launch_spmm<S, V>(d.a, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, d.mm_depth[lg][1]);
-        smooth_batch(d, d.mres.ptr, d.mpx.ptr, x, M, s);
+        residual_batch(d, d.mm_depth[lg][1], M, x, b, s, {d.dinv.ptr, (V)d.theta, d.md0.ptr, d.mpx.ptr});
+        smooth_batch(d, d.mres.ptr, d.mpx.ptr, x, M, s, true, widen);
     }
 
     template <int RB>

@@ -183,7 +183,16 @@ inline int columns_log2(uint32_t m) {
 // Y = A X for M row-interleaved columns (epilogue per dev::Epilogue), `batch` blocks in flight
 // (1, 2 or 4; 0 = the matrix's tuned depth for this column count).
 template <typename S, typename V>
-void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int batch = 0);
+void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int batch = 0,
+                 dev::Start<S, V> start = {nullptr, (V)0, nullptr, nullptr});
+// The forms of products and steps by plain 3 x 3 block rows for few columns (rows_sum_batch):
+// ROWS_BATCH_FORM + block rows per wavefront.
+constexpr int ROWS_BATCH_FORM = 112;
+constexpr uint32_t ROWS_BATCH_COLUMNS = 8;
+inline std::vector<int> rows_batch_forms() { return {ROWS_BATCH_FORM + 1, ROWS_BATCH_FORM + 2, ROWS_BATCH_FORM + 4}; }
+int rows_batch_rows(int form, uint32_t M);
+template <typename S, typename V>
+void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, dev::Start<S, V> start);
 // The batch depths worth trying for a matrix's batched product.
 // The variant codes a batched product (`product`) or Chebyshev step is timed over for M columns.
 std::vector<int> spmm_candidates(int rb, int cb, size_t value_size, uint32_t M, bool product = true, bool staged = false);
@@ -274,8 +283,10 @@ struct DeviceSystem {
     DeviceSliced<double> sliced;
     DeviceBsr<double> rows;  // a small system's pattern over `values`, for the row kernels
     int rows_form = 0;       // the product's form: 0 sliced, else of the row kernels (by timing)
-    // y = A x
+    mutable int rows_mm[8] = {-1, -1, -1, -1, -1, -1, -1, -1};  // the batched product's, per log2 of the column group (-1: not tuned)
+    // y = A x, and Y = A X for M row-interleaved columns
     void multiply(const double *x, double *y, hipStream_t s) const;
+    void multiply_batch(uint32_t M, const double *x, double *y, hipStream_t s) const;
     void upload_from_host(hipStream_t s);
     void build_from_device_values(hipStream_t s);
 };
@@ -369,7 +380,9 @@ class DevicePcgBatch {
     void initialise();
     void iterate();
     void precondition(const double *r, double *z);
-    void dot(const double *a, const double *b, size_t field, int kind, const uint32_t *mask, int mode = 0);
+    void dot(const double *a, const double *b, size_t field, int kind, const uint32_t *mask, int mode = 0,
+             dev::PcgScalars *mirror = nullptr, uint32_t tag = 0);
+    void wait_for_tag(uint32_t tag);
     void reset_direction(const uint32_t *mask);
     void upload_flags(uint32_t *device, const std::vector<uint32_t> &flags);
     const dev::PcgScalars *read_scalars();
@@ -386,11 +399,13 @@ class DevicePcgBatch {
     std::vector<Column> col_;
     DeviceBuffer<double> b_, x_, r_, z_, p_, ap_, tmp_, tmp2_, jacobi_, stage_;
     DeviceBuffer<dev::PcgScalars> scalars_;
-    DeviceBuffer<double> partials_;
+    DeviceBuffer<double> partials_, partials2_;
     DeviceBuffer<uint32_t> active_, mask_;
-    dev::PcgScalars *pinned_ = nullptr;
+    uint32_t rz_slot_ = 0;               // as DevicePcg's; stays 0 where the final sums have launches of their own
+    dev::PcgScalars *pinned_ = nullptr;  // fine-grained host memory the r.r kernel copies the columns' scalars into
+    dev::PcgScalars *mirror_ = nullptr;  // its device address
+    uint32_t readbacks_ = 0;             // tags of the copies so far
     uint32_t *pinned_flags_ = nullptr;
-    hipEvent_t copied_ = nullptr;
 };
 
 // ---- stress recovery --------------------------------------------------------------------------

@@ -1,0 +1,48 @@
+"""A small system's finest level by plain block rows for few columns, on the GPU: every column is bit for
+bit the single-column V-cycle and solve, in each form, where the columns fill a wavefront's chains and
+where they leave some idle."""
+import numpy as np
+import pytest
+
+import refcpu
+import solidfem_amd as sf
+from workloads import FINGERPRINT_PLATE, loaded
+
+pytestmark = pytest.mark.gpu
+
+ROWS_BATCH_FORM = 112
+
+
+def bits(a):
+    return np.ascontiguousarray(a, dtype=np.float64).view(np.uint64)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4])
+@pytest.mark.parametrize("precision", [0, 1, 2], ids=["double", "single-storage", "single"])
+def test_few_columns_by_rows_keep_each_columns_bits(ctx, forced_variant, rows, precision):
+    ref = refcpu.Problem(loaded(*FINGERPRINT_PLATE[:2]))
+    csr = sf.CsrMatrix.new(ctx, *ref.csr())
+    setup = sf.MultigridSetup.new(ctx, csr, ref.rigid_modes(), ref.free_positions(),
+                                  sf.MultigridOptions(coarse_dofs=100, precision=precision, coarse_solve=1))
+    while not setup.step(2 ** 62):
+        pass
+    mg = setup.finish()
+    opts = sf.PcgOptions(tolerance=1e-8, dot_order=sf.DotOrder.TREE)
+    forced_variant(ROWS_BATCH_FORM + rows)
+    rng = np.random.default_rng(rows)
+    # groups of 1, 2, 4 and 8 columns (a choice each), 3, 5 and 7 in them, and 9: past the forms and
+    # past the final sums formed by their consumers
+    for columns in (1, 2, 3, 4, 5, 7, 8, 9):
+        r = rng.standard_normal((columns, ref.free_dofs))
+        z = mg.apply_batch(r)
+        for m in range(columns):
+            assert np.array_equal(bits(z[m]), bits(mg.apply(r[m]))), f"{columns} columns: column {m}"
+        if precision != 2 or columns not in (3, 8, 9):
+            continue
+        batch = sf.PcgBatch.new(ctx, csr, mg, r, opts)
+        assert batch.step(100000)[0] == 0
+        x = batch.estimate()
+        for m in range(columns):
+            single = sf.Pcg.new(ctx, csr, mg, r[m], opts)
+            single.step(100000)
+            assert np.array_equal(bits(single.estimate()), bits(x[m])), f"{columns} columns: column {m}"
