@@ -931,7 +931,7 @@ void sf_pcg_destroy(sf_pcg *pcg) { delete pcg; }
 
 sf_status sf_recover_stress(sf_context *ctx, const sf_model *model, const double *displacements, double *point_values,
                             double *nodal_values) {
-    return guard([&] { recover_stress(model->model, displacements, point_values, nodal_values, ctx->ctx->stream); });
+    return guard([&] { recover_stress(model->model, displacements, point_values, nodal_values, ctx->ctx.get(), ctx->ctx->stream); });
 }
 sf_status sf_static_study_recover(sf_static_study *study, double *point_values, double *nodal_values) {
     return guard([&] {
@@ -939,7 +939,7 @@ sf_status sf_static_study_recover(sf_static_study *study, double *point_values, 
         std::vector<double> u(3 * study->model.mesh.nodes.size());
         const sf_status st = sf_static_study_displacements(study, u.data());
         if (st != SF_OK) throw Error(st, "the study's displacements are not available");
-        recover_stress(study->model, u.data(), point_values, nodal_values, study->ctx->stream);
+        recover_stress(study->model, u.data(), point_values, nodal_values, study->ctx.get(), study->ctx->stream);
         study->report.recovery_seconds += seconds() - t0;
     });
 }
@@ -951,7 +951,7 @@ sf_status sf_recovery_create(sf_context *ctx, const sf_model *model, const doubl
             throw Error(SF_ERR_INVALID_ARGUMENT, "a recovery needs a context, a model and displacements");
         auto r = std::make_unique<sf_recovery>();
         r->ctx = ctx->ctx;
-        r->recovery = std::make_unique<DeviceRecovery>(model->model, displacements, converged != 0, ctx->ctx->stream);
+        r->recovery = std::make_unique<DeviceRecovery>(model->model, displacements, converged != 0, ctx->ctx.get(), ctx->ctx->stream);
         *out = r.release();
     });
 }
@@ -963,7 +963,7 @@ sf_status sf_static_study_begin_recovery(sf_static_study *study, sf_recovery **o
         if (st != SF_OK) throw Error(st, "the study's displacements are not available");
         auto r = std::make_unique<sf_recovery>();
         r->ctx = study->ctx;
-        r->recovery = std::make_unique<DeviceRecovery>(study->model, u.data(), study->pcg->pcg->converged(), study->ctx->stream);
+        r->recovery = std::make_unique<DeviceRecovery>(study->model, u.data(), study->pcg->pcg->converged(), study->ctx.get(), study->ctx->stream);
         *out = r.release();
     });
 }
@@ -1012,7 +1012,7 @@ sf_status sf_error_estimation_create(const sf_model *model, sf_recovery *recover
         if (!model || !recovery || !out) throw Error(SF_ERR_INVALID_ARGUMENT, "an error estimate needs a model and a recovery");
         auto e = std::make_unique<sf_error_estimation>();
         e->ctx = recovery->ctx;
-        e->estimation = std::make_unique<DeviceErrorEstimation>(model->model, *recovery->recovery, recovery->ctx->stream);
+        e->estimation = std::make_unique<DeviceErrorEstimation>(model->model, *recovery->recovery, recovery->ctx.get(), recovery->ctx->stream);
         *out = e.release();
     });
 }
@@ -1021,7 +1021,7 @@ sf_status sf_static_study_begin_error_estimate(const sf_static_study *study, sf_
         if (!study || !recovery || !out) throw Error(SF_ERR_INVALID_ARGUMENT, "an error estimate needs a study and a recovery");
         auto e = std::make_unique<sf_error_estimation>();
         e->ctx = recovery->ctx;
-        e->estimation = std::make_unique<DeviceErrorEstimation>(study->model, *recovery->recovery, recovery->ctx->stream);
+        e->estimation = std::make_unique<DeviceErrorEstimation>(study->model, *recovery->recovery, recovery->ctx.get(), recovery->ctx->stream);
         *out = e.release();
     });
 }

@@ -30,6 +30,67 @@ Context::~Context() {
         (void)hipStreamSynchronize(stream);
         (void)hipStreamDestroy(stream);
     }
+    for (int i = 0; i < 2; ++i) {
+        if (stage[i]) (void)hipHostFree(stage[i]);
+        if (stage_done[i]) (void)hipEventDestroy(stage_done[i]);
+    }
+}
+
+void Context::need_stage() {
+    for (int i = 0; i < 2; ++i) {
+        if (!stage[i]) SF_HIP(hipHostMalloc((void **)&stage[i], STAGE, hipHostMallocDefault));
+        if (!stage_done[i]) SF_HIP(hipEventCreateWithFlags(&stage_done[i], hipEventDisableTiming));
+    }
+}
+
+static void copy_on_pool(void *to, const void *from, size_t bytes) {
+    parallel_for(bytes, size_t(256) << 10, [&](size_t first, size_t last) {
+        std::memcpy((unsigned char *)to + first, (const unsigned char *)from + first, last - first);
+    });
+}
+
+void staged_download(Context *ctx, void *host, const void *device, size_t bytes, hipStream_t s) {
+    std::unique_lock<std::mutex> hold;
+    if (ctx && bytes > Context::STAGE) hold = std::unique_lock<std::mutex>(ctx->stage_lock, std::try_to_lock);
+    if (!hold.owns_lock()) {
+        if (bytes) SF_HIP(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, s));
+        SF_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    ctx->need_stage();
+    const size_t pieces = (bytes + Context::STAGE - 1) / Context::STAGE;
+    auto size_of = [&](size_t k) { return std::min(Context::STAGE, bytes - k * Context::STAGE); };
+    for (size_t k = 0; k <= pieces; ++k) {
+        // piece k is on its way while piece k - 1, arrived, is copied out; its buffer held piece k - 2
+        if (k < pieces) {
+            SF_HIP(hipMemcpyAsync(ctx->stage[k % 2], (const unsigned char *)device + k * Context::STAGE, size_of(k), hipMemcpyDeviceToHost, s));
+            SF_HIP(hipEventRecord(ctx->stage_done[k % 2], s));
+        }
+        if (k > 0) {
+            SF_HIP(hipEventSynchronize(ctx->stage_done[(k - 1) % 2]));
+            copy_on_pool((unsigned char *)host + (k - 1) * Context::STAGE, ctx->stage[(k - 1) % 2], size_of(k - 1));
+        }
+    }
+}
+
+void staged_upload_bytes(Context *ctx, void *device, const void *host, size_t bytes, hipStream_t s) {
+    std::unique_lock<std::mutex> hold;
+    if (ctx && bytes > Context::STAGE) hold = std::unique_lock<std::mutex>(ctx->stage_lock, std::try_to_lock);
+    if (!hold.owns_lock()) {
+        if (bytes) SF_HIP(hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, s));
+        SF_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    ctx->need_stage();
+    const size_t pieces = (bytes + Context::STAGE - 1) / Context::STAGE;
+    for (size_t k = 0; k < pieces; ++k) {
+        if (k >= 2) SF_HIP(hipEventSynchronize(ctx->stage_done[k % 2]));  // piece k - 2 has left this buffer
+        const size_t n = std::min(Context::STAGE, bytes - k * Context::STAGE);
+        copy_on_pool(ctx->stage[k % 2], (const unsigned char *)host + k * Context::STAGE, n);
+        SF_HIP(hipMemcpyAsync((unsigned char *)device + k * Context::STAGE, ctx->stage[k % 2], n, hipMemcpyHostToDevice, s));
+        SF_HIP(hipEventRecord(ctx->stage_done[k % 2], s));
+    }
+    SF_HIP(hipStreamSynchronize(s));
 }
 
 template <typename T>

@@ -4,6 +4,7 @@
 
 #include <cmath>
 #include <functional>
+#include <mutex>
 #include <string>
 
 #include "sf_host.hpp"
@@ -17,7 +18,25 @@ struct Context {
     hipStream_t stream = nullptr;
     explicit Context(int dev);
     ~Context();
+    // Two pinned buffers for staged copies, allocated on first use and freed with the context; one copy
+    // at a time holds them.
+    static constexpr size_t STAGE = size_t(4) << 20;
+    std::mutex stage_lock;
+    unsigned char *stage[2] = {nullptr, nullptr};
+    hipEvent_t stage_done[2] = {nullptr, nullptr};
+    void need_stage();
 };
+// Large copies between host arrays and the device through the context's pinned buffers: the host pool
+// copies one piece (and takes the page faults of a fresh array) while the next is on its way. 49 MB to a
+// fresh host array took 4.5 ms in one hipMemcpy. Small copies, and any while another thread's copy
+// holds the buffers (or without a context), are plain ones. The copy is done on return.
+void staged_download(Context *ctx, void *host, const void *device, size_t bytes, hipStream_t s);
+void staged_upload_bytes(Context *ctx, void *device, const void *host, size_t bytes, hipStream_t s);
+template <typename T>
+void staged_upload(Context *ctx, DeviceBuffer<T> &to, const T *host, size_t n, hipStream_t s) {
+    if (n > to.count) to.resize(n);
+    staged_upload_bytes(ctx, to.ptr, host, n * sizeof(T), s);
+}
 
 // The row order and slot layout of a sliced matrix, planned on the host.
 struct SlicedPlan {
@@ -420,7 +439,8 @@ class DevicePcgBatch {
 // mesh node 7 -- the recovered stress and its von Mises.
 class DeviceRecovery {
    public:
-    DeviceRecovery(const Model &model, const double *u, bool converged, hipStream_t s);
+    // `ctx` (may be null) lends its staging to the large copies, for as long as the recovery lives.
+    DeviceRecovery(const Model &model, const double *u, bool converged, Context *ctx, hipStream_t s);
     // Up to `max_work` more units (an element, then a vertex's patch fit); `cancel` (may be empty)
     // is read before each. Returns whether every unit is done. A cancel throws
     // SF_ERR_MODEL_CANCELLED with the units before it done; a faulting element throws with its
@@ -443,10 +463,14 @@ class DeviceRecovery {
     const double *device_fits() const { return fit_.ptr; }
 
    private:
+    void build_incidence(const QuadMesh &mesh);
     void run_elements(size_t count);
     void run_fits(size_t count);
     void ensure_worst();
+    // a vertex's elements start where its slots do, unless the host built the lists
+    const uint32_t *vertex_starts() const { return vstart_.ptr ? vstart_.ptr : nstart_.ptr; }
 
+    Context *ctx_;
     hipStream_t s_;
     size_t elements_, nodes_, vertices_;
     int nq_;
@@ -468,7 +492,7 @@ class DeviceRecovery {
 // device; the running sums in element order on the host, so any slicing gives one run's bits.
 class DeviceErrorEstimation {
    public:
-    DeviceErrorEstimation(const Model &model, DeviceRecovery &recovery, hipStream_t s);
+    DeviceErrorEstimation(const Model &model, DeviceRecovery &recovery, Context *ctx, hipStream_t s);
     // Up to `max_elements` more elements, `cancel` (may be empty) read before each; whether every
     // element is done. Refuses a recovery of another mesh (SF_ERR_MODEL_RECOVERY_MESH_MISMATCH),
     // an unfinished or preview one (SF_ERR_MODEL_NOT_FINISHED); a cancel throws
@@ -499,7 +523,7 @@ class DeviceErrorEstimation {
 };
 
 // The whole recovery in one call; either output may be null.
-void recover_stress(const Model &model, const double *u, double *point_values, double *nodal_values, hipStream_t s);
+void recover_stress(const Model &model, const double *u, double *point_values, double *nodal_values, Context *ctx, hipStream_t s);
 
 // nodal_rotations (results.rs:262-305): half the curl of the displacement at every mesh node, the
 // element values at the node weighted by their Jacobian determinants and summed in element order.
