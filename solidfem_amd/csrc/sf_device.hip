@@ -725,15 +725,17 @@ class Hierarchy final : public DeviceMultigrid {
                     for (size_t i = 0; i < n; ++i) identity[i * n + i] = 1.0;
                     linv.upload(identity, s);
                     d.inverse.resize(n * n);
-                    for (size_t k = 0; k < n; ++k) {
-                        hipLaunchKernelGGL(factor_inverse_finish_row_kernel, dim3(grid_for(k + 1, 256)), dim3(256), 0, s, (uint32_t)n,
-                                           (uint32_t)k, (const double *)lt.ptr, linv.ptr);
-                        if (k + 1 < n)
-                            hipLaunchKernelGGL(factor_inverse_update_kernel, dim3(grid_for(k + 1, 256), (unsigned)(n - k - 1)), dim3(256), 0,
-                                               s, (uint32_t)n, (uint32_t)k, (const double *)lt.ptr, linv.ptr);
+                    const unsigned tiles = (unsigned)((n + DENSE_PANEL - 1) / DENSE_PANEL);
+                    for (uint32_t k0 = 0; k0 < n; k0 += DENSE_PANEL) {
+                        const uint32_t w = std::min<uint32_t>(DENSE_PANEL, (uint32_t)n - k0), below = (uint32_t)n - k0 - w;
+                        hipLaunchKernelGGL(factor_inverse_panel_kernel, dim3(grid_for(k0 + w, 64)), dim3(64), 0, s, (uint32_t)n, k0, w,
+                                           (const double *)lt.ptr, linv.ptr);
+                        if (below)
+                            hipLaunchKernelGGL(factor_inverse_trailing_kernel, dim3(grid_for(k0 + w, DENSE_PANEL), grid_for(below, DENSE_PANEL)),
+                                               dim3(256), 0, s, (uint32_t)n, k0, w, (const double *)lt.ptr, linv.ptr);
                     }
-                    hipLaunchKernelGGL(factor_inverse_entries_kernel, dim3(grid_for(n * n, 256)), dim3(256), 0, s, (uint32_t)n,
-                                       (const double *)linv.ptr, d.inverse.ptr);
+                    hipLaunchKernelGGL(factor_inverse_entries_kernel, dim3(tiles, tiles), dim3(256), 0, s, (uint32_t)n, (const double *)linv.ptr,
+                                       d.inverse.ptr);
                     SF_HIP(hipGetLastError());
                     SF_HIP(hipStreamSynchronize(s));  // lt and linv are freed on return
                 }

@@ -843,50 +843,95 @@ __global__ __launch_bounds__(COARSE_THREADS) void coarse_solve_kernel(uint32_t n
     for (uint32_t i = t; i < n; i += COARSE_THREADS) out[(size_t)i * stride] = (V)xs[i];
 }
 
-// The coarsest level's solve as a product with the f64 inverse (stored by columns: inv[k n + i]
-// is entry (i, k)), the right-hand side widened from V and staged through LDS, each row summed
-// in ascending k from zero: a fixed order, so the same bits on every run.
 // The explicit inverse of a coarse factor, L^-T L^-1. First linv = L^-1 by forward substitution
-// for all columns at once, one step per row k: row k is finished (divided by L[k][k]), then every
-// later row i takes the term L[i][k] linv[k][j] off its entries j <= k. Entry (i, j) thus computes
-// ((i == j) - sum over k from j to i - 1 of L[i][k] linv[k][j], subtracted in ascending k) /
-// L[i][i]; `lt` holds L by columns (lt[k n + i] = L[i][k]), linv starts as the identity. Then
-// entry (i, j) of the inverse = sum over k from max(i, j) of linv[k][i] linv[k][j], added in
-// ascending k from zero, stored at inv[j n + i] (the loads of each chunk of 16 terms are issued
-// before the terms are taken, in order).
-static __global__ void factor_inverse_finish_row_kernel(uint32_t n, uint32_t k, const double *__restrict__ lt, double *__restrict__ linv) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j > k) return;
-    linv[(size_t)k * n + j] = linv[(size_t)k * n + j] / lt[(size_t)k * n + k];
+// for all columns at once: row k is finished (divided by L[k][k]), then every later row i takes the
+// term L[i][k] linv[k][j] off its entries j <= k. Entry (i, j) thus computes ((i == j) - sum over k
+// from j to i - 1 of L[i][k] linv[k][j], subtracted in ascending k) / L[i][i]; `lt` holds L by columns
+// (lt[k n + i] = L[i][k]), linv starts as the identity. DENSE_PANEL rows are taken at a time: the
+// panel's own rows, one thread a column, then every later row takes the panel's terms in ascending k.
+// Then entry (i, j) of the inverse = sum over k from max(i, j) of linv[k][i] linv[k][j], added in
+// ascending k from zero, stored at inv[j n + i], by tiles staged through LDS; entries (i, j) and
+// (j, i) add the same products, so tiles on one side give both. A step per row took 2 n launches.
+constexpr uint32_t DENSE_PANEL = 32;  // columns or rows of a dense coarse level taken at a time
+static __global__ __launch_bounds__(64) void factor_inverse_panel_kernel(uint32_t n, uint32_t k0, uint32_t w, const double *__restrict__ lt,
+                                                                        double *__restrict__ linv) {
+    // d[k][r] = L[k0 + r][k0 + k]; past a last panel's w rows the identity, which leaves its zeros as they
+    // are, so that every step's loop is whole
+    __shared__ double d[DENSE_PANEL][DENSE_PANEL], v[DENSE_PANEL][64];
+    const uint32_t t = threadIdx.x;
+    for (uint32_t e = t; e < DENSE_PANEL * DENSE_PANEL; e += 64) {
+        const uint32_t k = e / DENSE_PANEL, r = e % DENSE_PANEL;
+        d[k][r] = r < k ? 0.0 : r < w ? lt[(size_t)(k0 + k) * n + k0 + r] : r == k ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    const uint32_t j = blockIdx.x * 64 + t;
+    if (j >= k0 + w) return;
+    // column j of the panel, in LDS: a loop short enough to stay in the instruction cache, where the
+    // unrolled one over registers (30 KB of instructions run once) took 70 us a panel. Where the column
+    // starts within the panel, the rows above its diagonal are zeros and stay so.
+    for (uint32_t r = 0; r < DENSE_PANEL; ++r) v[r][t] = r < w ? linv[(size_t)(k0 + r) * n + j] : 0.0;
+#pragma unroll 1
+    for (uint32_t k = 0; k < DENSE_PANEL; ++k) {
+        const double vk = v[k][t] / d[k][k];
+        v[k][t] = vk;
+#pragma unroll 4
+        for (uint32_t r = k + 1; r < DENSE_PANEL; ++r) v[r][t] = v[r][t] - d[k][r] * vk;
+    }
+    for (uint32_t r = 0; r < w; ++r) linv[(size_t)(k0 + r) * n + j] = v[r][t];
 }
-static __global__ void factor_inverse_update_kernel(uint32_t n, uint32_t k, const double *__restrict__ lt, double *__restrict__ linv) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x, i = k + 1 + blockIdx.y;
-    if (j > k || i >= n) return;
-    linv[(size_t)i * n + j] -= lt[(size_t)k * n + i] * linv[(size_t)k * n + j];
+static __global__ __launch_bounds__(256) void factor_inverse_trailing_kernel(uint32_t n, uint32_t k0, uint32_t w, const double *__restrict__ lt,
+                                                                            double *__restrict__ linv) {
+    __shared__ double l[DENSE_PANEL][DENSE_PANEL], x[DENSE_PANEL][DENSE_PANEL];  // by k
+    const uint32_t t = threadIdx.x, i0 = k0 + w + blockIdx.y * DENSE_PANEL, j0 = blockIdx.x * DENSE_PANEL;
+    for (uint32_t e = t; e < w * DENSE_PANEL; e += 256) {
+        const uint32_t k = e / DENSE_PANEL, c = e % DENSE_PANEL;
+        l[k][c] = i0 + c < n ? lt[(size_t)(k0 + k) * n + i0 + c] : 0.0;
+        x[k][c] = j0 + c < k0 + w ? linv[(size_t)(k0 + k) * n + j0 + c] : 0.0;
+    }
+    __syncthreads();
+    for (uint32_t e = t; e < DENSE_PANEL * DENSE_PANEL; e += 256) {
+        const uint32_t r = e / DENSE_PANEL, c = e % DENSE_PANEL, i = i0 + r, j = j0 + c;
+        if (i >= n || j >= k0 + w) continue;
+        double v = linv[(size_t)i * n + j];
+        for (uint32_t k = j > k0 ? j - k0 : 0; k < w; ++k) v = v - l[k][r] * x[k][c];  // j <= k0 + k
+        linv[(size_t)i * n + j] = v;
+    }
 }
 static __global__ __launch_bounds__(256) void factor_inverse_entries_kernel(uint32_t n, const double *__restrict__ linv,
                                                                            double *__restrict__ inv) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)n * n) return;
-    const uint32_t i = (uint32_t)(t % n), j = (uint32_t)(t / n);
-    constexpr uint32_t CHUNK = 16;
-    double v = 0.0;
-    uint32_t k = i > j ? i : j;
-    for (; k + CHUNK <= n; k += CHUNK) {
-        double p[CHUNK], q[CHUNK];
-#pragma unroll
-        for (uint32_t u = 0; u < CHUNK; ++u) {
-            p[u] = linv[(size_t)(k + u) * n + i];
-            q[u] = linv[(size_t)(k + u) * n + j];
+    if (blockIdx.x > blockIdx.y) return;  // j0 <= i0: the other side is its mirror
+    __shared__ double a[DENSE_PANEL][DENSE_PANEL], b[DENSE_PANEL][DENSE_PANEL];  // by k
+    const uint32_t t = threadIdx.x, i0 = blockIdx.y * DENSE_PANEL, j0 = blockIdx.x * DENSE_PANEL;
+    constexpr uint32_t PER = DENSE_PANEL * DENSE_PANEL / 256;
+    const uint32_t c = t % DENSE_PANEL, j = j0 + c;
+    double v[PER] = {};
+    for (uint32_t k0 = i0; k0 < n; k0 += DENSE_PANEL) {
+        for (uint32_t e = t; e < DENSE_PANEL * DENSE_PANEL; e += 256) {
+            const uint32_t k = e / DENSE_PANEL, r = e % DENSE_PANEL;
+            a[k][r] = k0 + k < n && i0 + r < n ? linv[(size_t)(k0 + k) * n + i0 + r] : 0.0;
+            b[k][r] = k0 + k < n && j0 + r < n ? linv[(size_t)(k0 + k) * n + j0 + r] : 0.0;
         }
+        __syncthreads();
+        const uint32_t w = n - k0 < DENSE_PANEL ? n - k0 : DENSE_PANEL;
 #pragma unroll
-        for (uint32_t u = 0; u < CHUNK; ++u) v += p[u] * q[u];
+        for (uint32_t u = 0; u < PER; ++u) {
+            const uint32_t r = t / DENSE_PANEL + u * (256 / DENSE_PANEL), first = i0 + r > j ? i0 + r : j;
+            for (uint32_t k = first > k0 ? first - k0 : 0; k < w; ++k) v[u] = v[u] + a[k][r] * b[k][c];
+        }
+        __syncthreads();
     }
-    for (; k < n; ++k) v += linv[(size_t)k * n + i] * linv[(size_t)k * n + j];
-    inv[(size_t)j * n + i] = v;
+#pragma unroll
+    for (uint32_t u = 0; u < PER; ++u) {
+        const uint32_t i = i0 + t / DENSE_PANEL + u * (256 / DENSE_PANEL);
+        if (i < n && j < n) {
+            inv[(size_t)j * n + i] = v[u];
+            inv[(size_t)i * n + j] = v[u];
+        }
+    }
 }
 
-// out = inv b, R rows per workgroup. inv is symmetric bit for bit (entry (i, j) and entry (j, i) add
+// The coarsest level's solve as a product with the f64 inverse, the right-hand side widened from V:
+// out = inv b, COARSE_ROWS rows per workgroup. inv is symmetric bit for bit (entry (i, j) and entry (j, i) add
 // the same products in the same order), so a row's entries are read as its column's, contiguous. All
 // threads form a chunk of the rows' terms into LDS with every load in flight at once; then row r of 16
 // lanes of the first wavefront adds row r's terms in ascending k from zero. Bound by that chain of n

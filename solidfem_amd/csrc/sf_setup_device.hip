@@ -428,18 +428,75 @@ __global__ void seed_settle_kernel(u32 rows, const u32 *__restrict__ starts, con
 // of the host's column loop, whose bits it has. The diagonal a[k][k] is read by step k's division
 // and by nothing after, so the roots are stored at the end (the value under each root is kept for
 // the host's refusal of a matrix that is not positive definite).
-__global__ void cholesky_finish_column_kernel(u32 n, u32 k, double *__restrict__ a, double *__restrict__ pivots) {
-    const u32 i = k + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double s = a[(size_t)k * n + k];
-    if (i == k) pivots[k] = s;
-    else a[(size_t)i * n + k] = a[(size_t)i * n + k] / sqrt(s);
+//
+// Columns are taken dev::DENSE_PANEL at a time: their own triangle by one workgroup, then the rows below it,
+// one thread a row, then the trailing triangle, each entry taking the panel's terms in ascending k. An
+// entry still receives its subtractions one per k in ascending k and its division last. Three launches a
+// panel, where a step per column took two launches a column: bound by launches (n = 251: 502 launches of
+// 1.7 to 2.7 us, now 24).
+__global__ __launch_bounds__(256) void cholesky_triangle_kernel(u32 n, u32 k0, u32 w, double *__restrict__ a, double *__restrict__ pivots) {
+    __shared__ double d[dev::DENSE_PANEL][dev::DENSE_PANEL + 1];
+    const u32 t = threadIdx.x;
+    for (u32 e = t; e < w * w; e += 256) d[e / w][e % w] = a[(size_t)(k0 + e / w) * n + k0 + e % w];
+    __syncthreads();
+    for (u32 k = 0; k < w; ++k) {
+        const double s = d[k][k];
+        if (t > k && t < w) d[t][k] = d[t][k] / sqrt(s);
+        if (t == 0) pivots[k0 + k] = s;
+        __syncthreads();
+        const u32 rest = w - k - 1;
+        for (u32 e = t; e < rest * rest; e += 256) {
+            const u32 i = k + 1 + e / rest, j = k + 1 + e % rest;
+            if (j <= i) d[i][j] = d[i][j] - d[i][k] * d[j][k];
+        }
+        __syncthreads();
+    }
+    for (u32 e = t; e < w * w; e += 256)
+        if (e % w <= e / w) a[(size_t)(k0 + e / w) * n + k0 + e % w] = d[e / w][e % w];
 }
-
-__global__ void cholesky_update_kernel(u32 n, u32 k, double *__restrict__ a) {
-    const u32 j = k + 1 + blockIdx.x * blockDim.x + threadIdx.x, i = k + 1 + blockIdx.y;
-    if (i >= n || j > i) return;
-    a[(size_t)i * n + j] -= a[(size_t)i * n + k] * a[(size_t)j * n + k];
+__global__ __launch_bounds__(64) void cholesky_rows_kernel(u32 n, u32 k0, double *__restrict__ a) {
+    // the panel's triangle by columns, roots on the diagonal; rows are below a whole panel only (w =
+    // DENSE_PANEL: the last panel has none)
+    constexpr u32 W = dev::DENSE_PANEL;
+    __shared__ double d[W][W], r[W][64];
+    const u32 t = threadIdx.x;
+    for (u32 e = t; e < W * W; e += 64) {
+        const u32 i = e / W, j = e % W;
+        const double v = a[(size_t)(k0 + i) * n + k0 + j];
+        d[j][i] = i == j ? sqrt(v) : v;
+    }
+    __syncthreads();
+    const u32 i = k0 + W + blockIdx.x * 64 + t;
+    if (i >= n) return;
+    double *row = a + (size_t)i * n + k0;
+    // the row in LDS and a loop short enough to stay in the instruction cache (factor_inverse_panel_kernel)
+    for (u32 k = 0; k < W; ++k) r[k][t] = row[k];
+#pragma unroll 1
+    for (u32 k = 0; k < W; ++k) {
+        const double rk = r[k][t] / d[k][k];
+        r[k][t] = rk;
+#pragma unroll 4
+        for (u32 j = k + 1; j < W; ++j) r[j][t] = r[j][t] - rk * d[k][j];
+    }
+    for (u32 k = 0; k < W; ++k) row[k] = r[k][t];
+}
+__global__ __launch_bounds__(256) void cholesky_trailing_kernel(u32 n, u32 k0, u32 w, double *__restrict__ a) {
+    if (blockIdx.x > blockIdx.y) return;  // tiles on or below the diagonal
+    __shared__ double li[dev::DENSE_PANEL][dev::DENSE_PANEL + 1], lj[dev::DENSE_PANEL][dev::DENSE_PANEL + 1];
+    const u32 t = threadIdx.x, i0 = k0 + w + blockIdx.y * dev::DENSE_PANEL, j0 = k0 + w + blockIdx.x * dev::DENSE_PANEL;
+    for (u32 e = t; e < dev::DENSE_PANEL * w; e += 256) {
+        const u32 r = e / w, k = e % w;
+        li[r][k] = i0 + r < n ? a[(size_t)(i0 + r) * n + k0 + k] : 0.0;
+        lj[r][k] = j0 + r < n ? a[(size_t)(j0 + r) * n + k0 + k] : 0.0;
+    }
+    __syncthreads();
+    for (u32 e = t; e < dev::DENSE_PANEL * dev::DENSE_PANEL; e += 256) {
+        const u32 r = e / dev::DENSE_PANEL, c = e % dev::DENSE_PANEL, i = i0 + r, j = j0 + c;
+        if (i >= n || j > i) continue;
+        double v = a[(size_t)i * n + j];
+        for (u32 k = 0; k < w; ++k) v = v - li[r][k] * lj[c][k];
+        a[(size_t)i * n + j] = v;
+    }
 }
 
 __global__ void cholesky_diagonal_kernel(u32 n, const double *__restrict__ pivots, double *__restrict__ a) {
@@ -789,13 +846,14 @@ bool DeviceSetup::factor(int level, size_t n, double *a) {
     } guard{s};
     DeviceBuffer<double> d_a, d_pivots(n);
     d_a.upload(a, n * n, s);
-    for (size_t k = 0; k < n; ++k) {
-        const size_t rest = n - k;  // rows k .. n - 1
-        hipLaunchKernelGGL(cholesky_finish_column_kernel, dim3((unsigned)((rest + 255) / 256)), dim3(256), 0, s, (u32)n, (u32)k, d_a.ptr,
-                           d_pivots.ptr);
-        if (rest > 1)
-            hipLaunchKernelGGL(cholesky_update_kernel, dim3((unsigned)((rest - 1 + 255) / 256), (unsigned)(rest - 1)), dim3(256), 0, s,
-                               (u32)n, (u32)k, d_a.ptr);
+    for (size_t k0 = 0; k0 < n; k0 += dev::DENSE_PANEL) {
+        const u32 w = (u32)std::min<size_t>(dev::DENSE_PANEL, n - k0);
+        const size_t rest = n - k0 - w;  // rows below the panel's triangle
+        hipLaunchKernelGGL(cholesky_triangle_kernel, dim3(1), dim3(256), 0, s, (u32)n, (u32)k0, w, d_a.ptr, d_pivots.ptr);
+        if (rest == 0) break;
+        hipLaunchKernelGGL(cholesky_rows_kernel, dim3((unsigned)((rest + 63) / 64)), dim3(64), 0, s, (u32)n, (u32)k0, d_a.ptr);
+        const unsigned tiles = (unsigned)((rest + dev::DENSE_PANEL - 1) / dev::DENSE_PANEL);
+        hipLaunchKernelGGL(cholesky_trailing_kernel, dim3(tiles, tiles), dim3(256), 0, s, (u32)n, (u32)k0, w, d_a.ptr);
     }
     hipLaunchKernelGGL(cholesky_diagonal_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (u32)n, (const double *)d_pivots.ptr,
                        d_a.ptr);
