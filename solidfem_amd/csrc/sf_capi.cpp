@@ -52,12 +52,14 @@ sf_status guard(F &&f) {
 }
 
 // SF_SETUP_AUTO takes levels of at least this many block rows to the device
-// (SOLIDFEM_SETUP_MIN_ROWS overrides it, read once).
+// (SOLIDFEM_SETUP_MIN_ROWS overrides it, read once). A level of about 1000 rows takes 13.4 ms on the
+// host (its 20 power iterations 8.4, on one thread) and 4.4 ms on the device; one of 340 takes 2.5 ms
+// on the host, no more on the device.
 size_t device_setup_rows() {
     static const size_t rows = [] {
         const char *e = std::getenv("SOLIDFEM_SETUP_MIN_ROWS");
         const long v = e ? std::atol(e) : 0;
-        return v > 0 ? (size_t)v : (size_t)4096;
+        return v > 0 ? (size_t)v : (size_t)256;
     }();
     return rows;
 }
