@@ -812,7 +812,8 @@ sf_status sf_multigrid_apply(sf_multigrid *mg, const double *r, double *z) {
             mg->in.resize(std::max<size_t>(n, 1));
             mg->out.resize(std::max<size_t>(n, 1));
         }
-        mg->in.upload(r, n, s);
+        // one wait for all of it: the caller's array outlives the call, so the copy in needs none of its own
+        if (n) SF_HIP(hipMemcpyAsync(mg->in.ptr, r, n * sizeof(double), hipMemcpyHostToDevice, s));
         mg->mg->apply(mg->in.ptr, mg->out.ptr, s);
         mg->out.download(z, n, s);
         SF_HIP(hipStreamSynchronize(s));

@@ -763,6 +763,13 @@ class Hierarchy final : public DeviceMultigrid {
         for (auto &g : graphs_) drop_graph(g);
     }
 
+    void apply_after(const FinalSum &sum, const double *r, double *z, hipStream_t s) override {
+        // the sum rides on the cycle's first kernel, the start, unless a graph of the cycle is replayed
+        // or the cycle has no start
+        if (lv_.empty() || !lv_[0].has_p || (use_graph && !Profiler::get().any_on())) return DeviceMultigrid::apply_after(sum, r, z, s);
+        launch_apply(r, z, s, sum);
+    }
+
     void apply(const double *r, double *z, hipStream_t s) override {
         if (lv_.empty()) return;
         if (use_graph && !Profiler::get().any_on()) {
@@ -819,22 +826,23 @@ class Hierarchy final : public DeviceMultigrid {
         g.done = nullptr;
     }
 
-    void launch_apply(const double *r, double *z, hipStream_t s) {
+    void launch_apply(const double *r, double *z, hipStream_t s, const FinalSum &sum = {}) {
         if constexpr (std::is_same<V, double>::value) {
-            cycle(0, r, z, s);
+            if (lv_[0].has_p) launch_start(lv_[0], r, z, s, sum);
+            cycle(0, r, z, s, lv_[0].has_p);
         } else {
             LevelDev<S, V> &d = lv_[0];
             const size_t n = d.n;
             if (d.has_p) {
                 // the rounding in, fused with the first start; the widening out, fused with the
                 // last step
-                const unsigned g = grid_for(d.rows, 256);
+                const unsigned g = grid_for(d.rows, 256) + (sum.partials ? 1 : 0);
                 if (d.rb == 3)
                     hipLaunchKernelGGL((convert_start_kernel<3, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, r, in_.ptr,
-                                       d.dinv.ptr, (V)d.theta, d.d0.ptr, out_.ptr);
+                                       d.dinv.ptr, (V)d.theta, d.d0.ptr, out_.ptr, sum);
                 else
                     hipLaunchKernelGGL((convert_start_kernel<6, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, r, in_.ptr,
-                                       d.dinv.ptr, (V)d.theta, d.d0.ptr, out_.ptr);
+                                       d.dinv.ptr, (V)d.theta, d.d0.ptr, out_.ptr, sum);
                 cycle(0, in_.ptr, out_.ptr, s, true, z);
             } else {
                 hipLaunchKernelGGL((convert_kernel<V, double>), dim3(grid_for(n, 256)), dim3(256), 0, s, n, r, in_.ptr);
@@ -1174,12 +1182,12 @@ class Hierarchy final : public DeviceMultigrid {
     }
 
     // The Chebyshev start z = D^-1 b / theta, d = z, x = z (cycle.rs:578-590).
-    static void launch_start(LevelDev<S, V> &d, const V *b, V *x, hipStream_t s) {
-        const unsigned g = grid_for(d.n, 256);
+    static void launch_start(LevelDev<S, V> &d, const V *b, V *x, hipStream_t s, const FinalSum &sum = {}) {
+        const unsigned g = grid_for(d.n, 256) + (sum.partials ? 1 : 0);
         if (d.rb == 3)
-            hipLaunchKernelGGL((cheb_start_kernel<3, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, d.dinv.ptr, b, (V)d.theta, d.d0.ptr, x);
+            hipLaunchKernelGGL((cheb_start_kernel<3, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, d.dinv.ptr, b, (V)d.theta, d.d0.ptr, x, sum);
         else
-            hipLaunchKernelGGL((cheb_start_kernel<6, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, d.dinv.ptr, b, (V)d.theta, d.d0.ptr, x);
+            hipLaunchKernelGGL((cheb_start_kernel<6, S, V>), dim3(g), dim3(256), 0, s, (uint32_t)d.rows, d.dinv.ptr, b, (V)d.theta, d.d0.ptr, x, sum);
     }
 
     // c.b = P^T d.res, with the coarser level's first start in the epilogue when `fuse`.
@@ -1560,6 +1568,17 @@ PcgScalars DevicePcg::read_scalars() {
     return *pinned_;
 }
 
+static void launch_final_sum(const FinalSum &sum, hipStream_t s) {
+    hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(DOT_THREADS), 0, s, DOT_BLOCKS, sum.partials, (int)FINAL_STORE, sum.out, sum.s,
+                       sum.mirror, sum.tag);
+    SF_HIP(hipGetLastError());
+}
+
+void DeviceMultigrid::apply_after(const FinalSum &sum, const double *r, double *z, hipStream_t s) {
+    launch_final_sum(sum, s);
+    apply(r, z, s);
+}
+
 void DevicePcg::iterate() {
     // pcg.rs:216-275. The branch taken when the recursive residual is above the tolerance (the
     // preconditioner, r.z and the new direction) is enqueued before the residual is read back, so
@@ -1579,10 +1598,15 @@ void DevicePcg::iterate() {
         hipLaunchKernelGGL(pcg_update_fused_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, s, n_, sc, rz_slot_,
                            (const double *)partials_.ptr, (const double *)p_.ptr, (const double *)ap_.ptr, x_.ptr, r_.ptr,
                            partials2_.ptr);
-        // r.r's final sum also copies the scalars into host memory, tagged for this readback
-        hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(DOT_THREADS), 0, s, DOT_BLOCKS, (const double *)partials2_.ptr,
-                           (int)FINAL_STORE, &sc->rr, sc, mirror_, tag);
-        precondition(r_.ptr, z_.ptr);
+        // r.r's final sum also copies the scalars into host memory, tagged for this readback; it rides
+        // on the V-cycle's first kernel
+        const FinalSum rr = {partials2_.ptr, &sc->rr, sc, mirror_, tag};
+        if (mg_) {
+            mg_->apply_after(rr, r_.ptr, z_.ptr, s);
+        } else {
+            launch_final_sum(rr, s);
+            precondition(r_.ptr, z_.ptr);
+        }
         hipLaunchKernelGGL((dot_partials_kernel<0>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, s, n_, (const double *)r_.ptr,
                            (const double *)z_.ptr, partials_.ptr);
         hipLaunchKernelGGL(pcg_direction_fused_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, s, n_, sc, rz_slot_,

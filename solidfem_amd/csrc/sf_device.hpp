@@ -264,6 +264,8 @@ class DeviceMultigrid {
     virtual ~DeviceMultigrid() = default;
     // z = M^-1 r, device pointers, f64 in and out.
     virtual void apply(const double *r, double *z, hipStream_t s) = 0;
+    // The same after a solve's final sum, which may ride on the first kernel.
+    virtual void apply_after(const dev::FinalSum &sum, const double *r, double *z, hipStream_t s);
     // One smoother application on `level` from a zero guess (f64 device vectors in and out).
     virtual void smooth_level(size_t level, const double *b, double *x, hipStream_t s) = 0;
     virtual void coarse_solve(const double *b, double *x, hipStream_t s) = 0;

@@ -587,11 +587,99 @@ __global__ __launch_bounds__(256) void rounding_bound_kernel(Sliced<double> a, c
     out[(size_t)row * RB + p] = bound * bound;
 }
 
-// The Chebyshev start (cycle.rs:591-610): z = D^-1 b, d = z / theta, x = d.
+// Scalars of a solve, resident on the device.
+struct PcgScalars {
+    double rz;         // r . z
+    double curvature;  // p . A p
+    double rr;         // r . r (recursive residual)
+    double rz_next;
+    double true_rr;    // ||b - A x||^2
+    double bound2;     // sum of squared row rounding bounds
+    double alpha;
+    double beta;
+    int32_t valid;     // the curvature test of pcg.rs:219-227 passed
+    uint32_t tag;      // host copies only: which readback the copy answers, written last
+};
+
+// Copies the scalars to host memory for the host to read without an event: every field first,
+// then, after a system-scope fence, the tag the host waits for.
+__device__ __forceinline__ void mirror_scalars(const PcgScalars *s, PcgScalars *mirror, uint32_t tag) {
+    mirror->rz = s->rz;
+    mirror->curvature = s->curvature;
+    mirror->rr = s->rr;
+    mirror->rz_next = s->rz_next;
+    mirror->true_rr = s->true_rr;
+    mirror->bound2 = s->bound2;
+    mirror->alpha = s->alpha;
+    mirror->beta = s->beta;
+    mirror->valid = s->valid;
+    __threadfence_system();
+    __hip_atomic_store(&mirror->tag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Deterministic dot products. TREE order is a fixed two-stage reduction: DOT_BLOCKS blocks each
+// sum a fixed grid-stride pattern through a fixed shuffle tree into one partial, then one block
+// sums the partials in the same fixed pattern (a second kernel: no atomics and no fences; a
+// one-launch form whose last block finishes the sum measured slower, its per-block release fences
+// costing more than the launch they save).
+// REFERENCE order is one thread summing in index order from zero, exactly
+// crates/solidfem-solve/src/pcg.rs:285-291.
+constexpr int DOT_BLOCKS = 512;
+constexpr int DOT_THREADS = 256;
+
+__device__ __forceinline__ double wave_sum(double v) {
+    // fixed butterfly: the same pairs add in the same order on every run
+#pragma unroll
+    for (int off = WAVE / 2; off > 0; off >>= 1) v = v + __shfl_xor(v, off, WAVE);
+    return v;
+}
+
+__device__ __forceinline__ double block_sum(double v) {
+    __shared__ double wsum[DOT_THREADS / WAVE];
+    v = wave_sum(v);
+    if ((threadIdx.x % WAVE) == 0) wsum[threadIdx.x / WAVE] = v;
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < DOT_THREADS / WAVE; ++w) s = s + wsum[w];
+    return s;  // valid in thread 0
+}
+
+// The final sum of a TREE dot product left to a kernel that has nothing to do with it: its first
+// workgroup (of DOT_THREADS threads) forms the sum as dot_final_kernel does, stores it and copies the
+// scalars to the host, while the others do the kernel's own work. Null partials: no sum.
+struct FinalSum {
+    const double *partials;
+    double *out;
+    PcgScalars *s;
+    PcgScalars *mirror;
+    uint32_t tag;
+};
+// Whether this workgroup formed the sum (and has no other work); `block` is its number among the rest.
+__device__ __forceinline__ bool final_sum(const FinalSum &f, uint32_t &block) {
+    block = blockIdx.x;
+    if (!f.partials) return false;
+    if (blockIdx.x > 0) {
+        --block;
+        return false;
+    }
+    double v = 0.0;
+    for (int i = threadIdx.x; i < DOT_BLOCKS; i += DOT_THREADS) v = v + f.partials[i];
+    const double total = block_sum(v);
+    if (threadIdx.x == 0) {
+        *f.out = total;
+        if (f.mirror) mirror_scalars(f.s, f.mirror, f.tag);
+    }
+    return true;
+}
+
+// The Chebyshev start (cycle.rs:591-610): z = D^-1 b, d = z / theta, x = d; with a solve's r . r left to it.
 template <int RB, typename S, typename V>
 __global__ __launch_bounds__(256) void cheb_start_kernel(uint32_t rows, const S *__restrict__ dinv, const V *__restrict__ b,
-                                                         V theta, V *__restrict__ d, V *__restrict__ x) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                                         V theta, V *__restrict__ d, V *__restrict__ x, FinalSum sum) {
+    uint32_t block;
+    if (final_sum(sum, block)) return;
+    const size_t i = (size_t)block * blockDim.x + threadIdx.x;
     if (i >= (size_t)rows * RB) return;
     const size_t row = i / RB, p = i - row * RB;
     const S *dr = dinv + row * RB * RB + p * RB;
@@ -655,12 +743,15 @@ __global__ void add_kernel(size_t n, V *__restrict__ x, const V *__restrict__ y)
 }
 
 // The finest level's right-hand side rounded in from f64 (the conversion of cycle.rs:226-243)
-// and the Chebyshev start on it (cheb_start_kernel), one thread per block row.
+// and the Chebyshev start on it (cheb_start_kernel), one thread per block row; with a solve's r . r left
+// to it.
 template <int RB, typename S, typename V>
 __global__ __launch_bounds__(256) void convert_start_kernel(uint32_t rows, const double *__restrict__ r, V *__restrict__ b,
                                                             const S *__restrict__ dinv, V theta, V *__restrict__ d,
-                                                            V *__restrict__ x) {
-    const size_t row = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                                            V *__restrict__ x, FinalSum sum) {
+    uint32_t block;
+    if (final_sum(sum, block)) return;
+    const size_t row = (size_t)block * blockDim.x + threadIdx.x;
     if (row >= rows) return;
     V bv[RB];
 #pragma unroll
@@ -966,64 +1057,6 @@ __global__ __launch_bounds__(256) void coarse_inverse_kernel(uint32_t n, const d
 }
 
 // ---- conjugate gradient vectors -------------------------------------------------------------
-
-// Scalars of a solve, resident on the device.
-struct PcgScalars {
-    double rz;         // r . z
-    double curvature;  // p . A p
-    double rr;         // r . r (recursive residual)
-    double rz_next;
-    double true_rr;    // ||b - A x||^2
-    double bound2;     // sum of squared row rounding bounds
-    double alpha;
-    double beta;
-    int32_t valid;     // the curvature test of pcg.rs:219-227 passed
-    uint32_t tag;      // host copies only: which readback the copy answers, written last
-};
-
-// Copies the scalars to host memory for the host to read without an event: every field first,
-// then, after a system-scope fence, the tag the host waits for.
-__device__ __forceinline__ void mirror_scalars(const PcgScalars *s, PcgScalars *mirror, uint32_t tag) {
-    mirror->rz = s->rz;
-    mirror->curvature = s->curvature;
-    mirror->rr = s->rr;
-    mirror->rz_next = s->rz_next;
-    mirror->true_rr = s->true_rr;
-    mirror->bound2 = s->bound2;
-    mirror->alpha = s->alpha;
-    mirror->beta = s->beta;
-    mirror->valid = s->valid;
-    __threadfence_system();
-    __hip_atomic_store(&mirror->tag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// Deterministic dot products. TREE order is a fixed two-stage reduction: DOT_BLOCKS blocks each
-// sum a fixed grid-stride pattern through a fixed shuffle tree into one partial, then one block
-// sums the partials in the same fixed pattern (a second kernel: no atomics and no fences; a
-// one-launch form whose last block finishes the sum measured slower, its per-block release fences
-// costing more than the launch they save).
-// REFERENCE order is one thread summing in index order from zero, exactly
-// crates/solidfem-solve/src/pcg.rs:285-291.
-constexpr int DOT_BLOCKS = 512;
-constexpr int DOT_THREADS = 256;
-
-__device__ __forceinline__ double wave_sum(double v) {
-    // fixed butterfly: the same pairs add in the same order on every run
-#pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) v = v + __shfl_xor(v, off, WAVE);
-    return v;
-}
-
-__device__ __forceinline__ double block_sum(double v) {
-    __shared__ double wsum[DOT_THREADS / WAVE];
-    v = wave_sum(v);
-    if ((threadIdx.x % WAVE) == 0) wsum[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0)
-        for (int w = 0; w < DOT_THREADS / WAVE; ++w) s = s + wsum[w];
-    return s;  // valid in thread 0
-}
 
 // MODE 0: a . b; MODE 1: sum of a.
 template <int MODE>
