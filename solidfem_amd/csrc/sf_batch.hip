@@ -45,6 +45,7 @@ std::vector<int> spmm_candidates(int rb, int cb, size_t value_size, uint32_t M, 
         c.push_back(OCT_FORM + 2);
     }
     if (staged && product) c.push_back(STAGED_FORM);
+    if (rb == 3 && M <= FEW_COLUMNS) c.push_back(FEW_FORM);
     return c;
 }
 
@@ -92,7 +93,8 @@ static void spmm_shape(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, c
 template <int RB, int CB, typename S, typename V, typename UNIT, int CPL>
 static void spmm_staged_unit(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
     const uint32_t units = (uint32_t)(CB * M * sizeof(V) / sizeof(UNIT));
-    const size_t lds = 2 * (size_t)stage_chunk(units, STAGE_UNITS<UNIT, V>) * units * sizeof(UNIT);
+    const uint32_t chunk = stage_chunk(units, STAGE_UNITS<UNIT, V>, M, STAGE_BLOCKS<RB * CB, S>);
+    const size_t lds = 2 * (size_t)chunk * (units * sizeof(UNIT) + RB * CB * sizeof(S));
     hipLaunchKernelGGL((spmm_staged_kernel<RB, CB, S, V, UNIT, CPL>), dim3((unsigned)((size_t)a.slices * Shape<RB>::NPW)), dim3(256), lds, s,
                        a.batch_view(), M, epi, x, y, b, st);
 }
@@ -123,6 +125,19 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
             SF_HIP(hipStreamSynchronize(s));
         }
         batch = tuned;
+    }
+    if (batch >= FEW_FORM) {
+        if (a.rb == 3 && M <= FEW_COLUMNS) {
+            with_columns(M, [&](auto columns) {
+                constexpr int MM = decltype(columns)::value;
+                const dim3 grid(grid_for(a.slices, 4)), block(256);
+                if (a.cb == 3) hipLaunchKernelGGL((spmm_few_kernel<3, 3, MM, S, V>), grid, block, 0, s, a.view(), epi, x, y, b, st);
+                else hipLaunchKernelGGL((spmm_few_kernel<3, 6, MM, S, V>), grid, block, 0, s, a.view(), epi, x, y, b, st);
+            });
+            SF_HIP(hipGetLastError());
+            return;
+        }
+        batch = 4;
     }
     if (batch >= STAGED_FORM) {
         // the staged form where it fits, else one column and four blocks in flight per lane
@@ -161,28 +176,23 @@ template void launch_spmm<float, float>(const DeviceSliced<float> &, uint32_t, c
                                         hipStream_t, int, Start<float, float>);
 
 // Rows per wavefront of a rows form for M columns: its chains, 3 M a row, fit the 64 lanes.
-int rows_batch_rows(int form, uint32_t M) {
-    int rpw = form - ROWS_BATCH_FORM;
-    while (rpw > 1 && (uint32_t)rpw * 3 * M > (uint32_t)WAVE) rpw /= 2;
-    return rpw;
-}
-template <int MM, int RPW, typename S, typename V>
-static void rows_batch_launch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
-    hipLaunchKernelGGL((rows_batch_kernel<3, 3, MM, RPW, S, V>), dim3((a.rows + RPW - 1) / RPW), dim3(WAVE),
-                       ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, a.view(), M, epi, x, y, b, st);
-}
-template <int MM, typename S, typename V>
-static void rows_batch_rpw(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int rpw, Start<S, V> st) {
-    if (rpw == 4) rows_batch_launch<MM, 4>(a, M, x, y, b, epi, s, st);
-    else if (rpw == 2) rows_batch_launch<MM, 2>(a, M, x, y, b, epi, s, st);
-    else rows_batch_launch<MM, 1>(a, M, x, y, b, epi, s, st);
+int rows_batch_rows(int form, uint32_t M) { return form - ROWS_BATCH_FORM == 4 && 12 * M <= (uint32_t)WAVE ? 4 : 2; }
+template <int M, int RPW, typename S, typename V>
+static void rows_batch_launch(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
+    hipLaunchKernelGGL((rows_batch_kernel<3, 3, M, RPW, S, V>), dim3((a.rows + RPW - 1) / RPW), dim3(WAVE),
+                       ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, a.view(), epi, x, y, b, st);
 }
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, Start<S, V> st) {
     if (a.rows == 0 || M == 0) return;
-    if (a.rb != 3 || a.cb != 3 || M > ROWS_BATCH_COLUMNS) throw Error(SF_ERR_INTERNAL, "no rows form for this block shape or column count");
-    if (M <= 4) rows_batch_rpw<4>(a, M, x, y, b, epi, s, rows_batch_rows(form, M), st);
-    else rows_batch_rpw<8>(a, M, x, y, b, epi, s, rows_batch_rows(form, M), st);
+    if (a.rb != 3 || a.cb != 3 || M > FEW_COLUMNS) throw Error(SF_ERR_INTERNAL, "no rows form for this block shape or column count");
+    with_columns(M, [&](auto columns) {
+        constexpr int MM = decltype(columns)::value;
+        if constexpr (12 * MM <= WAVE) {
+            if (rows_batch_rows(form, M) == 4) return rows_batch_launch<MM, 4>(a, x, y, b, epi, s, st);
+        }
+        rows_batch_launch<MM, 2>(a, x, y, b, epi, s, st);
+    });
     SF_HIP(hipGetLastError());
 }
 template void launch_rows_batch<double, double>(const DeviceBsr<double> &, uint32_t, const double *, double *, const double *, int, hipStream_t, int,
@@ -195,7 +205,7 @@ template void launch_rows_batch<float, float>(const DeviceBsr<float> &, uint32_t
 void DeviceSystem::multiply_batch(uint32_t M, const double *x, double *y, hipStream_t s) const {
     // the form by rows is chosen per group of column counts, as the sliced product's is
     int &form = rows_mm[columns_log2(M)];
-    if (rows.rows == 0 || M > ROWS_BATCH_COLUMNS) form = 0;
+    if (rows.rows == 0 || M > FEW_COLUMNS) form = 0;
     else if (form < 0) {
         DeviceBuffer<double> tx(host.cols * 3 * M), ty(host.rows * 3 * M);
         SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));

@@ -220,6 +220,189 @@ __global__ __launch_bounds__(256) void spmm_kernel(Sliced<S> a, int log2g, uint3
     if (then.dinv) start_columns<RB, CPL, S, V>(then, row, m0, M, sum);
 }
 
+// ---- few columns: a lane per scalar row ----
+
+// The columns of a scalar row, read or written: a vector where the count is one's, else one by one. The
+// count is a compile-time one: with a test of each column against a count known only at run time the
+// loads waited on one another (62 us a step for 5 columns of 6480 rows).
+template <int MM, typename V>
+__device__ __forceinline__ void load_few(const V *p, V (&out)[MM]) {
+    if constexpr (MM == 2 || MM % 4 == 0) {
+        load_columns<MM, V>(p, out);
+    } else {
+#pragma unroll
+        for (int m = 0; m < MM; ++m) out[m] = p[m];
+    }
+}
+template <int MM, typename V>
+__device__ __forceinline__ void store_few(V *p, const V (&in)[MM]) {
+    if constexpr (MM == 2 || MM % 4 == 0) {
+        store_columns<MM, V>(p, in);
+    } else {
+#pragma unroll
+        for (int m = 0; m < MM; ++m) p[m] = in[m];
+    }
+}
+
+// MM columns of row_product (the single-column kernels' lane mapping): a lane reads its row's values of
+// a block once and the columns of the x entries they meet, which the RB lanes of a block row share in
+// cache.
+template <int RB, int CB, int BATCH, int MM, typename S, typename V>
+__device__ __forceinline__ void row_product_few(const Sliced<S> &a, uint32_t slot0, uint32_t len, int j, int lane,
+                                                const V *__restrict__ x, V (&sum)[MM]) {
+    constexpr int NPW = Shape<RB>::NPW;
+#pragma unroll
+    for (int m = 0; m < MM; ++m) sum[m] = (V)0;
+    const uint32_t *cp = a.cols + (size_t)slot0 * NPW + j;
+    const S *vp = a.vals + ((size_t)slot0 * WAVE + lane) * CB;
+    auto columns = [&](uint32_t col, V(&xv)[CB][MM]) {
+#pragma unroll
+        for (int q = 0; q < CB; ++q) load_few<MM, V>(x + ((size_t)col * CB + q) * MM, xv[q]);
+    };
+    auto add = [&](const S(&v)[CB], const V(&xv)[CB][MM]) {
+#pragma unroll
+        for (int q = 0; q < CB; ++q)
+#pragma unroll
+            for (int m = 0; m < MM; ++m)
+                sum[m] = sum[m] + widen<V>(v[q]) * xv[q][m];
+    };
+    const uint32_t full = len - len % BATCH;
+    uint32_t c[BATCH];
+    if (full) {
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) c[b] = cp[(size_t)b * NPW];
+    }
+    for (uint32_t k = 0; k < full; k += BATCH) {
+        S v[BATCH][CB];
+        V xv[BATCH][CB][MM];
+        uint32_t cn[BATCH];
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b)
+#pragma unroll
+            for (int q = 0; q < CB; ++q) v[b][q] = vp[(size_t)(k + b) * WAVE * CB + q];
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) columns(c[b], xv[b]);
+        if (k + BATCH < full) {
+#pragma unroll
+            for (int b = 0; b < BATCH; ++b) cn[b] = cp[(size_t)(k + BATCH + b) * NPW];
+        }
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) add(v[b], xv[b]);
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) c[b] = cn[b];
+    }
+    for (uint32_t k = full; k < len; ++k) {
+        S v[CB];
+        V xv[CB][MM];
+#pragma unroll
+        for (int q = 0; q < CB; ++q) v[q] = vp[(size_t)k * WAVE * CB + q];
+        columns(cp[(size_t)k * NPW], xv);
+        add(v, xv);
+    }
+}
+// Blocks in flight per lane: what the columns of x leave of its registers.
+template <int MM>
+constexpr int FEW_DEPTH = MM <= 4 ? 4 : 2;
+
+// z[m] = sum over q in order from zero of drow[q] times the value of lane j RB + q (the block row's row q).
+template <int RB, int MM, typename S, typename V>
+__device__ __forceinline__ void block_times_few(const S *drow, int first_lane, bool live, const V (&mine)[MM], V (&z)[MM]) {
+#pragma unroll
+    for (int m = 0; m < MM; ++m) z[m] = (V)0;
+#pragma unroll
+    for (int q = 0; q < RB; ++q)
+#pragma unroll
+        for (int m = 0; m < MM; ++m) {
+            const V other = __shfl(mine[m], first_lane + q, WAVE);
+            if (live) z[m] = z[m] + widen<V>(drow[q]) * other;
+        }
+}
+
+// spmv_kernel and cheb_step_kernel for MM columns. The lane-group kernels read a block by lanes that
+// each walk whole block rows and hold few blocks in flight: on the 603k-unknown plate a batch of one
+// column took 2.4 times the single solve.
+template <int RB, int CB, int MM, typename S, typename V>
+__global__ __launch_bounds__(256) void spmm_few_kernel(Sliced<S> a, int epi, const V *__restrict__ x, V *__restrict__ y,
+                                                       const V *__restrict__ b, Start<S, V> then) {
+    constexpr int NPW = Shape<RB>::NPW;
+    const uint32_t slice = slice_of(a.order);
+    if (slice >= a.slices) return;  // whole wave leaves together
+    const int lane = threadIdx.x % WAVE;
+    const int j = lane / RB, p = lane - j * RB;
+    const bool in_wave = j < NPW;
+    const uint32_t pos = slice * NPW + (in_wave ? j : 0);
+    const uint32_t row = in_wave ? a.perm[pos] : NONE;
+    const bool live = row != NONE;
+    const size_t out = live ? ((size_t)row * RB + p) * MM : 0;
+    V value[MM] = {};
+    if (live) {
+        V sum[MM];
+        row_product_few<RB, CB, FEW_DEPTH<MM>, MM, S, V>(a, a.slice_start[slice], a.row_len[pos], j, lane, x, sum);
+        if (epi != EPI_STORE) load_few<MM, V>((epi == EPI_RESIDUAL ? b : y) + out, value);
+#pragma unroll
+        for (int m = 0; m < MM; ++m) value[m] = epi == EPI_STORE ? sum[m] : epi == EPI_RESIDUAL ? value[m] - sum[m] : value[m] + sum[m];
+        store_few<MM, V>(y + out, value);
+    }
+    if (!then.dinv) return;  // uniform: every lane takes part in the shuffles
+    V z[MM];
+    block_times_few<RB, MM, S, V>(then.dinv + (live ? (size_t)row * RB * RB + (size_t)p * RB : 0), in_wave ? j * RB : 0, live, value, z);
+    if (!live) return;
+#pragma unroll
+    for (int m = 0; m < MM; ++m) z[m] = z[m] / then.theta;
+    store_few<MM, V>(then.d + out, z);
+    store_few<MM, V>(then.x + out, z);
+}
+
+template <int RB, int MM, typename S, typename V>
+__global__ __launch_bounds__(256) void cheb_step_few_kernel(Sliced<S> a, const S *__restrict__ dinv, const V *__restrict__ d_in,
+                                                            const V *__restrict__ r_in, V keep, V step, V *__restrict__ d_out,
+                                                            V *__restrict__ r_out, V *__restrict__ x, V *__restrict__ sum_into,
+                                                            double *__restrict__ widen_into) {
+    constexpr int NPW = Shape<RB>::NPW;
+    const uint32_t slice = slice_of(a.order);
+    if (slice >= a.slices) return;  // whole wave leaves together
+    const int lane = threadIdx.x % WAVE;
+    const int j = lane / RB, p = lane - j * RB;
+    const bool in_wave = j < NPW;
+    const uint32_t pos = slice * NPW + (in_wave ? j : 0);
+    const uint32_t row = in_wave ? a.perm[pos] : NONE;
+    const bool live = row != NONE;
+    const size_t i = live ? ((size_t)row * RB + p) * MM : 0;
+    V r_new[MM] = {};
+    if (live) {
+        V ad[MM];
+        row_product_few<RB, RB, FEW_DEPTH<MM>, MM, S, V>(a, a.slice_start[slice], a.row_len[pos], j, lane, d_in, ad);
+        load_few<MM, V>(r_in + i, r_new);
+#pragma unroll
+        for (int m = 0; m < MM; ++m) r_new[m] = r_new[m] - ad[m];
+    }
+    V z[MM];
+    block_times_few<RB, MM, S, V>(dinv + (live ? (size_t)row * RB * RB + (size_t)p * RB : 0), in_wave ? j * RB : 0, live, r_new, z);
+    if (!live) return;
+    V dn[MM], xn[MM];
+    load_few<MM, V>(d_in + i, dn);
+    load_few<MM, V>(x + i, xn);
+#pragma unroll
+    for (int m = 0; m < MM; ++m) {
+        dn[m] = keep * dn[m] + step * z[m];
+        xn[m] = xn[m] + dn[m];
+    }
+    store_few<MM, V>(d_out + i, dn);
+    store_few<MM, V>(r_out + i, r_new);
+    store_few<MM, V>(x + i, xn);
+    if (!sum_into) return;
+    V total[MM];
+    load_few<MM, V>(sum_into + i, total);
+#pragma unroll
+    for (int m = 0; m < MM; ++m) total[m] = total[m] + xn[m];
+    store_few<MM, V>(sum_into + i, total);
+    if (!widen_into) return;
+    double wide[MM];
+#pragma unroll
+    for (int m = 0; m < MM; ++m) wide[m] = (double)total[m];
+    store_few<MM, double>(widen_into + i, wide);
+}
+
 // The same product with one wavefront per block row: the row's position, block columns and block
 // values are the same for every lane, so they are read through the scalar unit into registers
 // every lane uses, and only the M columns of x are vector loads. Lane m takes column m (lanes
@@ -280,18 +463,24 @@ __device__ __forceinline__ uint32_t node_of_wave(uint32_t order) {
 // round trip, and one barrier (two LDS buffers). Every sum is the lane-group form's: from zero, blocks
 // in order, block columns in order. x moves in units of UNIT: 16 bytes where a block's CB * M entries
 // are whole units, else single entries.
-constexpr int STAGE_BLOCKS = 32;  // at most this many blocks a chunk
+// A chunk holds at most STAGE_BLOCKS blocks (9 KB of values a buffer) and what x a thread's registers
+// carry: few columns take long chunks, so that a row of some hundred blocks is two or three (355 blocks
+// and 5 columns: 25.8 us a launch by 32). From 16 columns on 32 blocks: longer ones cost more of a CU's
+// workgroups than they save.
+template <int LEN, typename S>
+constexpr int STAGE_BLOCKS = 9216 / (LEN * (int)sizeof(S)) < 32 ? 32 : 9216 / (LEN * (int)sizeof(S)) > 128 ? 128 : 9216 / (LEN * (int)sizeof(S));
 template <typename UNIT, typename V>
 constexpr int STAGE_UNITS = sizeof(UNIT) == 16 && sizeof(V) < 16 ? 4 : 8;  // x units a thread holds
 // Blocks per chunk for `units` units of x per block.
-__host__ __device__ inline uint32_t stage_chunk(uint32_t units, uint32_t held) {
-    const uint32_t c = 256u * held / units;
-    return c < (uint32_t)STAGE_BLOCKS ? c : (uint32_t)STAGE_BLOCKS;
+__host__ __device__ inline uint32_t stage_chunk(uint32_t units, uint32_t held, uint32_t M, uint32_t most) {
+    const uint32_t c = 256u * held / units, cap = M < 16 || most < 32 ? most : 32;
+    return c < cap ? c : cap;
 }
 template <int RB, int CB, typename S, typename V, typename UNIT, int CPL>
 __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t M, int epi, const V *__restrict__ x,
                                                           V *__restrict__ y, const V *__restrict__ b, Start<S, V> then) {
-    constexpr int NPW = Shape<RB>::NPW, LEN = RB * CB, UX = STAGE_UNITS<UNIT, V>, UV = (STAGE_BLOCKS * LEN + 255) / 256;
+    constexpr int NPW = Shape<RB>::NPW, LEN = RB * CB, UX = STAGE_UNITS<UNIT, V>, BLOCKS = STAGE_BLOCKS<LEN, S>,
+                  UV = (BLOCKS * LEN + 255) / 256;
     const uint32_t pos = blockIdx.x;
     if (pos >= a.slices * (uint32_t)NPW) return;  // the whole workgroup leaves together
     const uint32_t row = a.perm[pos];
@@ -301,11 +490,12 @@ __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t 
     const uint32_t slot0 = a.slice_start[slice], len = a.row_len[pos];
     const uint32_t *__restrict__ cp = a.cols + (size_t)slot0 * NPW + j;
     const S *__restrict__ vp = a.vals + ((size_t)slot0 * WAVE + (size_t)j * RB) * CB;
-    __shared__ S values[2][STAGE_BLOCKS * LEN];
-    __shared__ uint32_t columns[2][STAGE_BLOCKS];
-    extern __shared__ __align__(16) unsigned char staged_x[];  // two buffers of chunk * CB * M entries of x
-    const uint32_t units = (uint32_t)(CB * M * sizeof(V) / sizeof(UNIT)), chunk = stage_chunk(units, UX);
-    UNIT *xs[2] = {reinterpret_cast<UNIT *>(staged_x), reinterpret_cast<UNIT *>(staged_x) + chunk * units};
+    __shared__ uint32_t columns[2][BLOCKS];
+    extern __shared__ __align__(16) unsigned char staged_x[];  // two buffers of chunk * CB * M entries of x, two of the values
+    const uint32_t units = (uint32_t)(CB * M * sizeof(V) / sizeof(UNIT)), chunk = stage_chunk(units, UX, M, BLOCKS);
+    // offsets and not an array of pointers, which would make every access a flat one
+    UNIT *const staged_units = reinterpret_cast<UNIT *>(staged_x);
+    S *const staged_values = reinterpret_cast<S *>(staged_x + (size_t)2 * chunk * units * sizeof(UNIT));
     const uint32_t t = threadIdx.x, across = M / CPL;
     const bool computes = t < (uint32_t)RB * across;
     const uint32_t p = computes ? t / across : 0, m = computes ? t % across * CPL : 0;
@@ -337,15 +527,15 @@ __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t 
     uint32_t column = t < chunk && chunk + t < len ? cp[(size_t)(chunk + t) * NPW] : 0;
     __syncthreads();
     fetch(0, columns[0]);
-    int buf = 0;
+    uint32_t buf = 0;
     for (uint32_t k0 = 0; k0 < len; k0 += chunk, buf ^= 1) {
         const uint32_t n = min(chunk, len - k0);
 #pragma unroll
         for (int u = 0; u < UX; ++u)
-            if (uk[u] < n) xs[buf][t + 256u * u] = xv[u];
+            if (uk[u] < n) staged_units[buf * chunk * units + t + 256u * u] = xv[u];
 #pragma unroll
         for (int u = 0; u < UV; ++u)
-            if (t + 256u * u < n * LEN) values[buf][t + 256u * u] = vv[u];
+            if (t + 256u * u < n * LEN) staged_values[buf * chunk * LEN + t + 256u * u] = vv[u];
         if (t < chunk) columns[buf ^ 1][t] = column;
         // one barrier per chunk: a buffer is written again two chunks on, which a wavefront reaches
         // only after the barrier between, and so after the others have read it
@@ -354,8 +544,8 @@ __global__ __launch_bounds__(256) void spmm_staged_kernel(Sliced<S> a, uint32_t 
         if (t < chunk && k2 + t < len) column = cp[(size_t)(k2 + t) * NPW];
         fetch(k0 + chunk, columns[buf ^ 1]);
         if (computes) {
-            const V *xb = reinterpret_cast<const V *>(xs[buf]) + m;
-            const S *vb = values[buf] + p * CB;
+            const V *xb = reinterpret_cast<const V *>(staged_units + buf * chunk * units) + m;
+            const S *vb = staged_values + buf * chunk * LEN + p * CB;
 #pragma unroll 4
             for (uint32_t k = 0; k < n; ++k)
 #pragma unroll
@@ -535,18 +725,18 @@ __global__ __launch_bounds__(256) void convert_start_batch_kernel(uint32_t rows,
 
 // ---- few columns of a small system ----
 
-// rows_sum for M <= MM columns: a wavefront (one workgroup) takes RPW block rows, 64 / RPW lanes each;
+// rows_sum for M columns (a compile-time count, as row_product_few's): a wavefront (one workgroup) takes RPW block rows, 64 / RPW lanes each;
 // every lane loads a block and the M columns of the x entries it meets and forms their terms into LDS,
 // then lane c adds chain c's terms in stored order: row entry and column c % (RB M) of row c / (RB M),
 // RPW RB M <= 64. One round trip per 64 / RPW blocks, where a lane walking its row pays one per few.
 template <int RB, int CB, typename V, int RPW>
 constexpr int ROWS_BATCH_STRIDE = WAVE / RPW * CB + 16 / sizeof(V);  // entries of a chain's room
-template <int RB, int CB, int MM, int RPW, typename S, typename V>
-__device__ __forceinline__ V rows_sum_batch(const Bsr<S> &a, V *terms, uint32_t M, int g, int sl, uint32_t start, uint32_t len,
+template <int RB, int CB, int M, int RPW, typename S, typename V>
+__device__ __forceinline__ V rows_sum_batch(const Bsr<S> &a, V *terms, int g, int sl, uint32_t start, uint32_t len,
                                             const V *__restrict__ x) {
     constexpr int LW = WAVE / RPW, STRIDE = ROWS_BATCH_STRIDE<RB, CB, V, RPW>;
     const uint32_t longest = longest_of_wave<RPW>(len), chain = threadIdx.x;
-    const bool adds = chain < (uint32_t)(RPW * RB) * M;
+    const bool adds = chain < (uint32_t)(RPW * RB * M);
     const uint32_t chain_len = (uint32_t)__shfl((int)len, adds ? (int)(chain / (RB * M)) * LW : 0, WAVE);
     V sum = (V)0;
     for (uint32_t k0 = 0; k0 < longest; k0 += LW) {
@@ -554,25 +744,19 @@ __device__ __forceinline__ V rows_sum_batch(const Bsr<S> &a, V *terms, uint32_t 
         if (k < len) {
             const uint32_t col = a.cols[start + k];
             S v[RB * CB];
-            V xv[MM][CB];
+            V xv[CB][M];
             const S *blk = a.vals + (size_t)(start + k) * RB * CB;
 #pragma unroll
             for (int e = 0; e < RB * CB; ++e) v[e] = blk[e];
 #pragma unroll
-            for (int m = 0; m < MM; ++m)
-                if ((uint32_t)m < M) {
+            for (int q = 0; q < CB; ++q) load_few<M, V>(x + ((size_t)col * CB + q) * M, xv[q]);
 #pragma unroll
-                    for (int q = 0; q < CB; ++q) xv[m][q] = x[((size_t)col * CB + q) * M + m];
-                }
+            for (int p = 0; p < RB; ++p)
 #pragma unroll
-            for (int m = 0; m < MM; ++m)
-                if ((uint32_t)m < M) {
+                for (int m = 0; m < M; ++m)
 #pragma unroll
-                    for (int p = 0; p < RB; ++p)
-#pragma unroll
-                        for (int q = 0; q < CB; ++q)
-                            terms[(size_t)((g * RB + p) * M + m) * STRIDE + sl * CB + q] = widen<V>(v[p * CB + q]) * xv[m][q];
-                }
+                    for (int q = 0; q < CB; ++q)
+                        terms[((g * RB + p) * M + m) * STRIDE + sl * CB + q] = widen<V>(v[p * CB + q]) * xv[q][m];
         }
         __syncthreads();
         if (adds && k0 < chain_len)
@@ -582,8 +766,8 @@ __device__ __forceinline__ V rows_sum_batch(const Bsr<S> &a, V *terms, uint32_t 
     return sum;
 }
 
-template <int RB, int CB, int MM, int RPW, typename S, typename V>
-__global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, uint32_t M, int epi, const V *__restrict__ x, V *__restrict__ y,
+template <int RB, int CB, int M, int RPW, typename S, typename V>
+__global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, int epi, const V *__restrict__ x, V *__restrict__ y,
                                                         const V *__restrict__ b, Start<S, V> then) {
     constexpr int LW = WAVE / RPW;
     extern __shared__ __align__(16) unsigned char rows_terms[];
@@ -593,11 +777,12 @@ __global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, uint32_t M, in
     const uint32_t row = first + lane / LW;
     const uint32_t start = row < a.rows ? a.starts[row] : 0u, len = row < a.rows ? a.starts[row + 1] - start : 0u;
     // this lane's chain: row entry p of `own`, column m
-    const uint32_t per = RB * M, within = lane % per, p = within / M, m = within - p * M, own = first + lane / per;
+    constexpr uint32_t per = RB * M;
+    const uint32_t within = lane % per, p = within / M, m = within - p * M, own = first + lane / per;
     const bool owner = lane < RPW * per && own < a.rows;
     const size_t out = owner ? ((size_t)own * RB + p) * M + m : 0;
     const V before = !owner || epi == EPI_STORE ? (V)0 : epi == EPI_RESIDUAL ? b[out] : y[out];
-    const V sum = rows_sum_batch<RB, CB, MM, RPW, S, V>(a, terms, M, (int)(lane / LW), (int)(lane % LW), start, len, x);
+    const V sum = rows_sum_batch<RB, CB, M, RPW, S, V>(a, terms, (int)(lane / LW), (int)(lane % LW), start, len, x);
     V value = (V)0;
     if (owner) {
         value = epi == EPI_STORE ? sum : epi == EPI_RESIDUAL ? before - sum : before + sum;
@@ -618,8 +803,8 @@ __global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, uint32_t M, in
     }
 }
 
-template <int RB, int MM, int RPW, typename S, typename V>
-__global__ __launch_bounds__(64) void cheb_rows_batch_kernel(Bsr<S> a, uint32_t M, const S *__restrict__ dinv, const V *__restrict__ d_in,
+template <int RB, int M, int RPW, typename S, typename V>
+__global__ __launch_bounds__(64) void cheb_rows_batch_kernel(Bsr<S> a, const S *__restrict__ dinv, const V *__restrict__ d_in,
                                                              const V *__restrict__ r_in, V keep, V step, V *__restrict__ d_out,
                                                              V *__restrict__ r_out, V *__restrict__ x, V *__restrict__ sum_into,
                                                              double *__restrict__ widen_into) {
@@ -630,7 +815,8 @@ __global__ __launch_bounds__(64) void cheb_rows_batch_kernel(Bsr<S> a, uint32_t 
     const uint32_t lane = threadIdx.x, first = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW;
     const uint32_t row = first + lane / LW;
     const uint32_t start = row < a.rows ? a.starts[row] : 0u, len = row < a.rows ? a.starts[row + 1] - start : 0u;
-    const uint32_t per = RB * M, within = lane % per, p = within / M, m = within - p * M, own = first + lane / per;
+    constexpr uint32_t per = RB * M;
+    const uint32_t within = lane % per, p = within / M, m = within - p * M, own = first + lane / per;
     const bool owner = lane < RPW * per && own < a.rows;
     const size_t i = owner ? ((size_t)own * RB + p) * M + m : 0;
     V r_old = (V)0, d_old = (V)0, x_old = (V)0, into = (V)0;
@@ -643,7 +829,7 @@ __global__ __launch_bounds__(64) void cheb_rows_batch_kernel(Bsr<S> a, uint32_t 
 #pragma unroll
         for (int q = 0; q < RB; ++q) drow[q] = dinv[(size_t)own * RB * RB + (size_t)p * RB + q];
     }
-    const V sum = rows_sum_batch<RB, RB, MM, RPW, S, V>(a, terms, M, (int)(lane / LW), (int)(lane % LW), start, len, d_in);
+    const V sum = rows_sum_batch<RB, RB, M, RPW, S, V>(a, terms, (int)(lane / LW), (int)(lane % LW), start, len, d_in);
     r_new[lane] = r_old - sum;
     __syncthreads();
     if (!owner) return;

@@ -477,6 +477,7 @@ std::map<std::string, int> &tuning_memo() {
 int fastest(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates, const std::string &what,
             const std::string &memo) {
     static const bool verbose = std::getenv("SOLIDFEM_TUNE_LOG") != nullptr;
+    if (candidates.size() == 1) return candidates.front();
     std::string key;
     if (!memo.empty()) {
         key = memo;
@@ -967,29 +968,32 @@ class Hierarchy final : public DeviceMultigrid {
     static void launch_cheb_batch(LevelDev<S, V> &d, int batch, uint32_t M, const V *d_in, const V *r_in, V keep, V stp,
                                   V *d_out, V *r_out, V *x, V *into, hipStream_t s, double *widen = nullptr) {
         if (d.a.slices == 0) return;
-        if (batch > ROWS_BATCH_FORM) {
-            const int rpw = rows_batch_rows(batch, M);
-            if (M <= 4) cheb_rows_batch_rpw<4>(d, rpw, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
-            else cheb_rows_batch_rpw<8>(d, rpw, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+        if (batch >= FEW_FORM) {
+            with_columns(M, [&](auto columns) {
+                hipLaunchKernelGGL((cheb_step_few_kernel<3, decltype(columns)::value, S, V>), dim3(grid_for(d.a.slices, 4)), dim3(256), 0, s,
+                                   d.a.view(), d.dinv.ptr, d_in, r_in, keep, stp, d_out, r_out, x, into, widen);
+            });
+        } else if (batch > ROWS_BATCH_FORM) {
+            with_columns(M, [&](auto columns) {
+                constexpr int MM = decltype(columns)::value;
+                if constexpr (12 * MM <= WAVE) {
+                    if (rows_batch_rows(batch, M) == 4)
+                        return cheb_rows_batch_launch<MM, 4>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+                }
+                cheb_rows_batch_launch<MM, 2>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+            });
         } else if (d.rb == 3) cheb_batch_rb<3>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
         else cheb_batch_rb<6>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
     }
-    template <int MM, int RPW>
-    static void cheb_rows_batch_launch(LevelDev<S, V> &d, uint32_t M, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out,
-                                       V *x, V *into, hipStream_t s, double *widen) {
-        hipLaunchKernelGGL((cheb_rows_batch_kernel<3, MM, RPW, S, V>), dim3((d.a_rows.rows + RPW - 1) / RPW), dim3(WAVE),
-                           ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, d.a_rows.view(), M, d.dinv.ptr, d_in,
-                           r_in, keep, stp, d_out, r_out, x, into, widen);
-    }
-    template <int MM>
-    static void cheb_rows_batch_rpw(LevelDev<S, V> &d, int rpw, uint32_t M, const V *d_in, const V *r_in, V keep, V stp, V *d_out,
-                                    V *r_out, V *x, V *into, hipStream_t s, double *widen) {
-        if (rpw == 4) cheb_rows_batch_launch<MM, 4>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
-        else if (rpw == 2) cheb_rows_batch_launch<MM, 2>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
-        else cheb_rows_batch_launch<MM, 1>(d, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+    template <int M, int RPW>
+    static void cheb_rows_batch_launch(LevelDev<S, V> &d, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out, V *x, V *into,
+                                       hipStream_t s, double *widen) {
+        hipLaunchKernelGGL((cheb_rows_batch_kernel<3, M, RPW, S, V>), dim3((d.a_rows.rows + RPW - 1) / RPW), dim3(WAVE),
+                           ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, d.a_rows.view(), d.dinv.ptr, d_in, r_in,
+                           keep, stp, d_out, r_out, x, into, widen);
     }
     // Whether the forms by plain block rows are candidates for a level's steps and residuals.
-    static bool rows_batch_level(const LevelDev<S, V> &d, uint32_t M) { return d.rb == 3 && d.a_rows.rows && M <= ROWS_BATCH_COLUMNS; }
+    static bool rows_batch_level(const LevelDev<S, V> &d, uint32_t M) { return d.rb == 3 && d.a_rows.rows && M <= FEW_COLUMNS; }
     static std::vector<int> with_rows_batch(std::vector<int> forms, const LevelDev<S, V> &d, uint32_t M) {
         if (rows_batch_level(d, M))
             for (int f : rows_batch_forms()) forms.push_back(f);
@@ -998,7 +1002,7 @@ class Hierarchy final : public DeviceMultigrid {
     // res = b - A x for M columns, optionally with the start of the smoothing that follows.
     static void residual_batch(LevelDev<S, V> &d, int form, uint32_t M, const V *x, const V *b, hipStream_t s,
                                Start<S, V> st = {nullptr, (V)0, nullptr, nullptr}) {
-        if (form > ROWS_BATCH_FORM) launch_rows_batch<S, V>(d.a_rows, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
+        if (form > ROWS_BATCH_FORM && form < FEW_FORM) launch_rows_batch<S, V>(d.a_rows, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
         else launch_spmm<S, V>(d.a, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
     }
 
@@ -1164,11 +1168,12 @@ class Hierarchy final : public DeviceMultigrid {
                 LevelDev<S, V> &c = lv_[l + 1];
                 SF_HIP(hipMemsetAsync(c.b.ptr, 0, c.n * sizeof(V), s));
                 SF_HIP(hipMemsetAsync(c.x.ptr, 0, c.n * sizeof(V), s));
+                const bool long_rows = d.r.blocks >= LONG_ROW * d.r.rows;
                 d.r.batch_spmv = tune_batch(s, [&](int batch) { launch_spmv<S, V>(d.r, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s, batch); },
-                                            {1, 2, 4, 8}, at + "restriction depth", "restriction " + shape_class(d.r) + vs_);
+                                            long_rows ? std::vector<int>{8} : std::vector<int>{1, 2, 4, 8}, at + "restriction depth", "restriction " + shape_class(d.r) + vs_);
                 // the sliced product at its best depth (0) against the rows_sum forms and four
                 // wavefronts per row
-                std::vector<int> restrict_forms = rows_forms(d.r.rb * d.r.cb * sizeof(V));
+                std::vector<int> restrict_forms = long_rows ? std::vector<int>{1, 2} : rows_forms(d.r.rb * d.r.cb * sizeof(V));
                 restrict_forms.push_back(WIDE_ROWS);
                 d.restrict_rows = forced_variant().load(std::memory_order_relaxed) == WIDE_ROWS ? WIDE_ROWS : fastest(s, [&](int rpw) {
                     if (!rpw) launch_spmv<S, V>(d.r, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s);

@@ -108,29 +108,27 @@ void build_bsr(DeviceBsr<T> &out, const HostBsr<double> &pattern, const double *
 constexpr int WIDE_ROWS = 96;
 constexpr int rows_form_code(int rows, int blocks) { return rows + 256 * (blocks - 1); }
 // The forms worth timing against the sliced kernel (0) for blocks of `bytes` in the vector's
-// precision: a lane keeps U blocks in registers and a wavefront 64 U of them in LDS.
+// precision: a lane keeps U blocks in registers and a wavefront 64 U of them in LDS. (Four blocks a
+// lane, and two with two rows a wavefront, were never the fastest by more than the timing's spread.)
 inline std::vector<int> rows_forms(size_t bytes) {
     std::vector<int> f{0, 1, 2, 4};
-    if (bytes <= 144) f.insert(f.end(), {rows_form_code(2, 2), rows_form_code(4, 2)});
-    if (bytes <= 72) f.insert(f.end(), {rows_form_code(4, 4), rows_form_code(8, 4)});
+    if (bytes <= 144) f.push_back(rows_form_code(4, 2));
     return f;
 }
 // Calls f(rows per wavefront, blocks per lane) as compile-time constants for one of rows_forms(BYTES).
 template <int BYTES, typename F>
 void with_rows_form(int form, F &&f) {
     using std::integral_constant;
-    if constexpr (BYTES <= 72) {
-        if (form == rows_form_code(4, 4)) return f(integral_constant<int, 4>{}, integral_constant<int, 4>{});
-        if (form == rows_form_code(8, 4)) return f(integral_constant<int, 8>{}, integral_constant<int, 4>{});
-    }
     if constexpr (BYTES <= 144) {
-        if (form == rows_form_code(2, 2)) return f(integral_constant<int, 2>{}, integral_constant<int, 2>{});
         if (form == rows_form_code(4, 2)) return f(integral_constant<int, 4>{}, integral_constant<int, 2>{});
     }
     if (form == 4) return f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
     if (form == 2) return f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
     return f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
 }
+// Rows of this many blocks on average are long: a lane per scalar row walks them in 40 to 115 us where
+// the row kernels take 10 to 25, so the sliced forms are not timed for them.
+constexpr size_t LONG_ROW = 64;
 // Systems of at most this many blocks also keep their finest level in plain block rows for the row
 // kernels, whose latency is shorter. Four rows per wavefront against the sliced kernel, f32 step: 9.0
 // against 10.3 us at 0.5M blocks, 16.4 against 16.3 us at 0.97M (f64 vectors), 61 against 59 us at 6.9M.
@@ -187,6 +185,23 @@ constexpr int PAIR_FORM = 32;
 constexpr int QUAD_FORM = 48;
 constexpr int OCT_FORM = 64;  // eight columns per lane
 constexpr int STAGED_FORM = 80;  // products only: one workgroup per block row, chunks staged in LDS
+constexpr int FEW_FORM = 128;    // a lane per scalar row with up to FEW_COLUMNS columns, blocks of three rows
+constexpr uint32_t FEW_COLUMNS = 8;
+// Calls f(M) as a compile-time constant for M of 1 to FEW_COLUMNS columns.
+template <typename F>
+void with_columns(uint32_t M, F &&f) {
+    using std::integral_constant;
+    switch (M) {
+        case 1: f(integral_constant<int, 1>{}); break;
+        case 2: f(integral_constant<int, 2>{}); break;
+        case 3: f(integral_constant<int, 3>{}); break;
+        case 4: f(integral_constant<int, 4>{}); break;
+        case 5: f(integral_constant<int, 5>{}); break;
+        case 6: f(integral_constant<int, 6>{}); break;
+        case 7: f(integral_constant<int, 7>{}); break;
+        default: f(integral_constant<int, 8>{}); break;
+    }
+}
 inline int form_columns(int code) {
     return code >= STAGED_FORM ? 1 : code >= OCT_FORM ? 8 : code >= QUAD_FORM ? 4 : code >= PAIR_FORM ? 2 : 1;
 }
@@ -207,8 +222,7 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
 // The forms of products and steps by plain 3 x 3 block rows for few columns (rows_sum_batch):
 // ROWS_BATCH_FORM + block rows per wavefront.
 constexpr int ROWS_BATCH_FORM = 112;
-constexpr uint32_t ROWS_BATCH_COLUMNS = 8;
-inline std::vector<int> rows_batch_forms() { return {ROWS_BATCH_FORM + 1, ROWS_BATCH_FORM + 2, ROWS_BATCH_FORM + 4}; }
+inline std::vector<int> rows_batch_forms() { return {ROWS_BATCH_FORM + 2, ROWS_BATCH_FORM + 4}; }
 int rows_batch_rows(int form, uint32_t M);
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, dev::Start<S, V> start);

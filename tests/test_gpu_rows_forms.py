@@ -17,7 +17,8 @@ def bits(a):
     return np.ascontiguousarray(a, dtype=np.float64).view(np.uint64)
 
 
-@pytest.mark.parametrize("rows", [1, 2, 4])
+# block rows per wavefront; 16: the form with a lane per scalar row (also on larger systems)
+@pytest.mark.parametrize("rows", [2, 4, 16])
 @pytest.mark.parametrize("precision", [0, 1, 2], ids=["double", "single-storage", "single"])
 def test_few_columns_by_rows_keep_each_columns_bits(ctx, forced_variant, rows, precision):
     ref = refcpu.Problem(loaded(*FINGERPRINT_PLATE[:2]))
