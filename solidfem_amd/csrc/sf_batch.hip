@@ -390,16 +390,20 @@ void DevicePcgBatch::iterate() {
         const size_t lds = (size_t)DOT_THREADS * m_ * sizeof(double);
         hipLaunchKernelGGL((dot_partials_batch_kernel<0>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_, m_, (const double *)p_.ptr,
                            (const double *)ap_.ptr, partials_.ptr);
-        hipLaunchKernelGGL(pcg_update_fused_batch_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_, m_, scalars_.ptr, rz_slot_,
-                           (const uint32_t *)active_.ptr, (const double *)partials_.ptr, (const double *)p_.ptr, (const double *)ap_.ptr,
-                           x_.ptr, r_.ptr, partials2_.ptr);
+        with_columns(m_, [&](auto columns) {
+            hipLaunchKernelGGL((pcg_update_fused_batch_kernel<decltype(columns)::value>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_,
+                               scalars_.ptr, rz_slot_, (const uint32_t *)active_.ptr, (const double *)partials_.ptr, (const double *)p_.ptr,
+                               (const double *)ap_.ptr, x_.ptr, r_.ptr, partials2_.ptr);
+        });
         hipLaunchKernelGGL(dot_final_batch_kernel, dim3(m_), dim3(DOT_THREADS), 0, s, DOT_BLOCKS, m_, (const double *)partials2_.ptr,
                            (int)FINAL_STORE, (uint32_t)offsetof(PcgScalars, rr), scalars_.ptr, (const uint32_t *)nullptr, mirror_, tag);
         precondition(r_.ptr, z_.ptr);
         hipLaunchKernelGGL((dot_partials_batch_kernel<0>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), lds, s, n_, m_, (const double *)r_.ptr,
                            (const double *)z_.ptr, partials_.ptr);
-        hipLaunchKernelGGL(pcg_direction_fused_batch_kernel, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, s, n_, m_, scalars_.ptr, rz_slot_,
-                           (const uint32_t *)active_.ptr, (const double *)partials_.ptr, (const double *)z_.ptr, p_.ptr);
+        with_columns(m_, [&](auto columns) {
+            hipLaunchKernelGGL((pcg_direction_fused_batch_kernel<decltype(columns)::value>), dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, s, n_,
+                               scalars_.ptr, rz_slot_, (const uint32_t *)active_.ptr, (const double *)partials_.ptr, (const double *)z_.ptr, p_.ptr);
+        });
         rz_slot_ ^= 1u;
     } else {
         dot(p_.ptr, ap_.ptr, offsetof(PcgScalars, curvature), FINAL_STORE, nullptr);

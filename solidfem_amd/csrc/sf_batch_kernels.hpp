@@ -1102,12 +1102,20 @@ static __global__ void mirror_columns_kernel(uint32_t M, const PcgScalars *s, Pc
 // does for one: a launch less each. FUSED_COLUMNS: each block reads every column's 512 partials, which
 // costs more than the launch it saves from about nine columns on.
 constexpr uint32_t FUSED_COLUMNS = 8;
-__device__ __forceinline__ void tree_totals(uint32_t M, const double *__restrict__ partials, double (&totals)[FUSED_COLUMNS]) {
+// M is a compile-time count, so that every column's partials are in flight at once.
+template <uint32_t M>
+__device__ __forceinline__ void tree_totals(const double *__restrict__ partials, double (&totals)[FUSED_COLUMNS]) {
     __shared__ double wsum[FUSED_COLUMNS][DOT_THREADS / WAVE];
+    static_assert(DOT_BLOCKS == 2 * DOT_THREADS, "two partials a thread");
+    double first[M], second[M];
+#pragma unroll
     for (uint32_t m = 0; m < M; ++m) {
-        double v = 0.0;
-        for (uint32_t i = threadIdx.x; i < (uint32_t)DOT_BLOCKS; i += DOT_THREADS) v = v + partials[(size_t)i * M + m];
-        v = wave_sum(v);
+        first[m] = partials[(size_t)threadIdx.x * M + m];
+        second[m] = partials[(size_t)(threadIdx.x + DOT_THREADS) * M + m];
+    }
+#pragma unroll
+    for (uint32_t m = 0; m < M; ++m) {
+        const double v = wave_sum((0.0 + first[m]) + second[m]);  // dot_final_batch_kernel's sums
         if (threadIdx.x % WAVE == 0) wsum[m][threadIdx.x / WAVE] = v;
     }
     __syncthreads();
@@ -1121,7 +1129,8 @@ __device__ __forceinline__ void tree_totals(uint32_t M, const double *__restrict
 
 // pcg_update_fused_kernel for M <= FUSED_COLUMNS columns: p . A p from its partials, the update of
 // pcg_update_batch_kernel, and the partials of the new r . r over dot_partials_batch_kernel's slots.
-static __global__ __launch_bounds__(DOT_THREADS) void pcg_update_fused_batch_kernel(size_t n, uint32_t M, PcgScalars *__restrict__ s, uint32_t slot,
+template <uint32_t M>
+__global__ __launch_bounds__(DOT_THREADS) void pcg_update_fused_batch_kernel(size_t n, PcgScalars *__restrict__ s, uint32_t slot,
                                                                                     const uint32_t *__restrict__ active,
                                                                                     const double *__restrict__ pap_partials,
                                                                                     const double *__restrict__ p,
@@ -1129,7 +1138,7 @@ static __global__ __launch_bounds__(DOT_THREADS) void pcg_update_fused_batch_ker
                                                                                     double *__restrict__ r, double *__restrict__ rr_partials) {
     extern __shared__ double ls[];  // DOT_THREADS x M
     __shared__ double totals[FUSED_COLUMNS];
-    tree_totals(M, pap_partials, totals);
+    tree_totals<M>(pap_partials, totals);
     const uint32_t u = threadIdx.x, groups = DOT_THREADS / M, m = u % M;
     const double curvature = totals[m], rz = rz_in(s + m, slot);
     const bool live_column = active[m] != 0;
@@ -1186,13 +1195,14 @@ static __global__ __launch_bounds__(DOT_THREADS) void pcg_update_fused_batch_ker
 
 // pcg_direction_fused_kernel for M <= FUSED_COLUMNS columns: r . z from its partials, beta, then
 // p = z + beta p in the active columns. Block 0 stores the next r . z in the other slot.
-static __global__ __launch_bounds__(DOT_THREADS) void pcg_direction_fused_batch_kernel(size_t n, uint32_t M, PcgScalars *__restrict__ s,
+template <uint32_t M>
+__global__ __launch_bounds__(DOT_THREADS) void pcg_direction_fused_batch_kernel(size_t n, PcgScalars *__restrict__ s,
                                                                                        uint32_t slot, const uint32_t *__restrict__ active,
                                                                                        const double *__restrict__ rz_partials,
                                                                                        const double *__restrict__ z, double *__restrict__ p) {
     __shared__ double totals[FUSED_COLUMNS];
     __shared__ double betas[FUSED_COLUMNS];
-    tree_totals(M, rz_partials, totals);
+    tree_totals<M>(rz_partials, totals);
     if (threadIdx.x < M) {
         const uint32_t m = threadIdx.x;
         const double beta = totals[m] / rz_in(s + m, slot);
