@@ -177,21 +177,22 @@ template void launch_spmm<float, float>(const DeviceSliced<float> &, uint32_t, c
 
 // Rows per wavefront of a rows form for M columns: its chains, 3 M a row, fit the 64 lanes.
 int rows_batch_rows(int form, uint32_t M) { return form - ROWS_BATCH_FORM == 4 && 12 * M <= (uint32_t)WAVE ? 4 : 2; }
-template <int M, int RPW, typename S, typename V>
+template <int RB, int M, int RPW, typename S, typename V>
 static void rows_batch_launch(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
-    hipLaunchKernelGGL((rows_batch_kernel<3, 3, M, RPW, S, V>), dim3((a.rows + RPW - 1) / RPW), dim3(WAVE),
-                       ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, a.view(), epi, x, y, b, st);
+    hipLaunchKernelGGL((rows_batch_kernel<RB, RB, M, RPW, S, V>), dim3((a.rows + RPW - 1) / RPW), dim3(WAVE),
+                       ((size_t)RPW * RB * M * ROWS_BATCH_STRIDE<RB, RB, V, RPW> * sizeof(V)), s, a.view(), epi, x, y, b, st);
 }
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, Start<S, V> st) {
     if (a.rows == 0 || M == 0) return;
-    if (a.rb != 3 || a.cb != 3 || M > FEW_COLUMNS) throw Error(SF_ERR_INTERNAL, "no rows form for this block shape or column count");
+    if (a.cb != a.rb || !rows_batch_fits<V>(a.rb, M)) throw Error(SF_ERR_INTERNAL, "no rows form for this block shape or column count");
     with_columns(M, [&](auto columns) {
         constexpr int MM = decltype(columns)::value;
+        if (a.rb == 6) return rows_batch_launch<6, MM, 1>(a, x, y, b, epi, s, st);
         if constexpr (12 * MM <= WAVE) {
-            if (rows_batch_rows(form, M) == 4) return rows_batch_launch<MM, 4>(a, x, y, b, epi, s, st);
+            if (rows_batch_rows(form, M) == 4) return rows_batch_launch<3, MM, 4>(a, x, y, b, epi, s, st);
         }
-        rows_batch_launch<MM, 2>(a, x, y, b, epi, s, st);
+        rows_batch_launch<3, MM, 2>(a, x, y, b, epi, s, st);
     });
     SF_HIP(hipGetLastError());
 }

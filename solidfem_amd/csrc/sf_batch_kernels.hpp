@@ -725,38 +725,44 @@ __global__ __launch_bounds__(256) void convert_start_batch_kernel(uint32_t rows,
 
 // ---- few columns of a small system ----
 
-// rows_sum for M columns (a compile-time count, as row_product_few's): a wavefront (one workgroup) takes RPW block rows, 64 / RPW lanes each;
-// every lane loads a block and the M columns of the x entries it meets and forms their terms into LDS,
-// then lane c adds chain c's terms in stored order: row entry and column c % (RB M) of row c / (RB M),
-// RPW RB M <= 64. One round trip per 64 / RPW blocks, where a lane walking its row pays one per few.
+// rows_sum for M columns (a compile-time count, as row_product_few's): a wavefront (one workgroup) takes
+// RPW block rows, 64 / RPW lanes each; every lane loads a block and the M columns of the x entries it
+// meets and forms their terms into LDS, then lane c adds chain c's terms in stored order: row entry and column c % (RB M) of row c / (RB M),
+// RPW RB M <= 64. One round trip per 64 / RPW blocks, where a lane walking its row pays one per few. A
+// block of six rows is shared by two lanes, three rows each: four columns' steps of the 603k-DOF
+// plate's level 2 (334 rows) take 5.3 us (17.9 with lanes walking rows), and batches of four solve in
+// 28.6 ms for 40.3 (55k-DOF plate), 14.9 for 18.6 (300k-DOF block), 10.6 for 14.2 (115k-DOF tube).
+template <int RB, int RPW>
+constexpr int ROWS_BATCH_BLOCKS = WAVE / RPW / (RB / 3);  // blocks of a row at a time
 template <int RB, int CB, typename V, int RPW>
-constexpr int ROWS_BATCH_STRIDE = WAVE / RPW * CB + 16 / sizeof(V);  // entries of a chain's room
+constexpr int ROWS_BATCH_STRIDE = ROWS_BATCH_BLOCKS<RB, RPW> * CB + 16 / sizeof(V);  // entries of a chain's room
 template <int RB, int CB, int M, int RPW, typename S, typename V>
 __device__ __forceinline__ V rows_sum_batch(const Bsr<S> &a, V *terms, int g, int sl, uint32_t start, uint32_t len,
                                             const V *__restrict__ x) {
-    constexpr int LW = WAVE / RPW, STRIDE = ROWS_BATCH_STRIDE<RB, CB, V, RPW>;
+    constexpr int PARTS = RB / 3, LW = ROWS_BATCH_BLOCKS<RB, RPW>, STRIDE = ROWS_BATCH_STRIDE<RB, CB, V, RPW>;
+    const int at = sl / PARTS, p0 = sl % PARTS * 3;
     const uint32_t longest = longest_of_wave<RPW>(len), chain = threadIdx.x;
     const bool adds = chain < (uint32_t)(RPW * RB * M);
-    const uint32_t chain_len = (uint32_t)__shfl((int)len, adds ? (int)(chain / (RB * M)) * LW : 0, WAVE);
+    const uint32_t chain_len = (uint32_t)__shfl((int)len, adds ? (int)(chain / (RB * M)) * (WAVE / RPW) : 0, WAVE);
     V sum = (V)0;
     for (uint32_t k0 = 0; k0 < longest; k0 += LW) {
-        const uint32_t k = k0 + sl;
+        const uint32_t k = k0 + at;
         if (k < len) {
             const uint32_t col = a.cols[start + k];
-            S v[RB * CB];
+            S v[3 * CB];
             V xv[CB][M];
-            const S *blk = a.vals + (size_t)(start + k) * RB * CB;
+            const S *blk = a.vals + ((size_t)(start + k) * RB + p0) * CB;
 #pragma unroll
-            for (int e = 0; e < RB * CB; ++e) v[e] = blk[e];
+            for (int e = 0; e < 3 * CB; ++e) v[e] = blk[e];
 #pragma unroll
             for (int q = 0; q < CB; ++q) load_few<M, V>(x + ((size_t)col * CB + q) * M, xv[q]);
 #pragma unroll
-            for (int p = 0; p < RB; ++p)
+            for (int p = 0; p < 3; ++p)
 #pragma unroll
                 for (int m = 0; m < M; ++m)
 #pragma unroll
                     for (int q = 0; q < CB; ++q)
-                        terms[((g * RB + p) * M + m) * STRIDE + sl * CB + q] = widen<V>(v[p * CB + q]) * xv[q][m];
+                        terms[((g * RB + p0 + p) * M + m) * STRIDE + at * CB + q] = widen<V>(v[p * CB + q]) * xv[q][m];
         }
         __syncthreads();
         if (adds && k0 < chain_len)

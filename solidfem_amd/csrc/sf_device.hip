@@ -968,6 +968,8 @@ class Hierarchy final : public DeviceMultigrid {
     static void launch_cheb_batch(LevelDev<S, V> &d, int batch, uint32_t M, const V *d_in, const V *r_in, V keep, V stp,
                                   V *d_out, V *r_out, V *x, V *into, hipStream_t s, double *widen = nullptr) {
         if (d.a.slices == 0) return;
+        // a choice made for another column count of the group
+        if (batch > ROWS_BATCH_FORM && batch < FEW_FORM && !rows_batch_fits<V>(d.rb, M)) batch = 2;
         if (batch >= FEW_FORM) {
             with_columns(M, [&](auto columns) {
                 hipLaunchKernelGGL((cheb_step_few_kernel<3, decltype(columns)::value, S, V>), dim3(grid_for(d.a.slices, 4)), dim3(256), 0, s,
@@ -976,32 +978,34 @@ class Hierarchy final : public DeviceMultigrid {
         } else if (batch > ROWS_BATCH_FORM) {
             with_columns(M, [&](auto columns) {
                 constexpr int MM = decltype(columns)::value;
+                if (d.rb == 6) return cheb_rows_batch_launch<6, MM, 1>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
                 if constexpr (12 * MM <= WAVE) {
                     if (rows_batch_rows(batch, M) == 4)
-                        return cheb_rows_batch_launch<MM, 4>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+                        return cheb_rows_batch_launch<3, MM, 4>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
                 }
-                cheb_rows_batch_launch<MM, 2>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+                cheb_rows_batch_launch<3, MM, 2>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
             });
         } else if (d.rb == 3) cheb_batch_rb<3>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
         else cheb_batch_rb<6>(d, batch, M, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
     }
-    template <int M, int RPW>
+    template <int RB, int M, int RPW>
     static void cheb_rows_batch_launch(LevelDev<S, V> &d, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out, V *x, V *into,
                                        hipStream_t s, double *widen) {
-        hipLaunchKernelGGL((cheb_rows_batch_kernel<3, M, RPW, S, V>), dim3((d.a_rows.rows + RPW - 1) / RPW), dim3(WAVE),
-                           ((size_t)RPW * 3 * M * ROWS_BATCH_STRIDE<3, 3, V, RPW> * sizeof(V)), s, d.a_rows.view(), d.dinv.ptr, d_in, r_in,
+        hipLaunchKernelGGL((cheb_rows_batch_kernel<RB, M, RPW, S, V>), dim3((d.a_rows.rows + RPW - 1) / RPW), dim3(WAVE),
+                           ((size_t)RPW * RB * M * ROWS_BATCH_STRIDE<RB, RB, V, RPW> * sizeof(V)), s, d.a_rows.view(), d.dinv.ptr, d_in, r_in,
                            keep, stp, d_out, r_out, x, into, widen);
     }
     // Whether the forms by plain block rows are candidates for a level's steps and residuals.
-    static bool rows_batch_level(const LevelDev<S, V> &d, uint32_t M) { return d.rb == 3 && d.a_rows.rows && M <= FEW_COLUMNS; }
+    static bool rows_batch_level(const LevelDev<S, V> &d, uint32_t M) { return d.a_rows.rows && rows_batch_fits<V>(d.rb, M); }
     static std::vector<int> with_rows_batch(std::vector<int> forms, const LevelDev<S, V> &d, uint32_t M) {
         if (rows_batch_level(d, M))
-            for (int f : rows_batch_forms()) forms.push_back(f);
+            for (int f : rows_batch_forms(d.rb)) forms.push_back(f);
         return forms;
     }
     // res = b - A x for M columns, optionally with the start of the smoothing that follows.
     static void residual_batch(LevelDev<S, V> &d, int form, uint32_t M, const V *x, const V *b, hipStream_t s,
                                Start<S, V> st = {nullptr, (V)0, nullptr, nullptr}) {
+        if (form > ROWS_BATCH_FORM && form < FEW_FORM && !rows_batch_fits<V>(d.rb, M)) form = 2;  // as launch_cheb_batch
         if (form > ROWS_BATCH_FORM && form < FEW_FORM) launch_rows_batch<S, V>(d.a_rows, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
         else launch_spmm<S, V>(d.a, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
     }

@@ -219,10 +219,17 @@ inline int columns_log2(uint32_t m) {
 template <typename S, typename V>
 void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int batch = 0,
                  dev::Start<S, V> start = {nullptr, (V)0, nullptr, nullptr});
-// The forms of products and steps by plain 3 x 3 block rows for few columns (rows_sum_batch):
-// ROWS_BATCH_FORM + block rows per wavefront.
+// The forms of products and steps by plain block rows for few columns (rows_sum_batch): 3 x 3 blocks
+// with ROWS_BATCH_FORM + block rows per wavefront, 6 x 6 blocks (one row a wavefront) with the first code.
 constexpr int ROWS_BATCH_FORM = 112;
-inline std::vector<int> rows_batch_forms() { return {ROWS_BATCH_FORM + 2, ROWS_BATCH_FORM + 4}; }
+inline std::vector<int> rows_batch_forms(int rb = 3) {
+    return rb == 3 ? std::vector<int>{ROWS_BATCH_FORM + 2, ROWS_BATCH_FORM + 4} : std::vector<int>{ROWS_BATCH_FORM + 2};
+}
+// Whether a form by rows takes blocks of rb rows and M columns: six rows' chains fit 64 KB of LDS.
+template <typename V>
+bool rows_batch_fits(int rb, uint32_t M) {
+    return M <= FEW_COLUMNS && (rb == 3 || (rb == 6 && (size_t)6 * M * (32 * 6 * sizeof(V) + 16) <= 65536));
+}
 int rows_batch_rows(int form, uint32_t M);
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, dev::Start<S, V> start);
