@@ -196,6 +196,31 @@ void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, cons
     });
     SF_HIP(hipGetLastError());
 }
+// y = a x for M columns by wide_rows_batch_kernel; false where its buffers fit no LDS (nothing launched).
+template <typename S, typename V>
+bool launch_wide_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, hipStream_t s, Start<S, V> st, bool launch) {
+    if (a.rb != 6 || (a.cb != 3 && a.cb != 6) || a.rows == 0 || M == 0 || M > FEW_COLUMNS) return false;
+    bool fits = false;
+    with_columns(M, [&](auto columns) {
+        constexpr int MM = decltype(columns)::value;
+        auto shape = [&](auto cb) {
+            constexpr int CB = decltype(cb)::value;
+            if constexpr (WideRowsBatch<CB, MM, V>::FITS) {
+                fits = true;
+                if (launch)
+                    hipLaunchKernelGGL((wide_rows_batch_kernel<CB, MM, S, V>), dim3(a.rows), dim3(WIDE_BATCH_THREADS), 0, s, a.view(), x, y, st);
+            }
+        };
+        if (a.cb == 3) shape(std::integral_constant<int, 3>{});
+        else shape(std::integral_constant<int, 6>{});
+    });
+    if (launch && fits) SF_HIP(hipGetLastError());
+    return fits;
+}
+template bool launch_wide_rows_batch<double, double>(const DeviceBsr<double> &, uint32_t, const double *, double *, hipStream_t, Start<double, double>, bool);
+template bool launch_wide_rows_batch<float, double>(const DeviceBsr<float> &, uint32_t, const double *, double *, hipStream_t, Start<float, double>, bool);
+template bool launch_wide_rows_batch<float, float>(const DeviceBsr<float> &, uint32_t, const float *, float *, hipStream_t, Start<float, float>, bool);
+
 template void launch_rows_batch<double, double>(const DeviceBsr<double> &, uint32_t, const double *, double *, const double *, int, hipStream_t, int,
                                                 Start<double, double>);
 template void launch_rows_batch<float, double>(const DeviceBsr<float> &, uint32_t, const double *, double *, const double *, int, hipStream_t, int,

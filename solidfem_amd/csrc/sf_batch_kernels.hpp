@@ -809,6 +809,92 @@ __global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, int epi, const
     }
 }
 
+// A restriction's few, long rows for M columns: a workgroup per block row of six. Three wavefronts load
+// the next CHUNK blocks and the M columns of the x entries they meet (a block shared by 192 / CHUNK
+// threads) and form their terms into LDS; the fourth adds the chunk before, a lane per chain (row entry
+// and column), in stored order. Bound by that chain of additions: 73 rows of 350 blocks, five columns,
+// f32: 9.0 us a launch, against 19.0 for the staged product. Batches of two to four solve in 0.85 to
+// 0.97 times the time (300k-DOF block, four columns: 14.9 -> 12.9 ms).
+constexpr uint32_t WIDE_BATCH_THREADS = 256, WIDE_BATCH_LDS = 65536 - 512;
+template <int CB, int M, typename V>
+struct WideRowsBatch {
+    static constexpr int stride(int chunk) { return chunk * CB + 16 / (int)sizeof(V); }  // entries of a chain's room
+    static constexpr uint32_t bytes(int chunk) { return 2u * 6 * M * stride(chunk) * sizeof(V); }
+    // the longest chunk whose two buffers fit the LDS; FITS: whether any does
+    static constexpr int CHUNK = bytes(64) <= WIDE_BATCH_LDS ? 64 : 32;
+    static constexpr bool FITS = bytes(CHUNK) <= WIDE_BATCH_LDS;
+    static constexpr int STRIDE = stride(CHUNK), PARTS = 192 / CHUNK, RP = 6 / PARTS;
+};
+template <int CB, int M, typename S, typename V>
+__global__ __launch_bounds__(256) void wide_rows_batch_kernel(Bsr<S> a, const V *__restrict__ x, V *__restrict__ y, Start<S, V> then) {
+    using W = WideRowsBatch<CB, M, V>;
+    constexpr int RB = 6, RP = W::RP, STRIDE = W::STRIDE;
+    constexpr uint32_t CHUNK = W::CHUNK, CHAINS = RB * M;
+    __shared__ __align__(16) V terms[2][CHAINS * STRIDE];
+    __shared__ V values[WAVE];
+    const uint32_t row = a.reverse ? xcd_reversed_block() : blockIdx.x;  // one workgroup per row: row < a.rows
+    const uint32_t start = a.starts[row], len = a.starts[row + 1] - start;
+    const uint32_t t = threadIdx.x, k = t / W::PARTS, p0 = t % W::PARTS * RP;
+    const bool loads = t < 192;  // k < CHUNK
+    const uint32_t chain = t - 192, p = chain / M, m = chain - p * M;
+    const bool adds = !loads && chain < CHAINS;
+    const size_t out = (size_t)row * CHAINS + chain;
+    S drow[RB];
+    if (then.dinv && adds) {
+#pragma unroll
+        for (int q = 0; q < RB; ++q) drow[q] = then.dinv[(size_t)row * RB * RB + (size_t)p * RB + q];
+    }
+    S v[RP * CB];
+    V xv[CB][M];
+    auto fetch = [&](uint32_t at, uint32_t col) {
+        if (loads && at < len) {
+            const S *blk = a.vals + ((size_t)(start + at) * RB + p0) * CB;
+#pragma unroll
+            for (int e = 0; e < RP * CB; ++e) v[e] = blk[e];
+#pragma unroll
+            for (int q = 0; q < CB; ++q) load_few<M, V>(x + ((size_t)col * CB + q) * M, xv[q]);
+        }
+    };
+    uint32_t col = loads && k < len ? a.cols[start + k] : 0u;
+    fetch(k, col);
+    col = loads && k + CHUNK < len ? a.cols[start + k + CHUNK] : 0u;
+    V sum = (V)0;
+    int buf = 0;
+    for (uint32_t k0 = 0; k0 < len; k0 += CHUNK, buf ^= 1) {
+        if (loads && k0 + k < len) {
+#pragma unroll
+            for (int r = 0; r < RP; ++r)
+#pragma unroll
+                for (int m1 = 0; m1 < M; ++m1)
+#pragma unroll
+                    for (int q = 0; q < CB; ++q)
+                        terms[buf][((p0 + r) * M + m1) * STRIDE + k * CB + q] = widen<V>(v[r * CB + q]) * xv[q][m1];
+        }
+        const uint32_t k1 = k0 + CHUNK, k2 = k1 + CHUNK;
+        if (k1 < len) {
+            fetch(k1 + k, col);
+            if (loads && k2 + k < len) col = a.cols[start + k2 + k];
+        }
+        // one barrier per chunk, as in wide_rows_kernel
+        __syncthreads();
+        if (adds) sum = add_terms<4>(sum, (const V *)terms[buf] + chain * STRIDE, (len - k0 < CHUNK ? len - k0 : CHUNK) * CB);
+    }
+    if (adds) {
+        y[out] = sum;
+        values[chain] = sum;
+    }
+    if (!then.dinv) return;  // uniform
+    __syncthreads();
+    if (adds) {
+        V z = (V)0;
+#pragma unroll
+        for (int q = 0; q < RB; ++q) z = z + widen<V>(drow[q]) * values[q * M + m];
+        const V dv = z / then.theta;
+        then.d[out] = dv;
+        then.x[out] = dv;
+    }
+}
+
 template <int RB, int M, int RPW, typename S, typename V>
 __global__ __launch_bounds__(64) void cheb_rows_batch_kernel(Bsr<S> a, const S *__restrict__ dinv, const V *__restrict__ d_in,
                                                              const V *__restrict__ r_in, V keep, V step, V *__restrict__ d_out,

@@ -1002,6 +1002,14 @@ class Hierarchy final : public DeviceMultigrid {
             for (int f : rows_batch_forms(d.rb)) forms.push_back(f);
         return forms;
     }
+    // The restriction y = R x for M columns, with the start of the coarser level's smoothing where given.
+    static void restrict_batch(LevelDev<S, V> &d, int form, uint32_t M, const V *x, V *y, hipStream_t s, Start<S, V> st) {
+        if (form == WIDE_ROWS) {
+            if (launch_wide_rows_batch<S, V>(d.r_rows, M, x, y, s, st, true)) return;
+            form = 2;  // a choice made for another column count of the group
+        }
+        launch_spmm<S, V>(d.r, M, x, y, nullptr, EPI_STORE, s, form, st);
+    }
     // res = b - A x for M columns, optionally with the start of the smoothing that follows.
     static void residual_batch(LevelDev<S, V> &d, int form, uint32_t M, const V *x, const V *b, hipStream_t s,
                                Start<S, V> st = {nullptr, (V)0, nullptr, nullptr}) {
@@ -1045,10 +1053,12 @@ class Hierarchy final : public DeviceMultigrid {
                 const size_t cneed = c.n * (size_t)M;
                 SF_HIP(hipMemsetAsync(c.mb.ptr, 0, cneed * sizeof(V), s));
                 SF_HIP(hipMemsetAsync(c.mx.ptr, 0, cneed * sizeof(V), s));
+                std::vector<int> restrict_forms = spmm_candidates(d.r.rb, d.r.cb, sizeof(S), M, true, staged_candidate(d.r, M));
+                if (launch_wide_rows_batch<S, V>(d.r_rows, M, d.mres.ptr, c.mb.ptr, s, {nullptr, (V)0, nullptr, nullptr}, false))
+                    restrict_forms.push_back(WIDE_ROWS);
                 d.mm_depth[lg][2] = tune_batch(s, [&](int batch) {
-                    launch_spmm<S, V>(d.r, M, d.mres.ptr, c.mb.ptr, nullptr, EPI_STORE, s, batch);
-                }, spmm_candidates(d.r.rb, d.r.cb, sizeof(S), M, true, staged_candidate(d.r, M)), "",
-                   "batch restriction " + group + shape_class(d.r) + vsize);
+                    restrict_batch(d, batch, M, d.mres.ptr, c.mb.ptr, s, {nullptr, (V)0, nullptr, nullptr});
+                }, restrict_forms, "", "batch restriction " + group + shape_class(d.r) + vsize);
                 d.mm_depth[lg][3] = tune_batch(s, [&](int batch) {
                     launch_spmm<S, V>(d.p, M, c.mx.ptr, d.mpx.ptr, nullptr, EPI_ADD, s, batch);
                 }, spmm_candidates(d.p.rb, d.p.cb, sizeof(S), M, true, staged_candidate(d.p, M)), "",
@@ -1121,7 +1131,7 @@ class Hierarchy final : public DeviceMultigrid {
         // restriction and residual with the start of the smoothing that follows, as cycle()
         const bool fuse = smooths_first(c);
         const Start<S, V> first = {fuse ? c.dinv.ptr : nullptr, (V)c.theta, c.md0.ptr, c.mx.ptr};
-        launch_spmm<S, V>(d.r, M, d.mres.ptr, c.mb.ptr, nullptr, EPI_STORE, s, d.mm_depth[lg][2], first);
+        restrict_batch(d, d.mm_depth[lg][2], M, d.mres.ptr, c.mb.ptr, s, first);
         cycle_batch(l + 1, c.mb.ptr, c.mx.ptr, M, s, fuse);
         launch_spmm<S, V>(d.p, M, c.mx.ptr, x, nullptr, EPI_ADD, s, d.mm_depth[lg][3]);
         residual_batch(d, d.mm_depth[lg][1], M, x, b, s, {d.dinv.ptr, (V)d.theta, d.md0.ptr, d.mpx.ptr});

@@ -103,7 +103,7 @@ void upload_bsr(DeviceBsr<T> &out, const HostBsr<double> &m, hipStream_t s);
 template <typename T>
 void build_bsr(DeviceBsr<T> &out, const HostBsr<double> &pattern, const double *values, hipStream_t s);
 // The forms of the row kernels: block rows per wavefront + 256 * (blocks a lane loads at once - 1),
-// or WIDE_ROWS: four wavefronts per block row (wide_rows_kernel, restrictions only).
+// or WIDE_ROWS: four wavefronts per block row (wide_rows_kernel, wide_rows_batch_kernel; restrictions only).
 // sf_force_variant(WIDE_ROWS) forces the latter on every restriction.
 constexpr int WIDE_ROWS = 96;
 constexpr int rows_form_code(int rows, int blocks) { return rows + 256 * (blocks - 1); }
@@ -233,6 +233,11 @@ bool rows_batch_fits(int rb, uint32_t M) {
 int rows_batch_rows(int form, uint32_t M);
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, dev::Start<S, V> start);
+// The restriction of few columns by wide_rows_batch_kernel (form WIDE_ROWS of a batched restriction).
+// False, and nothing launched, for another block shape, more columns or too large buffers; with
+// `launch` false it only answers.
+template <typename S, typename V>
+bool launch_wide_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, hipStream_t s, dev::Start<S, V> start, bool launch);
 // The batch depths worth trying for a matrix's batched product.
 // The variant codes a batched product (`product`) or Chebyshev step is timed over for M columns.
 std::vector<int> spmm_candidates(int rb, int cb, size_t value_size, uint32_t M, bool product = true, bool staged = false);

@@ -17,8 +17,9 @@ def bits(a):
     return np.ascontiguousarray(a, dtype=np.float64).view(np.uint64)
 
 
-# block rows per wavefront; 16: the form with a lane per scalar row (also on larger systems)
-@pytest.mark.parametrize("rows", [2, 4, 16])
+# block rows per wavefront; 16: the form with a lane per scalar row (also on larger systems); -16: the
+# restrictions with four wavefronts per row
+@pytest.mark.parametrize("rows", [2, 4, 16, -16])
 @pytest.mark.parametrize("precision", [0, 1, 2], ids=["double", "single-storage", "single"])
 def test_few_columns_by_rows_keep_each_columns_bits(ctx, forced_variant, rows, precision):
     ref = refcpu.Problem(loaded(*FINGERPRINT_PLATE[:2]))
@@ -30,7 +31,7 @@ def test_few_columns_by_rows_keep_each_columns_bits(ctx, forced_variant, rows, p
     mg = setup.finish()
     opts = sf.PcgOptions(tolerance=1e-8, dot_order=sf.DotOrder.TREE)
     forced_variant(ROWS_BATCH_FORM + rows)
-    rng = np.random.default_rng(rows)
+    rng = np.random.default_rng(rows + 16)
     # groups of 1, 2, 4 and 8 columns (a choice each), 3, 5 and 7 in them, and 9: past the forms and
     # past the final sums formed by their consumers
     for columns in (1, 2, 3, 4, 5, 7, 8, 9):
