@@ -549,10 +549,11 @@ void Server::serve(ServeSystem &system, const std::shared_ptr<Context> &ctx) {
         for (const auto &pr : st.model.prescribed) nodal[3 * (size_t)pr.first.first + pr.first.second] = pr.second;
         return nodal;
     };
-    // Fewer than four requests: each runs the single-column solve in turn (the same bits as a
-    // batch column). On the 300k-DOF block one column alone takes 9.7 ms against 34.6 ms as a
-    // one-column batch, two 19.3 ms against 34.1 ms, and four 38.2 ms against 31.1 ms. Requests
-    // that arrive meanwhile wait for the next round, where they batch together.
+    // One request runs the single-column solve (the same bits as a batch column), which a one-column
+    // batch does not beat (1.1 to 1.3 times its time). Two are a batch: on beams, tubes, a block and
+    // plates of 19k to 603k DOFs it takes 0.63 to 0.71 times two single solves (block of 300k DOFs 10.5
+    // ms against 16.5, plates of 55k 22.3 against 35.3, of 603k 286 against 429). Requests that arrive
+    // meanwhile wait for the next round, where they batch together.
     auto solve_alone = [&](u64 id, const std::vector<double> &b) {
         const sf_pcg_options pcg{options_.tolerance, 0, options_.dot_order, 0};
         sf_column_progress done{};
@@ -599,9 +600,8 @@ void Server::serve(ServeSystem &system, const std::shared_ptr<Context> &ctx) {
         cv_.notify_all();
         return true;
     };
-    if (ids.size() < 4) {
-        for (size_t k = 0; k < ids.size(); ++k)
-            if (!solve_alone(ids[k], rhs[k])) return;
+    if (ids.size() == 1) {
+        solve_alone(ids[0], rhs[0]);
         return;
     }
     const uint32_t M = (uint32_t)width;
