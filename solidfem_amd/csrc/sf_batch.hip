@@ -372,7 +372,7 @@ void DevicePcgBatch::restart(const double *rhs) {
     SF_HIP(hipStreamSynchronize(s));
     const size_t total = n_ * m_;
     if (rhs) {
-        stage_.upload(rhs, total, s);
+        staged_upload_bytes(ctx_.get(), stage_.ptr, rhs, total * sizeof(double), s);
         hipLaunchKernelGGL((interleave_kernel<double>), dim3(grid_for(total, 256)), dim3(256), 0, s, n_, m_, (const double *)stage_.ptr, b_.ptr);
     }
     SF_HIP(hipMemcpyAsync(r_.ptr, b_.ptr, total * 8, hipMemcpyDeviceToDevice, s));
@@ -537,8 +537,7 @@ void DevicePcgBatch::estimate(double *out) const {
     hipLaunchKernelGGL((deinterleave_kernel<double>), dim3(grid_for(total, 256)), dim3(256), 0, ctx_->stream, n_, m_,
                        (const double *)x_.ptr, stage_.ptr);
     SF_HIP(hipGetLastError());
-    stage_.download(out, total, ctx_->stream);
-    SF_HIP(hipStreamSynchronize(ctx_->stream));
+    staged_download(ctx_.get(), out, stage_.ptr, total * sizeof(double), ctx_->stream);
 }
 
 void DevicePcgBatch::estimate_column(uint32_t column, double *out) const {

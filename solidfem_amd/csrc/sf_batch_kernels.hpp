@@ -465,7 +465,7 @@ __device__ __forceinline__ uint32_t node_of_wave(uint32_t order) {
 // are whole units, else single entries.
 // A chunk holds at most STAGE_BLOCKS blocks (9 KB of values a buffer) and what x a thread's registers
 // carry: few columns take long chunks, so that a row of some hundred blocks is two or three (355 blocks
-// and 5 columns: 25.8 us a launch by 32). From 16 columns on 32 blocks: longer ones cost more of a CU's
+// and 5 columns: 18.5 us a launch, 25.8 by 32). From 16 columns on 32 blocks: longer ones cost more of a CU's
 // workgroups than they save.
 template <int LEN, typename S>
 constexpr int STAGE_BLOCKS = 9216 / (LEN * (int)sizeof(S)) < 32 ? 32 : 9216 / (LEN * (int)sizeof(S)) > 128 ? 128 : 9216 / (LEN * (int)sizeof(S));
