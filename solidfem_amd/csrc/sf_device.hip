@@ -463,6 +463,14 @@ int tune_batch(hipStream_t s, const std::function<void(int)> &launch, const std:
     return fastest(s, launch, candidates, what, memo);
 }
 
+int fastest_rows(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates, const std::string &what,
+                 const std::string &memo) {
+    const int forced = forced_variant().load(std::memory_order_relaxed) - ROWS_FORCED;
+    for (int c : candidates)
+        if (forced >= 0 && forced == c) return forced;
+    return fastest(s, launch, candidates, what, memo);
+}
+
 static int fastest_timed(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates,
                          const std::string &what);
 
@@ -1169,11 +1177,11 @@ class Hierarchy final : public DeviceMultigrid {
                                         {1, 2, 4, 8}, at + "residual depth", "residual " + a_class);
             if (d.a_rows.rows) {
                 // each kernel against its rows_sum forms (all the same bits); 0 is the sliced kernel
-                d.cheb_rows = fastest(s, [&](int rpw) {
+                d.cheb_rows = fastest_rows(s, [&](int rpw) {
                     if (!rpw) launch_cheb_step(d, d.a.batch_cheb, d.d0.ptr, d.b.ptr, (V)0, (V)0, d.d1.ptr, d.r0.ptr, d.x.ptr, nullptr, s);
                     else launch_cheb_rows(d, rpw, d.d0.ptr, d.b.ptr, (V)0, (V)0, d.d1.ptr, d.r0.ptr, d.x.ptr, nullptr, s);
                 }, rows_forms(d.rb * d.rb * sizeof(V)), at + "step rows per wave", "step rows " + a_class);
-                d.residual_rows = fastest(s, [&](int rpw) {
+                d.residual_rows = fastest_rows(s, [&](int rpw) {
                     if (!rpw) launch_spmv<S, V>(d.a, d.x.ptr, d.res.ptr, d.b.ptr, EPI_RESIDUAL, s);
                     else launch_long_rows<S, V>(d.a_rows, d.x.ptr, d.res.ptr, d.b.ptr, EPI_RESIDUAL, s, {nullptr, (V)0, nullptr, nullptr}, rpw);
                 }, rows_forms(d.rb * d.rb * sizeof(V)), at + "residual rows per wave", "residual rows " + a_class);
@@ -1189,7 +1197,7 @@ class Hierarchy final : public DeviceMultigrid {
                 // wavefronts per row
                 std::vector<int> restrict_forms = long_rows ? std::vector<int>{1, 2} : rows_forms(d.r.rb * d.r.cb * sizeof(V));
                 restrict_forms.push_back(WIDE_ROWS);
-                d.restrict_rows = forced_variant().load(std::memory_order_relaxed) == WIDE_ROWS ? WIDE_ROWS : fastest(s, [&](int rpw) {
+                d.restrict_rows = forced_variant().load(std::memory_order_relaxed) == WIDE_ROWS ? WIDE_ROWS : fastest_rows(s, [&](int rpw) {
                     if (!rpw) launch_spmv<S, V>(d.r, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s);
                     else launch_long_rows<S, V>(d.r_rows, d.res.ptr, c.b.ptr, nullptr, EPI_STORE, s, {nullptr, (V)0, nullptr, nullptr}, rpw);
                 }, restrict_forms, at + "restriction rows per wave", "restriction rows " + shape_class(d.r) + vs_);
@@ -1387,7 +1395,7 @@ void DeviceSystem::build_from_device_values(hipStream_t s) {
         rows.borrowed = values.ptr;
         DeviceBuffer<double> x(std::max<size_t>(host.cols * 3, 1)), y(std::max<size_t>(host.rows * 3, 1));
         SF_HIP(hipMemsetAsync(x.ptr, 0, x.bytes(), s));
-        rows_form = fastest(s, [&](int form) {
+        rows_form = fastest_rows(s, [&](int form) {
             if (!form) launch_spmv<double, double>(sliced, x.ptr, y.ptr, nullptr, EPI_STORE, s);
             else launch_long_rows<double, double>(rows, x.ptr, y.ptr, nullptr, EPI_STORE, s, {nullptr, 0.0, nullptr, nullptr}, form);
         }, rows_forms(9 * sizeof(double)), "system rows per wave", "system rows " + shape_class(sliced));

@@ -115,6 +115,8 @@ inline std::vector<int> rows_forms(size_t bytes) {
     if (bytes <= 144) f.push_back(rows_form_code(4, 2));
     return f;
 }
+// sf_force_variant(ROWS_FORCED + form) forces the form wherever rows_forms() has it among the candidates.
+constexpr int ROWS_FORCED = 1024;
 // Calls f(rows per wavefront, blocks per lane) as compile-time constants for one of rows_forms(BYTES).
 template <int BYTES, typename F>
 void with_rows_form(int form, F &&f) {
@@ -162,6 +164,9 @@ int tune_batch(hipStream_t s, const std::function<void(int)> &launch, const std:
 // same bits.
 int fastest(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates,
             const std::string &what = "", const std::string &memo = "");
+// fastest over forms of the row kernels, or the one that is forced.
+int fastest_rows(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates, const std::string &what,
+                 const std::string &memo);
 // A matrix's shape class for the tuning memo: block shape, value size, and the binary orders of
 // its block rows and of its mean blocks per row.
 template <typename T>

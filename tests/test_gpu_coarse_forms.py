@@ -73,3 +73,27 @@ def test_wide_restriction_rows_keep_the_cycles_bits(ctx, forced_variant, w, prec
     mg = multigrid(ctx, ref, precision, 100)
     assert mg.stats().levels >= 2
     assert np.array_equal(bits(mg.apply(r)), bits(expected))
+
+
+ROWS_FORCED = 1024
+
+
+# block rows per wavefront + 256 (blocks a lane loads at once - 1)
+@pytest.mark.parametrize("form", [1, 2, 4, 256 + 4])
+@pytest.mark.parametrize("precision", [0, 1, 2], ids=["double", "single-storage", "single"])
+@pytest.mark.parametrize("w", [block_config(0, divisions=(7, 5, 5)), plate_config(divisions=(5, 7, 2))], ids=["block", "plate"])
+def test_row_forms_keep_the_cycles_and_the_solves_bits(ctx, forced_variant, w, precision, form):
+    ref = refcpu.Problem(w)
+    r = np.random.default_rng(form).standard_normal(ref.free_dofs)
+
+    def results(code):
+        forced_variant(ROWS_FORCED + code)  # 0: the sliced forms
+        csr = sf.CsrMatrix.new(ctx, *ref.csr())
+        mg = multigrid(ctx, ref, precision, 100)
+        z = mg.apply(r)
+        solve = sf.Pcg.new(ctx, csr, mg, r, sf.PcgOptions(tolerance=1e-8, dot_order=sf.DotOrder.TREE))
+        solve.step(100000)
+        return bits(z), bits(solve.estimate())
+
+    for got, expected in zip(results(form), results(0)):
+        assert np.array_equal(got, expected)
