@@ -161,7 +161,7 @@ typedef struct sf_multigrid_options {
 
 /* Where a level's numeric setup phases run: the power iteration, the smoothed prolongator, A P
  * and P^T (A P) (setup.rs:390-449, :527-647). AUTO runs them on the device for levels of at
- * least 4096 block rows when the setup has a device context, HOST never, DEVICE for every
+ * least 256 block rows when the setup has a device context, HOST never, DEVICE for every
  * level (given a context). Aggregation, the tentative prolongator and the block inverses stay
  * on the host. The hierarchy is the same to the bit wherever the phases run. No counterpart in
  * the reference, whose setup runs on its host thread pool. */
@@ -812,8 +812,8 @@ sf_status sf_csr_tuned_depth(const sf_csr *csr, int32_t *depth);
  * read the environment (undefined behaviour in glibc); the environment is read once, as the
  * starting value.
  * sf_force_variant: every later tuning of a batch depth or batched form that has `code` among its
- *   candidates takes it (0: time the candidates, the default; SOLIDFEM_BATCH). Bits never depend
- *   on the variant.
+ *   candidates takes it (0: time the candidates, the default; SOLIDFEM_BATCH); 1024 + form does the
+ *   same for the row kernels' forms. Bits never depend on the variant.
  * sf_setup_slot_limit: device setup rows of more than `blocks` output blocks take the host path
  *   (0: the kernels' own limit of 1024; SOLIDFEM_SETUP_SLOT_LIMIT). Read when a setup begins. */
 sf_status sf_force_variant(int32_t code);

@@ -41,7 +41,7 @@ class Precision(enum.IntEnum):
 
 class SetupDevice(enum.IntEnum):
     """Where a level's numeric setup phases run (power iteration, smoothed prolongator, A P,
-    P^T A P): AUTO on the device for levels of at least 4096 block rows when the setup has a
+    P^T A P): AUTO on the device for levels of at least 256 block rows when the setup has a
     device context, HOST never, DEVICE for every level. The hierarchy's bits are the same."""
     AUTO = 0
     HOST = 1
