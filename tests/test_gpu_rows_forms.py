@@ -6,7 +6,7 @@ import pytest
 
 import refcpu
 import solidfem_amd as sf
-from workloads import FINGERPRINT_PLATE, loaded
+from workloads import FINGERPRINT_PLATE, block_config, loaded
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +48,24 @@ def test_few_columns_by_rows_keep_each_columns_bits(ctx, forced_variant, rows, p
             single = sf.Pcg.new(ctx, csr, mg, r[m], opts)
             single.step(100000)
             assert np.array_equal(bits(single.estimate()), bits(x[m])), f"{columns} columns: column {m}"
+
+
+def test_a_large_batchs_columns_arrive_and_return_in_pieces(ctx):
+    # 48 columns of 11,970 unknowns are 4.4 MiB: one whole pinned piece of 4 MiB and the rest
+    ref = refcpu.Problem(block_config(0, divisions=(9, 7, 7)))
+    columns = 48
+    assert 4 << 20 < columns * ref.free_dofs * 8 < 8 << 20
+    csr = sf.CsrMatrix.new(ctx, *ref.csr())
+    setup = sf.MultigridSetup.new(ctx, csr, ref.rigid_modes(), ref.free_positions(), sf.MultigridOptions(coarse_dofs=100, precision=2, coarse_solve=1))
+    while not setup.step(2 ** 62):
+        pass
+    mg = setup.finish()
+    opts = sf.PcgOptions(tolerance=1e-8, dot_order=sf.DotOrder.TREE)
+    r = np.random.default_rng(5).standard_normal((columns, ref.free_dofs))
+    batch = sf.PcgBatch.new(ctx, csr, mg, r, opts)
+    assert batch.step(100000)[0] == 0
+    x = batch.estimate()
+    for m in (0, 41, 42, 43, columns - 1):  # the pieces meet in column 43
+        single = sf.Pcg.new(ctx, csr, mg, r[m], opts)
+        single.step(100000)
+        assert np.array_equal(bits(single.estimate()), bits(x[m])), f"column {m}"
