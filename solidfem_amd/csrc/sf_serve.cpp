@@ -553,7 +553,8 @@ void Server::serve(ServeSystem &system, const std::shared_ptr<Context> &ctx) {
     // batch does not beat (1.1 to 1.3 times its time). Two are a batch: on beams, tubes, a block and
     // plates of 19k to 603k DOFs it takes 0.63 to 0.71 times two single solves (block of 300k DOFs 10.5
     // ms against 16.5, plates of 55k 22.3 against 35.3, of 603k 286 against 429). Requests that arrive
-    // meanwhile wait for the next round, where they batch together.
+    // during a single solve wait for the next round, where they batch together; those that arrive
+    // during a batch take its free columns, as far as the rule below lets them.
     auto solve_alone = [&](u64 id, const std::vector<double> &b) {
         const sf_pcg_options pcg{options_.tolerance, 0, options_.dot_order, 0};
         sf_column_progress done{};
@@ -648,17 +649,24 @@ void Server::serve(ServeSystem &system, const std::shared_ptr<Context> &ctx) {
             slot[m] = 0;
             cv_.notify_all();
         }
-        // continuous batching: waiting requests take the free columns
+        // Continuous batching: waiting requests take the free columns, unless a batch that could be wider
+        // sees twice its own width waiting. Then its open columns finish and the next round starts a wider
+        // one: its width is fixed, and a column costs less the wider the batch (block of 300k DOFs: 5.7 ms
+        // at width 2, 3.5 at 4, 2.6 at 8, 1.7 at 32; a tube of 31k DOFs: 2.3, 1.4, 1.2, 0.5). With less
+        // waiting, a new batch and the columns left idle while the last ones finish cost as much as the
+        // width saves. Six requests after two: 77 ms at width 2, 55 with the wider batch (plate of 55k DOFs).
         std::vector<uint32_t> free_cols;
         for (uint32_t m = 0; m < M; ++m)
             if (!slot[m]) free_cols.push_back(m);
         std::vector<u64> more;
         std::vector<std::vector<double>> more_rhs;
+        bool refill = true;
         {
             std::lock_guard<std::mutex> g(mu_);
             if (stop_) return;
+            refill = M >= options_.max_columns || system.waiting.size() < 2 * (size_t)M;
         }
-        if (!free_cols.empty()) take(free_cols.size(), more, more_rhs);
+        if (refill && !free_cols.empty()) take(free_cols.size(), more, more_rhs);
         if (!more.empty()) {
             std::vector<uint32_t> cols;
             std::vector<const double *> ptrs;

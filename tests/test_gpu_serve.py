@@ -4,6 +4,7 @@ Every answer must be bit for bit the answer of the same problem solved alone by 
 with the same options (crates/solidfem-elastic/src/study.rs:191-372), whatever else is in flight.
 """
 import dataclasses
+import time
 
 import numpy as np
 import pytest
@@ -161,3 +162,28 @@ def test_models_of_meshes_sent_as_text_equal_themselves_alone(ctx):
         assert np.array_equal(bits(srv.result(rid)), bits(ref)), k
     assert sum(s.cache_hit for s in states) == 2  # the second and third load cases of the shared mesh
     assert srv.stats()["builds"] == 3
+
+
+def test_a_narrow_batch_gives_way_to_many_waiting_requests(ctx):
+    # two requests wait while their system is built, so its first batch has two columns; the thirty
+    # that arrive once it runs are batched wider than two, and every answer is that of its request alone
+    loads = [block_config(c, divisions=(20, 14, 14)) for c in range(32)]
+    srv = server()
+    ids = [srv.submit(w) for w in loads[:2]]
+    while srv.status(ids[0]).state in (sf.ServeState.QUEUED, sf.ServeState.BUILDING):
+        time.sleep(0.0005)
+    submitted = []
+    for w in loads[2:]:
+        submitted.append(time.monotonic())
+        ids.append(srv.submit(w))
+    states = [srv.wait(i, 300.0) for i in ids]
+    assert all(s.state == sf.ServeState.DONE for s in states), states
+    ends = [t + s.latency_seconds for t, s in zip(submitted, states[2:])]
+    starts = [e - s.solve_seconds for e, s in zip(ends, states[2:])]
+    # requests in one batch are solved at the same time
+    together = max(sum(a <= 0.5 * (s + e) <= b for a, b in zip(starts, ends)) for s, e in zip(starts, ends))
+    assert together >= 8, (together, sorted(starts), sorted(ends))
+    for k in (0, 1, 2, 13, 31):
+        ref, iterations = alone(ctx, loads[k])
+        assert states[k].iterations == iterations
+        assert np.array_equal(bits(srv.result(ids[k])), bits(ref)), k
