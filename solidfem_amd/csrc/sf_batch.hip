@@ -113,18 +113,20 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
     if (a.slices == 0 || M == 0) return;
     if (M > MAX_COLUMNS) throw Error(SF_ERR_INVALID_ARGUMENT, "more columns than a batch carries");
     if (batch == 0) {
-        int &tuned = a.batch_mm[columns_log2(M)];
-        if (!tuned) {
-            // a product into scratch vectors of this shape, timed for each depth
-            DeviceBuffer<V> tx(std::max<size_t>(a.block_cols * a.cb * M, 1)), ty(std::max<size_t>(a.rows * a.rb * M, 1));
-            SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));
-            SF_HIP(hipMemsetAsync(ty.ptr, 0, ty.bytes(), s));
-            tuned = tune_batch(s, [&](int depth) { launch_spmm<S, V>(a, M, tx.ptr, ty.ptr, ty.ptr, EPI_STORE, s, depth); },
-                               spmm_candidates(a.rb, a.cb, sizeof(S), M, true, staged_candidate(a, M)), "",
-                               "batch product " + std::to_string(columns_log2(M)) + " " + shape_class(a) + "|" + std::to_string(sizeof(V)));
-            SF_HIP(hipStreamSynchronize(s));
+        batch = a.mm_form[M];
+        if (!batch) {
+            batch = a.mm_times[columns_log2(M)].form(M, a.mm_form[M], [](int) { return true; }, [&] {
+                // a product into scratch vectors of this shape, timed for each form
+                DeviceBuffer<V> tx(std::max<size_t>(a.block_cols * a.cb * M, 1)), ty(std::max<size_t>(a.rows * a.rb * M, 1));
+                SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));
+                SF_HIP(hipMemsetAsync(ty.ptr, 0, ty.bytes(), s));
+                GroupTimes t = tune_group(s, M, [&](int form) { launch_spmm<S, V>(a, M, tx.ptr, ty.ptr, ty.ptr, EPI_STORE, s, form); },
+                                          spmm_candidates(a.rb, a.cb, sizeof(S), M, true, staged_candidate(a, M)),
+                                          "batch product " + std::to_string(columns_log2(M)) + " " + shape_class(a) + "|" + std::to_string(sizeof(V)));
+                SF_HIP(hipStreamSynchronize(s));
+                return t;
+            });
         }
-        batch = tuned;
     }
     if (batch >= FEW_FORM) {
         if (a.rb == 3 && M <= FEW_COLUMNS) {
@@ -175,8 +177,6 @@ template void launch_spmm<float, double>(const DeviceSliced<float> &, uint32_t, 
 template void launch_spmm<float, float>(const DeviceSliced<float> &, uint32_t, const float *, float *, const float *, int,
                                         hipStream_t, int, Start<float, float>);
 
-// Rows per wavefront of a rows form for M columns: its chains, 3 M a row, fit the 64 lanes.
-int rows_batch_rows(int form, uint32_t M) { return form - ROWS_BATCH_FORM == 4 && 12 * M <= (uint32_t)WAVE ? 4 : 2; }
 template <int RB, int M, int RPW, typename S, typename V>
 static void rows_batch_launch(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
     hipLaunchKernelGGL((rows_batch_kernel<RB, RB, M, RPW, S, V>), dim3((a.rows + RPW - 1) / RPW), dim3(WAVE),
@@ -196,30 +196,41 @@ void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, cons
     });
     SF_HIP(hipGetLastError());
 }
-// y = a x for M columns by wide_rows_batch_kernel; false where its buffers fit no LDS (nothing launched).
-template <typename S, typename V>
-bool launch_wide_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, hipStream_t s, Start<S, V> st, bool launch) {
-    if (a.rb != 6 || (a.cb != 3 && a.cb != 6) || a.rows == 0 || M == 0 || M > FEW_COLUMNS) return false;
-    bool fits = false;
+// f(CB, M) as compile-time constants for a restriction of M columns that wide_rows_batch_kernel takes.
+template <typename S, typename V, typename F>
+static void with_wide_rows_batch(const DeviceBsr<S> &a, uint32_t M, F &&f) {
+    if (a.rb != 6 || (a.cb != 3 && a.cb != 6) || a.rows == 0 || M == 0 || M > FEW_COLUMNS) return;
     with_columns(M, [&](auto columns) {
-        constexpr int MM = decltype(columns)::value;
         auto shape = [&](auto cb) {
-            constexpr int CB = decltype(cb)::value;
-            if constexpr (WideRowsBatch<CB, MM, V>::FITS) {
-                fits = true;
-                if (launch)
-                    hipLaunchKernelGGL((wide_rows_batch_kernel<CB, MM, S, V>), dim3(a.rows), dim3(WIDE_BATCH_THREADS), 0, s, a.view(), x, y, st);
-            }
+            if constexpr (WideRowsBatch<decltype(cb)::value, decltype(columns)::value, V>::FITS) f(cb, columns);
         };
         if (a.cb == 3) shape(std::integral_constant<int, 3>{});
         else shape(std::integral_constant<int, 6>{});
     });
-    if (launch && fits) SF_HIP(hipGetLastError());
+}
+template <typename S, typename V>
+bool wide_rows_batch_fits(const DeviceBsr<S> &a, uint32_t M) {
+    bool fits = false;
+    with_wide_rows_batch<S, V>(a, M, [&](auto, auto) { fits = true; });
     return fits;
 }
-template bool launch_wide_rows_batch<double, double>(const DeviceBsr<double> &, uint32_t, const double *, double *, hipStream_t, Start<double, double>, bool);
-template bool launch_wide_rows_batch<float, double>(const DeviceBsr<float> &, uint32_t, const double *, double *, hipStream_t, Start<float, double>, bool);
-template bool launch_wide_rows_batch<float, float>(const DeviceBsr<float> &, uint32_t, const float *, float *, hipStream_t, Start<float, float>, bool);
+template <typename S, typename V>
+void launch_wide_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, hipStream_t s, Start<S, V> st) {
+    bool launched = false;
+    with_wide_rows_batch<S, V>(a, M, [&](auto cb, auto columns) {
+        hipLaunchKernelGGL((wide_rows_batch_kernel<decltype(cb)::value, decltype(columns)::value, S, V>), dim3(a.rows), dim3(WIDE_BATCH_THREADS), 0,
+                           s, a.view(), x, y, st);
+        launched = true;
+    });
+    if (!launched) throw Error(SF_ERR_INTERNAL, "no wide rows form for this block shape or column count");
+    SF_HIP(hipGetLastError());
+}
+template bool wide_rows_batch_fits<double, double>(const DeviceBsr<double> &, uint32_t);
+template bool wide_rows_batch_fits<float, double>(const DeviceBsr<float> &, uint32_t);
+template bool wide_rows_batch_fits<float, float>(const DeviceBsr<float> &, uint32_t);
+template void launch_wide_rows_batch<double, double>(const DeviceBsr<double> &, uint32_t, const double *, double *, hipStream_t, Start<double, double>);
+template void launch_wide_rows_batch<float, double>(const DeviceBsr<float> &, uint32_t, const double *, double *, hipStream_t, Start<float, double>);
+template void launch_wide_rows_batch<float, float>(const DeviceBsr<float> &, uint32_t, const float *, float *, hipStream_t, Start<float, float>);
 
 template void launch_rows_batch<double, double>(const DeviceBsr<double> &, uint32_t, const double *, double *, const double *, int, hipStream_t, int,
                                                 Start<double, double>);
@@ -229,20 +240,23 @@ template void launch_rows_batch<float, float>(const DeviceBsr<float> &, uint32_t
                                               Start<float, float>);
 
 void DeviceSystem::multiply_batch(uint32_t M, const double *x, double *y, hipStream_t s) const {
-    // the form by rows is chosen per group of column counts, as the sliced product's is
-    int &form = rows_mm[columns_log2(M)];
-    if (rows.rows == 0 || M > FEW_COLUMNS) form = 0;
-    else if (form < 0) {
-        DeviceBuffer<double> tx(host.cols * 3 * M), ty(host.rows * 3 * M);
-        SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));
-        launch_spmm<double, double>(sliced, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s);  // its own choice first
-        std::vector<int> forms = rows_batch_forms();
-        forms.insert(forms.begin(), 0);
-        form = tune_batch(s, [&](int f) {
-            if (!f) launch_spmm<double, double>(sliced, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s);
-            else launch_rows_batch<double, double>(rows, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s, f, {nullptr, 0.0, nullptr, nullptr});
-        }, forms, "", "batch system rows " + std::to_string(columns_log2(M)) + " " + shape_class(sliced));
-        SF_HIP(hipStreamSynchronize(s));
+    int form = 0;
+    if (rows.rows && M <= FEW_COLUMNS) {
+        form = rows_mm[M];
+        if (form < 0)
+            form = rows_times[columns_log2(M)].form(M, rows_mm[M], [](int) { return true; }, [&] {
+                DeviceBuffer<double> tx(host.cols * 3 * M), ty(host.rows * 3 * M);
+                SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));
+                launch_spmm<double, double>(sliced, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s);  // its own choice first
+                std::vector<int> forms = rows_batch_forms();
+                forms.insert(forms.begin(), 0);
+                GroupTimes t = tune_group(s, M, [&](int f) {
+                    if (!f) launch_spmm<double, double>(sliced, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s);
+                    else launch_rows_batch<double, double>(rows, M, tx.ptr, ty.ptr, nullptr, EPI_STORE, s, f, {nullptr, 0.0, nullptr, nullptr});
+                }, forms, "batch system rows " + std::to_string(columns_log2(M)) + " " + shape_class(sliced));
+                SF_HIP(hipStreamSynchronize(s));
+                return t;
+            });
     }
     if (form) launch_rows_batch<double, double>(rows, M, x, y, nullptr, EPI_STORE, s, form, {nullptr, 0.0, nullptr, nullptr});
     else launch_spmm<double, double>(sliced, M, x, y, nullptr, EPI_STORE, s);

@@ -471,8 +471,7 @@ int fastest_rows(hipStream_t s, const std::function<void(int)> &launch, const st
     return fastest(s, launch, candidates, what, memo);
 }
 
-static int fastest_timed(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates,
-                         const std::string &what);
+static std::vector<float> form_times(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates);
 
 namespace {
 std::mutex g_memo_lock;
@@ -480,7 +479,33 @@ std::map<std::string, int> &tuning_memo() {
     static std::map<std::string, int> memo;
     return memo;
 }
+std::map<std::string, GroupTimes> &group_memo() {
+    static std::map<std::string, GroupTimes> memo;
+    return memo;
+}
 }  // namespace
+
+GroupTimes tune_group(hipStream_t s, uint32_t M, const std::function<void(int)> &launch, const std::vector<int> &candidates, const std::string &memo) {
+    const int forced = forced_variant().load(std::memory_order_relaxed);
+    for (int c : candidates)
+        if (forced > 0 && forced == c) return {M, {{forced, 0.0f}}};
+    std::string key = memo;
+    for (int c : candidates) key += "," + std::to_string(c);
+    {
+        std::lock_guard<std::mutex> g(g_memo_lock);
+        auto it = group_memo().find(key);
+        if (it != group_memo().end()) return it->second;
+    }
+    const std::vector<float> least = form_times(s, launch, candidates);
+    static const bool verbose = std::getenv("SOLIDFEM_TUNE_LOG") != nullptr;
+    GroupTimes t{M, {}};
+    for (size_t c = 0; c < candidates.size(); ++c) {
+        t.times.push_back({candidates[c], least[c]});
+        if (verbose) std::fprintf(stderr, "[tune] %s: %u columns: form %d: %.2f us\n", memo.c_str(), M, candidates[c], least[c] * 1e3f / 3);
+    }
+    std::lock_guard<std::mutex> g(g_memo_lock);
+    return group_memo().emplace(key, t).first->second;
+}
 
 int fastest(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates, const std::string &what,
             const std::string &memo) {
@@ -497,20 +522,25 @@ int fastest(hipStream_t s, const std::function<void(int)> &launch, const std::ve
             return it->second;
         }
     }
-    const int best = fastest_timed(s, launch, candidates, what);
+    const std::vector<float> least = form_times(s, launch, candidates);
+    size_t best = 0;
+    for (size_t c = 0; c < candidates.size(); ++c) {
+        if (verbose) std::fprintf(stderr, "[tune] %s: variant %d: %.2f us\n", what.c_str(), candidates[c], least[c] * 1e3f / 3);
+        if (least[c] < least[best]) best = c;
+    }
+    if (verbose) std::fprintf(stderr, "[tune] %s: chose %d\n", what.c_str(), candidates[best]);
     if (!key.empty()) {
         std::lock_guard<std::mutex> g(g_memo_lock);
-        tuning_memo().emplace(key, best);
+        tuning_memo().emplace(key, candidates[best]);
     }
-    return best;
+    return candidates[best];
 }
 
-static int fastest_timed(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates,
-                         const std::string &what) {
+// The least time of three launches of each candidate.
+static std::vector<float> form_times(hipStream_t s, const std::function<void(int)> &launch, const std::vector<int> &candidates) {
     hipEvent_t e0, e1;
     SF_HIP(hipEventCreate(&e0));
     SF_HIP(hipEventCreate(&e1));
-    static const bool verbose = std::getenv("SOLIDFEM_TUNE_LOG") != nullptr;
     // two rounds over the candidates, each candidate's best kept: a drift in the GPU's state
     // during the first round (clocks, what the caches hold) does not decide the choice
     std::vector<float> least(candidates.size(), 1e30f);
@@ -526,19 +556,9 @@ static int fastest_timed(hipStream_t s, const std::function<void(int)> &launch, 
             SF_HIP(hipEventElapsedTime(&ms, e0, e1));
             least[c] = std::min(least[c], ms);
         }
-    int best = candidates.front();
-    float best_ms = 1e30f;
-    for (size_t c = 0; c < candidates.size(); ++c) {
-        if (verbose) std::fprintf(stderr, "[tune] %s: variant %d: %.2f us\n", what.c_str(), candidates[c], least[c] * 1e3f / 3);
-        if (least[c] < best_ms) {
-            best_ms = least[c];
-            best = candidates[c];
-        }
-    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (verbose) std::fprintf(stderr, "[tune] %s: chose %d\n", what.c_str(), best);
-    return best;
+    return least;
 }
 
 template <typename S, typename V>
@@ -616,9 +636,10 @@ struct LevelDev {
     DeviceBuffer<V> b, x, d0, d1, r0, r1, res, px;
     // the same work vectors for several columns (row-interleaved), grown on demand
     DeviceBuffer<V> mb, mx, md0, md1, mr0, mr1, mres, mpx;
-    // batch depths of the batched kernels per log2 of the column group: Chebyshev step, residual,
-    // restriction, prolongation (0 = not tuned yet)
-    int mm_depth[8][4] = {};
+    // The batched kernels' times per log2 of the column group, and the form taken for each count: Chebyshev
+    // step, residual, restriction, prolongation (0 = not chosen yet).
+    GroupTimes mm_times[8][4];
+    int mm_form[MAX_COLUMNS + 1][4] = {};
 };
 
 template <typename S, typename V>
@@ -976,8 +997,6 @@ class Hierarchy final : public DeviceMultigrid {
     static void launch_cheb_batch(LevelDev<S, V> &d, int batch, uint32_t M, const V *d_in, const V *r_in, V keep, V stp,
                                   V *d_out, V *r_out, V *x, V *into, hipStream_t s, double *widen = nullptr) {
         if (d.a.slices == 0) return;
-        // a choice made for another column count of the group
-        if (batch > ROWS_BATCH_FORM && batch < FEW_FORM && !rows_batch_fits<V>(d.rb, M)) batch = 2;
         if (batch >= FEW_FORM) {
             with_columns(M, [&](auto columns) {
                 hipLaunchKernelGGL((cheb_step_few_kernel<3, decltype(columns)::value, S, V>), dim3(grid_for(d.a.slices, 4)), dim3(256), 0, s,
@@ -1012,16 +1031,12 @@ class Hierarchy final : public DeviceMultigrid {
     }
     // The restriction y = R x for M columns, with the start of the coarser level's smoothing where given.
     static void restrict_batch(LevelDev<S, V> &d, int form, uint32_t M, const V *x, V *y, hipStream_t s, Start<S, V> st) {
-        if (form == WIDE_ROWS) {
-            if (launch_wide_rows_batch<S, V>(d.r_rows, M, x, y, s, st, true)) return;
-            form = 2;  // a choice made for another column count of the group
-        }
-        launch_spmm<S, V>(d.r, M, x, y, nullptr, EPI_STORE, s, form, st);
+        if (form == WIDE_ROWS) launch_wide_rows_batch<S, V>(d.r_rows, M, x, y, s, st);
+        else launch_spmm<S, V>(d.r, M, x, y, nullptr, EPI_STORE, s, form, st);
     }
     // res = b - A x for M columns, optionally with the start of the smoothing that follows.
     static void residual_batch(LevelDev<S, V> &d, int form, uint32_t M, const V *x, const V *b, hipStream_t s,
                                Start<S, V> st = {nullptr, (V)0, nullptr, nullptr}) {
-        if (form > ROWS_BATCH_FORM && form < FEW_FORM && !rows_batch_fits<V>(d.rb, M)) form = 2;  // as launch_cheb_batch
         if (form > ROWS_BATCH_FORM && form < FEW_FORM) launch_rows_batch<S, V>(d.a_rows, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
         else launch_spmm<S, V>(d.a, M, x, d.mres.ptr, b, EPI_RESIDUAL, s, form, st);
     }
@@ -1045,32 +1060,34 @@ class Hierarchy final : public DeviceMultigrid {
         const std::string group = std::to_string(lg) + " ", vsize = "|" + std::to_string(sizeof(V));
         for (size_t l = 0; l < lv_.size(); ++l) {
             LevelDev<S, V> &d = lv_[l];
-            if (d.mm_depth[lg][0]) continue;
+            if (d.mm_form[M][0]) continue;
             const size_t need = d.n * (size_t)M;
             V *vs[8] = {d.mb.ptr, d.mx.ptr, d.md0.ptr, d.md1.ptr, d.mr0.ptr, d.mr1.ptr, d.mres.ptr, d.mpx.ptr};
             for (V *v : vs) SF_HIP(hipMemsetAsync(v, 0, need * sizeof(V), s));
-            d.mm_depth[lg][0] = tune_batch(s, [&](int batch) {
-                launch_cheb_batch(d, batch, M, d.md0.ptr, d.mb.ptr, (V)0, (V)0, d.md1.ptr, d.mr0.ptr, d.mx.ptr, nullptr, s);
-            }, with_rows_batch(spmm_candidates(d.rb, d.rb, sizeof(S), M, false), d, M), "", "batch step " + group + shape_class(d.a) + vsize);
-            d.mm_depth[lg][1] = tune_batch(s, [&](int batch) {
-                residual_batch(d, batch, M, d.mx.ptr, d.mb.ptr, s);
-            }, with_rows_batch(spmm_candidates(d.rb, d.rb, sizeof(S), M, true, staged_candidate(d.a, M)), d, M), "",
-               "batch residual " + group + shape_class(d.a) + vsize);
+            auto tune = [&](int which, auto fits, const std::function<void(int)> &launch, const std::vector<int> &candidates, const std::string &memo) {
+                GroupTimes &times = d.mm_times[lg][which];
+                if (!times.columns) times = tune_group(s, M, launch, candidates, memo);
+                d.mm_form[M][which] = times.form(M, fits);
+            };
+            auto level_fits = [&](int form) { return form <= ROWS_BATCH_FORM || form >= FEW_FORM || rows_batch_fits<V>(d.rb, M); };
+            tune(0, level_fits, [&](int form) { launch_cheb_batch(d, form, M, d.md0.ptr, d.mb.ptr, (V)0, (V)0, d.md1.ptr, d.mr0.ptr, d.mx.ptr, nullptr, s); },
+                 with_rows_batch(spmm_candidates(d.rb, d.rb, sizeof(S), M, false), d, M), "batch step " + group + shape_class(d.a) + vsize);
+            tune(1, level_fits, [&](int form) { residual_batch(d, form, M, d.mx.ptr, d.mb.ptr, s); },
+                 with_rows_batch(spmm_candidates(d.rb, d.rb, sizeof(S), M, true, staged_candidate(d.a, M)), d, M),
+                 "batch residual " + group + shape_class(d.a) + vsize);
             if (d.has_p) {
                 LevelDev<S, V> &c = lv_[l + 1];
                 const size_t cneed = c.n * (size_t)M;
                 SF_HIP(hipMemsetAsync(c.mb.ptr, 0, cneed * sizeof(V), s));
                 SF_HIP(hipMemsetAsync(c.mx.ptr, 0, cneed * sizeof(V), s));
                 std::vector<int> restrict_forms = spmm_candidates(d.r.rb, d.r.cb, sizeof(S), M, true, staged_candidate(d.r, M));
-                if (launch_wide_rows_batch<S, V>(d.r_rows, M, d.mres.ptr, c.mb.ptr, s, {nullptr, (V)0, nullptr, nullptr}, false))
-                    restrict_forms.push_back(WIDE_ROWS);
-                d.mm_depth[lg][2] = tune_batch(s, [&](int batch) {
-                    restrict_batch(d, batch, M, d.mres.ptr, c.mb.ptr, s, {nullptr, (V)0, nullptr, nullptr});
-                }, restrict_forms, "", "batch restriction " + group + shape_class(d.r) + vsize);
-                d.mm_depth[lg][3] = tune_batch(s, [&](int batch) {
-                    launch_spmm<S, V>(d.p, M, c.mx.ptr, d.mpx.ptr, nullptr, EPI_ADD, s, batch);
-                }, spmm_candidates(d.p.rb, d.p.cb, sizeof(S), M, true, staged_candidate(d.p, M)), "",
-                   "batch prolongation " + group + shape_class(d.p) + vsize);
+                const bool wide = wide_rows_batch_fits<S, V>(d.r_rows, M);
+                if (wide) restrict_forms.push_back(WIDE_ROWS);
+                tune(2, [&](int form) { return form != WIDE_ROWS || wide; },
+                     [&](int form) { restrict_batch(d, form, M, d.mres.ptr, c.mb.ptr, s, {nullptr, (V)0, nullptr, nullptr}); }, restrict_forms,
+                     "batch restriction " + group + shape_class(d.r) + vsize);
+                tune(3, [](int) { return true; }, [&](int form) { launch_spmm<S, V>(d.p, M, c.mx.ptr, d.mpx.ptr, nullptr, EPI_ADD, s, form); },
+                     spmm_candidates(d.p.rb, d.p.cb, sizeof(S), M, true, staged_candidate(d.p, M)), "batch prolongation " + group + shape_class(d.p) + vsize);
             }
         }
         SF_HIP(hipStreamSynchronize(s));
@@ -1078,7 +1095,6 @@ class Hierarchy final : public DeviceMultigrid {
 
     // smooth() for M columns.
     void smooth_batch(LevelDev<S, V> &d, const V *b, V *x, V *sum_into, uint32_t M, hipStream_t s, bool started, double *widen = nullptr) {
-        const int lg = columns_log2(M);
         if (!started) {
             const unsigned g = grid_for(d.rows * (size_t)M, 256);
             if (d.rb == 3)
@@ -1103,7 +1119,7 @@ class Hierarchy final : public DeviceMultigrid {
             const V *r_in = k == 1 ? b : rr[(k - 1) & 1];
             const V keep = (V)d.steps[k - 1].first, stp = (V)d.steps[k - 1].second;
             V *into = k == steps ? sum_into : nullptr;
-            launch_cheb_batch(d, d.mm_depth[lg][0], M, d_in, r_in, keep, stp, dd[k & 1], rr[k & 1], x, into, s, into ? widen : nullptr);
+            launch_cheb_batch(d, d.mm_form[M][0], M, d_in, r_in, keep, stp, dd[k & 1], rr[k & 1], x, into, s, into ? widen : nullptr);
         }
         Profiler::get().end(3, token, s);
         if (steps == 0 && sum_into) {
@@ -1117,7 +1133,6 @@ class Hierarchy final : public DeviceMultigrid {
     // cycle() for M columns.
     void cycle_batch(size_t l, const V *b, V *x, uint32_t M, hipStream_t s, bool started = false, double *widen = nullptr) {
         LevelDev<S, V> &d = lv_[l];
-        const int lg = columns_log2(M);
         if (!d.has_p) {
             if (d.has_factor) {
                 if (d.inverse.ptr && d.n * (size_t)M <= COARSE_SUMS_MOST)
@@ -1135,14 +1150,14 @@ class Hierarchy final : public DeviceMultigrid {
         }
         LevelDev<S, V> &c = lv_[l + 1];
         smooth_batch(d, b, x, nullptr, M, s, started);
-        residual_batch(d, d.mm_depth[lg][1], M, x, b, s);
+        residual_batch(d, d.mm_form[M][1], M, x, b, s);
         // restriction and residual with the start of the smoothing that follows, as cycle()
         const bool fuse = smooths_first(c);
         const Start<S, V> first = {fuse ? c.dinv.ptr : nullptr, (V)c.theta, c.md0.ptr, c.mx.ptr};
-        restrict_batch(d, d.mm_depth[lg][2], M, d.mres.ptr, c.mb.ptr, s, first);
+        restrict_batch(d, d.mm_form[M][2], M, d.mres.ptr, c.mb.ptr, s, first);
         cycle_batch(l + 1, c.mb.ptr, c.mx.ptr, M, s, fuse);
-        launch_spmm<S, V>(d.p, M, c.mx.ptr, x, nullptr, EPI_ADD, s, d.mm_depth[lg][3]);
-        residual_batch(d, d.mm_depth[lg][1], M, x, b, s, {d.dinv.ptr, (V)d.theta, d.md0.ptr, d.mpx.ptr});
+        launch_spmm<S, V>(d.p, M, c.mx.ptr, x, nullptr, EPI_ADD, s, d.mm_form[M][3]);
+        residual_batch(d, d.mm_form[M][1], M, x, b, s, {d.dinv.ptr, (V)d.theta, d.md0.ptr, d.mpx.ptr});
         smooth_batch(d, d.mres.ptr, d.mpx.ptr, x, M, s, true, widen);
     }
 

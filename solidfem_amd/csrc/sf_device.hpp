@@ -47,6 +47,65 @@ struct SlicedPlan {
 };
 SlicedPlan plan_sliced(const int64_t *starts, const u32 *columns, size_t rows, int rb, int cb);
 
+// Columns one batched solve carries: a group of lanes per block row, one lane per column.
+constexpr uint32_t MAX_COLUMNS = 64;
+// A batched kernel's variant code: below NODE_FORM, the lane-group form with that depth (blocks in
+// flight); from NODE_FORM, the one-wavefront-per-block-row form with depth (code - NODE_FORM);
+// from PAIR_FORM, QUAD_FORM and OCT_FORM, the lane-group form whose lanes take two, four or
+// eight consecutive columns each (for M a multiple of that; otherwise the one-column form of the
+// same depth).
+constexpr int NODE_FORM = 16;
+constexpr int PAIR_FORM = 32;
+constexpr int QUAD_FORM = 48;
+constexpr int OCT_FORM = 64;  // eight columns per lane
+constexpr int STAGED_FORM = 80;  // products only: one workgroup per block row, chunks staged in LDS
+constexpr int WIDE_ROWS = 96;       // restrictions only: four wavefronts per block row
+constexpr int ROWS_BATCH_FORM = 112;  // plus 2 or 4: up to FEW_COLUMNS columns by plain block rows (rows_batch_forms)
+constexpr int FEW_FORM = 128;    // a lane per scalar row with up to FEW_COLUMNS columns, blocks of three rows
+constexpr uint32_t FEW_COLUMNS = 8;
+
+// Rows per wavefront of a rows form (3 x 3 blocks) for M columns: its chains, 3 M a row, fit the 64 lanes.
+inline int rows_batch_rows(int form, uint32_t M) { return form - ROWS_BATCH_FORM == 4 && 12 * M <= (uint32_t)dev::WAVE ? 4 : 2; }
+// The times of a batched kernel's forms at one column count, which choose the form for each count of its
+// group (1, 2, 3-4, 5-8, ...). The forms of few columns take time with the count (five columns to eight:
+// 1.3 to 1.9 times as long on a 31k-DOF tube), while a lane-group form takes the group's whole power of
+// two lanes whatever the count (within 3%): for more columns than were timed, the former are scaled up. A
+// form that does not take a count (its buffers fit no LDS), or takes it with fewer rows a wavefront, is
+// not that count's. With the first count's choice for the whole group, eight columns after five took 17.5
+// ms a solve of that tube in double, 11.9 with their own.
+struct GroupTimes {
+    uint32_t columns = 0;  // 0: not timed
+    std::vector<std::pair<int, float>> times;
+    template <typename F>
+    int form(uint32_t M, F &&fits) const {
+        int best = 2;  // two blocks in flight take every count
+        float least = 1e30f;
+        for (const auto &t : times) {
+            const bool per_column = t.first == WIDE_ROWS || t.first > ROWS_BATCH_FORM;
+            const float ms = per_column && M > columns ? t.second * (float)M / (float)columns : t.second;
+            if (t.first > ROWS_BATCH_FORM && t.first < FEW_FORM && rows_batch_rows(t.first, M) < rows_batch_rows(t.first, columns)) continue;
+            if (ms < least && fits(t.first)) {
+                least = ms;
+                best = t.first;
+            }
+        }
+        return best;
+    }
+    // The same for matrices that several threads may use: `chosen` is set, timing by `time` at first use.
+    template <typename F, typename T>
+    int form(uint32_t M, int &chosen, F &&fits, T &&time) {
+        static std::mutex lock;
+        {
+            std::lock_guard<std::mutex> g(lock);
+            if (columns) return chosen = form(M, fits);
+        }
+        GroupTimes t = time();
+        std::lock_guard<std::mutex> g(lock);
+        if (!columns) *this = std::move(t);
+        return chosen = form(M, fits);
+    }
+};
+
 template <typename T>
 struct DeviceSliced {
     int rb = 3, cb = 3;
@@ -56,7 +115,8 @@ struct DeviceSliced {
     DeviceBuffer<T> vals;
     int batch_spmv = 4;  // blocks in flight per lane, chosen by tune_batch
     int batch_cheb = 4;
-    mutable int batch_mm[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // batched product, per log2 of the column group
+    mutable GroupTimes mm_times[8];                 // the batched product's, per log2 of the column group
+    mutable int mm_form[MAX_COLUMNS + 1] = {};       // its form per column count (0: not chosen)
     mutable uint32_t passes = 0;  // launches so far, for the alternating traversal
     // The view one launch takes; each call is one pass (see dev::slice_of for the orders).
     dev::Sliced<T> view() const {
@@ -105,7 +165,6 @@ void build_bsr(DeviceBsr<T> &out, const HostBsr<double> &pattern, const double *
 // The forms of the row kernels: block rows per wavefront + 256 * (blocks a lane loads at once - 1),
 // or WIDE_ROWS: four wavefronts per block row (wide_rows_kernel, wide_rows_batch_kernel; restrictions only).
 // sf_force_variant(WIDE_ROWS) forces the latter on every restriction.
-constexpr int WIDE_ROWS = 96;
 constexpr int rows_form_code(int rows, int blocks) { return rows + 256 * (blocks - 1); }
 // The forms worth timing against the sliced kernel (0) for blocks of `bytes` in the vector's
 // precision: a lane keeps U blocks in registers and a wavefront 64 U of them in LDS. (Four blocks a
@@ -178,20 +237,6 @@ std::string shape_class(const DeviceSliced<T> &a) {
 
 // ---- several right-hand sides ------------------------------------------------------------------
 
-// Columns one batched solve carries: a group of lanes per block row, one lane per column.
-constexpr uint32_t MAX_COLUMNS = 64;
-// A batched kernel's variant code: below NODE_FORM, the lane-group form with that depth (blocks in
-// flight); from NODE_FORM, the one-wavefront-per-block-row form with depth (code - NODE_FORM);
-// from PAIR_FORM, QUAD_FORM and OCT_FORM, the lane-group form whose lanes take two, four or
-// eight consecutive columns each (for M a multiple of that; otherwise the one-column form of the
-// same depth).
-constexpr int NODE_FORM = 16;
-constexpr int PAIR_FORM = 32;
-constexpr int QUAD_FORM = 48;
-constexpr int OCT_FORM = 64;  // eight columns per lane
-constexpr int STAGED_FORM = 80;  // products only: one workgroup per block row, chunks staged in LDS
-constexpr int FEW_FORM = 128;    // a lane per scalar row with up to FEW_COLUMNS columns, blocks of three rows
-constexpr uint32_t FEW_COLUMNS = 8;
 // Calls f(M) as a compile-time constant for M of 1 to FEW_COLUMNS columns.
 template <typename F>
 void with_columns(uint32_t M, F &&f) {
@@ -226,7 +271,6 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
                  dev::Start<S, V> start = {nullptr, (V)0, nullptr, nullptr});
 // The forms of products and steps by plain block rows for few columns (rows_sum_batch): 3 x 3 blocks
 // with ROWS_BATCH_FORM + block rows per wavefront, 6 x 6 blocks (one row a wavefront) with the first code.
-constexpr int ROWS_BATCH_FORM = 112;
 inline std::vector<int> rows_batch_forms(int rb = 3) {
     return rb == 3 ? std::vector<int>{ROWS_BATCH_FORM + 2, ROWS_BATCH_FORM + 4} : std::vector<int>{ROWS_BATCH_FORM + 2};
 }
@@ -235,14 +279,17 @@ template <typename V>
 bool rows_batch_fits(int rb, uint32_t M) {
     return M <= FEW_COLUMNS && (rb == 3 || (rb == 6 && (size_t)6 * M * (32 * 6 * sizeof(V) + 16) <= 65536));
 }
-int rows_batch_rows(int form, uint32_t M);
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, dev::Start<S, V> start);
-// The restriction of few columns by wide_rows_batch_kernel (form WIDE_ROWS of a batched restriction).
-// False, and nothing launched, for another block shape, more columns or too large buffers; with
-// `launch` false it only answers.
+// The restriction of few columns by wide_rows_batch_kernel (form WIDE_ROWS of a batched restriction), and
+// whether it takes a matrix's block shape and M columns' buffers.
 template <typename S, typename V>
-bool launch_wide_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, hipStream_t s, dev::Start<S, V> start, bool launch);
+bool wide_rows_batch_fits(const DeviceBsr<S> &a, uint32_t M);
+template <typename S, typename V>
+void launch_wide_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, hipStream_t s, dev::Start<S, V> start);
+// The times of `candidates` at M columns, from the memo where its class has them, or the forced form alone.
+GroupTimes tune_group(hipStream_t s, uint32_t M, const std::function<void(int)> &launch, const std::vector<int> &candidates,
+                      const std::string &memo);
 // The batch depths worth trying for a matrix's batched product.
 // The variant codes a batched product (`product`) or Chebyshev step is timed over for M columns.
 std::vector<int> spmm_candidates(int rb, int cb, size_t value_size, uint32_t M, bool product = true, bool staged = false);
@@ -335,7 +382,8 @@ struct DeviceSystem {
     DeviceSliced<double> sliced;
     DeviceBsr<double> rows;  // a small system's pattern over `values`, for the row kernels
     int rows_form = 0;       // the product's form: 0 sliced, else of the row kernels (by timing)
-    mutable int rows_mm[8] = {-1, -1, -1, -1, -1, -1, -1, -1};  // the batched product's, per log2 of the column group (-1: not tuned)
+    mutable GroupTimes rows_times[4];                // the batched product's by rows, per log2 of the column group
+    mutable int rows_mm[FEW_COLUMNS + 1] = {-1, -1, -1, -1, -1, -1, -1, -1, -1};  // its form per column count (-1: not chosen, 0: sliced)
     // y = A x, and Y = A X for M row-interleaved columns
     void multiply(const double *x, double *y, hipStream_t s) const;
     void multiply_batch(uint32_t M, const double *x, double *y, hipStream_t s) const;

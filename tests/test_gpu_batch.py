@@ -5,6 +5,8 @@ batch runs that recurrence per column in lockstep. Every column must be bit for 
 single-column solve of that column -- and so, with the dot products in the reference's order,
 the oracle's solve of that load case -- whatever the other columns hold.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -218,3 +220,33 @@ def test_each_batched_form_gives_each_column_its_single_bits(ctx, forced_variant
         z = mg.apply_batch(r)
         for m in range(columns):
             assert np.array_equal(bits(z[m]), bits(mg.apply(r[m]))), f"{columns} columns: column {m}"
+
+
+@pytest.mark.parametrize("first,then", [(5, 8), (3, 4)])
+def test_a_batchs_speed_does_not_depend_on_its_groups_first_count(ctx, first, then):
+    # forms are timed once for a group of column counts (3 and 4, 5 to 8); where the first count's choice
+    # does not take a later one (double, six-row blocks: too much LDS), that one has a choice as good as
+    # its own would be: with the least-effort form instead, eight columns took 1.47 times as long
+    def part():
+        # another density of mesh per parameter: another shape class, so no choice is kept from before
+        w = sf.Workload(size=(60.0, 6.0, 6.0), divisions=(60 - first, 6, 6), clamp_axis=0, load_axis=0, load_value=60.0, youngs=200000.0,
+                        poisson=0.29, wall_cells=1, wall_thickness=1.0, traction_kind=1, traction_scale=1.0, traction_seed=3)
+        b = sf.StudyBuilder.new(ctx, sf.Model.from_workload(w), sf.PcgOptions(tolerance=1e-8, dot_order=sf.DotOrder.TREE),
+                                sf.MultigridOptions(precision=sf.Precision.DOUBLE, coarse_solve=1))
+        b.step(2 ** 62)
+        return b.finish()
+
+    def seconds(study, columns):
+        rhs = study.rhs() * np.random.default_rng(columns).uniform(0.5, 2.0, (columns, 1))
+        batch = sf.PcgBatch.new(ctx, study.system(), study.multigrid(), rhs, sf.PcgOptions(tolerance=1e-8, dot_order=sf.DotOrder.TREE))
+        best = 1e9
+        for _ in range(6):
+            batch.restart(rhs)
+            t = time.perf_counter()
+            batch.step(10000)
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    own, after = part(), part()
+    seconds(after, first)
+    assert seconds(after, then) < 1.2 * seconds(own, then)
