@@ -100,8 +100,11 @@ Server::~Server() {
 u64 Server::estimate(const ServeRequest &r) const {
     // A structured box of Tet10: (2 nx + 1)(2 ny + 1)(2 nz + 1) nodes with at most 27 blocks per
     // block row; a model's mesh: its nodes, and at most its 100 block pairs per element. The system
-    // holds the assembled f64 blocks twice (row-major and sliced), the hierarchy about 0.6 of that
-    // again in f64, and a full batch 14 vectors of every column.
+    // holds the assembled f64 blocks twice (row-major and sliced) and the finest level's in the V-cycle's
+    // storage; a small one that level and the system's pattern in plain block rows too. Transfers, coarser
+    // levels and one column's vectors take 48 B a block and half as much again as the finest level. That
+    // covers, by at most 60%, what beams, blocks and plates of 20k to 300k DOFs hold in each precision
+    // with 1 to 32 columns (without the plain rows and the transfers it was up to 47% short in double).
     const sf_workload &w = r.workload;
     double nodes, blocks;
     if (r.model) {
@@ -111,9 +114,17 @@ u64 Server::estimate(const ServeRequest &r) const {
         nodes = (2.0 * w.divisions[0] + 1) * (2.0 * w.divisions[1] + 1) * (2.0 * w.divisions[2] + 1);
         blocks = 27 * nodes;
     }
-    const double dofs = 3 * nodes;
-    const double system = blocks * (72 + 80) * 1.6 + dofs * 8 * 24;
-    const double batch = dofs * options_.max_columns * (10 * 8 + 1.4 * 8 * vector_size(options_.precision));
+    const double level = options_.precision == SF_PRECISION_DOUBLE ? 76 : 40;
+    const double rows = blocks <= (double)ROWS_BLOCKS ? level + 4 : 0;
+    const double system = 1.1 * blocks * (72 + 76 + level + rows + 48 + 1.5 * level);
+    // A full batch: nine f64 vectors of every column, eight in the V-cycle's precision (0.4 as much on the
+    // coarser levels), two more where that is not f64. The driver hands out large buffers in 2 MB units.
+    auto buffer = [](double bytes) {
+        constexpr double unit = 2 << 20;
+        return bytes > unit ? std::ceil(bytes / unit) * unit : bytes;
+    };
+    const double column = 3 * nodes * options_.max_columns, v = (double)vector_size(options_.precision);
+    const double batch = 9 * buffer(8 * column) + (v == 4 ? 10 : 8) * buffer(v * column) + 0.4 * 8 * v * column;
     return (u64)(system + batch);
 }
 

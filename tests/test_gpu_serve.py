@@ -8,6 +8,7 @@ import time
 
 import numpy as np
 import pytest
+import torch
 
 import solidfem_amd as sf
 from workloads import block_config, stretch_components, stretched_cube
@@ -187,3 +188,32 @@ def test_a_narrow_batch_gives_way_to_many_waiting_requests(ctx):
         ref, iterations = alone(ctx, loads[k])
         assert states[k].iterations == iterations
         assert np.array_equal(bits(srv.result(ids[k])), bits(ref)), k
+
+
+@pytest.mark.parametrize("size,divisions", [((100.0, 10.0, 10.0), (40, 4, 4)), ((32.0, 28.0, 28.0), (16, 14, 14)),
+                                            ((33.0, 31.0, 0.8), (33, 31, 2)), ((60.0, 40.0, 40.0), (30, 20, 20))],
+                         ids=["beam", "block", "plate", "large-block"])
+@pytest.mark.parametrize("precision", [0, 1, 2], ids=["double", "single-storage", "single"])
+@pytest.mark.parametrize("columns", [1, 2, 4, 32])
+def test_the_reservation_covers_what_a_system_and_its_batch_hold(ctx, size, divisions, precision, columns):
+    w = dataclasses.replace(block_config(0, divisions=divisions), size=size, load_value=size[2])
+    srv = server(precision=sf.Precision(precision), max_columns=columns)
+    rid = srv.submit(w)
+    assert srv.wait(rid, 120.0).state == sf.ServeState.DONE
+    reserved = srv.stats()["hbm_reserved"]
+    del srv
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    pcg = sf.PcgOptions(tolerance=OPTIONS["tolerance"], dot_order=OPTIONS["dot_order"])
+    mg = sf.MultigridOptions(precision=sf.Precision(precision), coarse_solve=OPTIONS["coarse_solve"])
+    before = free()
+    b = sf.StudyBuilder.new(ctx, sf.Model.from_workload(w), pcg, mg)
+    b.step(2 ** 62)
+    study = b.finish()
+    batch = sf.PcgBatch.new(ctx, study.system(), study.multigrid(), np.stack([study.rhs()] * columns), pcg)
+    batch.step(2)
+    held = before - free()
+    assert 0 < held <= reserved <= 1.6 * held, (held / 2 ** 20, reserved / 2 ** 20)
