@@ -270,7 +270,8 @@ __device__ __forceinline__ V add_terms(V sum, const V *t, uint32_t n) {
 // Adds onto acc, in order, the 16 bytes of terms that lanes FIRST .. FIRST + 3 of the lane's row of 16
 // hold, one instruction a term: the term comes from its lane with the addition. For double that is
 // fma(t, 1, acc), the same value, the product being exact. One block of instructions: between two
-// blocks the compiler would put a wait state each.
+// blocks the compiler would put a wait state each. The sum is written before the block's inputs are all
+// read, so its register is its own (an early clobber), also where it starts with an input's value.
 template <int FIRST>
 __device__ __forceinline__ void add_from_lanes(float &acc, float x, float y, float z, float w) {
 #define SF_ADD(N)                                                                          \
@@ -279,7 +280,7 @@ __device__ __forceinline__ void add_from_lanes(float &acc, float x, float y, flo
     "v_add_f32_dpp %0, %3, %0 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"           \
     "v_add_f32_dpp %0, %4, %0 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"
     asm("s_nop 1\n" SF_ADD(5) SF_ADD(6) SF_ADD(7) SF_ADD(8)
-        : "+v"(acc)
+        : "+&v"(acc)
         : "v"(x), "v"(y), "v"(z), "v"(w), "n"(FIRST), "n"(FIRST + 1), "n"(FIRST + 2), "n"(FIRST + 3));
 #undef SF_ADD
 }
@@ -289,7 +290,7 @@ __device__ __forceinline__ void add_from_lanes(double &acc, double x, double y) 
     "v_fmac_f64_dpp %0, %1, %3 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"             \
     "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"
     asm("s_nop 1\n" SF_ADD(4) SF_ADD(5) SF_ADD(6) SF_ADD(7)
-        : "+v"(acc)
+        : "+&v"(acc)
         : "v"(x), "v"(y), "v"(1.0), "n"(FIRST), "n"(FIRST + 1), "n"(FIRST + 2), "n"(FIRST + 3));
 #undef SF_ADD
 }
@@ -312,7 +313,7 @@ __device__ __forceinline__ void add_three_from_lanes(double (&acc)[3], const dou
     "v_fmac_f64_dpp %2, %" #C ", %16 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n"
 #define SF_LANE(N) SF_ADD(3, 6, 9, N) SF_ADD(4, 7, 10, N) SF_ADD(5, 8, 11, N)
     asm("s_nop 1\n" SF_LANE(12) SF_LANE(13) SF_LANE(14) SF_LANE(15)
-        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2])
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2])
         : "v"(t[0][0]), "v"(t[0][1]), "v"(t[0][2]), "v"(t[1][0]), "v"(t[1][1]), "v"(t[1][2]), "v"(t[2][0]), "v"(t[2][1]), "v"(t[2][2]),
           "n"(FIRST), "n"(FIRST + 1), "n"(FIRST + 2), "n"(FIRST + 3), "v"(1.0));
 #undef SF_LANE
