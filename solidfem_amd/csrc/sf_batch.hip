@@ -180,7 +180,7 @@ template void launch_spmm<float, float>(const DeviceSliced<float> &, uint32_t, c
 template <int RB, int M, int RPW, typename S, typename V>
 static void rows_batch_launch(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
     hipLaunchKernelGGL((rows_batch_kernel<RB, RB, M, RPW, S, V>), dim3((a.rows + RPW - 1) / RPW), dim3(WAVE),
-                       ((size_t)RPW * RB * M * ROWS_BATCH_STRIDE<RB, RB, V, RPW> * sizeof(V)), s, a.view(), epi, x, y, b, st);
+                       (ROWS_BATCH_LDS<RB, M, RPW, V>), s, a.view(), epi, x, y, b, st);
 }
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, Start<S, V> st) {

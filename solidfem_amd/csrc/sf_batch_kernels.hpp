@@ -736,6 +736,8 @@ template <int RB, int RPW>
 constexpr int ROWS_BATCH_BLOCKS = WAVE / RPW / (RB / 3);  // blocks of a row at a time
 template <int RB, int CB, typename V, int RPW>
 constexpr int ROWS_BATCH_STRIDE = ROWS_BATCH_BLOCKS<RB, RPW> * CB + 16 / sizeof(V);  // entries of a chain's room
+template <int RB, int M, int RPW, typename V>
+constexpr size_t ROWS_BATCH_LDS = (size_t)RPW * RB * M * ROWS_BATCH_STRIDE<RB, RB, V, RPW> * sizeof(V);  // all that a launch takes
 template <int RB, int CB, int M, int RPW, typename S, typename V>
 __device__ __forceinline__ V rows_sum_batch(const Bsr<S> &a, V *terms, int g, int sl, uint32_t start, uint32_t len,
                                             const V *__restrict__ x) {
@@ -776,9 +778,9 @@ template <int RB, int CB, int M, int RPW, typename S, typename V>
 __global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, int epi, const V *__restrict__ x, V *__restrict__ y,
                                                         const V *__restrict__ b, Start<S, V> then) {
     constexpr int LW = WAVE / RPW;
+    // the chains' terms, and after the sums (rows_sum_batch ends at a barrier) the block rows' values
     extern __shared__ __align__(16) unsigned char rows_terms[];
-    V *terms = reinterpret_cast<V *>(rows_terms);
-    __shared__ V values[WAVE];
+    V *terms = reinterpret_cast<V *>(rows_terms), *values = terms;
     const uint32_t lane = threadIdx.x, first = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW;
     const uint32_t row = first + lane / LW;
     const uint32_t start = row < a.rows ? a.starts[row] : 0u, len = row < a.rows ? a.starts[row + 1] - start : 0u;
@@ -901,9 +903,9 @@ __global__ __launch_bounds__(64) void cheb_rows_batch_kernel(Bsr<S> a, const S *
                                                              V *__restrict__ r_out, V *__restrict__ x, V *__restrict__ sum_into,
                                                              double *__restrict__ widen_into) {
     constexpr int LW = WAVE / RPW;
+    // the chains' terms, and after the sums the block rows' residuals
     extern __shared__ __align__(16) unsigned char rows_terms[];
-    V *terms = reinterpret_cast<V *>(rows_terms);
-    __shared__ V r_new[WAVE];
+    V *terms = reinterpret_cast<V *>(rows_terms), *r_new = terms;
     const uint32_t lane = threadIdx.x, first = (a.reverse ? xcd_reversed_block() : blockIdx.x) * RPW;
     const uint32_t row = first + lane / LW;
     const uint32_t start = row < a.rows ? a.starts[row] : 0u, len = row < a.rows ? a.starts[row + 1] - start : 0u;

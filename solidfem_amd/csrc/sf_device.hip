@@ -1019,8 +1019,7 @@ class Hierarchy final : public DeviceMultigrid {
     static void cheb_rows_batch_launch(LevelDev<S, V> &d, const V *d_in, const V *r_in, V keep, V stp, V *d_out, V *r_out, V *x, V *into,
                                        hipStream_t s, double *widen) {
         hipLaunchKernelGGL((cheb_rows_batch_kernel<RB, M, RPW, S, V>), dim3((d.a_rows.rows + RPW - 1) / RPW), dim3(WAVE),
-                           ((size_t)RPW * RB * M * ROWS_BATCH_STRIDE<RB, RB, V, RPW> * sizeof(V)), s, d.a_rows.view(), d.dinv.ptr, d_in, r_in,
-                           keep, stp, d_out, r_out, x, into, widen);
+                           (ROWS_BATCH_LDS<RB, M, RPW, V>), s, d.a_rows.view(), d.dinv.ptr, d_in, r_in, keep, stp, d_out, r_out, x, into, widen);
     }
     // Whether the forms by plain block rows are candidates for a level's steps and residuals.
     static bool rows_batch_level(const LevelDev<S, V> &d, uint32_t M) { return d.a_rows.rows && rows_batch_fits<V>(d.rb, M); }

@@ -274,7 +274,8 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
 inline std::vector<int> rows_batch_forms(int rb = 3) {
     return rb == 3 ? std::vector<int>{ROWS_BATCH_FORM + 2, ROWS_BATCH_FORM + 4} : std::vector<int>{ROWS_BATCH_FORM + 2};
 }
-// Whether a form by rows takes blocks of rb rows and M columns: six rows' chains fit 64 KB of LDS.
+// Whether a form by rows takes blocks of rb rows and M columns: six rows' chains, which are all the LDS a
+// workgroup takes (ROWS_BATCH_LDS), fit 64 KB.
 template <typename V>
 bool rows_batch_fits(int rb, uint32_t M) {
     return M <= FEW_COLUMNS && (rb == 3 || (rb == 6 && (size_t)6 * M * (32 * 6 * sizeof(V) + 16) <= 65536));

@@ -57,3 +57,24 @@ __global__ void f64_three(double *out, const double *in) {
     for op, total, term, other in adds:
         assert total != term, (op, total, term, other)
         assert op == "v_add_f32_dpp" or total != other, (op, total, term, other)
+
+
+def test_batched_rows_of_six_stay_within_64_kb_of_lds(tmp_path):
+    # what a launch asks for (the chains' terms: rows_batch_fits) and what the kernels declare besides
+    def asked(columns, size):
+        return 6 * columns * (32 * 6 * size + 16)
+
+    cases = [(v, size, m) for v, size in (("float", 4), ("double", 8)) for m in range(1, 9) if asked(m, size) <= 65536]
+    assert ("double", 8, 7) in cases and asked(7, 8) > 65536 - 512
+    text = assembly(tmp_path, "#include \"sf_batch_kernels.hpp\"\nnamespace sf::dev {\n" + "\n".join(
+        f"template __global__ void rows_batch_kernel<6, 6, {m}, 1, {v}, {v}>(Bsr<{v}>, int, const {v} *, {v} *, const {v} *, Start<{v}, {v}>);\n"
+        f"template __global__ void cheb_rows_batch_kernel<6, {m}, 1, {v}, {v}>(Bsr<{v}>, const {v} *, const {v} *, const {v} *, {v}, {v}, {v} *, {v} *,"
+        f" {v} *, {v} *, double *);" for v, _, m in cases) + "\n}\n")
+    declared = re.findall(r"\.group_segment_fixed_size: (\d+).*?\.name: +(\S+)", text, re.S)
+    found = 0
+    for static, name in declared:
+        kernel = re.search(r"(?:cheb_rows_batch_kernelILi6E|rows_batch_kernelILi6ELi6E)Li(\d)ELi1E([fd])", name)
+        if kernel:
+            found += 1
+            assert int(static) + asked(int(kernel[1]), 8 if kernel[2] == "d" else 4) <= 65536, (name, static)
+    assert found == 2 * len(cases)
