@@ -812,10 +812,15 @@ sf_status sf_multigrid_apply(sf_multigrid *mg, const double *r, double *z) {
             mg->in.resize(std::max<size_t>(n, 1));
             mg->out.resize(std::max<size_t>(n, 1));
         }
-        // one wait for all of it: the caller's array outlives the call, so the copy in needs none of its own
-        if (n) SF_HIP(hipMemcpyAsync(mg->in.ptr, r, n * sizeof(double), hipMemcpyHostToDevice, s));
-        mg->mg->apply(mg->in.ptr, mg->out.ptr, s);
-        mg->out.download(z, n, s);
+        // one wait for all of it: the copy in needs none of its own while the call lasts, nor where it fails
+        try {
+            if (n) SF_HIP(hipMemcpyAsync(mg->in.ptr, r, n * sizeof(double), hipMemcpyHostToDevice, s));
+            mg->mg->apply(mg->in.ptr, mg->out.ptr, s);
+            mg->out.download(z, n, s);
+        } catch (...) {
+            (void)hipStreamSynchronize(s);  // the caller's arrays are its own again on return
+            throw;
+        }
         SF_HIP(hipStreamSynchronize(s));
     });
 }
