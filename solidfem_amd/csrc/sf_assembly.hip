@@ -818,11 +818,15 @@ void upload_mesh(const QuadMesh &mesh, DeviceBuffer<double> &xyz, DeviceBuffer<u
     staged_upload(ctx, tets, reinterpret_cast<const uint32_t *>(mesh.tets.data()), 10 * mesh.tets.size(), s);
 }
 
-// The lists of incidence_of on the device, from the elements there: count, running sums, fill, and each
-// node's slots sorted (the fill's order is that of its atomics; sorted, it is element order). A vertex's
-// elements are its slots' (a vertex is only ever a corner), and a midside's first slot names its first
-// element. On the 120,000-element plate the host lists took 2 ms and their upload 1.5 ms.
-constexpr uint32_t INCIDENT_MOST = 256;  // slots of a node up to which the sort, one thread a node, is taken
+// The lists of incidence_of on the device, from the elements there: count, running sums, fill, and every
+// slot put where its rank among its node's says (the fill's order is that of its atomics; ranked, it is
+// element order). A vertex's elements are its slots' (a vertex is only ever a corner), and a midside's
+// first slot names its first element. On the 120,000-element plate the host lists took 2 ms and their
+// upload 1.5 ms.
+// Ranking reads a node's slots once per slot, all slots at once: a recovery about one vertex of 256 takes
+// 0.40 ms (0.44 with the host's lists; 2.3 with a thread a node sorting by insertion). A node's reads grow
+// with the square of its slots: 512 take what the host's lists do (0.49 ms), 1024 more (0.78 against 0.75).
+constexpr uint32_t INCIDENT_MOST = 256;  // slots of a node up to which the ranks are taken
 
 // starts[n + 1] counts node n's slots; flag is raised where a corner is no vertex or a midside is one
 __global__ void incidence_count_kernel(size_t slots, size_t vertices, const uint32_t *__restrict__ tets, uint32_t *__restrict__ starts,
@@ -875,34 +879,28 @@ __global__ void incidence_fill_kernel(size_t slots, const uint32_t *__restrict__
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < slots) at[atomicAdd(&cursor[tets[i]], 1u)] = (uint32_t)i;
 }
-__global__ void incidence_sort_kernel(size_t nodes, size_t vertices, const uint32_t *__restrict__ starts, const uint32_t *__restrict__ tets,
-                                      uint32_t *__restrict__ at, uint32_t *__restrict__ vert_at, uint32_t *__restrict__ ends) {
-    const size_t n = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= nodes) return;
-    const uint32_t k0 = starts[n], k1 = starts[n + 1];
-    for (uint32_t k = k0 + 1; k < k1; ++k) {
-        const uint32_t v = at[k];
-        uint32_t to = k;
-        for (; to > k0 && at[to - 1] > v; --to) at[to] = at[to - 1];
-        at[to] = v;
-    }
-    if (n < vertices) {
-        for (uint32_t k = k0; k < k1; ++k) vert_at[k] = at[k] / 10;
+__global__ void incidence_rank_kernel(size_t slots, size_t vertices, const uint32_t *__restrict__ starts, const uint32_t *__restrict__ tets,
+                                      const uint32_t *__restrict__ filled, uint32_t *__restrict__ at, uint32_t *__restrict__ vert_at,
+                                      uint32_t *__restrict__ ends) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= slots) return;
+    const uint32_t node = tets[i], k0 = starts[node], k1 = starts[node + 1];
+    uint32_t rank = 0;
+    for (uint32_t k = k0; k < k1; ++k) rank += filled[k] < (uint32_t)i ? 1u : 0u;
+    at[k0 + rank] = (uint32_t)i;
+    const uint32_t e = (uint32_t)(i / 10), slot = (uint32_t)(i % 10);
+    if (node < vertices) {
+        vert_at[k0 + rank] = e;
         return;
     }
+    if (rank) return;
     const uint32_t EA[6] = {0, 1, 2, 0, 1, 2}, EB[6] = {1, 2, 0, 3, 3, 3};
-    uint32_t a = 0, b = 0;
-    if (k1 > k0) {
-        const uint32_t e = at[k0] / 10, slot = at[k0] % 10 - 4;
 #pragma unroll
-        for (uint32_t k = 0; k < 6; ++k)
-            if (slot == k) {
-                a = tets[(size_t)e * 10 + EA[k]];
-                b = tets[(size_t)e * 10 + EB[k]];
-            }
-    }
-    ends[2 * (n - vertices)] = a;
-    ends[2 * (n - vertices) + 1] = b;
+    for (uint32_t k = 0; k < 6; ++k)
+        if (slot == 4 + k) {
+            ends[2 * (node - vertices)] = tets[(size_t)e * 10 + EA[k]];
+            ends[2 * (node - vertices) + 1] = tets[(size_t)e * 10 + EB[k]];
+        }
 }
 
 }  // namespace
@@ -924,11 +922,11 @@ DeviceRecovery::DeviceRecovery(const Model &model, const double *u, bool converg
     nearest_.upload(nearest_points(nq_), s);
     if (field_.kind == SF_MATERIAL_POINTS) field_table_.upload(field_.points(nq_), s);
     clock.lap("recovery: uploads");
+    nodevals_.resize(elements_ * 10 * 7);
     build_incidence(model.mesh);
     clock.lap("recovery: incidence lists");
     points_.resize(elements_ * nq_ * 10);
     material_.resize(elements_ * nq_ * 2);
-    nodevals_.resize(elements_ * 10 * 7);
     worst_.resize(nodes_ * 6);
     fit_.resize(std::max<size_t>(vertices_, 1) * 29);
     nodal_.resize(nodes_ * 7);
@@ -955,9 +953,11 @@ void DeviceRecovery::build_incidence(const QuadMesh &mesh) {
             nat_.resize(slots);
             vat_.resize(std::max<size_t>(elements_ * 4, 1));
             SF_HIP(hipMemcpyAsync(cursor.ptr, nstart_.ptr, nstart_.bytes(), hipMemcpyDeviceToDevice, s_));
-            hipLaunchKernelGGL(incidence_fill_kernel, grid_of(slots), dim3(256), 0, s_, slots, (const uint32_t *)tets_.ptr, cursor.ptr, nat_.ptr);
-            hipLaunchKernelGGL(incidence_sort_kernel, grid_of(nodes_), dim3(256), 0, s_, nodes_, vertices_, (const uint32_t *)nstart_.ptr,
-                               (const uint32_t *)tets_.ptr, nat_.ptr, vat_.ptr, ends_.ptr);
+            // the lists as filled take room that the elements' values have not begun to use (70 doubles each)
+            uint32_t *filled = reinterpret_cast<uint32_t *>(nodevals_.ptr);
+            hipLaunchKernelGGL(incidence_fill_kernel, grid_of(slots), dim3(256), 0, s_, slots, (const uint32_t *)tets_.ptr, cursor.ptr, filled);
+            hipLaunchKernelGGL(incidence_rank_kernel, grid_of(slots), dim3(256), 0, s_, slots, vertices_, (const uint32_t *)nstart_.ptr,
+                               (const uint32_t *)tets_.ptr, (const uint32_t *)filled, nat_.ptr, vat_.ptr, ends_.ptr);
             SF_HIP(hipGetLastError());
             SF_HIP(hipStreamSynchronize(s_));  // the cursors are freed on return
             return;
