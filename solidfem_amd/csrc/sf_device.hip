@@ -1060,9 +1060,11 @@ class Hierarchy final : public DeviceMultigrid {
         for (size_t l = 0; l < lv_.size(); ++l) {
             LevelDev<S, V> &d = lv_[l];
             if (d.mm_form[M][0]) continue;
+            const bool timed = d.mm_times[lg][0].columns != 0;  // for another count of the group
             const size_t need = d.n * (size_t)M;
             V *vs[8] = {d.mb.ptr, d.mx.ptr, d.md0.ptr, d.md1.ptr, d.mr0.ptr, d.mr1.ptr, d.mres.ptr, d.mpx.ptr};
-            for (V *v : vs) SF_HIP(hipMemsetAsync(v, 0, need * sizeof(V), s));
+            for (V *v : vs)
+                if (!timed) SF_HIP(hipMemsetAsync(v, 0, need * sizeof(V), s));
             auto tune = [&](int which, auto fits, const std::function<void(int)> &launch, const std::vector<int> &candidates, const std::string &memo) {
                 GroupTimes &times = d.mm_times[lg][which];
                 if (!times.columns) times = tune_group(s, M, launch, candidates, memo);
@@ -1077,8 +1079,8 @@ class Hierarchy final : public DeviceMultigrid {
             if (d.has_p) {
                 LevelDev<S, V> &c = lv_[l + 1];
                 const size_t cneed = c.n * (size_t)M;
-                SF_HIP(hipMemsetAsync(c.mb.ptr, 0, cneed * sizeof(V), s));
-                SF_HIP(hipMemsetAsync(c.mx.ptr, 0, cneed * sizeof(V), s));
+                for (V *v : {c.mb.ptr, c.mx.ptr})
+                    if (!timed) SF_HIP(hipMemsetAsync(v, 0, cneed * sizeof(V), s));
                 std::vector<int> restrict_forms = spmm_candidates(d.r.rb, d.r.cb, sizeof(S), M, true, staged_candidate(d.r, M));
                 const bool wide = wide_rows_batch_fits<S, V>(d.r_rows, M);
                 if (wide) restrict_forms.push_back(WIDE_ROWS);
