@@ -1259,6 +1259,19 @@ static __global__ void jacobi_kernel(size_t n, const double *__restrict__ inv, c
     if (i < n) z[i] = r[i] * inv[i];
 }
 
+// A sliced matrix's block columns row after row (Bsr's order), from the slots they lie in: one thread a row.
+template <int NPW>
+__global__ void plain_columns_kernel(size_t positions, const uint32_t *__restrict__ slice_start, const uint32_t *__restrict__ row_len,
+                                     const uint32_t *__restrict__ perm, const uint32_t *__restrict__ cols, const uint32_t *__restrict__ starts,
+                                     uint32_t *__restrict__ out) {
+    const size_t pos = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (pos >= positions) return;
+    const uint32_t row = perm[pos];
+    if (row == NONE) return;
+    const uint32_t slice = (uint32_t)(pos / NPW), j = (uint32_t)(pos % NPW), to = starts[row], len = row_len[pos];
+    for (uint32_t k = 0; k < len; ++k) out[to + k] = cols[((size_t)slice_start[slice] + k) * NPW + j];
+}
+
 // Sliced values from a row-major block array: slot i of the sliced layout takes value
 // src[map[i]] rounded to T (the precision conversion of block.rs:26-35).
 template <typename T>
