@@ -185,10 +185,14 @@ static void rows_batch_launch(const DeviceBsr<S> &a, const V *x, V *y, const V *
 template <typename S, typename V>
 void launch_rows_batch(const DeviceBsr<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int form, Start<S, V> st) {
     if (a.rows == 0 || M == 0) return;
-    if (a.cb != a.rb || !rows_batch_fits<V>(a.rb, M)) throw Error(SF_ERR_INTERNAL, "no rows form for this block shape or column count");
+    if (a.cb != a.rb || !rows_batch_fits<V>(a.rb, M) || epi == EPI_ADD)
+        throw Error(SF_ERR_INTERNAL, "no rows form for this block shape, column count or epilogue");
     with_columns(M, [&](auto columns) {
         constexpr int MM = decltype(columns)::value;
-        if (a.rb == 6) return rows_batch_launch<6, MM, 1>(a, x, y, b, epi, s, st);
+        static_assert(rows_batch_fits<V>(6, MM) == (ROWS_BATCH_LDS<6, MM, 1, V> <= 65536), "the rule counts what a launch takes");
+        if constexpr (rows_batch_fits<V>(6, MM)) {
+            if (a.rb == 6) return rows_batch_launch<6, MM, 1>(a, x, y, b, epi, s, st);
+        }
         if constexpr (12 * MM <= WAVE) {
             if (rows_batch_rows(form, M) == 4) return rows_batch_launch<3, MM, 4>(a, x, y, b, epi, s, st);
         }

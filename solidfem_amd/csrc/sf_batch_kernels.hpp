@@ -789,11 +789,11 @@ __global__ __launch_bounds__(64) void rows_batch_kernel(Bsr<S> a, int epi, const
     const uint32_t within = lane % per, p = within / M, m = within - p * M, own = first + lane / per;
     const bool owner = lane < RPW * per && own < a.rows;
     const size_t out = owner ? ((size_t)own * RB + p) * M + m : 0;
-    const V before = !owner || epi == EPI_STORE ? (V)0 : epi == EPI_RESIDUAL ? b[out] : y[out];
+    const V before = !owner || epi == EPI_STORE ? (V)0 : b[out];
     const V sum = rows_sum_batch<RB, CB, M, RPW, S, V>(a, terms, (int)(lane / LW), (int)(lane % LW), start, len, x);
     V value = (V)0;
     if (owner) {
-        value = epi == EPI_STORE ? sum : epi == EPI_RESIDUAL ? before - sum : before + sum;
+        value = epi == EPI_STORE ? sum : before - sum;
         y[out] = value;
     }
     if (!then.dinv) return;  // uniform

@@ -404,23 +404,16 @@ template <int RB, int CB, int RPW, int U, typename S, typename V>
 static void long_rows_epi(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
     const dim3 grid((a.rows + RPW - 1) / RPW), block(WAVE);
     if (epi == EPI_STORE) hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_STORE, RPW, U>), grid, block, 0, s, a.view(), x, y, b, st);
-    else if (epi == EPI_RESIDUAL)
-        hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_RESIDUAL, RPW, U>), grid, block, 0, s, a.view(), x, y, b, st);
-    else hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_ADD, RPW, U>), grid, block, 0, s, a.view(), x, y, b, st);
-}
-
-template <int RB, int CB, typename S, typename V>
-static void wide_rows_epi(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st) {
-    const dim3 grid(a.rows), block(WideRows<RB, CB, V>::THREADS);
-    if (epi == EPI_STORE) hipLaunchKernelGGL((wide_rows_kernel<RB, CB, S, V, EPI_STORE>), grid, block, 0, s, a.view(), x, y, b, st);
-    else if (epi == EPI_RESIDUAL) hipLaunchKernelGGL((wide_rows_kernel<RB, CB, S, V, EPI_RESIDUAL>), grid, block, 0, s, a.view(), x, y, b, st);
-    else hipLaunchKernelGGL((wide_rows_kernel<RB, CB, S, V, EPI_ADD>), grid, block, 0, s, a.view(), x, y, b, st);
+    else hipLaunchKernelGGL((long_rows_kernel<RB, CB, S, V, EPI_RESIDUAL, RPW, U>), grid, block, 0, s, a.view(), x, y, b, st);
 }
 
 template <int RB, int CB, typename S, typename V>
 static void long_rows_shape(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st, int rpw) {
-    if constexpr (RB == 6) {  // the restrictions and the coarse levels
-        if (rpw == WIDE_ROWS) return wide_rows_epi<RB, CB>(a, x, y, b, epi, s, st);
+    if constexpr (RB == 6) {
+        if (rpw == WIDE_ROWS) {  // restrictions, which store
+            hipLaunchKernelGGL((wide_rows_kernel<RB, CB, S, V>), dim3(a.rows), dim3(WideRows<RB, CB, V>::THREADS), 0, s, a.view(), x, y, st);
+            return;
+        }
     }
     with_rows_form<RB * CB * (int)sizeof(V)>(rpw, [&](auto rows, auto blocks) {
         long_rows_epi<RB, CB, decltype(rows)::value, decltype(blocks)::value>(a, x, y, b, epi, s, st);
@@ -430,6 +423,7 @@ static void long_rows_shape(const DeviceBsr<S> &a, const V *x, V *y, const V *b,
 template <typename S, typename V>
 void launch_long_rows(const DeviceBsr<S> &a, const V *x, V *y, const V *b, int epi, hipStream_t s, Start<S, V> st, int rpw) {
     if (a.rows == 0) return;
+    if (epi == EPI_ADD || (rpw == WIDE_ROWS && epi != EPI_STORE)) throw Error(SF_ERR_INTERNAL, "no rows form with this epilogue");
     if (a.rb == 6 && a.cb == 3) long_rows_shape<6, 3>(a, x, y, b, epi, s, st, rpw);
     else if (a.rb == 6 && a.cb == 6) long_rows_shape<6, 6>(a, x, y, b, epi, s, st, rpw);
     else if (a.rb == 3 && a.cb == 3) long_rows_shape<3, 3>(a, x, y, b, epi, s, st, rpw);
@@ -631,7 +625,7 @@ struct LevelDev {
     size_t rows = 0, n = 0;
     DeviceSliced<S> a, p, r;
     DeviceBsr<S> r_rows;          // the same transpose in plain block rows, for long_rows_kernel
-    int restrict_rows = 0;  // 0: the sliced restriction; else long_rows_kernel with this many rows per wave (by timing)
+    int restrict_rows = 0;  // 0: the sliced restriction; else a form of the row kernels, or WIDE_ROWS (by timing)
     DeviceBsr<S> a_rows;          // coarse levels and small systems: A in plain block rows, for the row kernels
     int cheb_rows = 0, residual_rows = 0;  // the same choice for the steps and residuals (by timing)
     DeviceBuffer<S> dinv;
@@ -1012,7 +1006,10 @@ class Hierarchy final : public DeviceMultigrid {
         } else if (batch > ROWS_BATCH_FORM) {
             with_columns(M, [&](auto columns) {
                 constexpr int MM = decltype(columns)::value;
-                if (d.rb == 6) return cheb_rows_batch_launch<6, MM, 1>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+                if constexpr (rows_batch_fits<V>(6, MM)) {
+                    if (d.rb == 6) return cheb_rows_batch_launch<6, MM, 1>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);
+                }
+                if (d.rb == 6) throw Error(SF_ERR_INTERNAL, "no rows form for this column count");
                 if constexpr (12 * MM <= WAVE) {
                     if (rows_batch_rows(batch, M) == 4)
                         return cheb_rows_batch_launch<3, MM, 4>(d, d_in, r_in, keep, stp, d_out, r_out, x, into, s, widen);

@@ -264,8 +264,8 @@ inline int columns_log2(uint32_t m) {
     while ((1u << g) < m) ++g;
     return g;
 }
-// Y = A X for M row-interleaved columns (epilogue per dev::Epilogue), `batch` blocks in flight
-// (1, 2 or 4; 0 = the matrix's tuned depth for this column count).
+// Y = A X for M row-interleaved columns (epilogue per dev::Epilogue) in the form `batch` (a code as above;
+// 0 = the matrix's tuned form for this column count).
 template <typename S, typename V>
 void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V *b, int epi, hipStream_t s, int batch = 0,
                  dev::Start<S, V> start = {nullptr, (V)0, nullptr, nullptr});
@@ -277,7 +277,7 @@ inline std::vector<int> rows_batch_forms(int rb = 3) {
 // Whether a form by rows takes blocks of rb rows and M columns: six rows' chains, which are all the LDS a
 // workgroup takes (ROWS_BATCH_LDS), fit 64 KB.
 template <typename V>
-bool rows_batch_fits(int rb, uint32_t M) {
+constexpr bool rows_batch_fits(int rb, uint32_t M) {
     return M <= FEW_COLUMNS && (rb == 3 || (rb == 6 && (size_t)6 * M * (32 * 6 * sizeof(V) + 16) <= 65536));
 }
 template <typename S, typename V>

@@ -437,7 +437,7 @@ __device__ __forceinline__ V rows_sum(const Bsr<S> &a, RowTerms<RB, CB, V, RPW, 
     return sum;
 }
 
-// y = A x with an epilogue (as spmv_kernel) by rows_sum, for matrices with few or long rows: the
+// y = A x or y = b - A x (as spmv_kernel) by rows_sum, for matrices with few or long rows: the
 // stored transposes of the prolongators, whose rows gather every fine row of an aggregate's
 // neighbourhood, the coarse levels, and systems too small to fill the chip with a lane per row.
 template <int RB, int CB, typename S, typename V, int EPI, int RPW, int U>
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(64) void long_rows_kernel(Bsr<S> a, const V *__rest
     const bool owner = live && sl < RB;
     const size_t out = (size_t)row * RB + (owner ? sl : 0);
     // what the epilogue reads is fetched before the sums
-    const V before = !owner || EPI == EPI_STORE ? (V)0 : EPI == EPI_RESIDUAL ? b[out] : y[out];
+    const V before = !owner || EPI == EPI_STORE ? (V)0 : b[out];
     S drow[RB];
     if (then.dinv && owner) {
 #pragma unroll
@@ -461,7 +461,7 @@ __global__ __launch_bounds__(64) void long_rows_kernel(Bsr<S> a, const V *__rest
     }
     const V sum = rows_sum<RB, CB, RPW, U, S, V>(a, terms, g, sl, start, len, x);
     if (owner) {
-        const V value = EPI == EPI_STORE ? sum : EPI == EPI_RESIDUAL ? before - sum : before + sum;
+        const V value = EPI == EPI_STORE ? sum : before - sum;
         y[out] = value;
         values[g][sl] = value;
     }
@@ -495,9 +495,8 @@ struct WideRows {
     static constexpr int STRIDE = CHUNK * CB + 16 / sizeof(V);  // rows on different banks, 16-byte aligned
     static_assert(RB % PARTS == 0 && CHUNK * PARTS <= THREADS, "whole rows per thread");
 };
-template <int RB, int CB, typename S, typename V, int EPI>
-__global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__restrict__ x, V *__restrict__ y, const V *__restrict__ b,
-                                                        Start<S, V> then) {
+template <int RB, int CB, typename S, typename V>
+__global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__restrict__ x, V *__restrict__ y, Start<S, V> then) {
     using W = WideRows<RB, CB, V>;
     constexpr int RP = RB / W::PARTS;
     __shared__ __align__(16) V terms[2][RB][W::STRIDE];
@@ -511,8 +510,7 @@ __global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__res
     const uint32_t p = t / 16 < (uint32_t)RB ? t / 16 : RB - 1;
     const bool owner = t / 16 < (uint32_t)RB && t % 16 == 0;
     const size_t out = (size_t)row * RB + p;
-    // what the epilogue reads is fetched before the sums
-    const V before = !owner || EPI == EPI_STORE ? (V)0 : EPI == EPI_RESIDUAL ? b[out] : y[out];
+    // what the start reads is fetched before the sums
     S drow[RB];
     if (then.dinv && owner) {
 #pragma unroll
@@ -552,9 +550,8 @@ __global__ __launch_bounds__(256) void wide_rows_kernel(Bsr<S> a, const V *__res
         if (adds) sum = add_row_terms(sum, (const V *)terms[buf][p], (len - k0 < (uint32_t)W::CHUNK ? len - k0 : (uint32_t)W::CHUNK) * CB);
     }
     if (owner) {
-        const V value = EPI == EPI_STORE ? sum : EPI == EPI_RESIDUAL ? before - sum : before + sum;
-        y[out] = value;
-        values[p] = value;
+        y[out] = sum;
+        values[p] = sum;
     }
     if (then.dinv) {  // uniform
         __syncthreads();
