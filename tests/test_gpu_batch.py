@@ -54,6 +54,23 @@ def test_batched_v_cycle_is_bit_identical_per_column(ctx, precision, coarse_solv
     assert np.array_equal(bits(mg.apply_batch(r)), bits(z)), "a second application differs"
 
 
+@pytest.mark.parametrize("precision", [0, 1, 2], ids=["double", "single-storage", "single"])
+@pytest.mark.parametrize("columns", [1, 6, 33])
+def test_a_batched_v_cycle_of_one_smoothing_step_is_bit_identical_per_column(ctx, precision, columns):
+    # a smoother of degree one has no later step to add its result, nor to widen it to f64
+    ref = refcpu.Problem(loaded(*FINGERPRINT_PLATE[:2]))
+    csr = sf.CsrMatrix.new(ctx, *ref.csr())
+    setup = sf.MultigridSetup.new(ctx, csr, ref.rigid_modes(), ref.free_positions(),
+                                  sf.MultigridOptions(coarse_dofs=100, precision=precision, smoother_degree=1))
+    while not setup.step(2 ** 62):
+        pass
+    mg = setup.finish()
+    r = np.random.default_rng(columns).standard_normal((columns, ref.free_dofs))
+    z = mg.apply_batch(r)
+    for m in range(columns):
+        assert np.array_equal(bits(z[m]), bits(mg.apply(r[m]))), f"column {m}"
+
+
 def test_batched_solve_reproduces_the_oracle_per_load_case(ctx):
     # five random-traction load cases of the clamped block, one hierarchy, the reference's order
     cases = [block_config(c, divisions=(6, 4, 4)) for c in range(5)]

@@ -32,8 +32,9 @@ def serial(first, terms):
 
 
 # 54 and 108 unknowns: one panel; 162, the first past it: two; 600: panels of 9 columns; 1260: of 4, and two chunks of 1024;
+# 3000, the most that a level is factored for: panels of one column, three chunks, 158 KB of LDS;
 # 64 columns of the inverse's product are past the form of eight sums a workgroup from 600 on, 3 columns within it
-@pytest.mark.parametrize("divisions", [(1, 1, 1), (2, 1, 1), (3, 1, 1), (4, 2, 2), (6, 3, 2)])
+@pytest.mark.parametrize("divisions", [(1, 1, 1), (2, 1, 1), (3, 1, 1), (4, 2, 2), (6, 3, 2), (4, 2, 12)])
 def test_coarse_solves_follow_their_serial_orders(ctx, divisions):
     ref = refcpu.Problem(loaded([float(d) for d in divisions], list(divisions)))
     mg_ref = refcpu.Multigrid(ref, refcpu.options(precision=0, coarse_dofs=100000))

@@ -120,11 +120,13 @@ def test_a_coarse_factor_of_hundreds_of_unknowns_is_factored_on_the_device_to_th
 
 
 def test_automatic_placement_on_a_larger_plate(ctx):
-    # about 36,000 block rows: level 0 runs on the device, the coarse levels on the host
+    # levels of 32,400, 11,320, 365, 25 and 3 block rows: the first three run on the device, which takes
+    # those of at least 256, the fourth (with a coarser one behind it) on the host
     ref = refcpu.Problem(plate_config(divisions=(40, 40, 2)))
-    auto = run_setup(ctx, ref, sf.MultigridOptions(precision=sf.Precision.SINGLE))
-    host = run_setup(ctx, ref, sf.MultigridOptions(precision=sf.Precision.SINGLE, setup_device=sf.SetupDevice.HOST))
-    assert auto.level_matrix(0)["starts"].size - 1 >= 4096
+    auto = run_setup(ctx, ref, sf.MultigridOptions(precision=sf.Precision.SINGLE, coarse_dofs=100))
+    host = run_setup(ctx, ref, sf.MultigridOptions(precision=sf.Precision.SINGLE, coarse_dofs=100, setup_device=sf.SetupDevice.HOST))
+    rows = [auto.level_matrix(l)["starts"].size - 1 for l in range(auto.level_count())]
+    assert sum(n >= 256 for n in rows[:-1]) >= 2 and any(n < 256 for n in rows[:-1]), rows
     assert_same_setup(auto, host)
 
 
