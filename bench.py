@@ -503,7 +503,7 @@ def main():
     recovery_ms = (time.perf_counter() - t) * 1e3
     line["stress_recovery"] = {"ms": round(recovery_ms, 2), "elements": int(points.shape[0]),
                                "nodes": int(nodal.shape[0]), "peak_nodal_von_mises": float(nodal[:, 6].max()),
-                               "note": "host incidence lists, uploads and downloads included"}
+                               "note": "incidence lists, uploads and downloads included"}
     log(f"stress recovery of the plate: {recovery_ms:.1f} ms, peak nodal von Mises {nodal[:, 6].max():.4g} MPa")
     # the error estimate of that recovery (error_estimate.rs): 14-point integrals per element on the
     # device, the sums in element order on the host

@@ -1065,7 +1065,9 @@ __global__ __launch_bounds__(256) void coarse_inverse_batch_kernel(uint32_t n, u
 // of 16 lanes adds each sum's terms in ascending k (add_row_terms). n = 377 rows and 5 columns took
 // 20 us with the tiles above, 12 workgroups in a chain of round trips.
 constexpr uint32_t COARSE_SUMS = 8, COARSE_SUMS_CHUNK = 512;
-constexpr size_t COARSE_SUMS_MOST = 16384;  // sums up to which this form is taken: two waves of the chip's workgroups
+// Sums up to which this form is taken, two waves of the chip's workgroups. n = 774, an iteration of a
+// 220k-DOF plate: 16 columns 882 us (908 with the tiles), 32 1344 (1329), 64 2418 (2363).
+constexpr size_t COARSE_SUMS_MOST = 16384;
 template <typename V>
 __global__ __launch_bounds__(256) void coarse_inverse_sums_kernel(uint32_t n, uint32_t M, const double *__restrict__ inv,
                                                                   const V *__restrict__ rhs, V *__restrict__ out) {
@@ -1194,7 +1196,8 @@ static __global__ void mirror_columns_kernel(uint32_t M, const PcgScalars *s, Pc
 
 // For few columns, the final sums formed by every block of the kernel that uses them, as tree_total
 // does for one: a launch less each. FUSED_COLUMNS: each block reads every column's 512 partials, which
-// costs more than the launch it saves from about nine columns on.
+// at eight columns costs what it saves on a 300k-DOF block (733 us an iteration against 736 with sums of
+// their own; one column 345 against 353) and less on smaller systems (plate of 55k DOFs 289 against 300).
 constexpr uint32_t FUSED_COLUMNS = 8;
 // M is a compile-time count, so that every column's partials are in flight at once.
 template <uint32_t M>

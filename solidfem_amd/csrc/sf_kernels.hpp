@@ -841,9 +841,11 @@ __global__ void convert_kernel(size_t n, const From *__restrict__ in, To *__rest
 // next panel of `width` columns into the other LDS buffer meanwhile, so no step waits on global
 // memory. A factor that fits one buffer is one panel, read once for both substitutions. Forward, a
 // block of 64 rows stays in registers, one per lane, for its own columns, then the later rows take
-// those columns' terms. Bound by the n^2 / 2 dependent subtractions of the back substitution and 2 n
-// dependent divisions (100 cycles each): n = 90 took 104 us with every step through LDS and a lane
-// folding the products.
+// those columns' terms. Not bound by its chain: n = 90 takes 67 us, of which its n^2 / 2 dependent
+// subtractions (2.5 ns) and 2 n divisions (42 ns) are 17; the rest is what each row of the back
+// substitution does around them (products to LDS and back, the division, x to LDS, a fence each). With every
+// step through LDS and a lane folding the products it took 104. One V-cycle call that is this solve alone
+// (25 us of it copies): n = 108 110 us (156 before), 360 0.60 ms (1.02), 756 2.25 (3.89), 1296 6.3 (12.5).
 constexpr uint32_t COARSE_MAX = 3072;
 constexpr uint32_t COARSE_THREADS = 256;
 constexpr uint32_t COARSE_PANEL = 5600;  // entries of one of the two panel buffers
