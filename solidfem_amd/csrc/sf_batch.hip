@@ -115,7 +115,7 @@ void launch_spmm(const DeviceSliced<S> &a, uint32_t M, const V *x, V *y, const V
     if (batch == 0) {
         batch = a.mm_form[M];
         if (!batch) {
-            batch = a.mm_times[columns_log2(M)].form(M, a.mm_form[M], [](int) { return true; }, [&] {
+            batch = a.mm_times[columns_log2(M)].form(M, a.mm_form[M], [&](int form) { return form != STAGED_FORM || staged_candidate(a, M); }, [&] {
                 // a product into scratch vectors of this shape, timed for each form
                 DeviceBuffer<V> tx(std::max<size_t>(a.block_cols * a.cb * M, 1)), ty(std::max<size_t>(a.rows * a.rb * M, 1));
                 SF_HIP(hipMemsetAsync(tx.ptr, 0, tx.bytes(), s));

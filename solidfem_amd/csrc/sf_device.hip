@@ -1074,7 +1074,9 @@ class Hierarchy final : public DeviceMultigrid {
                 if (!times.columns) times = tune_group(s, M, launch, candidates, memo);
                 d.mm_form[M][which] = times.form(M, fits);
             };
-            auto level_fits = [&](int form) { return form <= ROWS_BATCH_FORM || form >= FEW_FORM || rows_batch_fits<V>(d.rb, M); };
+            auto level_fits = [&](int form) {
+                return form == STAGED_FORM ? staged_candidate(d.a, M) : form <= ROWS_BATCH_FORM || form >= FEW_FORM || rows_batch_fits<V>(d.rb, M);
+            };
             tune(0, level_fits, [&](int form) { launch_cheb_batch(d, form, M, d.md0.ptr, d.mb.ptr, (V)0, (V)0, d.md1.ptr, d.mr0.ptr, d.mx.ptr, nullptr, s); },
                  with_rows_batch(spmm_candidates(d.rb, d.rb, sizeof(S), M, false), d, M), "batch step " + group + shape_class(d.a) + vsize);
             tune(1, level_fits, [&](int form) { residual_batch(d, form, M, d.mx.ptr, d.mb.ptr, s); },
@@ -1088,10 +1090,10 @@ class Hierarchy final : public DeviceMultigrid {
                 std::vector<int> restrict_forms = spmm_candidates(d.r.rb, d.r.cb, sizeof(S), M, true, staged_candidate(d.r, M));
                 const bool wide = wide_rows_batch_fits<S, V>(d.r_rows, M);
                 if (wide) restrict_forms.push_back(WIDE_ROWS);
-                tune(2, [&](int form) { return form != WIDE_ROWS || wide; },
+                tune(2, [&](int form) { return form == WIDE_ROWS ? wide : form != STAGED_FORM || staged_candidate(d.r, M); },
                      [&](int form) { restrict_batch(d, form, M, d.mres.ptr, c.mb.ptr, s, {nullptr, (V)0, nullptr, nullptr}); }, restrict_forms,
                      "batch restriction " + group + shape_class(d.r) + vsize);
-                tune(3, [](int) { return true; }, [&](int form) { launch_spmm<S, V>(d.p, M, c.mx.ptr, d.mpx.ptr, nullptr, EPI_ADD, s, form); },
+                tune(3, [&](int form) { return form != STAGED_FORM || staged_candidate(d.p, M); }, [&](int form) { launch_spmm<S, V>(d.p, M, c.mx.ptr, d.mpx.ptr, nullptr, EPI_ADD, s, form); },
                      spmm_candidates(d.p.rb, d.p.cb, sizeof(S), M, true, staged_candidate(d.p, M)), "batch prolongation " + group + shape_class(d.p) + vsize);
             }
         }

@@ -64,15 +64,21 @@ constexpr int ROWS_BATCH_FORM = 112;  // plus 2 or 4: up to FEW_COLUMNS columns 
 constexpr int FEW_FORM = 128;    // a lane per scalar row with up to FEW_COLUMNS columns, blocks of three rows
 constexpr uint32_t FEW_COLUMNS = 8;
 
+// Columns a lane takes in a form.
+inline int form_columns(int code) {
+    return code >= STAGED_FORM ? 1 : code >= OCT_FORM ? 8 : code >= QUAD_FORM ? 4 : code >= PAIR_FORM ? 2 : 1;
+}
 // Rows per wavefront of a rows form (3 x 3 blocks) for M columns: its chains, 3 M a row, fit the 64 lanes.
 inline int rows_batch_rows(int form, uint32_t M) { return form - ROWS_BATCH_FORM == 4 && 12 * M <= (uint32_t)dev::WAVE ? 4 : 2; }
 // The times of a batched kernel's forms at one column count, which choose the form for each count of its
 // group (1, 2, 3-4, 5-8, ...). The forms of few columns take time with the count (five columns to eight:
 // 1.3 to 1.9 times as long on a 31k-DOF tube), while a lane-group form takes the group's whole power of
 // two lanes whatever the count (within 3%): for more columns than were timed, the former are scaled up. A
-// form that does not take a count (its buffers fit no LDS), or takes it with fewer rows a wavefront, is
-// not that count's. With the first count's choice for the whole group, eight columns after five took 17.5
-// ms a solve of that tube in double, 11.9 with their own.
+// count leaves out a form that does not take it (no LDS for its buffers, no workgroup for its sums), that
+// takes it with fewer rows a wavefront, or whose lanes' columns do not divide it (it would run as the
+// one-column form of its depth, which is timed itself). With the first count's choice for its whole group,
+// eight columns after five took 17.5 ms a solve of that tube in double, 11.9 with their own, and 45 after
+// 64 on a 55k-DOF plate 159, 140 with theirs.
 struct GroupTimes {
     uint32_t columns = 0;  // 0: not timed
     std::vector<std::pair<int, float>> times;
@@ -84,6 +90,7 @@ struct GroupTimes {
             const bool per_column = t.first == WIDE_ROWS || t.first > ROWS_BATCH_FORM;
             const float ms = per_column && M > columns ? t.second * (float)M / (float)columns : t.second;
             if (t.first > ROWS_BATCH_FORM && t.first < FEW_FORM && rows_batch_rows(t.first, M) < rows_batch_rows(t.first, columns)) continue;
+            if (M % (uint32_t)form_columns(t.first)) continue;
             if (ms < least && fits(t.first)) {
                 least = ms;
                 best = t.first;
@@ -251,9 +258,6 @@ void with_columns(uint32_t M, F &&f) {
         case 7: f(integral_constant<int, 7>{}); break;
         default: f(integral_constant<int, 8>{}); break;
     }
-}
-inline int form_columns(int code) {
-    return code >= STAGED_FORM ? 1 : code >= OCT_FORM ? 8 : code >= QUAD_FORM ? 4 : code >= PAIR_FORM ? 2 : 1;
 }
 inline int form_depth(int code) {
     return code >= STAGED_FORM ? 0 : code >= OCT_FORM ? code - OCT_FORM : code >= QUAD_FORM ? code - QUAD_FORM : code >= PAIR_FORM ? code - PAIR_FORM : code >= NODE_FORM ? code - NODE_FORM : code;

@@ -52,6 +52,22 @@ def test_few_columns_by_rows_keep_each_columns_bits(ctx, forced_variant, rows, p
             assert np.array_equal(bits(single.estimate()), bits(x[m])), f"{columns} columns: column {m}"
 
 
+def test_a_staged_group_takes_odd_counts_past_a_workgroup_in_another_form(ctx, forced_variant):
+    # rows of six and 64 columns, two a thread, are 192 threads' sums, 45 columns, one a thread, 270
+    ref = refcpu.Problem(loaded(*FINGERPRINT_PLATE[:2]))
+    csr = sf.CsrMatrix.new(ctx, *ref.csr())
+    setup = sf.MultigridSetup.new(ctx, csr, ref.rigid_modes(), ref.free_positions(), sf.MultigridOptions(coarse_dofs=100, precision=2, coarse_solve=1))
+    while not setup.step(2 ** 62):
+        pass
+    mg = setup.finish()
+    forced_variant(80)
+    for columns in (64, 45, 43, 42):
+        r = np.random.default_rng(columns).standard_normal((columns, ref.free_dofs))
+        z = mg.apply_batch(r)
+        for m in range(columns):
+            assert np.array_equal(bits(z[m]), bits(mg.apply(r[m]))), f"{columns} columns: column {m}"
+
+
 def test_a_large_batchs_columns_arrive_and_return_in_pieces(ctx):
     # 48 columns of 11,970 unknowns are 4.4 MiB: one whole pinned piece of 4 MiB and the rest
     ref = refcpu.Problem(block_config(0, divisions=(9, 7, 7)))
